@@ -296,8 +296,11 @@ int sym_near_shares(const Ctx& c, int64_t n)
     return (int)std::min<int64_t>(16, std::max<int64_t>(1, (target + blocks - 1) / blocks));
 }
 
-// The symmetric sweep, begun: buffers; the rest of the evaluation forked
-// onto the context's second stream (ws) after the gather and the mass
+// particles from which, with lists, the rest of the evaluation runs beside the far field
+constexpr int kForkMin = 20480;
+
+// The symmetric sweep, begun: buffers; with lists and at least kForkMin
+// particles, the rest of the evaluation forked onto the context's second stream (ws) after the gather and the mass
 // check; the far field on s, launched first so that its workgroups are
 // placed first and no event stands between it and the work before it; the
 // near field's lists on ws.  The far field needs only the slot-ordered
@@ -345,12 +348,16 @@ int sym_sweep_begin(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_
     S.accsum = c.sym_accsum;
     hipError_t e;
     ws = s;
-    // With gravity alone, only the in-group gravity (enqueued by
-    // sym_sweep_end) runs on the second stream, in the issue cycles the far
-    // field's wavefronts leave (Plummer N = 16384: 0.103 -> 0.099 ms per step
-    // against both in order on s; launched before the far field it delayed
-    // it, 0.101).
-    if (sym_has_far(S)) {
+    // The rest beside the far field only with lists and many particles: a
+    // wavefront of another kernel on its SIMD takes the far field's from 2
+    // to 4 clocks per instruction (far_rotation.hpp), so what runs beside it
+    // has to be worth more than that.  Gravity alone in order on s: Plummer
+    // N = 16384 86.1 -> 73.4 us per step, 50021 unequal masses 482 -> 460;
+    // the default solids at N = 16384 (lists) 207 -> 190 us.  Beside it:
+    // collision N = 131072 2.72 against 2.86 ms, liquid N = 65536 0.872
+    // against 0.902, collision N = 33000 0.51 against 0.56.
+    if (sym_has_far(S) && L.want_nbr && L.n >= kForkMin) {
+        S.far_done = true;
         if (c.no_alloc && (!c.side || !c.ev_fork || !c.ev_join))
             return fail(c, GRASPH_E_NOMEM, "the second stream would need creating");
         if (!c.side && (e = hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking)) != hipSuccess)
@@ -366,17 +373,11 @@ int sym_sweep_begin(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_
         }
         ws = c.side;
         // Below ~50k particles the far field's window is short next to the
-        // lists' work: there the lists take issue priority, so they and the
-        // passes after them end inside it (collision N = 32768: 0.435 ->
-        // 0.410 ms per step, N = 16384: 0.290 -> 0.283; liquid N = 32768:
-        // 0.420 -> 0.387); from 65536 on the side stream ends inside the
-        // window without it, and its VALU work would lengthen the far field
-        // (collision N = 65536: 0.985 -> 1.008 ms, liquid N = 65536: 0.945
-        // -> 1.005, collision N = 131072: 3.79 -> 3.86).  Once the lists have
-        // grown long (capacity past 512: bodies in contact), the lists and
-        // the passes after them outlast the far field at any size, and the
-        // priority shortens the step (collision N = 131072 after impact:
-        // 5.87 -> 5.57 ms).
+        // lists' work, and once the lists have grown long (capacity past
+        // 512: bodies in contact) the lists and the passes after them outlast
+        // it at any size: there issue priority over the far field shortens
+        // the step (collision N = 32768: 0.435 -> 0.410 ms, N = 131072 after
+        // impact: 5.87 -> 5.57).
         S.list_prio = c.sym_list_priority == 1 ||
                       (c.sym_list_priority == 2 && (L.n < 49152 || c.max_neighbours > 512));
     }
@@ -389,6 +390,10 @@ int sym_sweep_end(Ctx& c, SymLaunch& S, const DevParams& P, hipStream_t s, hipSt
 {
     hipError_t e;
     S.add_acc = add_acc;
+    if (!S.far_done) {
+        ProfScope ps(&c, s, KC_FAR);
+        if ((e = launch_sym_far(S, P, s)) != hipSuccess) return hip_fail(c, e, "far-field launch");
+    }
     {
         // the gravity inside the groups last: only the combine needs it
         ProfScope ps(&c, ws, KC_SWEEP);

@@ -227,6 +227,7 @@ struct SymLaunch {
     bool grav, want_nbr;
     bool finish;        // as SweepLaunch::finish
     bool add_acc;       // acc already holds the SPH terms: the combine adds the gravity to them
+    bool far_done;      // the far field is already enqueued (beside what follows)
     bool list_prio;     // the lists' wavefronts take issue priority over the far field's beside them
     int list_shares;    // its list kernel cut into this many shares (own list planes, merged after)
     int nshares;        // near field cut into this many shares per block (own list planes, merged after)

@@ -15,29 +15,25 @@
 //  - far field: every pair of slots in different groups is computed once,
 //    for both sides (Newton's third law).  One wavefront owns a group (16
 //    slots per lane).  The later groups' particles come 16 at a time, one
-//    per lane of each 16-lane DPP row; rotation k (row_ror:k) pairs a lane's
-//    slots with the partner k lanes away in its row.  A lane sums its own
-//    slots' gravity in registers, and the partner side of each rotation
-//    over its 16 slots in one accumulator per rotation, so nothing crosses
-//    lanes until the 16 x 16 x 16 pairs of the chunk are done; 15 DPP adds
-//    per component then gather each partner's rotations in its own lane,
-//    two swaps add the four rows, and the values are stored as the
-//    (group, partner) partial straight away;
+//    per lane of each 16-lane DPP row, and go once round the row
+//    (far_rotation.hpp); a lane sums its own slots' gravity in registers,
+//    and each partner's sum travels with it.  Two swaps then add the four
+//    rows, and the values are stored as the (group, partner) partial
+//    straight away;
 //  - a combine kernel adds, per slot and in a fixed order, the near sum,
 //    the far own-side fragments and the far partner-side partials
 //    (compensated), then finishes the acceleration as the one-range sweep.
 // Per far pair: 3 sub, 3 FMA for r^2 + H^2, one v_rsq_f32, 2 mul, 3 FMA for
 // the own side and 3 FMA for the partner side (2 more mul with unequal
-// masses), plus, per chunk and lane, 45 DPP moves of the partners' x, y, z
-// (a DPP move with several uses is not folded into them) and 51 for the
-// reduction, over 256 pairs: ~15.4 VALU instructions per wavefront and
-// partner for two interactions per lane and slot, against ~12 for one
-// interaction in the one-sided sweep.
+// masses), plus 6 DPP instructions per rotation of 16 pairs: for two
+// interactions per lane and slot, against 11 and a v_rsq_f32 for one in the
+// one-sided sweep.
 // Every sum is in a fixed order, so results do not vary from run to run.
 #include <algorithm>
 #include <utility>
 #include <vector>
 
+#include "far_rotation.hpp"
 #include "sweep_core.hpp"
 #include "sym_geometry.hpp"
 
@@ -248,98 +244,6 @@ __global__ __launch_bounds__(kBlock) void near_kernel(const float4* __restrict__
     near_blocks<GRAV, NBR, SOFT, false>(xs, 0, n, nb, nwords, bits, box, I, sl, ns, lane, cnt, part, P, R, 1.0f);
 }
 
-// Own slots of a lane in the far field: position, mass and the plain
-// gravity sums of the current unit.  At the end of a unit those go into
-// the wavefront's LDS sums (lsum[1024 c + slot], component c: plain sums of
-// at most kFoldsPerFlush units), and every kFoldsPerFlush units and at the
-// end of the row the LDS sums go into the row's own-side fragment in global
-// memory (float4 sums at frag[frag_elem(slot)], their corrections 64
-// further), compensated.  Neither level takes registers from the pair loop,
-// and the fragment is written about once per row.
-struct FarOwn {
-    float x[kNI], y[kNI], z[kNI], m[kNI];
-    float ax[kNI], ay[kNI], az[kNI];
-    float* lsum;
-    float4* frag;
-    int folds;   // units in lsum since the last flush (0: lsum holds nothing)
-    bool fresh;  // nothing flushed into the fragment yet: the first flush writes it
-    bool plain;  // every fragment is flushed once: no correction planes
-};
-
-// ------------------------------------------------------------------ rotated far segment
-// The partners of a chunk sit one per lane of a DPP row (16 partners, the
-// same 16 in all four rows).  Rotation k pairs lane l's slots with the
-// partner of row lane (l - k) & 15: DPP row_ror:k reads it straight into the
-// subtraction, so no instruction moves partner data.  The partner side of
-// rotation k is summed over the lane's slots into its own accumulator
-// (P[k]: lane l holds partner (l - k) & 15's sum), so nothing crosses lanes
-// until the chunk's 16 x 16 x 4 pairs are done; then 15 DPP adds per
-// component bring partner p's rotations to row lane p (row_ror:16-k reads
-// lane (p + k) & 15), and two swaps add the four rows.  Per chunk and lane:
-// 64 pairs at 15 instructions, plus 51 for the reduction (0.8 per pair,
-// against 54 / 32 for a reduction of 8 broadcast partners).
-
-template <int K>
-__device__ __forceinline__ float ror(float v)
-{
-    if constexpr (K == 0)
-        return v;
-    else
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + K, 0xf, 0xf, true));
-}
-
-constexpr int kRow = 16;  // partners per rotated chunk (one DPP row)
-
-// Rotation K of a chunk: the lane's kNI slots against partner (l - K) & 15
-// of its row; own side into o.a*, partner side into P[K].
-template <int K, bool UM, bool SOFT>
-__device__ __forceinline__ void far_rotation(const float4 pj, FarOwn& o, const float H2, float (&P)[kRow][3])
-{
-    const float jx = ror<K>(pj.x), jy = ror<K>(pj.y), jz = ror<K>(pj.z);
-    const float jm = UM ? 1.0f : ror<K>(pj.w);
-#pragma unroll
-    for (int q = 0; q < kNI; ++q) {
-        const float dx = jx - o.x[q], dy = jy - o.y[q], dz = jz - o.z[q];
-        const float d2 = SOFT ? fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, H2))) : fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        const float inv = __builtin_amdgcn_rsqf(d2);
-        float s = inv * inv;
-        s = s * inv;
-        if (!SOFT) s = (d2 > 0.0f) ? s : 0.0f;  // coincident particles exert nothing (computeDerivatives.h:226)
-        float sa = s, sb = s;
-        if (!UM) {
-            sa = jm * s;
-            sb = s * o.m[q];
-        }
-        o.ax[q] = fmaf(dx, sa, o.ax[q]); o.ay[q] = fmaf(dy, sa, o.ay[q]); o.az[q] = fmaf(dz, sa, o.az[q]);
-        if (q == 0) {
-            P[K][0] = dx * sb; P[K][1] = dy * sb; P[K][2] = dz * sb;
-        } else {
-            P[K][0] = fmaf(dx, sb, P[K][0]); P[K][1] = fmaf(dy, sb, P[K][1]); P[K][2] = fmaf(dz, sb, P[K][2]);
-        }
-    }
-}
-
-// partner p's rotations to row lane p: P[K] of lane (p + K) & 15 holds them
-template <int K>
-__device__ __forceinline__ void fold_rotation(const float (&P)[kRow][3], float (&T)[3])
-{
-#pragma unroll
-    for (int c = 0; c < 3; ++c) T[c] = ror<kRow - K>(P[K][c]) + T[c];
-}
-
-template <bool UM, bool SOFT, int... K>
-__device__ __forceinline__ void far_rotations(const float4 pj, FarOwn& o, const float H2, float (&P)[kRow][3],
-                                              std::integer_sequence<int, K...>)
-{
-    (far_rotation<K, UM, SOFT>(pj, o, H2, P), ...);
-}
-template <int... K>
-__device__ __forceinline__ void fold_rotations(const float (&P)[kRow][3], float (&T)[3],
-                                               std::integer_sequence<int, K...>)
-{
-    (fold_rotation<K + 1>(P, T), ...);
-}
-
 // One chunk of 16 partners (pj: row lane l holds partner l) against the
 // lane's kNI slots.  Own side into o.a*; returns the partner side: lanes
 // 0-15 hold partner l's x, lanes 16-31 partner l - 16's z, lanes 32-47
@@ -347,13 +251,19 @@ __device__ __forceinline__ void fold_rotations(const float (&P)[kRow][3], float 
 template <bool UM, bool SOFT>
 __device__ __forceinline__ float far_chunk_rot(const float4 pj, FarOwn& o, const float H2)
 {
-    float P[kRow][3];
-    far_rotations<UM, SOFT>(pj, o, H2, P, std::make_integer_sequence<int, kRow>{});
-    float T[3] = {P[0][0], P[0][1], P[0][2]};
-    fold_rotations(P, T, std::make_integer_sequence<int, kRow - 1>{});
+    FarPartner p{pj.x, pj.y, pj.z, pj.w, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int k = 0; k < kRow; ++k) {
+        if constexpr (SOFT)
+            far_rotation_soft<UM>(p, o, H2);
+        else
+            far_rotation_hard<UM>(p, o);
+    }
+    // the last rotation's contribution, then home
+    const float tx = ror<1>(ror<1>(p.tx) + p.px), ty = ror<1>(ror<1>(p.ty) + p.py), tz = ror<1>(ror<1>(p.tz) + p.pz);
     // rows 0 + 2 and 1 + 3: x to lanes 0-31, y to lanes 32-63; z everywhere
-    const float xy = swap32_sum(T[0], T[1]);
-    const float zz = swap32_sum(T[2], T[2]);
+    const float xy = swap32_sum(tx, ty);
+    const float zz = swap32_sum(tz, tz);
     // row 0: x, row 1: z, row 2: y (row 3: z again)
     return swap16_sum(xy, zz);
 }

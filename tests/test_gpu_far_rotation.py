@@ -1,0 +1,35 @@
+"""The far field's softened pair block (csrc/far_rotation.hpp) at the edges of
+its tiles: one far group of a single particle, a last chunk that is partly
+empty, whole groups, equal and unequal masses, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import grasph2_amd as g
+from grasph2_amd import ics
+from oracle import pyoracle as O
+
+from tests._util import vec_errors
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("n", [1025, 1039, 2048, 2065, 3583])
+def test_far_pairs_match_fp64(n, uniform):
+    print("far rotation n=%d uniform=%s" % (n, uniform), flush=True)
+    h, prm = ics.plummer(n, seed=n)
+    if not uniform:
+        h["posm"][:, 3] *= np.random.default_rng(n).uniform(0.5, 2.0, size=n).astype(np.float32)
+    ctx = g.Context(0)
+    ctx.set_option("sweep_symmetric", 1)
+    d = g.DeviceParticles.from_host(h)
+    ctx.compute_derivatives(d, prm)
+    g.hip.synchronize()
+    got = d.download(["acc"])["acc"]
+    d.free()
+    ctx.close()
+    ref = O.compute_derivatives(prm, h, "f64")["acc"]
+    mx, norm = vec_errors(got, ref)
+    # a slot adds at most 512 terms in plain FP32 before they are compensated: random-walk rounding of
+    # sqrt(512) half-ulps is 7e-7 of the partial sums, a tenth of that norm-wise over ~10 partials
+    assert mx < 1e-5 and norm < 1e-6, (mx, norm)
