@@ -3,9 +3,11 @@
 // A batch packs many instances back to back (see grasph_batch in
 // grasph2.h).  Per step:
 //   order   per-instance Morton order (eager, every reorder_interval steps)
-//   sweep   one persistent launch: every wavefront pulls (instance, tile)
-//           items from an atomic counter, longest instances first, so the
-//           uneven instances keep all CUs busy to the end
+//   lists   the neighbour lists of every instance (lists.hip)
+//   sweep   gravity: the symmetric sweep (sym_sweep.hip), or one persistent
+//           launch whose wavefronts pull (instance, tile) items from an atomic
+//           counter, longest instances first, so the uneven instances keep
+//           all CUs busy to the end
 //   passes  density / strain / record / accel and the leapfrog, one launch
 //           each over all instances, a block never straddling two instances
 // grasph_batch_step captures one step as a HIP graph and replays it.
@@ -57,10 +59,7 @@ struct BatchState {
     int4* d_sblk = nullptr;  // 256-slot blocks of the instances in the symmetric sweep
     int n_sblk = 0;
     int64_t sym_min = -1;    // the size threshold the tables were built with (-1: none)
-    int sym_max_words = 0;
     bool sym_plain = true;  // SymBatchTables::plain
-    float4* d_sbox = nullptr;
-    uint32_t* d_sbits = nullptr;
     float4* d_snear = nullptr;
     float4* d_sapart = nullptr;
     float* d_sbpart = nullptr;
@@ -78,7 +77,9 @@ struct BatchState {
     const void* order_src = nullptr;
     int64_t evals_since_order = 0;
 
-    // neighbour lists and pass records
+    // neighbour lists (and their boxes: fine ones, then coarse ones) and pass records
+    float4* d_box = nullptr;
+    int64_t n_fine = 0;
     int* d_nbr = nullptr;
     int* d_cnt = nullptr;
     int64_t nbr_cap = 0;  // slots * kmax allocated
@@ -89,9 +90,6 @@ struct BatchState {
     // graph of one step
     hipStream_t gs = nullptr;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
-    // the symmetric sweep's far field: its own stream, forked and joined
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_lists = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::string graph_key;
@@ -121,15 +119,14 @@ void drop_graph(BatchState& b)
 void free_tables(BatchState& b)
 {
     void* ps[] = {b.d_insts, b.d_prm, b.d_inst_of, b.d_items, b.d_blk, b.d_queue, b.d_bbox, b.d_keys, b.d_keys_alt,
-                  b.d_vals, b.d_perm, b.d_sort_tmp, b.d_ts, b.d_um, b.d_xs, b.d_sinst, b.d_srows, b.d_sbox,
-                  b.d_sbits, b.d_snear, b.d_sapart, b.d_sbpart, b.d_sblk};
+                  b.d_vals, b.d_perm, b.d_sort_tmp, b.d_ts, b.d_um, b.d_xs, b.d_sinst, b.d_srows, b.d_box,
+                  b.d_snear, b.d_sapart, b.d_sbpart, b.d_sblk};
     for (void* p : ps) free_ptr(p);
-    b.d_sinst = nullptr; b.d_srows = nullptr; b.d_sbox = nullptr; b.d_sbits = nullptr; b.d_snear = nullptr;
+    b.d_sinst = nullptr; b.d_srows = nullptr; b.d_box = nullptr; b.d_snear = nullptr;
     b.d_sapart = nullptr; b.d_sbpart = nullptr; b.d_sblk = nullptr;
     b.n_srows = 0;
     b.n_sblk = 0;
     b.sym_min = -1;
-    b.sym_max_words = 0;
     b.sym_plain = true;
     b.d_insts = nullptr; b.d_prm = nullptr; b.d_inst_of = nullptr; b.d_items = nullptr; b.d_blk = nullptr;
     b.d_queue = nullptr; b.d_bbox = nullptr; b.d_keys = nullptr; b.d_keys_alt = nullptr; b.d_vals = nullptr;
@@ -227,10 +224,13 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
         std::vector<DevParams> prm(n_inst);
         std::vector<int> inst_of((size_t)p->n);
         std::vector<int4> blk;
+        int fine0 = 0, coarse0 = 0;
         for (int k = 0; k < n_inst; ++k) {
             prm[k] = make_dev_params(&bt->params[k]);
             const int64_t off = bt->offsets[k], n = bt->offsets[k + 1] - off;
-            insts[k] = BatchInst{(int)off, (int)n, prm[k].H2, prm[k].cand};
+            insts[k] = BatchInst{(int)off, (int)n, prm[k].H2, fine0, coarse0};
+            fine0 += (int)fine_boxes(n);
+            coarse0 += (int)coarse_boxes(n);
             for (int64_t i = off; i < off + n; ++i) inst_of[(size_t)i] = k;
             for (int64_t s = off; s < off + n; s += 256)
                 blk.push_back(make_int4(k, (int)s, (int)std::min<int64_t>(s + 256, off + n), 0));
@@ -253,10 +253,12 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
             hipMalloc((void**)&b.d_keys_alt, nt * sizeof(uint64_t)) != hipSuccess ||
             hipMalloc((void**)&b.d_vals, nt * sizeof(int)) != hipSuccess ||
             hipMalloc((void**)&b.d_perm, nt * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&b.d_xs, nt * sizeof(float4)) != hipSuccess) {
+            hipMalloc((void**)&b.d_xs, nt * sizeof(float4)) != hipSuccess ||
+            hipMalloc((void**)&b.d_box, 2 * (size_t)std::max(1, fine0 + coarse0) * sizeof(float4)) != hipSuccess) {
             (void)hipGetLastError();
             return fail(c, GRASPH_E_NOMEM, "device allocation of the batch order failed");
         }
+        b.n_fine = fine0;
         b.sort_bytes = batch_order_tmp_bytes((int)p->n, b.key_bits);
         if (hipMalloc(&b.d_sort_tmp, std::max<size_t>(b.sort_bytes, 1)) != hipSuccess) {
             (void)hipGetLastError();
@@ -292,15 +294,11 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
         b.rec_cap = cap;
     }
     // the symmetric sweep's tables, here and not at first use: a step may be under graph capture then
-    if (c.batch_symmetric && (b.flags & (GRASPH_SPH | GRASPH_SELF_GRAVITY)) && (r = ensure_sym(c, b))) return r;
+    if (c.batch_symmetric && (b.flags & GRASPH_SELF_GRAVITY) && (r = ensure_sym(c, b))) return r;
     if (!b.gs) {
         if (hipStreamCreateWithFlags(&b.gs, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&b.ev_in, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&b.ev_out, hipEventDisableTiming) != hipSuccess ||
-            hipStreamCreateWithFlags(&b.side, hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&b.ev_fork, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&b.ev_join, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&b.ev_lists, hipEventDisableTiming) != hipSuccess)
+            hipEventCreateWithFlags(&b.ev_out, hipEventDisableTiming) != hipSuccess)
             return hip_fail(c, hipGetLastError(), "batch stream");
     }
     return 0;
@@ -378,10 +376,37 @@ int batch_gather(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
     return 0;
 }
 
+bool all_soft(const BatchState& b)
+{
+    for (const auto& q : b.params)
+        if (!(q.H > 0.0f)) return false;
+    return true;
+}
+
+// the neighbour lists of every instance (batch_gather must have run for the current positions)
+int batch_lists(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s)
+{
+    ListLaunch L;
+    std::memset(&L, 0, sizeof L);
+    L.xs = slot_order(c, b) ? b.d_xs : (const float4*)p->posm;
+    L.n = (int)b.ntotal;
+    L.fine = b.d_box;
+    L.coarse = b.d_box + 2 * b.n_fine;
+    L.nbr = b.d_nbr;
+    L.nbr_cnt = b.d_cnt;
+    L.kmax = b.kmax;
+    L.blk = b.d_blk;
+    L.n_blk = b.n_blk;
+    L.insts = b.d_insts;
+    ProfScope ps(&c, s, KC_SWEEP);
+    hipError_t e = launch_batch_lists(L, s);
+    if (e != hipSuccess) return hip_fail(c, e, "batched neighbour list launch");
+    return 0;
+}
+
 // the persistent sweep; with a slot order, batch_gather must have run for the current positions
 int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done = false)
 {
-    const uint32_t f = b.flags;
     const DevParams P = make_dev_params(&b.params[0]);
     hipError_t e = launch_reset_queue(b.d_queue, 1, s);
     if (e != hipSuccess) return hip_fail(c, e, "batch work counter reset");
@@ -394,25 +419,15 @@ int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStrea
     L.insts = b.d_insts;
     L.queue = b.d_queue;
     L.acc = (float4*)p->acc;
-    L.nbr = b.d_nbr;
-    L.nbr_cnt = b.d_cnt;
-    L.ntotal = (int)b.ntotal;
-    L.kmax = b.kmax;
     L.waves_per_block = c.batch_wpb;
     L.blocks = device_cus(c) * c.batch_bpc;
     L.ni_max = b.items_ni_max;
-    L.grav = f & GRASPH_SELF_GRAVITY;
-    L.want_nbr = f & GRASPH_SPH;
-    bool soft = true;
-    for (const auto& q : b.params) soft = soft && q.H > 0.0f;
-    L.soft = soft;
-    if (L.grav) {
-        if (!mass_done) {
-            e = launch_mass_check((const float4*)p->posm, b.d_insts, b.n_inst, 0, b.d_um, s);
-            if (e != hipSuccess) return hip_fail(c, e, "batch mass check launch");
-        }
-        L.umass = b.d_um;
+    L.soft = all_soft(b);
+    if (!mass_done) {
+        e = launch_mass_check((const float4*)p->posm, b.d_insts, b.n_inst, 0, b.d_um, s);
+        if (e != hipSuccess) return hip_fail(c, e, "batch mass check launch");
     }
+    L.umass = b.d_um;
     ProfScope ps(&c, s, KC_SWEEP);
     e = launch_batch_sweep(L, P, s);
     if (e != hipSuccess) return hip_fail(c, e, "batched sweep launch");
@@ -423,7 +438,7 @@ int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStrea
 int ensure_sym(Ctx& c, BatchState& b)
 {
     if (b.d_sinst && b.sym_min == c.batch_symmetric_min) return 0;
-    const SymBatchTables T = sym_batch_tables(b.offsets, (b.flags & GRASPH_SPH) != 0, c.batch_symmetric_min);
+    const SymBatchTables T = sym_batch_tables(b.offsets, c.batch_symmetric_min);
     int r;
     free_ptr(b.d_sinst); free_ptr(b.d_srows); free_ptr(b.d_sblk);
     b.d_sinst = nullptr; b.d_srows = nullptr; b.d_sblk = nullptr;
@@ -434,17 +449,12 @@ int ensure_sym(Ctx& c, BatchState& b)
     b.n_srows = (int)T.rows.size();
     b.n_sblk = (int)T.blk.size();
     b.sym_min = c.batch_symmetric_min;
-    b.sym_max_words = T.max_words;
     b.sym_plain = T.plain;
     // fresh arrays for the new tables (upload()-style: free, then allocate)
-    void* old[] = {b.d_sbox, b.d_sbits, b.d_snear, b.d_sapart, b.d_sbpart};
+    void* old[] = {b.d_snear, b.d_sapart, b.d_sbpart};
     for (void* q : old) free_ptr(q);
-    b.d_sbox = nullptr; b.d_sbits = nullptr; b.d_snear = nullptr; b.d_sapart = nullptr; b.d_sbpart = nullptr;
+    b.d_snear = nullptr; b.d_sapart = nullptr; b.d_sbpart = nullptr;
     int64_t cap = 0;
-    if ((r = grow(c, b.d_sbox, cap, std::max<int64_t>(T.box_elems, 1), "batch symmetric-sweep boxes"))) return r;
-    cap = 0;
-    if ((r = grow(c, b.d_sbits, cap, std::max<int64_t>(T.bits_elems, 1), "batch symmetric-sweep near bits"))) return r;
-    cap = 0;
     if ((r = grow(c, b.d_snear, cap, std::max<int64_t>(2 * b.ntotal, 1), "batch symmetric-sweep near sums"))) return r;
     cap = 0;
     if ((r = grow(c, b.d_sapart, cap, std::max<int64_t>(T.apart_elems, 1), "batch symmetric-sweep own sums"))) return r;
@@ -455,120 +465,57 @@ int ensure_sym(Ctx& c, BatchState& b)
     return 0;
 }
 
-// The symmetric sweep over the batch's larger instances, begun (after
-// launch_sweep_only, which has then run the mass check: mass_done): the far
-// field forked onto b.side (fork; else in order on s), the near field's
-// lists on s; sym_batch_end adds its in-group gravity, joins and combines.
-// The far field reads only the slot-ordered positions and the mass
-// records, written on s before the fork.
-int sym_batch_begin(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done, bool fork,
-                    SymBatchLaunch& L)
+// The symmetric gravity sweep over the batch's larger instances, in order on
+// s (mass_done: launch_sweep_only has run the mass check).  add_acc: acc
+// holds the SPH terms, the gravity joins them.
+int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done, bool add_acc)
 {
     int r;
     if ((r = ensure_sym(c, b))) return r;
-    const uint32_t f = b.flags;
+    SymBatchLaunch L;
     std::memset(&L, 0, sizeof L);
     L.perm = slot_order(c, b);
     L.xs = L.perm ? b.d_xs : (const float4*)p->posm;
     L.ntotal = (int)b.ntotal;
     L.n_inst = b.n_inst;
-    L.grav = f & GRASPH_SELF_GRAVITY;
-    L.want_nbr = f & GRASPH_SPH;
+    L.grav = true;
     L.finish = false;  // the finishing launch of the batch follows
-    bool soft = true;
-    for (const auto& q : b.params) soft = soft && q.H > 0.0f;
-    L.soft = soft;
+    L.add_acc = add_acc;
+    L.soft = all_soft(b);
     L.sinst = b.d_sinst;
     L.insts = b.d_insts;
     L.prm = b.d_prm;
     L.blk = b.d_sblk;
     L.n_blk = b.n_sblk;
-    L.inst_of = b.d_inst_of;
     L.rows = b.d_srows;
     L.nrows = b.n_srows;
-    L.max_words = b.sym_max_words;
     L.plain = b.sym_plain;
     L.queue = b.d_queue + 1;
     L.wgs = c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(device_cus(c));
     L.acc = (float4*)p->acc;
-    L.nbr = b.d_nbr;
-    L.nbr_cnt = b.d_cnt;
-    L.kmax = b.kmax;
     L.vel = (const float4*)p->vel;
     L.xvel = (float4*)p->xvel;
     L.maxvsig = p->maxvsig;
-    L.box = b.d_sbox;
-    L.bits = b.d_sbits;
     L.near_part = b.d_snear;
     L.apart = b.d_sapart;
     L.bpart = b.d_sbpart;
     hipError_t e;
-    if (L.grav) {
-        if (!mass_done) {
-            e = launch_mass_check((const float4*)p->posm, b.d_insts, b.n_inst, 0, b.d_um, s);
-            if (e != hipSuccess) return hip_fail(c, e, "batch mass check launch");
-        }
-        L.umass = b.d_um;
+    if (!mass_done) {
+        e = launch_mass_check((const float4*)p->posm, b.d_insts, b.n_inst, 0, b.d_um, s);
+        if (e != hipSuccess) return hip_fail(c, e, "batch mass check launch");
     }
+    L.umass = b.d_um;
     if (sym_batch_has_far(L)) {
-        hipStream_t fs = s;
-        if (fork) {
-            if ((e = hipEventRecord(b.ev_fork, s)) != hipSuccess || (e = hipStreamWaitEvent(b.side, b.ev_fork, 0)))
-                return hip_fail(c, e, "batched far-field fork");
-            fs = b.side;
-        }
-        {
-            ProfScope ps(&c, fs, KC_FAR);
-            if ((e = launch_sym_batch_far(L, fs)) != hipSuccess) return hip_fail(c, e, "batched far-field launch");
-        }
+        ProfScope ps(&c, s, KC_FAR);
+        if ((e = launch_sym_batch_far(L, s)) != hipSuccess) return hip_fail(c, e, "batched far-field launch");
     }
     {
         ProfScope ps(&c, s, KC_SWEEP);
-        if ((e = launch_sym_batch_lists(L, s)) != hipSuccess) return hip_fail(c, e, "batched near-field list launch");
+        if ((e = launch_sym_batch_ingroup(L, s)) != hipSuccess) return hip_fail(c, e, "batched in-group gravity launch");
     }
-    if (fork && sym_batch_has_far(L)) {
-        // the gravity inside the groups needs only the positions: after the
-        // far field on its stream, once the lists are done, so that it shares
-        // the vector units with the memory-bound passes on s rather than with
-        // the list kernel, which the passes wait for
-        if (L.want_nbr && ((e = hipEventRecord(b.ev_lists, s)) != hipSuccess ||
-                           (e = hipStreamWaitEvent(b.side, b.ev_lists, 0)) != hipSuccess))
-            return hip_fail(c, e, "batched list event");
-        {
-            ProfScope ps(&c, b.side, KC_SWEEP);
-            if ((e = launch_sym_batch_ingroup(L, b.side)) != hipSuccess)
-                return hip_fail(c, e, "batched near-field gravity launch");
-            L.ingroup_done = true;
-        }
-        if ((e = hipEventRecord(b.ev_join, b.side)) != hipSuccess) return hip_fail(c, e, "batched far-field join event");
-    }
-    return 0;
-}
-
-int sym_batch_end(Ctx& c, BatchState& b, SymBatchLaunch& L, hipStream_t s, bool forked, bool add_acc)
-{
-    hipError_t e;
-    if (!L.ingroup_done) {
-        // the gravity inside the groups last on s: only the combine needs it
-        ProfScope ps(&c, s, KC_SWEEP);
-        if ((e = launch_sym_batch_ingroup(L, s)) != hipSuccess)
-            return hip_fail(c, e, "batched near-field gravity launch");
-    }
-    if (forked && sym_batch_has_far(L) && (e = hipStreamWaitEvent(s, b.ev_join, 0)) != hipSuccess)
-        return hip_fail(c, e, "batched far-field join");
-    L.add_acc = add_acc;
     ProfScope ps(&c, s, KC_SWEEP);
     if ((e = launch_sym_batch_combine(L, s)) != hipSuccess) return hip_fail(c, e, "batched symmetric combine launch");
     return 0;
-}
-
-// the whole symmetric sweep in order on s (the autotuner times it)
-int launch_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done)
-{
-    SymBatchLaunch L;
-    int r;
-    if ((r = sym_batch_begin(c, b, p, s, mass_done, false, L))) return r;
-    return sym_batch_end(c, b, L, s, false, false);
 }
 
 int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s);
@@ -595,13 +542,12 @@ int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
     const DevParams P = make_dev_params(&b.params[0]);  // flags; values come from the per-instance table
     int r;
     if ((r = batch_gather(c, b, p, s))) return r;
-    // the one-sided persistent sweep takes the items (with the symmetric
-    // sweep on: the smaller instances), the symmetric sweep the rest; its
-    // far field is forked onto a stream of its own and overlaps the rest
-    const bool sym = (sph || grav) && c.batch_symmetric;
-    SymBatchLaunch SL;
-    if (sym && (r = sym_batch_begin(c, b, p, s, false, true, SL))) return r;
-    if ((sph || grav) && b.n_items > 0 && (r = launch_sweep_only(c, b, p, s, sym))) return r;
+    if (sph && (r = batch_lists(c, b, p, s))) return r;
+    // gravity: the one-sided persistent sweep takes the items (with the
+    // symmetric sweep on: the smaller instances), the symmetric sweep the rest
+    const bool sym = grav && c.batch_symmetric;
+    const bool items = grav && b.n_items > 0;
+    if (items && (r = launch_sweep_only(c, b, p, s))) return r;
 
     const int* perm = slot_order(c, b);
     NbrLaunch N;
@@ -623,11 +569,10 @@ int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
     N.acc = (float4*)p->acc;
     N.xvel = (float4*)p->xvel;
     N.maxvsig = p->maxvsig;
-    N.acc_has_gravity = grav;
     N.T = tables(b);
     hipError_t e;
     if (!sph) {
-        if (sym && (r = sym_batch_end(c, b, SL, s, true, false))) return r;
+        if (sym && (r = run_sym_sweep_batch(c, b, p, s, items, false))) return r;
         ProfScope ps(&c, s, KC_OTHER);
         e = launch_finish(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "batched finish launch");
@@ -647,23 +592,18 @@ int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
         e = launch_prep(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "batched record launch");
     }
-    // With every instance in the symmetric sweep, the acceleration pass runs
-    // while the far field is still going and writes the SPH terms alone; the
-    // combine then adds the gravity to them.  Otherwise it adds the SPH
-    // terms to the gravity of the sweeps.
-    const bool accel_first = sym && b.n_items == 0;
-    if (accel_first) {
-        N.acc_has_gravity = false;
+    // With every instance in the symmetric sweep, the acceleration pass
+    // writes the SPH terms alone and the combine adds the gravity to them.
+    // Otherwise it adds the SPH terms to the gravity of the sweeps.
+    const bool accel_first = sym && !items;
+    if (sym && !accel_first && (r = run_sym_sweep_batch(c, b, p, s, items, false))) return r;
+    N.acc_has_gravity = grav && !accel_first;
+    {
         ProfScope ps(&c, s, KC_ACCEL);
         e = launch_accel(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "batched acceleration launch");
     }
-    if (sym && (r = sym_batch_end(c, b, SL, s, true, accel_first && grav))) return r;
-    if (accel_first) return 0;
-    ProfScope ps(&c, s, KC_ACCEL);
-    e = launch_accel(N, P, s);
-    if (e != hipSuccess) return hip_fail(c, e, "batched acceleration launch");
-    return 0;
+    return accel_first ? run_sym_sweep_batch(c, b, p, s, false, true) : 0;
 }
 
 int batch_integrate_launch(Ctx& c, BatchState& b, const grasph_particles* p, int nfs, hipStream_t s)
@@ -718,13 +658,13 @@ std::string graph_key(const Ctx& c, const BatchState& b, const grasph_particles*
       << (c.reorder_interval > 0) << ' ' << c.batch_wpb << ' ' << c.batch_bpc << ' ' << (const void*)b.d_nbr << ' '
       << (const void*)b.d_rec << ' ' << (const void*)b.d_items << ' ' << (const void*)b.d_xs << ' '
       << c.batch_symmetric << ' ' << c.batch_symmetric_min << ' '
-      << (const void*)b.d_sinst << ' ' << (const void*)b.d_sbpart << ' ' << (const void*)b.d_sblk;
+      << (const void*)b.d_box << ' ' << (const void*)b.d_sinst << ' ' << (const void*)b.d_sbpart << ' '
+      << (const void*)b.d_sblk;
     return k.str();
 }
 
-// time the batched sweep (min of reps), milliseconds: the one-sided
-// persistent sweep alone, or (all) with the symmetric sweep of the larger instances
-int time_sweep(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, int reps, double* ms, bool all = false)
+// time the one-sided persistent sweep (min of reps), milliseconds
+int time_sweep(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, int reps, double* ms)
 {
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
@@ -735,8 +675,7 @@ int time_sweep(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, 
     c.profile = false;
     for (int k = 0; k < reps + 1 && !r; ++k) {
         (void)hipEventRecord(e0, s);
-        if (!all || b.n_items > 0) r = launch_sweep_only(c, b, p, s);
-        if (!r && all && c.batch_symmetric) r = launch_sym_sweep_batch(c, b, p, s, b.n_items > 0);
+        r = launch_sweep_only(c, b, p, s);
         (void)hipEventRecord(e1, s);
         if (!r && hipEventSynchronize(e1) == hipSuccess) {
             float t = 0;
@@ -806,10 +745,6 @@ void destroy_batch_state(BatchState* b)
     if (b->ev_in) (void)hipEventDestroy(b->ev_in);
     if (b->ev_out) (void)hipEventDestroy(b->ev_out);
     if (b->gs) (void)hipStreamDestroy(b->gs);
-    if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
-    if (b->ev_join) (void)hipEventDestroy(b->ev_join);
-    if (b->ev_lists) (void)hipEventDestroy(b->ev_lists);
-    if (b->side) (void)hipStreamDestroy(b->side);
     for (grasph_ctx* x : b->loop)
         if (x) grasph_destroy(x);
     delete b;
@@ -973,9 +908,11 @@ int grasph_autotune(grasph_ctx* ctx, const grasph_particles* p, const grasph_bat
         }
     }
     if ((r = grasph::ensure_order(c, B, p, s, false))) return r;
+    // gravity only: without it there is no sweep to tune
+    const bool grav = B.flags & GRASPH_SELF_GRAVITY, sym_allowed = grav && c.batch_symmetric;
+    int64_t sym_min = grav ? -1 : c.batch_symmetric ? c.batch_symmetric_min : -1;
     // the one-sided persistent sweep over every instance for its launch shape
-    const bool sym_allowed = c.batch_symmetric && (B.flags & (GRASPH_SPH | GRASPH_SELF_GRAVITY));
-    c.batch_symmetric = 0;
+    if (grav) c.batch_symmetric = 0;
     // launch shape with one particle per lane everywhere
     for (int q = 0; q < 4; ++q) c.batch_ni[q] = 1;
     if ((r = grasph::prepare(c, p, b))) return r;
@@ -984,6 +921,7 @@ int grasph_autotune(grasph_ctx* ctx, const grasph_particles* p, const grasph_bat
     double best = 1e30;
     int bw = 4, bb = 8;
     for (const auto& sh : shapes) {
+        if (!grav) break;
         c.batch_wpb = sh[0];
         c.batch_bpc = sh[1];
         double t;
@@ -1000,7 +938,7 @@ int grasph_autotune(grasph_ctx* ctx, const grasph_particles* p, const grasph_bat
     int present[4] = {0, 0, 0, 0};
     for (int k = 0; k < B.n_inst; ++k) present[grasph::bucket_of(B.offsets[k + 1] - B.offsets[k])] = 1;
     for (int q = 0; q < 4; ++q) {
-        if (!present[q]) continue;
+        if (!present[q] || !grav) continue;
         c.batch_ni[q] = 2;
         if ((r = grasph::prepare(c, p, b))) return r;
         double t;
@@ -1011,10 +949,8 @@ int grasph_autotune(grasph_ctx* ctx, const grasph_particles* p, const grasph_bat
             c.batch_ni[q] = 1;
     }
     // the symmetric sweep from which size bucket on (or for none), timed
-    // as whole derivative evaluations: the sweeps alone rank the candidates
-    // near 0, 4096 and 8192 within their noise, while the passes beside
-    // the far field set the step apart (16.5 against 17.1 ms per step)
-    int64_t sym_min = -1;
+    // as whole derivative evaluations (the sweeps alone rank the candidates
+    // near 0, 4096 and 8192 within their noise)
     if (sym_allowed) {
         const int64_t cands[] = {0, 2048, 4096, 8192, -1};
         double best_all = 1e30;

@@ -155,11 +155,6 @@ int ensure_order(Ctx& c, const grasph_particles* p, hipStream_t s, bool count_ev
 
 const int* order_of(Ctx& c) { return c.reorder_interval > 0 ? c.perm : nullptr; }
 
-// The list capacity an earlier evaluation asked for: once the copy of its
-// largest neighbour count has landed (queried, never waited for), a count
-// above max_neighbours raises it to 1.25 times that count, in steps of 32,
-// at most 4096 and at most 16 GiB of list planes.  Overflowing particles
-// take the exact all-partner scan meanwhile, so the results do not change.
 // whether work enqueued on s is being captured into a graph (then the
 // event query and the copy would break the capture)
 bool stream_capturing(hipStream_t s)
@@ -172,51 +167,44 @@ bool stream_capturing(hipStream_t s)
     return st != hipStreamCaptureStatusNone;
 }
 
-void grow_list_capacity(Ctx& c, int64_t n, int slices, hipStream_t s)
+// The list capacity an earlier evaluation asked for: a list that overflowed
+// has stored its count in pinned host memory (read, never waited for); a
+// count above max_neighbours raises it to 1.25 times that count, in steps of
+// 32, at most 4096 and at most 16 GiB of lists.  Overflowing particles take
+// the exact all-partner scan meanwhile, so the results do not change.
+void grow_list_capacity(Ctx& c, int64_t n, hipStream_t s)
 {
-    if (!c.list_max_pending || c.capturing || stream_capturing(s)) return;
-    const hipError_t q = hipEventQuery(c.list_max_ev);
-    if (q != hipSuccess) {
-        (void)hipGetLastError();  // not ready (or unknown): look again next time
-        return;
-    }
-    c.list_max_pending = false;
-    const int m = *c.list_max_host;
+    if (!c.list_max_host) return;
+    const int m = *(volatile int*)c.list_max_host;
+    if (m <= 0 || c.capturing || stream_capturing(s)) return;
+    *(volatile int*)c.list_max_host = 0;
     if (!c.max_neighbours_grow || m <= c.max_neighbours) return;
     int64_t k = ((int64_t)m + m / 4 + 31) / 32 * 32;
-    const int64_t cap = (int64_t(16) << 30) / (4 * std::max<int64_t>(1, n) * std::max(1, slices));
+    const int64_t cap = (int64_t(16) << 30) / (4 * std::max<int64_t>(1, n));
     k = std::min<int64_t>(std::min<int64_t>(k, 4096), cap / 32 * 32);
     if (k > c.max_neighbours) c.max_neighbours = (int)k;
 }
 
-// After the lists of an evaluation are final: their largest count, reduced
-// on ws and copied to pinned host memory behind an event (not while the
-// caller's stream is being captured into a graph, nor without growth).
-int watch_list_counts(Ctx& c, int64_t n, hipStream_t s, hipStream_t ws)
+// where the list kernel reports overflowed lists (not when capacities are fixed)
+int ensure_list_watch(Ctx& c, hipStream_t s)
 {
-    if (!c.max_neighbours_grow || c.no_alloc || c.capturing || stream_capturing(s)) return 0;
+    if (!c.max_neighbours_grow || c.no_alloc || c.list_max_host || c.capturing || stream_capturing(s)) return 0;
     hipError_t e;
     if (!c.list_max_dev && (e = hipMalloc((void**)&c.list_max_dev, sizeof(int))) != hipSuccess)
         return hip_fail(c, e, "neighbour-count maximum");
-    if (!c.list_max_host && (e = hipHostMalloc((void**)&c.list_max_host, sizeof(int), hipHostMallocDefault)) != hipSuccess)
+    if ((e = hipHostMalloc((void**)&c.list_max_host, sizeof(int), hipHostMallocDefault)) != hipSuccess) {
+        c.list_max_host = nullptr;
         return hip_fail(c, e, "pinned neighbour-count maximum");
-    if (!c.list_max_ev && (e = hipEventCreateWithFlags(&c.list_max_ev, hipEventDisableTiming)) != hipSuccess)
-        return hip_fail(c, e, "neighbour-count event");
-    ProfScope ps(&c, ws, KC_OTHER);
-    if ((e = launch_count_max(c.nbr_cnt, (int)n, c.list_max_dev, ws)) != hipSuccess ||
-        (e = hipMemcpyAsync(c.list_max_host, c.list_max_dev, sizeof(int), hipMemcpyDeviceToHost, ws)) != hipSuccess ||
-        (e = hipEventRecord(c.list_max_ev, ws)) != hipSuccess)
-        return hip_fail(c, e, "neighbour-count watch");
-    c.list_max_pending = true;
+    }
+    *c.list_max_host = 0;
     return 0;
 }
 
-// lists for `slices` slices: slices planes of list_plane(n, kmax) entries
-// (slots rounded up to tiles of 64) and slices * n counts
-int ensure_nbr(Ctx& c, int64_t n, int slices)
+// list_plane(n, kmax) entries (slots rounded up to tiles of 64) and n counts
+int ensure_nbr(Ctx& c, int64_t n)
 {
     const int k = c.max_neighbours;
-    const int64_t need_n = (n + 63) / 64 * 64 * slices;
+    const int64_t need_n = (n + 63) / 64 * 64;
     if (c.nbr && c.nbr_cap_n >= need_n && c.nbr_cap_k >= k) return 0;
     if (c.no_alloc) return fail(c, GRASPH_E_NOMEM, "the neighbour list would need a device allocation");
     if (c.nbr) (void)hipFree(c.nbr);
@@ -240,10 +228,7 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
     L.perm = order_of(c);
     L.n = (int)p->n;
     L.acc = (float4*)p->acc;
-    L.nbr = c.nbr;
-    L.nbr_cnt = c.nbr_cnt;
     L.pot = c.pot;
-    L.kmax = c.max_neighbours;
     L.vel = (const float4*)p->vel;
     L.xvel = (float4*)p->xvel;
     L.maxvsig = p->maxvsig;
@@ -287,7 +272,7 @@ constexpr int64_t kSymAutoMinGravity = 16384;
 
 int sym_wgs(const Ctx& c) { return c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(c.cus); }
 
-// shares of the symmetric sweep's near field: ~16 wavefronts per SIMD, at most 16
+// shares of the symmetric sweep's in-group gravity: ~16 wavefronts per SIMD, at most 16
 int sym_near_shares(const Ctx& c, int64_t n)
 {
     if (c.sym_near_shares > 0) return c.sym_near_shares;
@@ -296,111 +281,53 @@ int sym_near_shares(const Ctx& c, int64_t n)
     return (int)std::min<int64_t>(16, std::max<int64_t>(1, (target + blocks - 1) / blocks));
 }
 
-// particles from which, with lists, the rest of the evaluation runs beside the far field
-constexpr int kForkMin = 20480;
-
-// The symmetric sweep, begun: buffers; with lists and at least kForkMin
-// particles, the rest of the evaluation forked onto the context's second stream (ws) after the gather and the mass
-// check; the far field on s, launched first so that its workgroups are
-// placed first and no event stands between it and the work before it; the
-// near field's lists on ws.  The far field needs only the slot-ordered
-// positions and the mass record; the work enqueued on ws after this (list
-// merge, the SPH passes) runs beside it.  sym_sweep_end enqueues the near
-// field's in-group gravity on ws, joins ws to s and combines on s.
-int sym_sweep_begin(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t s, SymLaunch& S,
-                    hipStream_t& ws)
+// The symmetric gravity sweep, in order on s: the far field, the in-group
+// gravity, the combine (add_acc: acc holds the SPH terms, the gravity joins
+// them).  Nothing runs beside the far field: a wavefront of another kernel on
+// its SIMD takes the far field's from 2 to 4 clocks per instruction
+// (far_rotation.hpp; with the lists and passes beside it on a second stream
+// the collision of 131072 took 2.71 ms per step, in order 2.70, and every
+// smaller one gains: 16384 default solids 207 -> 138 us).
+int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t s, bool add_acc)
 {
     const int64_t col_elems = c.sym_partial_bytes / (int64_t)sizeof(float);
-    const SymGeom G = sym_geometry(L.n, sym_wgs(c), L.want_nbr, L.near_shares, col_elems);
+    const SymGeom G = sym_geometry(L.n, sym_wgs(c), L.near_shares, col_elems);
     int r;
-    if ((r = grow(c, c.sym_box, c.sym_box_cap, G.box_elems, "symmetric sweep boxes")) ||
-        (r = grow(c, c.sym_bits, c.sym_bits_cap, G.bits_elems, "symmetric sweep near bits")) ||
-        (r = grow(c, c.sym_near, c.sym_near_cap, G.near_elems, "symmetric sweep near sums")) ||
+    if ((r = grow(c, c.sym_near, c.sym_near_cap, G.near_elems, "symmetric sweep near sums")) ||
         (r = grow(c, c.sym_apart, c.sym_apart_cap, G.apart_elems, "symmetric sweep own-side sums")) ||
         (r = grow(c, c.sym_bpart, c.sym_bpart_cap, G.bpart_elems, "symmetric sweep partner-side sums")) ||
-        (G.ncols > 1 && L.grav &&
+        (G.ncols > 1 &&
          (r = grow(c, c.sym_accsum, c.sym_accsum_cap, 2 * (int64_t)L.n, "symmetric sweep column sums"))))
         return r;
+    SymLaunch S;
     std::memset(&S, 0, sizeof S);
     S.xs = L.xs ? L.xs : L.posm;
     S.perm = L.perm;
     S.n = L.n;
     S.grav = L.grav;
-    S.want_nbr = L.want_nbr;
     S.finish = L.finish;
+    S.add_acc = add_acc;
     S.nshares = L.near_shares;
-    S.list_shares = L.nslices;
     S.acc = L.acc;
-    S.nbr = L.nbr;
-    S.nbr_cnt = L.nbr_cnt;
-    S.kmax = L.kmax;
     S.vel = L.vel;
     S.xvel = L.xvel;
     S.maxvsig = L.maxvsig;
     S.umass = L.umass;
     S.wgs = G.wgs;
-    S.box = c.sym_box;
-    S.bits = c.sym_bits;
     S.near_part = c.sym_near;
     S.apart = c.sym_apart;
     S.bpart = c.sym_bpart;
     S.col_elems = col_elems;
     S.accsum = c.sym_accsum;
     hipError_t e;
-    ws = s;
-    // The rest beside the far field only with lists and many particles: a
-    // wavefront of another kernel on its SIMD takes the far field's from 2
-    // to 4 clocks per instruction (far_rotation.hpp), so what runs beside it
-    // has to be worth more than that.  Gravity alone in order on s: Plummer
-    // N = 16384 86.1 -> 73.4 us per step, 50021 unequal masses 482 -> 460;
-    // the default solids at N = 16384 (lists) 207 -> 190 us.  Beside it:
-    // collision N = 131072 2.72 against 2.86 ms, liquid N = 65536 0.872
-    // against 0.902, collision N = 33000 0.51 against 0.56.
-    if (sym_has_far(S) && L.want_nbr && L.n >= kForkMin) {
-        S.far_done = true;
-        if (c.no_alloc && (!c.side || !c.ev_fork || !c.ev_join))
-            return fail(c, GRASPH_E_NOMEM, "the second stream would need creating");
-        if (!c.side && (e = hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking)) != hipSuccess)
-            return hip_fail(c, e, "second stream");
-        if ((!c.ev_fork && (e = hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming)) != hipSuccess) ||
-            (!c.ev_join && (e = hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming)) != hipSuccess))
-            return hip_fail(c, e, "fork and join events");
-        if ((e = hipEventRecord(c.ev_fork, s)) != hipSuccess || (e = hipStreamWaitEvent(c.side, c.ev_fork, 0)) != hipSuccess)
-            return hip_fail(c, e, "fork");
-        {
-            ProfScope ps(&c, s, KC_FAR);
-            if ((e = launch_sym_far(S, P, s)) != hipSuccess) return hip_fail(c, e, "far-field launch");
-        }
-        ws = c.side;
-        // Below ~50k particles the far field's window is short next to the
-        // lists' work, and once the lists have grown long (capacity past
-        // 512: bodies in contact) the lists and the passes after them outlast
-        // it at any size: there issue priority over the far field shortens
-        // the step (collision N = 32768: 0.435 -> 0.410 ms, N = 131072 after
-        // impact: 5.87 -> 5.57).
-        S.list_prio = c.sym_list_priority == 1 ||
-                      (c.sym_list_priority == 2 && (L.n < 49152 || c.max_neighbours > 512));
-    }
-    ProfScope ps(&c, ws, KC_SWEEP);
-    if ((e = launch_sym_lists(S, P, ws)) != hipSuccess) return hip_fail(c, e, "near-field list launch");
-    return 0;
-}
-
-int sym_sweep_end(Ctx& c, SymLaunch& S, const DevParams& P, hipStream_t s, hipStream_t ws, bool add_acc)
-{
-    hipError_t e;
-    S.add_acc = add_acc;
-    if (!S.far_done) {
+    if (sym_has_far(S)) {
         ProfScope ps(&c, s, KC_FAR);
         if ((e = launch_sym_far(S, P, s)) != hipSuccess) return hip_fail(c, e, "far-field launch");
     }
     {
-        // the gravity inside the groups last: only the combine needs it
-        ProfScope ps(&c, ws, KC_SWEEP);
-        if ((e = launch_sym_ingroup(S, P, ws)) != hipSuccess) return hip_fail(c, e, "near-field gravity launch");
+        ProfScope ps(&c, s, KC_SWEEP);
+        if ((e = launch_sym_ingroup(S, P, s)) != hipSuccess) return hip_fail(c, e, "in-group gravity launch");
     }
-    if (ws != s && ((e = hipEventRecord(c.ev_join, ws)) != hipSuccess || (e = hipStreamWaitEvent(s, c.ev_join, 0))))
-        return hip_fail(c, e, "join");
     ProfScope ps(&c, s, KC_SWEEP);
     if ((e = launch_sym_combine(S, P, s)) != hipSuccess) return hip_fail(c, e, "symmetric combine launch");
     return 0;
@@ -487,35 +414,23 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     // the order only matters for the neighbour branch: gravity alone runs in index order
     if (need_list && (r = ensure_order(c, p, s, true))) return r;
     const bool sweep_grav = accel_pass && grav;
-    const bool sym_on = c.sweep_symmetric == 1 ||
-                        (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity));
-    const bool sym = sym_on && (sweep_grav || need_list);
+    const bool sym = sweep_grav &&
+                     (c.sweep_symmetric == 1 ||
+                      (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity)));
     int slices = 1, slice_len = (int)n;
-    if ((sweep_grav || need_list) && !sym) choose_slices(c, n, c.sweep_ni, &slices, &slice_len);
-    int near_shares = 1;
-    if (sym) {
-        // the near field's list shares take the slices' list planes; with
-        // long lists (after a collision's impact) one share: the merge of
-        // shares would move every entry again (1e8 entries: 1.4 ms), and
-        // the one list kernel still ends inside the far field's window
-        near_shares = sym_near_shares(c, n);
-        slices = (int64_t)n * c.max_neighbours >= (int64_t(1) << 26) ? 1 : near_shares;
-    }
+    if (sweep_grav && !sym) choose_slices(c, n, c.sweep_ni, &slices, &slice_len);
     if (need_list) {
-        grow_list_capacity(c, n, slices, s);
-        if ((r = ensure_nbr(c, n, slices))) return r;
+        grow_list_capacity(c, n, s);
+        if ((r = ensure_nbr(c, n)) || (r = ensure_list_watch(c, s))) return r;
         c.last_list_n = n;
-        c.last_list_slices = slices;
     }
-    if (slices > 1 && sweep_grav && !sym) {
-        if ((r = grow(c, c.part, c.part_cap, 2 * n * slices, "sweep partial sums"))) return r;
-    }
+    if (slices > 1 && (r = grow(c, c.part, c.part_cap, 2 * n * slices, "sweep partial sums"))) return r;
     const DevParams P = make_dev_params(prm);
 
     // slot-ordered positions for the sweep and the passes' slot records
     const int* perm = need_list ? order_of(c) : nullptr;
     const float4* xs = (const float4*)p->posm;
-    const int gather_blocks = (int)((n + 255) / 256);
+    const int gather_blocks = (int)((n + kGatherBlock - 1) / kGatherBlock);
     bool mass_flags = false;  // the gather makes the equal-mass check's per-block flags
     if (need_list) {
         const bool reads_vel = strain_pass || (accel_pass && sph);
@@ -523,26 +438,45 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         mass_flags = sweep_grav;
         if ((perm && (r = grow(c, c.xs, c.xs_cap, n, "slot-ordered positions"))) ||
             (r = grow(c, c.rec, c.rec_cap, n, "slot records")) ||
+            (r = grow(c, c.box, c.box_cap, 2 * (fine_boxes(n) + coarse_boxes(n)), "neighbour-search boxes")) ||
             (mass_flags && (r = grow(c, c.mass_flags, c.mass_flags_cap, gather_blocks, "mass-check flags"))))
             return r;
         ProfScope ps(&c, s, KC_REORDER);
         hipError_t e = launch_gather(perm, (int)n, (const float4*)p->posm, reads_vel ? (const float4*)p->vel : nullptr,
                                      gdens ? p->density : nullptr, perm ? c.xs : nullptr, c.rec, s,
-                                     mass_flags ? c.mass_flags : nullptr);
+                                     mass_flags ? c.mass_flags : nullptr, c.box, c.box + 2 * fine_boxes(n),
+                                     c.list_max_dev);
         if (e != hipSuccess) return hip_fail(c, e, "slot-order gather launch");
         if (perm) xs = c.xs;
     }
 
-    // one all-pairs sweep
+    if (need_list) {
+        ListLaunch N;
+        std::memset(&N, 0, sizeof N);
+        N.xs = xs;
+        N.n = (int)n;
+        N.H2 = P.H2;
+        N.fine = c.box;
+        N.coarse = c.box + 2 * fine_boxes(n);
+        N.nbr = c.nbr;
+        N.nbr_cnt = c.nbr_cnt;
+        N.kmax = c.max_neighbours;
+        N.max_dev = c.list_max_dev;
+        N.max_host = c.max_neighbours_grow ? c.list_max_host : nullptr;
+        ProfScope ps(&c, s, KC_SWEEP);
+        hipError_t e = launch_lists(N, s);
+        if (e != hipSuccess) return hip_fail(c, e, "neighbour list launch");
+    }
+
+    // gravity
     SweepLaunch L = sweep_base(c, p);
     L.perm = perm;
     L.xs = xs;
     L.grav = sweep_grav;
-    L.want_nbr = need_list;
     L.want_pot = false;
     L.finish = accel_pass && !sph;
     L.nslices = slices;
-    L.near_shares = near_shares;
+    L.near_shares = sym ? sym_near_shares(c, n) : 1;
     L.slice_len = slice_len;
     L.part = c.part;
     if (sweep_grav) {
@@ -553,67 +487,43 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         if (e != hipSuccess) return hip_fail(c, e, "mass check launch");
         L.umass = c.umass;
     }
-    SymLaunch S;
-    hipStream_t ws = s;  // the near field and the passes: the forked stream beside the far field, or s
-    if (sym) {
-        if ((r = sym_sweep_begin(c, L, P, s, S, ws))) return r;
-    } else if ((r = run_sweep(c, L, P, s))) {
-        return r;
-    }
-    if (need_list && slices > 1) {
-        // one list per particle for the passes (walking per-slice lists costs them up to 2x)
-        ProfScope ps(&c, ws, KC_OTHER);
-        hipError_t e = launch_merge_lists(c.nbr, c.nbr_cnt, (int)n, c.max_neighbours, slices, ws);
-        if (e != hipSuccess) return hip_fail(c, e, "list merge launch");
-        c.last_list_slices = 1;
-    }
-    if (need_list && (r = watch_list_counts(c, n, s, ws))) return r;
+    if (!sym && (sweep_grav || L.finish) && (r = run_sweep(c, L, P, s))) return r;
 
     NbrLaunch N = nbr_base(c, p);
     N.perm = perm;
     N.xs = xs;
     N.rec = c.rec;
     if (dens_pass) {
-        ProfScope ps(&c, ws, KC_DENSITY);
-        hipError_t e = launch_density(N, p->density, P, ws);
+        ProfScope ps(&c, s, KC_DENSITY);
+        hipError_t e = launch_density(N, p->density, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "density pass launch");
     }
     if (strain_pass) {
-        ProfScope ps(&c, ws, KC_STRAIN);
-        hipError_t e = launch_strain(N, P, ws);
+        ProfScope ps(&c, s, KC_STRAIN);
+        hipError_t e = launch_strain(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "strain pass launch");
     }
     if (accel_pass && sph && !strain_pass) {
-        ProfScope ps(&c, ws, KC_OTHER);
-        hipError_t e = launch_prep(N, P, ws);
+        ProfScope ps(&c, s, KC_OTHER);
+        hipError_t e = launch_prep(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "record pass launch");
     }
-    // With the symmetric sweep, the acceleration pass runs while the far
-    // field is still going and writes the SPH terms alone; the combine then
-    // adds the gravity to them.  Otherwise it adds the SPH terms to the
-    // gravity of the sweep.
-    const bool accel_first = sym && accel_pass && sph;
-    if (accel_first) {
-        N.acc_has_gravity = false;
-        ProfScope ps(&c, ws, KC_ACCEL);
-        hipError_t e = launch_accel(N, P, ws);
+    // The acceleration pass adds the SPH terms to the one-sided sweep's
+    // gravity; the symmetric sweep's combine adds its gravity to them.
+    if (accel_pass && sph) {
+        N.acc_has_gravity = grav && !sym;
+        ProfScope ps(&c, s, KC_ACCEL);
+        hipError_t e = launch_accel(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "acceleration pass launch");
     }
     if (accel_pass && (f & GRASPH_VARIABLE_TIMESTEP)) {
         // calcAcceleration::do_after sets nextTS = max_timestep
         // (computeDerivatives.h:305-308): the next integrate(pb, true) takes
         // min(max_timestep, this step's criteria), so dt can grow again.
-        // Enqueued beside the far field when there is one (ws joins s below).
-        hipError_t e = launch_vts_set_next(c.ts, 1, nullptr, P, 1, ws);
+        hipError_t e = launch_vts_set_next(c.ts, 1, nullptr, P, 1, s);
         if (e != hipSuccess) return hip_fail(c, e, "time-step reset launch");
     }
-    if (sym && (r = sym_sweep_end(c, S, P, s, ws, accel_first && grav))) return r;
-    if (accel_pass && sph && !accel_first) {
-        N.acc_has_gravity = grav;
-        ProfScope ps(&c, s, KC_ACCEL);
-        hipError_t e = launch_accel(N, P, s);
-        if (e != hipSuccess) return hip_fail(c, e, "acceleration pass launch");
-    }
+    if (sym) return run_sym_sweep(c, L, P, s, sph);
     return 0;
 }
 
@@ -646,6 +556,10 @@ void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav
         sh.sort_tmp_bytes = reorder_tmp_bytes((int)n);
         sh.sort_tmp = k.take<unsigned char>((int64_t)std::max<size_t>(sh.sort_tmp_bytes, 1));
         sh.bbox = k.take<float>(257 * 6);
+        // the boxes go where the sort's keys were: 32 B per 8 and per 512 slots
+        // in 8 B per slot (below 64 slots: in room of their own)
+        sh.box_cap = 2 * (fine_boxes(n) + coarse_boxes(n));
+        sh.box = n < 64 ? k.take<float4>(sh.box_cap) : reinterpret_cast<float4*>(sh.keys);
         sh.xs = k.take<float4>(n);
         sh.xs_cap = n;
         sh.rec = k.take<SlotRec>(n);
@@ -654,7 +568,7 @@ void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav
             sh.mass_flags_cap = (n + 255) / 256;
             sh.mass_flags = k.take<int>(sh.mass_flags_cap);
         }
-        sh.nbr_cap_n = (n + 63) / 64 * 64 * slices;
+        sh.nbr_cap_n = (n + 63) / 64 * 64;
         sh.nbr_cap_k = sh.max_neighbours;
         sh.nbr = k.take<int>(sh.nbr_cap_n * sh.max_neighbours);
         sh.nbr_cnt = k.take<int>(sh.nbr_cap_n);
@@ -698,7 +612,7 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
     // until the arrays fit
     sh.sweep_slices = c.sweep_slices;
     int slices = 1, len = (int)n;
-    if (grav || lists) choose_slices(sh, n, sh.sweep_ni, &slices, &len);
+    if (grav) choose_slices(sh, n, sh.sweep_ni, &slices, &len);
     size_t need = 0;
     for (;;) {
         Carve m{nullptr, 0};
@@ -840,7 +754,7 @@ int grasph_destroy(grasph_ctx* ctx)
     c.batch = nullptr;
     void* bufs[] = {c.perm, c.keys,   c.keys_alt, c.vals, c.sort_tmp, c.bbox,
                     c.nbr,  c.nbr_cnt, c.rec,     c.pot,  c.red,      c.part, c.ts, c.umass,
-                    c.xs,   c.sym_box, c.sym_bits, c.sym_near, c.sym_apart, c.sym_bpart, c.sym_accsum, c.mass_flags};
+                    c.xs,   c.box, c.sym_near, c.sym_apart, c.sym_bpart, c.sym_accsum, c.mass_flags};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (auto& ev : c.ev_pending) {
@@ -848,12 +762,8 @@ int grasph_destroy(grasph_ctx* ctx)
         (void)hipEventDestroy(ev.b);
     }
     for (auto e : c.ev_free) (void)hipEventDestroy(e);
-    if (c.ev_fork) (void)hipEventDestroy(c.ev_fork);
-    if (c.ev_join) (void)hipEventDestroy(c.ev_join);
-    if (c.list_max_ev) (void)hipEventDestroy(c.list_max_ev);
     if (c.list_max_dev) (void)hipFree(c.list_max_dev);
     if (c.list_max_host) (void)hipHostFree(c.list_max_host);
-    if (c.side) (void)hipStreamDestroy(c.side);
     delete ctx;
     return 0;
 }
@@ -1097,25 +1007,17 @@ int grasph_get_neighbour_stats(grasph_ctx* ctx, int64_t* pairs, int32_t* max_cou
     if (max_count) *max_count = 0;
     if (overflowed) *overflowed = 0;
     if (!c.nbr_cnt || c.last_list_n <= 0) return 0;
-    const size_t n = (size_t)c.last_list_n, S = (size_t)c.last_list_slices;
-    std::vector<int> cnt(n * S);
+    const size_t n = (size_t)c.last_list_n;
+    std::vector<int> cnt(n);
     hipError_t e = hipDeviceSynchronize();
-    if (e == hipSuccess)
-        e = hipMemcpy(cnt.data(), c.nbr_cnt, cnt.size() * sizeof(int), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(cnt.data(), c.nbr_cnt, n * sizeof(int), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return grasph::hip_fail(c, e, "neighbour counts copy");
     int64_t tot = 0, over = 0;
     int32_t mx = 0;
-    for (size_t t = 0; t < n; ++t) {
-        int sum = 0;
-        bool o = false;
-        for (size_t s = 0; s < S; ++s) {
-            const int v = cnt[s * n + t];
-            sum += v;
-            o = o || v > c.max_neighbours;
-        }
-        tot += sum;
-        if (sum > mx) mx = sum;
-        if (o) ++over;
+    for (const int v : cnt) {
+        tot += v;
+        mx = std::max<int32_t>(mx, v);
+        over += v > c.max_neighbours;
     }
     if (pairs) *pairs = tot;
     if (max_count) *max_count = mx;

@@ -43,14 +43,12 @@ struct Ctx {
     // options
     int max_neighbours = 160;      // list capacity of this context's single-instance evaluations (grows)
     int max_neighbours_set = 160;  // the capacity last set: batches and their launch-loop contexts start from it
-    // grow max_neighbours after an evaluation whose lists overflowed: its
-    // largest count is reduced on the device and copied to pinned host
-    // memory; a later call reads it once the copy has landed (no wait)
+    // grow max_neighbours after an evaluation whose lists overflowed: the
+    // list kernel stores its largest count in pinned host memory, and a later
+    // call reads what has landed there (no wait)
     int max_neighbours_grow = 1;
-    int* list_max_dev = nullptr;
+    int* list_max_dev = nullptr;   // of the evaluation under way (the gather clears it)
     int* list_max_host = nullptr;
-    hipEvent_t list_max_ev = nullptr;
-    bool list_max_pending = false;
     int reorder_interval = 8;  // particles move little in 8 steps: the order only affects speed
     int sweep_ni = 1;  // i particles per lane in the single-instance sweep
     int sweep_slices = 0;  // j-split of the single-instance sweep (0: chosen from the occupancy)
@@ -90,21 +88,17 @@ struct Ctx {
     float* bbox = nullptr;  // [nblocks][6] partial bounds then final [6]
     int64_t reorder_cap = 0;
 
-    // neighbour lists: one plane per slice (list_plane entries; entry k of
-    // slot t at list_entry(t, k, kmax)), counts nbr_cnt[plane * n + slot]
+    // neighbour lists: entry k of slot t at list_entry(t, k, kmax), counts nbr_cnt[slot]
     int* nbr = nullptr;
     int* nbr_cnt = nullptr;
     int64_t nbr_cap_n = 0;
     int nbr_cap_k = 0;
+    float4* box = nullptr;  // the lists' boxes: fine, then coarse
+    int64_t box_cap = 0;
     int64_t last_list_n = 0;  // particles of the last neighbour list built
-    int last_list_slices = 1;
     float4* part = nullptr;   // partial sums of a j-split sweep
     int64_t part_cap = 0;
     // work arrays of the symmetric sweep
-    float4* sym_box = nullptr;
-    int64_t sym_box_cap = 0;
-    uint32_t* sym_bits = nullptr;
-    int64_t sym_bits_cap = 0;
     float4* sym_near = nullptr;
     int64_t sym_near_cap = 0;
     float4* sym_apart = nullptr;
@@ -137,12 +131,6 @@ struct Ctx {
     int64_t launches[GRASPH_NKERNEL_CLASSES] = {};
     bool capturing = false;  // no timing events while a graph is being captured
 
-    // beside the symmetric sweep's far field (on the caller's stream), the
-    // rest of the evaluation runs on a second stream (default priority,
-    // non-blocking), forked from and joined to the caller's
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-
     struct BatchState* batch = nullptr;
 
     // The allocation-free entry point runs the derivative path on a
@@ -174,18 +162,14 @@ struct SweepLaunch {
     const int* perm;
     int n;
     float4* acc;        // gravity (written when grav)
-    int* nbr;           // written when want_nbr
-    int* nbr_cnt;
     float* pot;         // written when want_pot
-    int kmax;
-    bool grav, want_nbr, want_pot;
+    bool grav, want_pot;
     bool finish;        // apply environmentAcceleration, zero xvel / maxvsig (SPH off)
     const float4* vel;
     float4* xvel;
     float* maxvsig;
     int ni;             // i particles per lane (1 or 2)
-    int nslices;        // j-split: slices of slice_len j (lists and counts per slice); the
-                        // symmetric sweep: its near field's list shares (planes)
+    int nslices;        // j-split: slices of slice_len j
     int near_shares;    // the symmetric sweep: shares of its in-group gravity
     int slice_len;
     float4* part;       // [nslices][n][2] partial sums when nslices > 1
@@ -193,24 +177,20 @@ struct SweepLaunch {
 };
 hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s);
 
-// The symmetric single-instance sweep (sym_sweep.hip): super-blocks of 256
-// slots, groups of 4 super-blocks; gravity inside a group through the
-// candidate sweep, between groups once per unordered pair; neighbour lists
-// from the blocks of 64 whose boxes come within H.  Sizes of its work
-// arrays, in elements.
+// The symmetric single-instance gravity sweep (sym_sweep.hip): groups of
+// 1024 slots; inside a group one-sided, between groups once per unordered
+// pair.  Sizes of its work arrays, in elements.
 struct SymGeom {
-    int nb, groups, wgs, nwords;
+    int nb, groups, wgs;
     int64_t nsb, units;   // super-blocks; far work units
     int split;            // pieces per partner super-block in a far unit (1, 2 or 4)
-    int64_t box_elems;    // float4: bounding box per block of 64
-    int64_t bits_elems;   // uint32: near-block bit matrix (lists wanted)
     int64_t near_elems;   // float4: near-field partial per slot and share
     int64_t apart_elems;  // float4: far own-side fragments (kFragElems each)
     bool plain;           // no far workgroup flushes a fragment twice: no correction planes
     int64_t bpart_elems;  // float: far partner-side partials (of the widest column batch)
     int ncols;            // column batches of the far field (1: the whole far field at once)
 };
-SymGeom sym_geometry(int64_t n, int wgs, bool want_nbr, int nshares, int64_t col_elems = INT64_MAX);
+SymGeom sym_geometry(int64_t n, int wgs, int nshares, int64_t col_elems = INT64_MAX);
 // one column batch [c0, c1) of the far field's partner groups
 struct SymCol {
     int c0, c1;
@@ -224,34 +204,24 @@ struct SymLaunch {
     const float4* xs;   // slot-ordered positions + masses
     const int* perm;    // slot -> particle, or null
     int n;
-    bool grav, want_nbr;
+    bool grav;
     bool finish;        // as SweepLaunch::finish
     bool add_acc;       // acc already holds the SPH terms: the combine adds the gravity to them
-    bool far_done;      // the far field is already enqueued (beside what follows)
-    bool list_prio;     // the lists' wavefronts take issue priority over the far field's beside them
-    int list_shares;    // its list kernel cut into this many shares (own list planes, merged after)
-    int nshares;        // near field cut into this many shares per block (own list planes, merged after)
+    int nshares;        // in-group gravity cut into this many shares per block of 64 slots
     float4* acc;
-    int* nbr;           // a list per slot and share
-    int* nbr_cnt;
-    int kmax;
     const float4* vel;
     float4* xvel;
     float* maxvsig;
     const float* umass; // {uniform, mass} (grav)
     int wgs;            // workgroups of the far kernel
-    float4* box;
-    uint32_t* bits;
     float4* near_part;
     float4* apart;        // own-side fragments (kFragElems each)
     float* bpart;
     int64_t col_elems;    // partner-side partials (floats) a column batch of the far field may take
     float4* accsum;       // running sums between column batches: 2 float4 per slot (column-batched far field)
 };
-// the symmetric sweep in four launches: the near field's lists and its
-// in-group gravity, the far field (no dependence among them: they may run
-// on two streams), then the combine
-hipError_t launch_sym_lists(const SymLaunch& L, const DevParams& P, hipStream_t s);
+// the symmetric sweep in three launches: the in-group gravity, the far
+// field, then the combine
 hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_t s);
 hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s);
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s);
@@ -261,10 +231,9 @@ bool sym_has_far(const SymLaunch& L);
 struct BatchInst;
 struct SymInst {
     int off, n;         // slots [off, off + n)
-    int nb, nwords;     // blocks of 64; words per near-bit row
-    int nsb, nrows;     // super-blocks; far rows (groups with later super-blocks)
-    int box0, row0;     // its first block box and first far row in the batch's arrays
-    int64_t bits0;      // first word of its near-bit matrix
+    int nb;             // blocks of 64
+    int nsb, nrows;     // groups; far rows (groups with later ones)
+    int row0;           // its first far row in the batch's arrays
     int64_t bpart0;     // first float of its partner-side partials
 };
 struct SymRow {
@@ -274,57 +243,66 @@ struct SymBatchTables {
     std::vector<SymInst> insts;  // every instance; those below min_n have n = 0
     std::vector<SymRow> rows;    // longest first
     std::vector<int4> blk;       // 256-slot blocks (instance, first, end) of the instances in the sweep
-    int max_words = 0;
-    int64_t box_elems = 0, bits_elems = 0, apart_elems = 0, bpart_elems = 0;
+    int64_t apart_elems = 0, bpart_elems = 0;
     bool plain = true;  // no row piece flushes its fragment twice
 };
 // instances of at least min_n particles take the symmetric sweep
-SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, bool want_nbr, int64_t min_n);
+SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n);
 struct SymBatchLaunch {
     const float4* xs;     // slot-ordered positions + masses of the batch
     const int* perm;      // slot -> particle, or null
     int ntotal, n_inst;
-    bool grav, want_nbr, finish, soft;
+    bool grav, finish, soft;
     bool add_acc;         // acc already holds the SPH terms: the combine adds the gravity to them
     const SymInst* sinst;
     const BatchInst* insts;
     const DevParams* prm;
     const int4* blk;      // 256-slot blocks of the instances in the sweep
     int n_blk;
-    const int* inst_of;
     const SymRow* rows;
     int nrows;
-    int max_words;
     int* queue;           // one work counter
     int wgs;
     bool plain;           // SymBatchTables::plain
-    bool ingroup_done;    // the in-group gravity was enqueued after the far field on its stream
     const float* umass;   // {uniform, mass} per instance
     float4* acc;
-    int* nbr;
-    int* nbr_cnt;
-    int kmax;
     const float4* vel;
     float4* xvel;
     float* maxvsig;
-    float4* box;
-    uint32_t* bits;
     float4* near_part;
     float4* apart;        // own-side fragments (kFragElems each)
     float* bpart;
 };
-// the batched symmetric sweep in four launches, as the single-instance one
-hipError_t launch_sym_batch_lists(const SymBatchLaunch& L, hipStream_t s);
+// the batched symmetric sweep in three launches, as the single-instance one
 hipError_t launch_sym_batch_ingroup(const SymBatchLaunch& L, hipStream_t s);
 hipError_t launch_sym_batch_far(const SymBatchLaunch& L, hipStream_t s);
 hipError_t launch_sym_batch_combine(const SymBatchLaunch& L, hipStream_t s);
 inline bool sym_batch_has_far(const SymBatchLaunch& L) { return L.ntotal > 0 && L.n_blk > 0 && L.grav && L.nrows > 0; }
 
-// Fold the per-slice lists of a j-split sweep into one list per particle
-// (slice 0's arrays; a count above kmax means "scan the instance").
-hipError_t launch_merge_lists(int* nbr, int* cnt, int n, int kmax, int nslices, hipStream_t s);
-// out[0] = the largest of cnt[0, n) (one workgroup)
-hipError_t launch_count_max(const int* cnt, int n, int* out, hipStream_t s);
+// Neighbour lists (lists.hip): bounding boxes of every kBoxFine and every
+// kBoxCoarse consecutive slots of an instance, two float4 (lo, hi) each, then
+// one list per slot.
+constexpr int kBoxFine = 8, kBoxCoarse = 512;
+inline int64_t fine_boxes(int64_t n) { return (n + kBoxFine - 1) / kBoxFine; }
+inline int64_t coarse_boxes(int64_t n) { return (n + kBoxCoarse - 1) / kBoxCoarse; }
+struct BatchInst;
+struct ListLaunch {
+    const float4* xs;  // slot-ordered positions
+    int n;
+    float H2;          // one instance
+    float4* fine;      // boxes: one instance's come from the gather, a batch's are made here
+    float4* coarse;
+    int* nbr;
+    int* nbr_cnt;
+    int kmax;
+    int* max_dev;      // largest count of an overflowed list: of this evaluation (0 before it), and
+    int* max_host;     // the host's copy; null: not reported
+    const int4* blk;   // batch: 256-slot blocks of all instances
+    int n_blk;
+    const BatchInst* insts;
+};
+hipError_t launch_lists(const ListLaunch& L, hipStream_t s);
+hipError_t launch_batch_lists(const ListLaunch& L, hipStream_t s);
 
 // Per-slot record of the neighbour passes (64 bytes, slot order): position
 // and mass; velocity and density; the acceleration pass's j-side terms
@@ -338,7 +316,7 @@ struct BatchInst {
     int off;     // first particle
     int n;       // particle count
     float H2;    // smoothing length squared
-    float cand;  // neighbour-candidate threshold on r^2 + H^2
+    int fine0, coarse0;  // its first fine and coarse box in the batch's arrays
 };
 
 // Block descriptors of the per-particle passes over a batch: block b covers
@@ -396,6 +374,45 @@ __device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_bl
     return m;
 }
 
+// The boxes of the kBoxCoarse slots first + threadIdx.x of an instance of n
+// (a workgroup of as many threads; p: this thread's slot, act: below n) into
+// the instance's fine and coarse arrays.
+__device__ inline void block_boxes(const float4 p, const bool act, const int first, const int n,
+                                   float4* __restrict__ fine, float4* __restrict__ coarse)
+{
+    constexpr int kWaves = kBoxCoarse / 64;
+    __shared__ float red[6][kWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float v[6] = {act ? p.x : INFINITY,  act ? p.y : INFINITY,  act ? p.z : INFINITY,
+                  act ? p.x : -INFINITY, act ? p.y : -INFINITY, act ? p.z : -INFINITY};
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            v[c] = fminf(v[c], __shfl_xor(v[c], o, 64));
+            v[c + 3] = fmaxf(v[c + 3], __shfl_xor(v[c + 3], o, 64));
+        }
+        if (o == kBoxFine / 2 && (lane & (kBoxFine - 1)) == 0 && act) {
+            const int f = (first + (int)threadIdx.x) / kBoxFine;
+            fine[2 * f] = make_float4(v[0], v[1], v[2], 0.0f);
+            fine[2 * f + 1] = make_float4(v[3], v[4], v[5], 0.0f);
+        }
+    }
+    if (lane == 0)
+#pragma unroll
+        for (int c = 0; c < 6; ++c) red[c][wave] = v[c];
+    __syncthreads();  // every thread of the workgroup gets here
+    if (threadIdx.x == 0 && first < n) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            v[c] = red[c][0];
+            for (int w = 1; w < kWaves; ++w) v[c] = c < 3 ? fminf(v[c], red[c][w]) : fmaxf(v[c], red[c][w]);
+        }
+        coarse[2 * (first / kBoxCoarse)] = make_float4(v[0], v[1], v[2], 0.0f);
+        coarse[2 * (first / kBoxCoarse) + 1] = make_float4(v[3], v[4], v[5], 0.0f);
+    }
+}
+
 struct BatchSweepLaunch {
     const float4* xs;   // particles in slot order (posm itself when perm is null)
     const int* perm;
@@ -404,14 +421,10 @@ struct BatchSweepLaunch {
     const BatchInst* insts;
     int* queue;         // work counter, zero before the launch
     float4* acc;
-    int* nbr;
-    int* nbr_cnt;
-    int ntotal;
-    int kmax;
     int blocks;           // persistent grid
     int waves_per_block;  // 1, 2 or 4
-    bool grav, want_nbr, soft;
-    const float* umass;   // {uniform, mass} per instance, or null
+    bool soft;
+    const float* umass;   // {uniform, mass} per instance
     int ni_max;           // largest ni of the items (1 or 2)
 };
 hipError_t launch_batch_sweep(const BatchSweepLaunch& L, const DevParams& P, hipStream_t s);
@@ -528,10 +541,13 @@ hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s);
 // Slot-ordered copies for the sweep and the list passes (perm null: the
 // identity): xs[t] = posm[perm[t]] when xs is given, and the slot records'
 // position/mass and velocity/density (vel or density null: zeros there).
-// slot-ordered copies; with mass_flags (one int per 256 slots) also the
-// per-block half of the equal-mass check, which launch_mass_final completes
+// With mass_flags (one int per kGatherBlock slots) also the per-block half of
+// the equal-mass check, which launch_mass_final completes; with fine and
+// coarse the lists' boxes (one instance), and list_max cleared.
+constexpr int kGatherBlock = kBoxCoarse;
 hipError_t launch_gather(const int* perm, int n, const float4* posm, const float4* vel, const float* density,
-                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags = nullptr);
+                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags = nullptr,
+                         float4* fine = nullptr, float4* coarse = nullptr, int* list_max = nullptr);
 hipError_t launch_mass_final(const float4* posm, const int* mass_flags, int nflags, float* umass, hipStream_t s);
 
 // environmentAcceleration and the zero XVEL / MAXVSIG stores of

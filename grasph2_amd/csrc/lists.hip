@@ -1,0 +1,227 @@
+// lists.hip -- the neighbour lists (0 < r^2 <= H^2, src/computeDerivatives.h
+// :72,122,238) that the passes of nbr_passes.hip walk (gfx950).
+//
+// Boxes: every 8 consecutive slots of an instance have a bounding box, and
+// every 512 slots one.  In slot (Morton) order these are small, and a box
+// farther than H from a particle holds none of its neighbours: the box gaps
+// and their squared sum round like the exact pair distance (rounding is
+// monotonic), so they never exceed it.
+//
+// One wavefront makes the lists of 8 slots.  Lane l tests box l of 64 boxes
+// of 512 against the 8 slots' own box, then lane l box l of the 64 boxes of 8
+// in each that is near; every near one is 8 partners j, and lane l = 8 i + j
+// takes the pair (i, j).  The 64 lanes' hits in one ballot give slot i its
+// partners as a byte in slot order, so a partner's place in the list is the
+// count so far plus the bits below it: the lists come out in increasing slot
+// order, complete and one to a slot, whatever the launch shape.
+//
+// What bounds it: the vector issue, ~25 instructions per 64 pairs.  A box of
+// 8 slots meets ~70 boxes within H = 2.5 spacings, so a slot is tested
+// against ~560 partners for its ~65 neighbours; blocks of 64 slots against
+// blocks of 64 partners, one slot per lane, tested ~1900 and appended lane by
+// lane in branches.  Partners are read into vector registers (the 8 rows of
+// lanes share a 128-byte line): a scalar operand would halve the issue rate
+// (far_rotation.hpp).  Measured: N = 131072 collision 115 us, where blocks of
+// 64 with their shares, merge and count maximum took 300; 20011 particles
+// 50 us instead of 135; 65536 squeezed ones (430 partners each) 253
+// instead of 640.
+#include "internal.hpp"
+
+namespace grasph {
+namespace {
+
+constexpr int kBoxThreads = kBoxCoarse;  // slots of a coarse box: one workgroup
+constexpr int kTile = 64;                // slots per workgroup of the list kernel
+constexpr int kListThreads = 8 * kTile;
+constexpr int kBoxList = 384;            // near fine boxes a wavefront collects before it tests them
+constexpr int kAhead = 4;                // boxes' partners in flight
+
+// whether two boxes come within H of each other
+__device__ __forceinline__ bool boxes_near(const float4 lo, const float4 hi, const float4 l2, const float4 h2,
+                                           const float H2)
+{
+    const float gx = fmaxf(0.0f, fmaxf(l2.x - hi.x, lo.x - h2.x));
+    const float gy = fmaxf(0.0f, fmaxf(l2.y - hi.y, lo.y - h2.y));
+    const float gz = fmaxf(0.0f, fmaxf(l2.z - hi.z, lo.z - h2.z));
+    return dist2_exact(gx, gy, gz) <= H2;
+}
+
+__device__ __forceinline__ float lane_value(const float v, const int lane)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// boxes of a batch: block b of the 256-slot block table makes the coarse box
+// its instance-relative slots begin, if they begin one
+__global__ __launch_bounds__(kBoxThreads) void batch_box_kernel(const float4* __restrict__ xs,
+                                                                const int4* __restrict__ blk,
+                                                                const BatchInst* __restrict__ insts,
+                                                                float4* __restrict__ fine, float4* __restrict__ coarse)
+{
+    const int4 bl = blk[blockIdx.x];
+    const BatchInst I = insts[bl.x];
+    const int first = bl.y - I.off;
+    if (first % kBoxCoarse) return;  // the whole workgroup leaves
+    const int t = first + (int)threadIdx.x;
+    const bool act = t < I.n;
+    const float4 p = act ? xs[I.off + t] : make_float4(0.f, 0.f, 0.f, 0.f);
+    block_boxes(p, act, first, I.n, fine + 2 * (size_t)I.fine0, coarse + 2 * (size_t)I.coarse0);
+}
+
+template <bool BATCH>
+__global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __restrict__ xs, const int n0,
+                                                            const float4* __restrict__ fine0,
+                                                            const float4* __restrict__ coarse0,
+                                                            int* __restrict__ nbr, int* __restrict__ nbr_cnt,
+                                                            const int kmax, const float h2,
+                                                            const int4* __restrict__ blk,
+                                                            const BatchInst* __restrict__ insts,
+                                                            int* __restrict__ max_dev, int* __restrict__ max_host)
+{
+    __shared__ int boxes[kTile / kBoxFine][kBoxList];  // one wavefront's row is its own: no barrier
+    // XCD-contiguous (xcd_block): neighbouring tiles read the same partners
+    const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    int off = 0, n = n0, first;  // the instance's slots [off, off + n); this wavefront's 8, instance-relative
+    float H2 = h2;
+    const float4 *fine = fine0, *coarse = coarse0;
+    if (BATCH) {
+        const int4 bl = blk[tile / 4];  // 256 slots: four tiles
+        const BatchInst I = insts[bl.x];
+        off = I.off;
+        n = I.n;
+        H2 = I.H2;
+        fine += 2 * (size_t)I.fine0;
+        coarse += 2 * (size_t)I.coarse0;
+        first = bl.y - off + kTile * (tile % 4) + kBoxFine * wave;
+    } else {
+        first = kTile * tile + kBoxFine * wave;
+    }
+    if (first >= n) return;  // whole wavefronts leave
+    int* const box = boxes[wave];
+    const int i = lane >> 3, j = lane & 7;
+    const int t = first + i;
+    float xi = __int_as_float(0x7fc00000), yi = xi, zi = xi;  // NaN: a slot past the end hits nothing
+    if (t < n) {
+        const float4 p = xs[off + t];
+        xi = p.x; yi = p.y; zi = p.z;
+    }
+    const int nf = (n + kBoxFine - 1) / kBoxFine, nc = (n + kBoxCoarse - 1) / kBoxCoarse;
+    const float4 lo = fine[2 * (first / kBoxFine)], hi = fine[2 * (first / kBoxFine) + 1];
+    // eight slots that span a jump of the slot order have a box that says
+    // little: there (wider than H^2's reach both ways) the boxes are tested
+    // against the particles one by one (without it one such wavefront tested
+    // every particle: N = 200003, 1736 us instead of 207)
+    const float wide = fmaxf(hi.x - lo.x, fmaxf(hi.y - lo.y, hi.z - lo.z));
+    const bool jump = __builtin_amdgcn_readfirstlane(wide * wide > 4.0f * H2);
+    const int own = min(kBoxFine, n - first);
+    auto near = [&](const float4 l2, const float4 h2) -> bool {
+        if (!jump) return boxes_near(lo, hi, l2, h2, H2);
+        bool any = false;
+        for (int q = 0; q < own; ++q) {
+            const float x = lane_value(xi, 8 * q), y = lane_value(yi, 8 * q), z = lane_value(zi, 8 * q);
+            const float4 p = make_float4(x, y, z, 0.0f);
+            any = any || boxes_near(p, p, l2, h2, H2);
+        }
+        return any;
+    };
+    int* const list = nbr + list_entry(off + t, 0, kmax);
+    const uint32_t bit = 1u << j, below = bit - 1u;
+    const int shift = 8 * (i & 3);
+    // the instance's last fine box may be short: its bits, the same in every byte
+    const uint64_t tail = n % kBoxFine ? 0x0101010101010101ull * ((1u << (n % kBoxFine)) - 1u) : ~0ull;
+    const float4* const xj = xs + off;
+    int cnt = 0;
+    // The pairs of this wavefront's slots with the partners of the m boxes in
+    // box[]: kAhead boxes' partners in flight while one is tested.
+    auto test_boxes = [&](const int m) {
+        for (int b0 = 0; b0 < m; b0 += 64) {
+            const int mb = min(64, m - b0);
+            const int mine64 = box[b0 + min(lane, mb - 1)];
+            float3 q[kAhead];
+            int f[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                f[u] = __builtin_amdgcn_readlane(mine64, min(u, mb - 1));
+                q[u] = *reinterpret_cast<const float3*>(xj + min(kBoxFine * f[u] + j, n - 1));
+            }
+            for (int k0 = 0; k0 < mb; k0 += kAhead) {
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {
+                    const int fb = f[u];
+                    const float r2 = dist2_exact(xi - q[u].x, yi - q[u].y, zi - q[u].z);
+                    uint64_t hits = __builtin_amdgcn_ballot_w64(is_neighbour(r2, H2));
+                    f[u] = __builtin_amdgcn_readlane(mine64, min(k0 + u + kAhead, mb - 1));
+                    q[u] = *reinterpret_cast<const float3*>(xj + min(kBoxFine * f[u] + j, n - 1));
+                    if (k0 + u >= mb) hits = 0;
+                    if (fb == nf - 1) hits &= tail;
+                    if (!hits) continue;
+                    const uint32_t half = lane < 32 ? (uint32_t)hits : (uint32_t)(hits >> 32);
+                    const uint32_t mine = (half >> shift) & 0xffu;
+                    const int k = cnt + __builtin_popcount(mine & below);
+                    if ((mine & bit) && k < kmax) list[64 * (size_t)k] = off + kBoxFine * fb + j;
+                    cnt += __builtin_popcount(mine);
+                }
+            }
+        }
+    };
+    int m = 0;  // boxes collected
+    for (int c0 = 0; c0 < nc; c0 += 64) {
+        const int c = min(c0 + lane, nc - 1);
+        uint64_t mc = __builtin_amdgcn_ballot_w64(c0 + lane < nc && near(coarse[2 * c], coarse[2 * c + 1]));
+        while (mc) {
+            // two coarse boxes at a time, their fine boxes' loads in flight together
+            const int f0 = (c0 + __builtin_ctzll(mc)) * (kBoxCoarse / kBoxFine);
+            mc &= mc - 1;
+            const int f1 = mc ? (c0 + __builtin_ctzll(mc)) * (kBoxCoarse / kBoxFine) : nf;  // nf: none
+            mc &= mc - 1;
+            const int fa = min(f0 + lane, nf - 1), fb = min(f1 + lane, nf - 1);
+            const float4 la = fine[2 * fa], ha = fine[2 * fa + 1], lb = fine[2 * fb], hb = fine[2 * fb + 1];
+            const uint64_t ma = __builtin_amdgcn_ballot_w64(f0 + lane < nf && near(la, ha));
+            const uint64_t mb = __builtin_amdgcn_ballot_w64(f1 + lane < nf && near(lb, hb));
+            const uint64_t lower = (1ull << lane) - 1ull;
+            if ((ma >> lane) & 1) box[m + __builtin_popcountll(ma & lower)] = f0 + lane;
+            m += __builtin_popcountll(ma);
+            if ((mb >> lane) & 1) box[m + __builtin_popcountll(mb & lower)] = f1 + lane;
+            m += __builtin_popcountll(mb);
+            if (m > kBoxList - 128) {
+                test_boxes(m);
+                m = 0;
+            }
+        }
+    }
+    test_boxes(m);
+    if (j == 0 && t < n) nbr_cnt[off + t] = cnt;
+    // a list that overflowed reports the largest count: to the device's
+    // maximum of this evaluation, and to the host's when it raises that one
+    // (two wavefronts' host stores may land in either order: the host then
+    // sees the smaller, and the next evaluation's overflow corrects it)
+    if (max_host && __builtin_amdgcn_ballot_w64(t < n && cnt > kmax)) {
+        int m = t < n ? cnt : 0;
+        for (int o = 32; o >= 8; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+        if (lane == 0 && atomicMax(max_dev, m) < m)
+            __hip_atomic_store(max_host, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+}  // namespace
+
+hipError_t launch_lists(const ListLaunch& L, hipStream_t s)
+{
+    if (L.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(list_kernel<false>, dim3((L.n + kTile - 1) / kTile), dim3(kListThreads), 0, s, L.xs, L.n,
+                       L.fine, L.coarse, L.nbr, L.nbr_cnt, L.kmax, L.H2, nullptr, nullptr, L.max_dev, L.max_host);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_lists(const ListLaunch& L, hipStream_t s)
+{
+    if (L.n <= 0 || L.n_blk <= 0) return hipSuccess;
+    hipLaunchKernelGGL(batch_box_kernel, dim3(L.n_blk), dim3(kBoxThreads), 0, s, L.xs, L.blk, L.insts, L.fine,
+                       L.coarse);
+    hipLaunchKernelGGL(list_kernel<true>, dim3(4 * L.n_blk), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
+                       L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk, L.insts, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+}  // namespace grasph

@@ -154,17 +154,19 @@ __global__ __launch_bounds__(kBlock) void batch_keys(const float4* __restrict__ 
 // slot-ordered copies: xs[t] = posm[perm[t]] (when xs is given) and the
 // slot records' {x y z m} and {vx vy vz rho}; with mass_flags, also the
 // first half of the equal-mass check: flag b is set when a mass of block b
-// differs from particle 0's, bit for bit
-__global__ __launch_bounds__(kBlock) void gather_kernel(const int* __restrict__ perm, const int n,
-                                                        const float4* __restrict__ posm, const float4* __restrict__ vel,
-                                                        const float* __restrict__ density, float4* __restrict__ xs,
-                                                        SlotRec* __restrict__ rec, int* __restrict__ mass_flags)
+// differs from particle 0's, bit for bit; with fine, also the lists' boxes
+// (in a kernel of their own they took 5 us at any size)
+__global__ __launch_bounds__(kGatherBlock) void gather_kernel(
+    const int* __restrict__ perm, const int n, const float4* __restrict__ posm, const float4* __restrict__ vel,
+    const float* __restrict__ density, float4* __restrict__ xs, SlotRec* __restrict__ rec,
+    int* __restrict__ mass_flags, float4* __restrict__ fine, float4* __restrict__ coarse, int* __restrict__ list_max)
 {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
+    const int t = blockIdx.x * kGatherBlock + threadIdx.x;
     int bad = 0;
+    float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
     if (t < n) {
         const int i = perm ? perm[t] : t;
-        const float4 p = posm[i];
+        p = posm[i];
         if (xs) xs[t] = p;
         if (rec) {
             const float4 v = vel ? vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -173,21 +175,25 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(const int* __restrict__ 
         }
         if (mass_flags) bad = __float_as_int(p.w) != __float_as_int(posm[0].w);
     }
+    if (list_max && t == 0) *list_max = 0;
     if (mass_flags) {  // uniform: the whole workgroup reaches the barrier
         bad = __syncthreads_or(bad);
         if (threadIdx.x == 0) mass_flags[blockIdx.x] = bad;
     }
+    if (fine) block_boxes(p, t < n, blockIdx.x * kGatherBlock, n, fine, coarse);
 }
 
 }  // namespace
 
 hipError_t launch_gather(const int* perm, int n, const float4* posm, const float4* vel, const float* density,
-                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags)
+                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags, float4* fine, float4* coarse,
+                         int* list_max)
 {
     if (n <= 0) return hipSuccess;
-    if (!posm || (xs && !perm)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(gather_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, perm, n, posm, vel,
-                       density, xs, rec, mass_flags);
+    if (!posm || (xs && !perm) || (fine && !coarse)) return hipErrorInvalidValue;
+    static_assert(kGatherBlock == kBoxCoarse, "a workgroup of the gather makes one coarse box");
+    hipLaunchKernelGGL(gather_kernel, dim3((n + kGatherBlock - 1) / kGatherBlock), dim3(kGatherBlock), 0, s, perm, n,
+                       posm, vel, density, xs, rec, mass_flags, fine, coarse, list_max);
     return hipGetLastError();
 }
 

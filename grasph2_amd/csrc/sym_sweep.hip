@@ -1,17 +1,11 @@
-// sym_sweep.hip -- the single-instance all-pairs sweep evaluated once per
-// unordered pair (gfx950).
+// sym_sweep.hip -- the all-pairs gravity sweep evaluated once per unordered
+// pair (gfx950).
 //
 // Same results as the sweep of sweep.hip (softened gravity of
-// calcAcceleration, src/computeDerivatives.h:229-235, plus the neighbour
-// lists of :72,122,238), organised by groups of 1024 consecutive slots:
-//  - near field, one wavefront per block of 64 slots, partner blocks in
-//    increasing slot order through the candidate sweep of sweep_core.hpp:
-//    the blocks of its own group with gravity, and (when lists are wanted)
-//    every other block whose bounding box comes within H of its own,
-//    distance test only -- every SPH neighbour of a slot lies in such a
-//    block (the box distance, rounded like the pair distance, never exceeds
-//    it), so the lists come out complete and in slot order, exactly as the
-//    one-range sweep writes them;
+// calcAcceleration, src/computeDerivatives.h:229-235), organised by groups
+// of 1024 consecutive slots:
+//  - in-group gravity, one wavefront per block of 64 slots (and share of the
+//    group's partners), one-sided through the pair loop of sweep_core.hpp;
 //  - far field: every pair of slots in different groups is computed once,
 //    for both sides (Newton's third law).  One wavefront owns a group (16
 //    slots per lane).  The later groups' particles come 16 at a time, one
@@ -20,7 +14,7 @@
 //    and each partner's sum travels with it.  Two swaps then add the four
 //    rows, and the values are stored as the (group, partner) partial
 //    straight away;
-//  - a combine kernel adds, per slot and in a fixed order, the near sum,
+//  - a combine kernel adds, per slot and in a fixed order, the in-group sum,
 //    the far own-side fragments and the far partner-side partials
 //    (compensated), then finishes the acceleration as the one-range sweep.
 // Per far pair: 3 sub, 3 FMA for r^2 + H^2, one v_rsq_f32, 2 mul, 3 FMA for
@@ -57,85 +51,21 @@ __device__ __forceinline__ float swap16_sum(float p, float q)
 }
 // ------------------------------------------------------------------ kernels
 
-// Bounding box of every block of 64 slots (one wavefront per block).
-__global__ __launch_bounds__(kBlock) void block_box_kernel(const float4* __restrict__ xs, const int n, const int nb,
-                                                           float4* __restrict__ box)
-{
-    const int blk = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    if (blk >= nb) return;  // whole wavefronts leave together
-    const int t = 64 * blk + lane;
-    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    if (t < n) {
-        const float4 p = xs[t];
-        v[0] = v[3] = p.x; v[1] = v[4] = p.y; v[2] = v[5] = p.z;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v[c] = fminf(v[c], __shfl_xor(v[c], o, 64));
-            v[c + 3] = fmaxf(v[c + 3], __shfl_xor(v[c + 3], o, 64));
-        }
-    }
-    if (lane == 0) {
-        box[2 * blk] = make_float4(v[0], v[1], v[2], 0.0f);
-        box[2 * blk + 1] = make_float4(v[3], v[4], v[5], 0.0f);
-    }
-}
-
-// near[I][J] (bit J % 32 of word I * nwords + J / 32) for blocks of 64:
-// boxes within H.  The per-axis gaps and their squared sum round like the
-// exact pair distance, so a pair with r^2 <= H^2 never sits in two blocks
-// whose box distance exceeds H^2.  Symmetric by construction.
-__global__ __launch_bounds__(kBlock) void near_bits_kernel(const float4* __restrict__ box, const int nb,
-                                                           const int nwords, const float H2,
-                                                           uint32_t* __restrict__ bits)
-{
-    const int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= (int64_t)nb * nwords) return;
-    const int I = (int)(idx / nwords), w = (int)(idx - (int64_t)I * nwords);
-    const float4 lo = box[2 * I], hi = box[2 * I + 1];
-    uint32_t word = 0;
-    for (int b = 0; b < 32; ++b) {
-        const int J = 32 * w + b;
-        if (J >= nb) break;
-        const float4 l2 = box[2 * J], h2 = box[2 * J + 1];
-        const float gx = fmaxf(0.0f, fmaxf(l2.x - hi.x, lo.x - h2.x));
-        const float gy = fmaxf(0.0f, fmaxf(l2.y - hi.y, lo.y - h2.y));
-        const float gz = fmaxf(0.0f, fmaxf(l2.z - hi.z, lo.z - h2.z));
-        if (dist2_exact(gx, gy, gz) <= H2) word |= 1u << b;
-    }
-    bits[idx] = word;
-}
-
-// Near field of the 64 slots of block I of the instance whose slots are
-// [base, base + n), share `sl` of `ns`: the partner
-// blocks are the blocks of its group (gravity, and the distance test when
-// lists are wanted) and, with bits, the other blocks near it (distance test
-// only); in increasing order they are cut into ns runs of equal count, and
-// this wavefront takes run sl.  A block of the distance test only is swept
-// only if some slot of block I comes within H of its box (box: the
-// instance's block boxes): the point-to-box gaps and their squared sum
-// round like the exact pair distance (lo <= x <= hi, rounding is monotonic),
-// so they never exceed the distance to a particle in the box, and a skipped
-// block holds no neighbour.  Blocks whose own box is large (a jump of the
-// slot order) skip most of their box neighbours this way.  Writes the slot's compensated gravity
-// partial (slot-indexed, two float4) and its list and count -- all in the
-// planes of share sl, which later fold in share order.
-template <bool GRAV, bool NBR, bool SOFT, bool UM>
-__device__ __forceinline__ void near_blocks(const float4* __restrict__ xs, const int base, const int n, const int nb,
-                                            const int nwords, const uint32_t* __restrict__ bits,
-                                            const float4* __restrict__ box, const int I,
-                                            const int sl, const int ns, const int lane, int* __restrict__ nbr_cnt,
-                                            float4* __restrict__ near_part, const DevParams& P, const Rare& R,
-                                            const float m)
+// In-group gravity of the 64 slots of block I of the instance whose slots are
+// [base, base + n), share `sl` of `ns`: the blocks of its group are cut into
+// ns runs of equal count, and this wavefront takes run sl.  Writes the slot's
+// compensated gravity partial (slot-indexed, two float4) in the plane of
+// share sl; the combine folds the planes in share order.
+template <bool SOFT, bool UM>
+__device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, const int base, const int n, const int nb,
+                                              const int I, const int sl, const int ns, const int lane,
+                                              float4* __restrict__ near_part, const float H2, const float m)
 {
     constexpr int kGroupBlocks = kGroup / 64;  // 16
     const int t = base + 64 * I + lane;  // slots of the instance: [base, base + n)
     const bool act = 64 * I + lane < n;
     float xi[1], yi[1], zi[1];
-    xi[0] = yi[0] = zi[0] = __int_as_float(0x7fc00000);  // NaN: inactive slots never branch
+    xi[0] = yi[0] = zi[0] = 0.0f;
     if (act) {
         const float4 p = xs[t];
         xi[0] = p.x; yi[0] = p.y; zi[0] = p.z;
@@ -143,105 +73,29 @@ __device__ __forceinline__ void near_blocks(const float4* __restrict__ xs, const
     Acc<1> a;
     a.ax[0] = a.ay[0] = a.az[0] = a.phi[0] = 0.0f;
     a.sx[0] = a.sy[0] = a.sz[0] = a.sphi[0] = CSum{0.0f, 0.0f};
-    a.cnt[0] = 0;
-    const int G0 = (I / kGroupBlocks) * kGroupBlocks, G1 = min(nb, G0 + kGroupBlocks);  // own group's blocks
-    const bool use_bits = NBR && bits;
-    const uint32_t* row = use_bits ? bits + (size_t)I * nwords : nullptr;
-    // the own group's blocks lie in one word (groups of 16 blocks are 16-aligned)
-    const int gw = G0 >> 5;
-    const uint32_t gmask = (uint32_t)(((1ull << (G1 - G0)) - 1) << (G0 - 32 * gw));
-    // the row through the constant address space: a uniform address there
-    // becomes a scalar load (a global pointer gives a vector load and a wait
-    // per word)
-    const __attribute__((address_space(4))) uint32_t* crow = (const __attribute__((address_space(4))) uint32_t*)row;
-    auto word_of = [&](int w) -> uint32_t {
-        uint32_t word = use_bits ? crow[w] : 0u;
-        if ((GRAV || !use_bits) && w == gw) word |= gmask;
-        return word;
-    };
-    // the boxes through the constant address space too (scalar loads)
-    const __attribute__((address_space(4))) float* cbox = (const __attribute__((address_space(4))) float*)box;
-    auto lane_near = [&](int J) -> bool {
-        const __attribute__((address_space(4))) float* c = cbox + 8 * J;  // lo.xyzw, hi.xyzw
-        const float gx = fmaxf(0.0f, fmaxf(c[0] - xi[0], xi[0] - c[4]));
-        const float gy = fmaxf(0.0f, fmaxf(c[1] - yi[0], yi[0] - c[5]));
-        const float gz = fmaxf(0.0f, fmaxf(c[2] - zi[0], zi[0] - c[6]));
-        return __builtin_amdgcn_ballot_w64(act && dist2_exact(gx, gy, gz) <= P.H2) != 0;
-    };
-    const int w0 = use_bits ? 0 : gw, w1 = use_bits ? nwords : gw + 1;
-    int total = 0;
-#pragma unroll 8
-    for (int w = w0; w < w1; ++w) total += __builtin_popcount(word_of(w));
-    const int r0 = (int)((int64_t)sl * total / ns), r1 = (int)((int64_t)(sl + 1) * total / ns);
-    // blocks of this share, consecutive ones of one kind (own group or not) swept as one range
-    int rank = 0, run0 = -1, run1 = -1;
-    bool run_grav = false;
-    auto flush = [&]() {
-        if (run0 < 0) return;
-        const int j0 = base + 64 * run0, j1 = base + min(n, 64 * run1);
-        if (GRAV && run_grav)
-            sweep_range<1, GRAV, NBR, false, SOFT, UM>(xs, j0, j1, xi, yi, zi, a, t, P.H2, P.cand, R, m);
-        else
-            sweep_range<1, false, NBR, false, SOFT, UM>(xs, j0, j1, xi, yi, zi, a, t, P.H2, P.cand, R, m);
-        run0 = -1;
-    };
-    for (int w = w0; w < w1 && rank < r1; ++w) {
-        uint32_t word = word_of(w);
-        const int c = __builtin_popcount(word);
-        if (rank + c <= r0) {
-            rank += c;
-            continue;
-        }
-        while (word && rank < r1) {
-            const int J = 32 * w + __builtin_ctz(word);
-            word &= word - 1;
-            if (rank++ < r0) continue;
-            const bool g = J >= G0 && J < G1;
-            if (use_bits && !(GRAV && g) && !lane_near(J)) continue;
-            if (run0 >= 0 && (J != run1 || g != run_grav)) flush();
-            if (run0 < 0) {
-                run0 = J;
-                run_grav = g;
-            }
-            run1 = J + 1;
-        }
-    }
-    flush();
+    const int G0 = (I / kGroupBlocks) * kGroupBlocks, total = min(nb, G0 + kGroupBlocks) - G0;  // own group's blocks
+    const int r0 = G0 + sl * total / ns, r1 = G0 + (sl + 1) * total / ns;
+    if (r0 < r1)
+        sweep_range<1, true, false, SOFT, UM>(xs, base + 64 * r0, base + min(n, 64 * r1), xi, yi, zi, a, H2, 0.0f, m);
     if (!act) return;
-    if (GRAV) {
-        near_part[2 * (size_t)t] = make_float4(a.sx[0].s, a.sy[0].s, a.sz[0].s, 0.0f);
-        near_part[2 * (size_t)t + 1] = make_float4(a.sx[0].c, a.sy[0].c, a.sz[0].c, 0.0f);
-    }
-    if (NBR) nbr_cnt[t] = a.cnt[0];
+    near_part[2 * (size_t)t] = make_float4(a.sx[0].s, a.sy[0].s, a.sz[0].s, 0.0f);
+    near_part[2 * (size_t)t + 1] = make_float4(a.sx[0].c, a.sy[0].c, a.sz[0].c, 0.0f);
 }
 
-template <bool GRAV, bool NBR, bool SOFT>
-__global__ __launch_bounds__(kBlock) void near_kernel(const float4* __restrict__ xs, const int n, const int nb,
-                                                      const int nwords, const uint32_t* __restrict__ bits,
-                                                      const float4* __restrict__ box, int* __restrict__ nbr,
-                                                      int* __restrict__ nbr_cnt,
-                                                      const int kmax, float4* __restrict__ near_part,
-                                                      const DevParams P, const float* __restrict__ umass,
-                                                      const int prio)
+template <bool SOFT>
+__global__ __launch_bounds__(kBlock) void ingroup_kernel(const float4* __restrict__ xs, const int n, const int nb,
+                                                         float4* __restrict__ near_part, const float H2,
+                                                         const float* __restrict__ umass)
 {
-    // issue priority over the far field's wavefronts, which run beside this
-    // kernel on the other stream (see the list_prio option of SymLaunch)
-    if (prio) __builtin_amdgcn_s_setprio(3);
     const int I = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kBlock + threadIdx.x) >> 6));
     const int lane = threadIdx.x & 63;
     if (I >= nb) return;
-    // share blockIdx.y of gridDim.y: its list, count and partial planes
-    const int sl = blockIdx.y, ns = gridDim.y;
-    const Rare R = make_rare(nbr + (size_t)sl * list_plane(n, kmax), kmax, P.H2);
-    int* const cnt = nbr_cnt + (size_t)sl * n;
+    const int sl = blockIdx.y, ns = gridDim.y;  // share sl of ns
     float4* const part = near_part + 2 * (size_t)sl * n;
-    if constexpr (GRAV) {
-        if (umass && umass[0] != 0.0f) {
-            near_blocks<GRAV, NBR, SOFT, true>(xs, 0, n, nb, nwords, bits, box, I, sl, ns, lane, cnt, part, P, R, umass[1]);
-            return;
-        }
-    }
-    near_blocks<GRAV, NBR, SOFT, false>(xs, 0, n, nb, nwords, bits, box, I, sl, ns, lane, cnt, part, P, R, 1.0f);
+    if (umass[0] != 0.0f)
+        ingroup_block<SOFT, true>(xs, 0, n, nb, I, sl, ns, lane, part, H2, umass[1]);
+    else
+        ingroup_block<SOFT, false>(xs, 0, n, nb, I, sl, ns, lane, part, H2, 1.0f);
 }
 
 // One chunk of 16 partners (pj: row lane l holds partner l) against the
@@ -718,74 +572,14 @@ __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
 // (instance, group) from a counter, longest first, so each row's own-side
 // sums leave as one fragment, numbered by the instance's first row + g.
 
-// Bounding boxes of the 64-slot blocks of every instance (the batch's
-// 256-slot block table, one wavefront per 64 slots).
-__global__ __launch_bounds__(kBlock) void sym_batch_box_kernel(const float4* __restrict__ xs,
-                                                               const int4* __restrict__ blk,
-                                                               const SymInst* __restrict__ sinst,
-                                                               float4* __restrict__ box)
+template <bool SOFT>
+__global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4* __restrict__ xs,
+                                                                   const int4* __restrict__ blk,
+                                                                   const SymInst* __restrict__ sinst,
+                                                                   const BatchInst* __restrict__ insts,
+                                                                   float4* __restrict__ near_part,
+                                                                   const float* __restrict__ umass)
 {
-    const int4 bl = blk[blockIdx.x];
-    const int lane = threadIdx.x & 63, first = bl.y + 64 * (threadIdx.x >> 6);
-    if (first >= bl.z) return;  // whole wavefronts leave together
-    const SymInst S = sinst[bl.x];
-    const int I = (first - S.off) >> 6, t = first + lane;
-    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    if (t < bl.z) {
-        const float4 p = xs[t];
-        v[0] = v[3] = p.x; v[1] = v[4] = p.y; v[2] = v[5] = p.z;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v[c] = fminf(v[c], __shfl_xor(v[c], o, 64));
-            v[c + 3] = fmaxf(v[c + 3], __shfl_xor(v[c + 3], o, 64));
-        }
-    }
-    if (lane == 0) {
-        box[2 * (size_t)(S.box0 + I)] = make_float4(v[0], v[1], v[2], 0.0f);
-        box[2 * (size_t)(S.box0 + I) + 1] = make_float4(v[3], v[4], v[5], 0.0f);
-    }
-}
-
-// near-block bits of instance blockIdx.y (as near_bits_kernel, per instance)
-__global__ __launch_bounds__(kBlock) void sym_batch_bits_kernel(const float4* __restrict__ box,
-                                                                const SymInst* __restrict__ sinst,
-                                                                const BatchInst* __restrict__ insts,
-                                                                uint32_t* __restrict__ bits)
-{
-    const SymInst S = sinst[blockIdx.y];
-    const int idx = blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= S.nb * S.nwords) return;
-    const float H2 = insts[blockIdx.y].H2;
-    const int I = idx / S.nwords, w = idx - I * S.nwords;
-    const float4* bx = box + 2 * (size_t)S.box0;
-    const float4 lo = bx[2 * I], hi = bx[2 * I + 1];
-    uint32_t word = 0;
-    for (int b = 0; b < 32; ++b) {
-        const int J = 32 * w + b;
-        if (J >= S.nb) break;
-        const float4 l2 = bx[2 * J], h2 = bx[2 * J + 1];
-        const float gx = fmaxf(0.0f, fmaxf(l2.x - hi.x, lo.x - h2.x));
-        const float gy = fmaxf(0.0f, fmaxf(l2.y - hi.y, lo.y - h2.y));
-        const float gz = fmaxf(0.0f, fmaxf(l2.z - hi.z, lo.z - h2.z));
-        if (dist2_exact(gx, gy, gz) <= H2) word |= 1u << b;
-    }
-    bits[S.bits0 + idx] = word;
-}
-
-template <bool GRAV, bool NBR, bool SOFT>
-__global__ __launch_bounds__(kBlock) void sym_batch_near_kernel(
-    const float4* __restrict__ xs, const int4* __restrict__ blk, const SymInst* __restrict__ sinst,
-    const uint32_t* __restrict__ bits, const float4* __restrict__ box, int* __restrict__ nbr,
-    int* __restrict__ nbr_cnt, const int kmax, const int ntotal, float4* __restrict__ near_part,
-    const DevParams* __restrict__ prm, const float* __restrict__ umass)
-{
-    // the lists issue ahead of the far field's wavefronts beside them: the
-    // passes wait for them (ensemble of 512: 16.25-16.30 -> 15.98-16.03 ms
-    // per step, with the passes' own priority)
-    if (NBR) __builtin_amdgcn_s_setprio(3);
     const int4 bl = blk[xcd_block((int)blockIdx.x, (int)gridDim.x)];  // XCD-contiguous (xcd_block)
     const int lane = threadIdx.x & 63;
     const int first = __builtin_amdgcn_readfirstlane(bl.y + 64 * (int)(threadIdx.x >> 6));
@@ -793,19 +587,11 @@ __global__ __launch_bounds__(kBlock) void sym_batch_near_kernel(
     const int k = bl.x;
     const SymInst S = sinst[k];
     const int I = (first - S.off) >> 6;
-    const DevParams P = prm[k];
-    const Rare R = make_rare(nbr, kmax, P.H2);
-    const uint32_t* b = NBR ? bits + S.bits0 : nullptr;
-    const float4* bx = NBR ? box + 2 * (size_t)S.box0 : nullptr;
-    if constexpr (GRAV) {
-        if (umass[2 * k] != 0.0f) {
-            near_blocks<GRAV, NBR, SOFT, true>(xs, S.off, S.n, S.nb, S.nwords, b, bx, I, 0, 1, lane, nbr_cnt, near_part, P,
-                                               R, umass[2 * k + 1]);
-            return;
-        }
-    }
-    near_blocks<GRAV, NBR, SOFT, false>(xs, S.off, S.n, S.nb, S.nwords, b, bx, I, 0, 1, lane, nbr_cnt, near_part, P, R,
-                                        1.0f);
+    const float H2 = insts[k].H2;
+    if (umass[2 * k] != 0.0f)
+        ingroup_block<SOFT, true>(xs, S.off, S.n, S.nb, I, 0, 1, lane, near_part, H2, umass[2 * k + 1]);
+    else
+        ingroup_block<SOFT, false>(xs, S.off, S.n, S.nb, I, 0, 1, lane, near_part, H2, 1.0f);
 }
 
 // one piece of a far row of an instance of the batch: group R.g against
@@ -923,23 +709,6 @@ __global__ __launch_bounds__(kBlock) void sym_batch_combine_kernel(
     acc[i] = make_float4(ax, ay, az, 0.0f);
 }
 
-template <bool GRAV, bool NBR, bool SOFT>
-void launch_batch_near(const SymBatchLaunch& L, hipStream_t s)
-{
-    hipLaunchKernelGGL((sym_batch_near_kernel<GRAV, NBR, SOFT>), dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk,
-                       L.sinst, L.bits, L.box, L.nbr, L.nbr_cnt, L.kmax, L.ntotal, L.near_part, L.prm, L.umass);
-}
-
-template <bool GRAV, bool NBR, bool SOFT>
-void launch_near(const SymLaunch& L, const SymGeom& G, const DevParams& P, hipStream_t s)
-{
-    const int blocks = (G.nb + kBlock / 64 - 1) / (kBlock / 64);
-    hipLaunchKernelGGL((near_kernel<GRAV, NBR, SOFT>), dim3(blocks, L.nshares), dim3(kBlock), 0, s, L.xs, L.n, G.nb,
-                       G.nwords,
-                       L.want_nbr ? L.bits : nullptr, L.want_nbr ? L.box : nullptr, L.nbr, L.nbr_cnt, L.kmax,
-                       L.near_part, P, L.umass, L.list_prio ? 1 : 0);
-}
-
 }  // namespace
 
 int sym_default_workgroups(int cus)
@@ -960,7 +729,7 @@ SymCol sym_column(int64_t nsb, int split, int wanted, int c0, int c1)
     return C;
 }
 
-SymGeom sym_geometry(int64_t n, int wgs, bool want_nbr, int nshares, int64_t col_elems)
+SymGeom sym_geometry(int64_t n, int wgs, int nshares, int64_t col_elems)
 {
     SymGeom G;
     G.nb = (int)((n + 63) / 64);
@@ -969,9 +738,6 @@ SymGeom sym_geometry(int64_t n, int wgs, bool want_nbr, int nshares, int64_t col
     G.split = far_split(n, wgs);
     G.units = row_prefix(rows_with_units(G.nsb), G.nsb, G.split);
     G.wgs = far_workgroups(wgs, G.units);
-    G.nwords = (G.nb + 31) / 32;
-    G.box_elems = 2 * (int64_t)G.nb;
-    G.bits_elems = want_nbr ? (int64_t)G.nb * G.nwords : 0;
     G.near_elems = 2 * n * nshares;
     G.apart_elems = (int64_t)kFragElems * (G.groups + wgs);
     G.plain = fragments_plain((G.units + G.wgs - 1) / G.wgs);
@@ -986,37 +752,21 @@ SymGeom sym_geometry(int64_t n, int wgs, bool want_nbr, int nshares, int64_t col
     return G;
 }
 
-// near field, neighbour lists: boxes, near bits, the distance tests
-hipError_t launch_sym_lists(const SymLaunch& L, const DevParams& P, hipStream_t s)
-{
-    if (L.n <= 0 || !L.want_nbr) return hipSuccess;
-    if (L.list_shares < 1) return hipErrorInvalidValue;
-    SymLaunch M = L;
-    M.nshares = L.list_shares;  // the list kernel's shares (list planes), not the in-group gravity's
-    const SymGeom G = sym_geometry(M.n, M.wgs, M.want_nbr, M.nshares);
-    hipLaunchKernelGGL(block_box_kernel, dim3((G.nb + kBlock / 64 - 1) / (kBlock / 64)), dim3(kBlock), 0, s, L.xs, L.n,
-                       G.nb, L.box);
-    const int64_t words = (int64_t)G.nb * G.nwords;
-    hipLaunchKernelGGL(near_bits_kernel, dim3((unsigned)((words + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, L.box,
-                       G.nb, G.nwords, P.H2, L.bits);
-    if (P.H2 > 0.0f) launch_near<false, true, true>(M, G, P, s); else launch_near<false, true, false>(M, G, P, s);
-    return hipGetLastError();
-}
-
-// near field, gravity inside the groups (the partials of the combine)
+// gravity inside the groups (the partials of the combine)
 hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0 || !L.grav) return hipSuccess;
     if (L.nshares < 1) return hipErrorInvalidValue;
-    SymLaunch M = L;
-    M.want_nbr = false;  // own group only, no bits
-    M.list_prio = false;
-    const SymGeom G = sym_geometry(M.n, M.wgs, false, M.nshares);
-    if (P.H2 > 0.0f) launch_near<true, false, true>(M, G, P, s); else launch_near<true, false, false>(M, G, P, s);
+    const int nb = (L.n + 63) / 64;
+    const dim3 grid((nb + kBlock / 64 - 1) / (kBlock / 64), L.nshares);
+    if (P.H2 > 0.0f)
+        hipLaunchKernelGGL(ingroup_kernel<true>, grid, dim3(kBlock), 0, s, L.xs, L.n, nb, L.near_part, P.H2, L.umass);
+    else
+        hipLaunchKernelGGL(ingroup_kernel<false>, grid, dim3(kBlock), 0, s, L.xs, L.n, nb, L.near_part, P.H2, L.umass);
     return hipGetLastError();
 }
 
-bool sym_has_far(const SymLaunch& L) { return L.n > 0 && L.grav && sym_geometry(L.n, L.wgs, false, 1).units > 0; }
+bool sym_has_far(const SymLaunch& L) { return L.n > 0 && L.grav && sym_geometry(L.n, L.wgs, 1).units > 0; }
 
 template <bool SOFT>
 void launch_far_column(const SymLaunch& L, const SymCol& C, const int split, const DevParams& P, hipStream_t s)
@@ -1040,7 +790,7 @@ void launch_column_combine(const SymLaunch& L, const SymCol& C, const int split,
 hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (!sym_has_far(L)) return hipSuccess;
-    const SymGeom G = sym_geometry(L.n, L.wgs, L.want_nbr, L.nshares, L.col_elems);
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.nshares, L.col_elems);
     if (G.ncols == 1) {
         if (P.H2 > 0.0f)
             hipLaunchKernelGGL((far_kernel<true>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
@@ -1063,7 +813,7 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0 || !(L.grav || L.finish)) return hipSuccess;
-    const SymGeom G = sym_geometry(L.n, L.wgs, L.want_nbr, L.nshares, L.col_elems);
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.nshares, L.col_elems);
     if (G.ncols > 1 && sym_has_far(L)) {
         // the last column batch's combine, which finishes
         const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
@@ -1092,12 +842,12 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
     return hipGetLastError();
 }
 
-SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, bool want_nbr, int64_t min_n)
+SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n)
 {
     SymBatchTables T;
     const int n_inst = (int)offsets.size() - 1;
-    int box0 = 0, row0 = 0;
-    int64_t bits0 = 0, bpart0 = 0;
+    int row0 = 0;
+    int64_t bpart0 = 0;
     for (int k = 0; k < n_inst; ++k) {
         const int64_t n = offsets[k + 1] - offsets[k];
         const bool sym = n >= min_n && n > 0;
@@ -1108,12 +858,9 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, bool want_n
             for (int64_t s = offsets[k]; s < offsets[k + 1]; s += 256)
                 T.blk.push_back(make_int4(k, (int)s, (int)std::min<int64_t>(s + 256, offsets[k + 1]), 0));
         S.nb = (int)((S.n + 63) / 64);
-        S.nwords = (S.nb + 31) / 32;
         S.nsb = (int)((S.n + kSB - 1) / kSB);
         S.nrows = (int)rows_with_units(S.nsb);
-        S.box0 = box0;
         S.row0 = row0;
-        S.bits0 = bits0;
         S.bpart0 = bpart0;
         for (int g = 0; g < S.nrows; ++g) {
             const int64_t u = row_units(g, S.nsb);
@@ -1123,36 +870,25 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, bool want_n
                 T.plain = T.plain && fragments_plain(2 * (int64_t)units);  // two far units per partner group
             }
         }
-        T.max_words = std::max(T.max_words, S.nb * S.nwords);
-        box0 += S.nb;
         row0 += S.nrows;
-        if (want_nbr) bits0 += (int64_t)S.nb * S.nwords;
         bpart0 += 3 * bpart_group_base((S.nsb + kGroupSB - 1) / kGroupSB);
         T.insts.push_back(S);
     }
     std::stable_sort(T.rows.begin(), T.rows.end(), [](const SymRow& a, const SymRow& b) { return a.units > b.units; });
-    T.box_elems = 2 * (int64_t)box0;
-    T.bits_elems = bits0;
     T.apart_elems = (int64_t)kFragElems * kBatchPieces * row0;
     T.bpart_elems = bpart0;
     return T;
 }
 
-hipError_t launch_sym_batch_lists(const SymBatchLaunch& L, hipStream_t s)
-{
-    if (L.ntotal <= 0 || L.n_blk <= 0 || !L.want_nbr) return hipSuccess;
-    hipLaunchKernelGGL(sym_batch_box_kernel, dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk, L.sinst, L.box);
-    if (L.max_words > 0)
-        hipLaunchKernelGGL(sym_batch_bits_kernel, dim3((L.max_words + kBlock - 1) / kBlock, L.n_inst), dim3(kBlock),
-                           0, s, L.box, L.sinst, L.insts, L.bits);
-    if (L.soft) launch_batch_near<false, true, true>(L, s); else launch_batch_near<false, true, false>(L, s);
-    return hipGetLastError();
-}
-
 hipError_t launch_sym_batch_ingroup(const SymBatchLaunch& L, hipStream_t s)
 {
     if (L.ntotal <= 0 || L.n_blk <= 0 || !L.grav) return hipSuccess;
-    if (L.soft) launch_batch_near<true, false, true>(L, s); else launch_batch_near<true, false, false>(L, s);
+    if (L.soft)
+        hipLaunchKernelGGL(sym_batch_ingroup_kernel<true>, dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk, L.sinst,
+                           L.insts, L.near_part, L.umass);
+    else
+        hipLaunchKernelGGL(sym_batch_ingroup_kernel<false>, dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk, L.sinst,
+                           L.insts, L.near_part, L.umass);
     return hipGetLastError();
 }
 

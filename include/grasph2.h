@@ -151,8 +151,8 @@ int grasph_destroy(grasph_ctx* ctx);
  * sums four ways: equal to FP32 rounding), "max_neighbours_grow" (1 = after an
  * single-instance evaluation whose lists overflowed, a later one raises
  * max_neighbours to 1.25 times the largest count seen, in steps of 32, up
- * to 4096 and 16 GiB of lists; the count travels to the host behind an
- * event and is read without waiting, and not during graph capture; the
+ * to 4096 and 16 GiB of lists; the count is stored in host memory by the
+ * list kernel and read without waiting, and not during graph capture; the
  * default; 0 = fixed; batches keep the capacity last set),
  * "reorder_interval"
  * (Morton re-sort every k derivative evaluations, default 8; 0 = never;
@@ -175,11 +175,10 @@ int grasph_destroy(grasph_ctx* ctx);
  * field runs in column batches of partner groups, each with its share of
  * the partials, the running sums kept between batches in 32 B per particle;
  * results agree with the unbatched far field to FP32 rounding),
- * "sym_near_shares" (wavefronts per 64 particles in its near field, 1-16,
- * 0 = chosen from the occupancy), "sym_list_priority" (its near-field list
- * kernel takes issue priority over the far field running beside it: 1 = yes,
- * 0 = no, 2 = below 49152 particles or once max_neighbours has grown past
- * 512, the default), "batch_symmetric" (1 = batches use the
+ * "sym_near_shares" (wavefronts per 64 particles in its in-group gravity, 1-16,
+ * 0 = chosen from the occupancy), "sym_list_priority" (0, 1 or 2: kept for
+ * callers that set it; without effect, as the lists no longer run beside the
+ * far field), "batch_symmetric" (1 = batches use the
  * symmetric sweep for their instances of at least "batch_symmetric_min"
  * particles (default 0), the smaller ones the one-sided persistent sweep,
  * the default; gravity then equals the single-instance path's to FP32
@@ -332,12 +331,10 @@ int grasph_reduce_invariants(grasph_ctx* ctx, const grasph_particles* p,
 /* Per-kernel timing recorded while option "profile" is 1: accumulated
  * milliseconds and launch counts (recorded intervals) per kernel class, in
  * the order sweep, density, strain, accel, integrate, reorder, other, far.
- * "far" is the far-field kernel of the symmetric sweep, which runs on the
- * caller's stream while the near field, the list merge and the SPH passes
- * run beside it on the context's second stream; "sweep" holds the rest of
- * the all-pairs sweep (with the symmetric sweep three intervals per
- * evaluation: near-field lists, in-group gravity, combine).  Synchronises the recorded events.  Resets the counters when
- * reset != 0. */
+ * "far" is the far-field kernel of the symmetric sweep; "sweep" holds the
+ * rest of the all-pairs work (neighbour lists, in-group gravity, combine, or
+ * the one-sided sweep).  Synchronises the recorded events.  Resets the
+ * counters when reset != 0. */
 #define GRASPH_NKERNEL_CLASSES 8
 int grasph_get_kernel_times(grasph_ctx* ctx, double ms[GRASPH_NKERNEL_CLASSES],
                             int64_t launches[GRASPH_NKERNEL_CLASSES], int reset);
