@@ -1,13 +1,18 @@
-// reorder.hip -- Morton (Z-order) ordering of the particles (gfx950).
+// reorder.hip -- Hilbert-curve ordering of the particles (gfx950).
 //
-// The sweep and the neighbour passes map slot t to particle perm[t] and
+// The list kernel and the neighbour passes map slot t to particle perm[t] and
 // read the particles through slot-ordered copies (gather_kernel: positions,
-// velocities, densities).  Along a Z-order curve consecutive slots are
-// spatial neighbours, so the 64 lanes of a wavefront share most of their
-// SPH partners, consecutive j of the sweep are close together (few j chunks
-// hold neighbour candidates), and the list passes' gathers of neighbour data
-// hit the same cache lines.  The order changes the summation order of the
-// (compensated) sums, not which pairs are summed.
+// velocities, densities).  Along a space-filling curve consecutive slots are
+// spatial neighbours, so the 64 lanes of a wavefront share most of their SPH
+// partners, the boxes of consecutive slots are small (lists.hip), and the
+// list passes' gathers of neighbour data hit the same cache lines.  The order
+// changes the summation order of the (compensated) sums, not which pairs are
+// summed.
+//
+// Hilbert's curve, on cubic cells, rather than Morton's on the bounding box's
+// own proportions: it has no jumps inside the particles.  Two spheres of 8192,
+// H = 2.5 spacings: a box of 8 slots comes within H of 51 others instead of
+// 90, and 1.5% of them instead of 10% are longer than 2 H.
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "internal.hpp"
@@ -80,24 +85,65 @@ __device__ inline uint32_t spread10(uint32_t v)
     return v;
 }
 
-__global__ __launch_bounds__(kBlock) void morton_keys(const float4* __restrict__ posm, const int n,
-                                                      const float* __restrict__ box, uint32_t* __restrict__ keys,
-                                                      int* __restrict__ vals)
+// place along the Hilbert curve of a cell of the 1024^3 grid (J. Skilling,
+// "Programming the Hilbert curve", AIP Conf. Proc. 707 (2004) 381: from the
+// axes to the transposed index, whose bits then interleave)
+__device__ inline uint32_t hilbert_index(uint32_t x, uint32_t y, uint32_t z)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float4 p = posm[i];
-    uint32_t q[3];
+    uint32_t c[3] = {x, y, z};
+    for (uint32_t q = 512; q > 1; q >>= 1) {
+        const uint32_t low = q - 1;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint32_t t = (c[0] ^ c[d]) & low;
+            if (c[d] & q) {
+                c[0] ^= low;
+            } else {
+                c[0] ^= t;
+                c[d] ^= t;
+            }
+        }
+    }
+    c[1] ^= c[0];
+    c[2] ^= c[1];
+    uint32_t t = 0;
+    for (uint32_t q = 512; q > 1; q >>= 1)
+        if (c[2] & q) t ^= q - 1;
+    return (spread10(c[0] ^ t) << 2) | (spread10(c[1] ^ t) << 1) | spread10(c[2] ^ t);
+}
+
+// p's place along the curve through the box {lo xyz, hi xyz}.  The cells are
+// cubes of a 1024th of the longest side; across a side less than an eighth of
+// it they are finer (bodies far apart keep their resolution across the line
+// between them).
+__device__ inline uint32_t curve_key(const float4 p, const float* __restrict__ box)
+{
     const float c[3] = {p.x, p.y, p.z};
+    float ext[3], longest = 0.0f;
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const float lo = box[d], hi = box[3 + d];
-        const float ext = hi - lo;
-        float u = (ext > 0.0f) ? (c[d] - lo) / ext : 0.0f;
+        ext[d] = box[3 + d] - box[d];
+        longest = fmaxf(longest, ext[d]);
+    }
+    uint32_t q[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float side = fminf(longest, 8.0f * ext[d]);
+        float u = (side > 0.0f) ? (c[d] - box[d]) / side : 0.0f;
         if (!(u >= 0.0f)) u = 0.0f;  // NaN and negatives
         if (u > 1.0f) u = 1.0f;
         q[d] = (uint32_t)(u * 1023.0f);
     }
-    keys[i] = (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+    return hilbert_index(q[0], q[1], q[2]);
+}
+
+__global__ __launch_bounds__(kBlock) void curve_keys(const float4* __restrict__ posm, const int n,
+                                                     const float* __restrict__ box, uint32_t* __restrict__ keys,
+                                                     int* __restrict__ vals)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    keys[i] = curve_key(posm[i], box);
     vals[i] = i;
 }
 
@@ -136,18 +182,7 @@ __global__ __launch_bounds__(kBlock) void batch_keys(const float4* __restrict__ 
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const int k = inst_of[i];
-    const float4 p = posm[i];
-    const float c[3] = {p.x, p.y, p.z};
-    uint32_t q[3];
-    for (int d = 0; d < 3; ++d) {
-        const float lo = box[6 * k + d], hi = box[6 * k + 3 + d];
-        const float ext = hi - lo;
-        float u = (ext > 0.0f) ? (c[d] - lo) / ext : 0.0f;
-        if (!(u >= 0.0f)) u = 0.0f;
-        if (u > 1.0f) u = 1.0f;
-        q[d] = (uint32_t)(u * 1023.0f);
-    }
-    keys[i] = ((uint64_t)k << 30) | (uint64_t)((spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]));
+    keys[i] = ((uint64_t)k << 30) | (uint64_t)curve_key(posm[i], box + 6 * k);
     vals[i] = i;
 }
 
@@ -233,7 +268,7 @@ hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s)
     static_assert(kBoxBlocks <= kBlock, "bbox_final folds at most one box per thread");
     hipLaunchKernelGGL(bbox_final, dim3(1), dim3(kBlock), 0, s, c.bbox, kBoxBlocks);
     const int blocks = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(morton_keys, dim3(blocks), dim3(kBlock), 0, s, posm, n, c.bbox + kBoxBlocks * 6, c.keys,
+    hipLaunchKernelGGL(curve_keys, dim3(blocks), dim3(kBlock), 0, s, posm, n, c.bbox + kBoxBlocks * 6, c.keys,
                        c.vals);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
