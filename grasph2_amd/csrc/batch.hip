@@ -407,7 +407,6 @@ int batch_lists(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s)
 // the persistent sweep; with a slot order, batch_gather must have run for the current positions
 int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done = false)
 {
-    const DevParams P = make_dev_params(&b.params[0]);
     hipError_t e = launch_reset_queue(b.d_queue, 1, s);
     if (e != hipSuccess) return hip_fail(c, e, "batch work counter reset");
     BatchSweepLaunch L;
@@ -429,7 +428,7 @@ int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStrea
     }
     L.umass = b.d_um;
     ProfScope ps(&c, s, KC_SWEEP);
-    e = launch_batch_sweep(L, P, s);
+    e = launch_batch_sweep(L, s);
     if (e != hipSuccess) return hip_fail(c, e, "batched sweep launch");
     return 0;
 }

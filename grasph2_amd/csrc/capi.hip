@@ -47,25 +47,28 @@ ProfScope::~ProfScope()
     c->ev_pending.push_back(Ctx::Ev{a, b, cls});
 }
 
-// j-split of the single-instance sweep: enough slices for ~16 wavefronts
-// per SIMD (measured: the sweep keeps gaining up to there, as more resident
-// waves hide the scalar-load and rare-path latency), at most 32 slices of
-// at least 512 j each; slice length a multiple of 8.
-void choose_slices(const Ctx& c, int64_t n, int ni, int* slices, int* slice_len)
+// The one-sided sweep's shape: one slot per lane below kOwnFour particles,
+// four from there on (Plummer steps at 6000: 26.9 us with one, 27.4 with
+// four; at 8192: 47 and 31), and as many shares of the partners as give ~16
+// (four slots per lane: 8) wavefronts per compute unit, of 32 partners or
+// more (1000 particles: 28 us with one share per slot block, 14 with 16).
+constexpr int64_t kOwnFour = 6144;
+
+OwnPlan own_plan(const Ctx& c, int64_t n, int slices)
 {
-    int S = c.sweep_slices;
-    if (S <= 0) {
-        const int64_t waves = (n + 64 * ni - 1) / (64 * ni);
-        const int64_t target = 16 * 4 * (int64_t)c.cus;
-        S = (int)std::min<int64_t>(32, std::max<int64_t>(1, (target + waves - 1) / waves));
-        S = (int)std::max<int64_t>(1, std::min<int64_t>(S, n / 512));
+    OwnPlan p;
+    p.ni = c.sweep_ni == 2 ? 2 : n >= kOwnFour ? 4 : 1;
+    const int max_waves = p.ni == 4 ? 8 : 16;  // LDS: the wavefronts' sums in 64 KiB
+    if (slices <= 0) {
+        const int64_t blocks = (n + 64 * p.ni - 1) / (64 * p.ni), target = (p.ni == 4 ? 8 : 16) * (int64_t)c.cus;
+        slices = (int)std::max<int64_t>(1, std::min<int64_t>((target + blocks - 1) / blocks, n / 32));
+        if (slices > max_waves) slices = slices / max_waves * max_waves;  // whole workgroups
+        slices = std::min(slices, 64);
     }
-    int64_t len = (n + S - 1) / S;
-    len = (len + 7) / 8 * 8;
-    if (len < 8) len = 8;
-    *slice_len = (int)len;
-    *slices = (int)((n + len - 1) / len);
-    if (*slices < 1) *slices = 1;
+    p.waves = std::min(slices, max_waves);
+    p.planes = (slices + p.waves - 1) / p.waves;
+    p.len = (int)(((n + p.slices() - 1) / p.slices() + 7) / 8 * 8);
+    return p;
 }
 
 namespace {
@@ -232,7 +235,6 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
     L.vel = (const float4*)p->vel;
     L.xvel = (float4*)p->xvel;
     L.maxvsig = p->maxvsig;
-    L.ni = c.sweep_ni;
     return L;
 }
 
@@ -272,13 +274,12 @@ constexpr int64_t kSymAutoMinGravity = 16384;
 
 int sym_wgs(const Ctx& c) { return c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(c.cus); }
 
-// shares of the symmetric sweep's in-group gravity: ~16 wavefronts per SIMD, at most 16
-int sym_near_shares(const Ctx& c, int64_t n)
+// the power of two at most `shares` (1-16)
+int near_waves_of(int shares)
 {
-    if (c.sym_near_shares > 0) return c.sym_near_shares;
-    const int64_t blocks = (n + 63) / 64;
-    const int64_t target = 16 * 4 * (int64_t)c.cus;
-    return (int)std::min<int64_t>(16, std::max<int64_t>(1, (target + blocks - 1) / blocks));
+    int w = 1;
+    while (2 * w <= shares) w *= 2;
+    return w;
 }
 
 // The symmetric gravity sweep, in order on s: the far field, the in-group
@@ -291,7 +292,7 @@ int sym_near_shares(const Ctx& c, int64_t n)
 int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t s, bool add_acc)
 {
     const int64_t col_elems = c.sym_partial_bytes / (int64_t)sizeof(float);
-    const SymGeom G = sym_geometry(L.n, sym_wgs(c), L.near_shares, col_elems);
+    const SymGeom G = sym_geometry(L.n, sym_wgs(c), col_elems);
     int r;
     if ((r = grow(c, c.sym_near, c.sym_near_cap, G.near_elems, "symmetric sweep near sums")) ||
         (r = grow(c, c.sym_apart, c.sym_apart_cap, G.apart_elems, "symmetric sweep own-side sums")) ||
@@ -307,7 +308,9 @@ int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t 
     S.grav = L.grav;
     S.finish = L.finish;
     S.add_acc = add_acc;
-    S.nshares = L.near_shares;
+    // wavefronts per 64 slots (Plummer steps at 16384: 81.3 us with 4, 77.3
+    // with 8, 77.8 with 16; at 50021: 437 with 1, 416 with 4, 418 with 8)
+    S.near_waves = c.sym_near_shares > 0 ? near_waves_of(c.sym_near_shares) : L.n < 32768 ? 8 : 4;
     S.acc = L.acc;
     S.vel = L.vel;
     S.xvel = L.xvel;
@@ -417,14 +420,16 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     const bool sym = sweep_grav &&
                      (c.sweep_symmetric == 1 ||
                       (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity)));
-    int slices = 1, slice_len = (int)n;
-    if (sweep_grav && !sym) choose_slices(c, n, c.sweep_ni, &slices, &slice_len);
+    const OwnPlan plan = own_plan(c, n, c.sweep_slices);
+    const bool masses = sweep_grav && (sym || n >= kMassCheckMin);  // the equal-mass check
     if (need_list) {
         grow_list_capacity(c, n, s);
         if ((r = ensure_nbr(c, n)) || (r = ensure_list_watch(c, s))) return r;
         c.last_list_n = n;
     }
-    if (slices > 1 && (r = grow(c, c.part, c.part_cap, 2 * n * slices, "sweep partial sums"))) return r;
+    if (sweep_grav && !sym && plan.planes > 1 &&
+        (r = grow(c, c.part, c.part_cap, 2 * n * plan.planes, "sweep partial sums")))
+        return r;
     const DevParams P = make_dev_params(prm);
 
     // slot-ordered positions for the sweep and the passes' slot records
@@ -435,7 +440,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     if (need_list) {
         const bool reads_vel = strain_pass || (accel_pass && sph);
         const bool gdens = reads_vel && !dens_pass;  // else the density pass fills the records' densities
-        mass_flags = sweep_grav;
+        mass_flags = masses;
         if ((perm && (r = grow(c, c.xs, c.xs_cap, n, "slot-ordered positions"))) ||
             (r = grow(c, c.rec, c.rec_cap, n, "slot records")) ||
             (r = grow(c, c.box, c.box_cap, 2 * (fine_boxes(n) + coarse_boxes(n)), "neighbour-search boxes")) ||
@@ -475,11 +480,12 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     L.grav = sweep_grav;
     L.want_pot = false;
     L.finish = accel_pass && !sph;
-    L.nslices = slices;
-    L.near_shares = sym ? sym_near_shares(c, n) : 1;
-    L.slice_len = slice_len;
+    L.ni = plan.ni;
+    L.waves = plan.waves;
+    L.planes = plan.planes;
+    L.slice_len = plan.len;
     L.part = c.part;
-    if (sweep_grav) {
+    if (masses) {
         // equal masses let the sweep factor the mass out of the gravity sum
         ProfScope ps(&c, s, KC_OTHER);
         hipError_t e = mass_flags ? launch_mass_final(L.posm, c.mass_flags, gather_blocks, c.umass, s)
@@ -543,9 +549,9 @@ struct Carve {
 };
 
 // The work arrays computeDerivatives needs on the one-sided sweep with
-// `slices` j-slices, re-sorted every call: cut from `k` into `sh` (its
+// `planes` planes of partial sums, re-sorted every call: cut from `k` into `sh` (its
 // capacities set to exactly what the path asks of grow / ensure_*).
-void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav, int slices)
+void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav, int planes)
 {
     if (lists) {
         sh.perm = k.take<int>(n);
@@ -573,8 +579,8 @@ void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav
         sh.nbr = k.take<int>(sh.nbr_cap_n * sh.max_neighbours);
         sh.nbr_cnt = k.take<int>(sh.nbr_cap_n);
     }
-    if (slices > 1 && grav) {
-        sh.part_cap = 2 * n * slices;
+    if (planes > 1 && grav) {
+        sh.part_cap = 2 * n * planes;
         sh.part = k.take<float4>(sh.part_cap);
     }
 }
@@ -608,19 +614,17 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
     sh.ts = c.ts;
     sh.umass = c.umass;
 
-    // the j-split: as many slices as the allocating path would take, fewer
-    // until the arrays fit
-    sh.sweep_slices = c.sweep_slices;
-    int slices = 1, len = (int)n;
-    if (grav) choose_slices(sh, n, sh.sweep_ni, &slices, &len);
+    // the j-split: as the allocating path would take it, fewer planes until
+    // the arrays fit
+    OwnPlan plan = own_plan(sh, n, c.sweep_slices);
+    if (!grav) plan = own_plan(sh, n, 1);
     size_t need = 0;
     for (;;) {
         Carve m{nullptr, 0};
-        carve_derivative_arrays(sh, m, n, lists, grav, slices);
+        carve_derivative_arrays(sh, m, n, lists, grav, plan.planes);
         need = m.used;
-        if (need <= (size_t)GRASPH_NOALLOC_SCRATCH_BYTES || slices == 1) break;
-        sh.sweep_slices = slices - 1;
-        choose_slices(sh, n, sh.sweep_ni, &slices, &len);
+        if (need <= (size_t)GRASPH_NOALLOC_SCRATCH_BYTES || plan.planes == 1) break;
+        plan = own_plan(sh, n, plan.waves * (plan.planes - 1));
     }
     if (need > (size_t)GRASPH_NOALLOC_SCRATCH_BYTES)
         return fail(c, GRASPH_E_INVALID,
@@ -628,12 +632,12 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
                         std::to_string(need) + " bytes of scratch with these flags and max_neighbours = " +
                         std::to_string(c.max_neighbours) + "; the scratch array holds " +
                         std::to_string((long long)GRASPH_NOALLOC_SCRATCH_BYTES));
-    sh.sweep_slices = slices;
+    sh.sweep_slices = plan.slices();
     Carve k{static_cast<char*>(c.scratch), (size_t)GRASPH_NOALLOC_SCRATCH_BYTES};
-    carve_derivative_arrays(sh, k, n, lists, grav, slices);
+    carve_derivative_arrays(sh, k, n, lists, grav, plan.planes);
     r = derivatives(sh, p, prm, stream, 0);
     if (r) c.err = sh.err;
-    c.noalloc_slices = slices;
+    c.noalloc_slices = plan.slices();
     return r;
 }
 

@@ -168,11 +168,11 @@ struct SweepLaunch {
     const float4* vel;
     float4* xvel;
     float* maxvsig;
-    int ni;             // i particles per lane (1 or 2)
-    int nslices;        // j-split: slices of slice_len j
-    int near_shares;    // the symmetric sweep: shares of its in-group gravity
-    int slice_len;
-    float4* part;       // [nslices][n][2] partial sums when nslices > 1
+    // one-sided gravity: ni particles per lane (1, 2 or 4); `waves` wavefronts
+    // of a workgroup and `planes` workgroups share their particles' partners,
+    // slice_len (a multiple of 8) each
+    int ni, waves, planes, slice_len;
+    float4* part;       // [planes][n][2] partial sums when planes > 1
     const float* umass; // {uniform, mass} from launch_mass_check, or null
 };
 hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s);
@@ -181,16 +181,16 @@ hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 // 1024 slots; inside a group one-sided, between groups once per unordered
 // pair.  Sizes of its work arrays, in elements.
 struct SymGeom {
-    int nb, groups, wgs;
+    int groups, wgs;
     int64_t nsb, units;   // super-blocks; far work units
     int split;            // pieces per partner super-block in a far unit (1, 2 or 4)
-    int64_t near_elems;   // float4: near-field partial per slot and share
+    int64_t near_elems;   // float4: in-group sums and their corrections per slot
     int64_t apart_elems;  // float4: far own-side fragments (kFragElems each)
     bool plain;           // no far workgroup flushes a fragment twice: no correction planes
     int64_t bpart_elems;  // float: far partner-side partials (of the widest column batch)
     int ncols;            // column batches of the far field (1: the whole far field at once)
 };
-SymGeom sym_geometry(int64_t n, int wgs, int nshares, int64_t col_elems = INT64_MAX);
+SymGeom sym_geometry(int64_t n, int wgs, int64_t col_elems = INT64_MAX);
 // one column batch [c0, c1) of the far field's partner groups
 struct SymCol {
     int c0, c1;
@@ -207,7 +207,7 @@ struct SymLaunch {
     bool grav;
     bool finish;        // as SweepLaunch::finish
     bool add_acc;       // acc already holds the SPH terms: the combine adds the gravity to them
-    int nshares;        // in-group gravity cut into this many shares per block of 64 slots
+    int near_waves;     // in-group gravity: wavefronts sharing 64 slots
     float4* acc;
     const float4* vel;
     float4* xvel;
@@ -231,7 +231,6 @@ bool sym_has_far(const SymLaunch& L);
 struct BatchInst;
 struct SymInst {
     int off, n;         // slots [off, off + n)
-    int nb;             // blocks of 64
     int nsb, nrows;     // groups; far rows (groups with later ones)
     int row0;           // its first far row in the batch's arrays
     int64_t bpart0;     // first float of its partner-side partials
@@ -427,7 +426,7 @@ struct BatchSweepLaunch {
     const float* umass;   // {uniform, mass} per instance
     int ni_max;           // largest ni of the items (1 or 2)
 };
-hipError_t launch_batch_sweep(const BatchSweepLaunch& L, const DevParams& P, hipStream_t s);
+hipError_t launch_batch_sweep(const BatchSweepLaunch& L, hipStream_t s);
 // umass[2k] = 1 when every particle of instance k (insts null: the n
 // particles of one instance) has the same mass, umass[2k + 1] = that mass.
 // With insts null, umass must hold 2 + 256 floats (per-block flags follow).
@@ -624,8 +623,18 @@ inline int check_particles(Ctx& c, const grasph_particles* p)
     return 0;
 }
 
-// j-split of the single-instance one-sided sweep for n particles at ni per lane
-void choose_slices(const Ctx& c, int64_t n, int ni, int* slices, int* slice_len);
+// How the one-sided gravity sweep of n particles is cut: `slices` (0:
+// chosen from the count) shares of the partners, as many wavefronts of a
+// workgroup as take them, the rest in planes.
+struct OwnPlan {
+    int ni, waves, planes, len;
+    int slices() const { return waves * planes; }
+};
+OwnPlan own_plan(const Ctx& c, int64_t n, int slices);
+// particles from which the one-sided sweep looks whether all masses are equal
+// (the check's launch costs more than the multiply per pair it saves: Plummer
+// 1000 14.2 -> 10 us per step without it)
+constexpr int64_t kMassCheckMin = 6144;
 
 // arrays each pass needs, by configuration; 0 or a GRASPH_E_INVALID code
 int check_derivative_arrays(Ctx& c, const grasph_particles* p, uint32_t f, int which);

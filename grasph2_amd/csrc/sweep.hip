@@ -1,61 +1,156 @@
-// sweep.hip -- the one-sided O(N^2) gravity sweep (gfx950).
+// sweep.hip -- the one-sided O(N^2) sweeps (gfx950): gravity, and the
+// potential of the invariants.
 //
-// It sums the softened gravity of calcAcceleration
+// Gravity sums the softened gravity of calcAcceleration
 // (src/computeDerivatives.h:229-235) over every pair, in place of the tiled
-// device loop do_for_each_pair_fast_impl (src/particles/algorithms.h:270-309),
-// or the potential.  The neighbour lists come from lists.hip.
+// device loop do_for_each_pair_fast_impl (src/particles/algorithms.h:270-309);
+// it serves the particle counts below the symmetric sweep's (sym_sweep.hip),
+// the allocation-free entry point and, persistently, the smaller instances
+// of a batch.  The neighbour lists come from lists.hip.
 //
-// Mapping: NI i particles per lane (slots t and t + 64 for NI = 2).  The
-// particle stream xs is in slot order: with a Morton order the positions
+// The particle stream xs is in slot order: with a curve order the positions
 // gathered as xs[t] = posm[perm[t]], without one posm itself.  Results go to
-// particle perm[t].  All lanes visit the same j at the same time, so the j
-// stream (float4 x,y,z,m) is read with scalar loads into SGPRs -- no LDS, no
-// barriers -- in chunks of 8, two SGPR buffers in ping-pong so the next
-// chunk loads while this one computes.
-// Per pair: 3 sub, 3 FMA for r^2 + H^2, one v_rsq_f32, 2 mul (3 with
-// unequal masses), 3 FMA (a second transcendental per pair in place of a
-// multiply, rsqrt * rcp, measured 12% slower).  Sums are plain FP32 over
-// blocks of 128 j, then compensated (TwoSum) into the running total.
+// particle perm[t].  The pair loop is own_block.hpp's: up to 16 wavefronts of
+// a workgroup share 64 or 256 own slots and add their sums in LDS; with more
+// shares than that, planes of workgroups write partial sums that a second
+// kernel adds.  Sums are plain FP32 over blocks of 128 partners, then
+// compensated (TwoSum).
 //
 // The batched kernel runs the same code persistently over a queue of work
 // items (instance, 64 NI slots) ordered longest instance first; each
 // wavefront takes the next item with one atomic add.
 #include <algorithm>
 
-#include "sweep_core.hpp"
+#include "own_block.hpp"
 
 namespace grasph {
 namespace {
 
+constexpr int kBlock = 256;
 constexpr int kMassBlocks = 256;  // blocks of the single-instance mass check (flags after umass[0..1])
 
-template <int NI, bool GRAV, bool POT, bool SOFT>
-__global__ __launch_bounds__(kBlock) void sweep_kernel(const float4* __restrict__ xs, const int* __restrict__ perm,
-                                                       const int n, float4* __restrict__ acc,
-                                                       float* __restrict__ pot, const int finish,
-                                                       const float4* __restrict__ vel, float4* __restrict__ xvel,
-                                                       float* __restrict__ maxvsig, const DevParams P,
-                                                       const int slice_len, float4* __restrict__ part,
-                                                       const float* __restrict__ umass)
+// Workgroup (own block blockIdx.x, plane blockIdx.y): its wavefronts' shares
+// of slice_len partners start at plane * waves * slice_len.  One plane: the
+// accelerations; several: the plane's partial sums (2 float4 per particle).
+template <int NI, bool SOFT>
+__global__ __launch_bounds__(64 * kOwnMaxWaves) void own_kernel(const float4* __restrict__ xs,
+                                                                const int* __restrict__ perm, const int n,
+                                                                float4* __restrict__ acc, const int finish,
+                                                                float4* __restrict__ xvel,
+                                                                float* __restrict__ maxvsig, const DevParams P,
+                                                                const int slice_len, float4* __restrict__ part,
+                                                                const float* __restrict__ umass)
 {
-    const int wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    const int s0 = wave * 64 * NI + lane;
-    // slice blockIdx.y of the j range
-    const int sl = blockIdx.y;
-    const int j0 = sl * slice_len;
-    int j1 = min(n, j0 + slice_len);
-    if (!(GRAV || POT)) j1 = j0;  // nothing pairwise to do: skip the j loop
-    float4* const pp = part ? part + 2 * (size_t)sl * n : nullptr;
-    if constexpr (GRAV && !POT) {
-        if (umass && umass[0] != 0.0f) {  // {uniform, mass} of the partners, wave-uniform
-            sweep_slots<NI, GRAV, POT, SOFT, true>(xs, perm, s0, n, j0, j1, acc, pot, finish, vel, xvel, maxvsig, P,
-                                                   P.H2, P.cand, umass[1], pp);
+    extern __shared__ float lds[];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
+    const int o0 = 64 * NI * blockIdx.x, j0 = (int)blockIdx.y * waves * slice_len;
+    float4* const pp = part ? part + 2 * (size_t)blockIdx.y * n : nullptr;
+    auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
+        const int i = perm ? perm[t] : t;
+        if (pp) {
+            pp[2 * (size_t)i] = make_float4(x.s, y.s, z.s, 0.0f);
+            pp[2 * (size_t)i + 1] = make_float4(x.c, y.c, z.c, 0.0f);
             return;
         }
+        float ax = x.value(), ay = y.value(), az = z.value();
+        if (finish) {
+            environment_acceleration(P, ax, ay, az);
+            if (xvel) xvel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (maxvsig) maxvsig[i] = 0.0f;
+        }
+        acc[i] = make_float4(ax, ay, az, 0.0f);
+    };
+    if (umass && umass[0] != 0.0f)  // {uniform, mass} of the particles
+        own_block<NI, true, SOFT>(xs, o0, n, j0, n, slice_len, P.H2, umass[1], wave, waves, lds, store);
+    else
+        own_block<NI, false, SOFT>(xs, o0, n, j0, n, slice_len, P.H2, 1.0f, wave, waves, lds, store);
+}
+
+// Without gravity: what a sweep's finish leaves (environment, zero xvel / maxvsig).
+__global__ __launch_bounds__(kBlock) void no_gravity_kernel(const int n, float4* __restrict__ acc,
+                                                            float4* __restrict__ xvel, float* __restrict__ maxvsig,
+                                                            const DevParams P)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    environment_acceleration(P, ax, ay, az);
+    if (xvel) xvel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (maxvsig) maxvsig[i] = 0.0f;
+    acc[i] = make_float4(ax, ay, az, 0.0f);
+}
+
+// pot[i] = -sum_{j != i} m_j / sqrt(r^2 + H^2), one particle per lane: all
+// lanes visit the same j, read with scalar loads in chunks of 8, two buffers
+// in ping-pong.  Softened, the self pair is in the sum and is taken back
+// where r^2, as the oracle rounds it, is 0 (cand: softened squared distance
+// that every such pair stays below).
+constexpr int kChunk = 8;
+template <bool SOFT>
+__device__ __forceinline__ void pot_chunk(const float4 (&pj)[kChunk], const float xi, const float yi, const float zi,
+                                          float& phi, const float H2, const float cand)
+{
+    float d2[kChunk];
+#pragma unroll
+    for (int c = 0; c < kChunk; ++c) {
+        const float dx = pj[c].x - xi, dy = pj[c].y - yi, dz = pj[c].z - zi;
+        d2[c] = SOFT ? fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, H2))) : fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+        const float inv = __builtin_amdgcn_rsqf(d2[c]);
+        phi += SOFT ? pj[c].w * inv : ((d2[c] > 0.0f) ? pj[c].w * inv : 0.0f);
     }
-    sweep_slots<NI, GRAV, POT, SOFT, false>(xs, perm, s0, n, j0, j1, acc, pot, finish, vel, xvel, maxvsig, P, P.H2,
-                                            P.cand, 1.0f, pp);
+    if (SOFT) {
+        float mn = d2[0];
+#pragma unroll
+        for (int c = 0; c < kChunk; ++c) mn = fminf(mn, d2[c]);
+        if (mn <= cand) {
+#pragma unroll
+            for (int c = 0; c < kChunk; ++c)
+                if (d2[c] <= cand && dist2_exact(xi - pj[c].x, yi - pj[c].y, zi - pj[c].z) == 0.0f)
+                    phi -= pj[c].w * __builtin_amdgcn_rsqf(d2[c]);
+        }
+    }
+}
+
+template <bool SOFT>
+__global__ __launch_bounds__(kBlock) void pot_kernel(const float4* __restrict__ posm, const int n,
+                                                     float* __restrict__ pot, const float H2, const float cand)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const float4 p = posm[min(i, n - 1)];
+    float phi = 0.0f;
+    CSum sum{0.0f, 0.0f};
+    const int nchunks = n / kChunk, nfull = nchunks * kChunk;
+    float4 A[kChunk], B[kChunk];
+    if (nchunks > 0) {
+#pragma unroll
+        for (int c = 0; c < kChunk; ++c) A[c] = posm[c];
+    }
+    auto fold = [&]() {
+        sum.add(phi);
+        phi = 0.0f;
+    };
+    int k = 0;
+    for (; k + 1 < nchunks; k += 2) {
+        const int jb = k * kChunk;
+#pragma unroll
+        for (int c = 0; c < kChunk; ++c) B[c] = posm[jb + kChunk + c];
+        pot_chunk<SOFT>(A, p.x, p.y, p.z, phi, H2, cand);
+        // next A: chunk k + 2, or chunk k + 1 again when k + 2 is past the end
+        const int ja = ((k + 2 < nchunks) ? (k + 2) : (k + 1)) * kChunk;
+#pragma unroll
+        for (int c = 0; c < kChunk; ++c) A[c] = posm[ja + c];
+        pot_chunk<SOFT>(B, p.x, p.y, p.z, phi, H2, cand);
+        if (((k + 1) % (kFold / kChunk)) == kFold / kChunk - 1) fold();
+    }
+    if (k < nchunks) pot_chunk<SOFT>(A, p.x, p.y, p.z, phi, H2, cand);
+    if (nfull < n) {  // the last partial chunk, padded with far-away massless partners
+#pragma unroll
+        for (int c = 0; c < kChunk; ++c)
+            A[c] = (nfull + c < n) ? posm[nfull + c] : make_float4(3.0e18f, 3.0e18f, 3.0e18f, 0.0f);
+        pot_chunk<SOFT>(A, p.x, p.y, p.z, phi, H2, cand);
+    }
+    fold();
+    if (i < n) pot[i] = -sum.value();
 }
 
 // {1, m} when every particle of [off, off + n) has mass m (bit for bit),
@@ -118,18 +213,18 @@ __global__ __launch_bounds__(kBlock) void mass_final_kernel(const float4* __rest
     }
 }
 
-// Sum the slices' partial gravity in slice order (compensated) and finish
-// the acceleration as a one-slice sweep would.
-__global__ __launch_bounds__(kBlock) void combine_kernel(const float4* __restrict__ part, const int nslices,
-                                                         const int n, const float4* __restrict__ posm,
-                                                         float4* __restrict__ acc, const int finish,
-                                                         const float4* __restrict__ vel, float4* __restrict__ xvel,
-                                                         float* __restrict__ maxvsig, const DevParams P)
+// Sum the planes' partial gravity in plane order (compensated) and finish
+// the acceleration as a one-plane sweep would.
+__global__ __launch_bounds__(64) void combine_kernel(const float4* __restrict__ part, const int nplanes, const int n,
+                                                     float4* __restrict__ acc, const int finish,
+                                                     float4* __restrict__ xvel, float* __restrict__ maxvsig,
+                                                     const DevParams P)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= n) return;
     CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
-    for (int s = 0; s < nslices; ++s) {
+#pragma unroll 8
+    for (int s = 0; s < nplanes; ++s) {
         const float4 a = part[2 * ((size_t)s * n + i)], c = part[2 * ((size_t)s * n + i) + 1];
         x.add(a.x); y.add(a.y); z.add(a.z);
         x.c += c.x; y.c += c.y; z.c += c.z;
@@ -145,43 +240,42 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(const float4* __restric
 
 // Persistent sweep over a batch of independent instances.  Item w =
 // (inst, slot0, ni) covers slots [slot0, slot0 + 64 ni) of instance inst
-// with ni particles per lane (chosen per size bucket); the instance's
-// particles are [off, off + n) and its slots are the same range of perm.
+// with ni particles per lane (chosen per size bucket) against all of the
+// instance's particles [off, off + n); its slots are the same range of perm.
 // Every wavefront leaves the loop once the counter passes n_items.  NIMAX
-// is the largest ni of the items: the two-per-lane code needs about twice
-// the registers, so a batch without such items gets the leaner kernel.
+// is the largest ni of the items.
 template <int NIMAX, bool SOFT>
 __global__ __launch_bounds__(kBlock) void batch_sweep_kernel(const float4* __restrict__ xs,
                                                              const int* __restrict__ perm,
                                                              const int4* __restrict__ items, const int n_items,
                                                              const BatchInst* __restrict__ insts,
                                                              int* __restrict__ queue, float4* __restrict__ acc,
-                                                             const DevParams P, const float* __restrict__ umass)
+                                                             const float* __restrict__ umass)
 {
-    const int lane = threadIdx.x & 63;
+    __shared__ float lds[own_lds_floats(1, 1) * (kBlock / 64)];
+    float* const tile = lds + own_lds_floats(1, 1) * (threadIdx.x >> 6);  // one wavefront's
+    auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
+        acc[perm ? perm[t] : t] = make_float4(x.value(), y.value(), z.value(), 0.0f);
+    };
     for (;;) {
         int w = 0;
-        if (lane == 0) w = atomicAdd(queue, 1);
+        if ((threadIdx.x & 63) == 0) w = atomicAdd(queue, 1);
         w = __builtin_amdgcn_readfirstlane(w);
         if (w >= n_items) break;
         const int4 it = items[w];
         const BatchInst I = insts[it.x];
-        const int s0 = it.y + lane, e = I.off + I.n;
-        const bool um = umass && umass[2 * it.x] != 0.0f;
-        const float m = um ? umass[2 * it.x + 1] : 1.0f;
-        if (um) {
-            if (NIMAX == 2 && it.z == 2)
-                sweep_slots<NIMAX, true, false, SOFT, true>(xs, perm, s0, e, I.off, e, acc, nullptr, 0, nullptr,
-                                                            nullptr, nullptr, P, I.H2, 0.0f, m);
+        const int e = I.off + I.n;
+        const bool um = I.n >= kMassCheckMin && umass[2 * it.x] != 0.0f;  // as one instance
+        const float m = umass[2 * it.x + 1];
+        if (NIMAX == 2 && it.z == 2) {
+            if (um)
+                own_block<NIMAX, true, SOFT>(xs, it.y, e, I.off, e, I.n, I.H2, m, 0, 1, tile, store);
             else
-                sweep_slots<1, true, false, SOFT, true>(xs, perm, s0, e, I.off, e, acc, nullptr, 0, nullptr, nullptr,
-                                                        nullptr, P, I.H2, 0.0f, m);
-        } else if (NIMAX == 2 && it.z == 2) {
-            sweep_slots<NIMAX, true, false, SOFT, false>(xs, perm, s0, e, I.off, e, acc, nullptr, 0, nullptr, nullptr,
-                                                         nullptr, P, I.H2, 0.0f, m);
+                own_block<NIMAX, false, SOFT>(xs, it.y, e, I.off, e, I.n, I.H2, 1.0f, 0, 1, tile, store);
+        } else if (um) {
+            own_block<1, true, SOFT>(xs, it.y, e, I.off, e, I.n, I.H2, m, 0, 1, tile, store);
         } else {
-            sweep_slots<1, true, false, SOFT, false>(xs, perm, s0, e, I.off, e, acc, nullptr, 0, nullptr, nullptr,
-                                                     nullptr, P, I.H2, 0.0f, m);
+            own_block<1, false, SOFT>(xs, it.y, e, I.off, e, I.n, I.H2, 1.0f, 0, 1, tile, store);
         }
     }
 }
@@ -194,47 +288,29 @@ __global__ void reset_queue_kernel(int* __restrict__ queue, const int n)
     if (i < n) queue[i] = 0;
 }
 
-template <int NI, bool GRAV, bool POT, bool SOFT>
-hipError_t launch_t(const SweepLaunch& L, const DevParams& P, hipStream_t s)
+template <int NI, bool SOFT>
+hipError_t launch_own(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 {
-    const int waves = (L.n + 64 * NI - 1) / (64 * NI);
-    const int blocks = (waves + kBlock / 64 - 1) / (kBlock / 64);
-    const int ns = L.nslices > 1 ? L.nslices : 1;
-    hipLaunchKernelGGL((sweep_kernel<NI, GRAV, POT, SOFT>), dim3(blocks, ns), dim3(kBlock), 0, s,
-                       L.xs ? L.xs : L.posm, L.perm, L.n, L.acc, L.pot, L.finish ? 1 : 0, L.vel, L.xvel, L.maxvsig, P,
-                       ns > 1 ? L.slice_len : L.n, ns > 1 ? L.part : nullptr, L.umass);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || ns == 1 || !(GRAV || L.finish)) return e;
-    hipLaunchKernelGGL(combine_kernel, dim3((L.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, L.part, ns, L.n, L.posm,
-                       L.acc, L.finish ? 1 : 0, L.vel, L.xvel, L.maxvsig, P);
+    const dim3 grid((unsigned)((L.n + 64 * NI - 1) / (64 * NI)), (unsigned)L.planes);
+    hipLaunchKernelGGL((own_kernel<NI, SOFT>), grid, dim3(64 * L.waves), sizeof(float) * own_lds_floats(NI, L.waves),
+                       s, L.xs ? L.xs : L.posm, L.perm, L.n, L.acc, L.finish ? 1 : 0, L.xvel, L.maxvsig, P,
+                       L.slice_len, L.planes > 1 ? L.part : nullptr, L.umass);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || L.planes == 1) return e;
+    hipLaunchKernelGGL(combine_kernel, dim3((L.n + 63) / 64), dim3(64), 0, s, L.part, L.planes, L.n, L.acc,
+                       L.finish ? 1 : 0, L.xvel, L.maxvsig, P);
     return hipGetLastError();
 }
 
-template <int NI>
-hipError_t launch_ni(const SweepLaunch& L, const DevParams& P, hipStream_t s)
-{
-    const bool soft = P.H2 > 0.0f;
-    const int key = (L.grav ? 4 : 0) | (L.want_pot ? 2 : 0) | (soft ? 1 : 0);
-    switch (key) {
-        case 0: return launch_t<NI, false, false, false>(L, P, s);
-        case 1: return launch_t<NI, false, false, true>(L, P, s);
-        case 2: return launch_t<NI, false, true, false>(L, P, s);
-        case 3: return launch_t<NI, false, true, true>(L, P, s);
-        case 4: return launch_t<NI, true, false, false>(L, P, s);
-        case 5: return launch_t<NI, true, false, true>(L, P, s);
-        default: return hipErrorInvalidValue;  // the potential sweep runs alone
-    }
-}
-
 template <bool SOFT>
-hipError_t launch_b(const BatchSweepLaunch& L, const DevParams& P, hipStream_t s)
+hipError_t launch_b(const BatchSweepLaunch& L, hipStream_t s)
 {
     if (L.ni_max == 2)
         hipLaunchKernelGGL((batch_sweep_kernel<2, SOFT>), dim3(L.blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
-                           L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, P, L.umass);
+                           L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, L.umass);
     else
         hipLaunchKernelGGL((batch_sweep_kernel<1, SOFT>), dim3(L.blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
-                           L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, P, L.umass);
+                           L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, L.umass);
     return hipGetLastError();
 }
 
@@ -243,7 +319,29 @@ hipError_t launch_b(const BatchSweepLaunch& L, const DevParams& P, hipStream_t s
 hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0) return hipSuccess;
-    return L.ni == 2 ? launch_ni<2>(L, P, s) : launch_ni<1>(L, P, s);
+    const bool soft = P.H2 > 0.0f;
+    if (L.want_pot) {
+        const dim3 grid((L.n + kBlock - 1) / kBlock);
+        if (soft)
+            hipLaunchKernelGGL(pot_kernel<true>, grid, dim3(kBlock), 0, s, L.posm, L.n, L.pot, P.H2, P.cand);
+        else
+            hipLaunchKernelGGL(pot_kernel<false>, grid, dim3(kBlock), 0, s, L.posm, L.n, L.pot, P.H2, P.cand);
+        return hipGetLastError();
+    }
+    if (!L.grav) {
+        if (L.finish)
+            hipLaunchKernelGGL(no_gravity_kernel, dim3((L.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, L.n, L.acc,
+                               L.xvel, L.maxvsig, P);
+        return hipGetLastError();
+    }
+    if (L.waves < 1 || L.waves > kOwnMaxWaves || L.planes < 1 || L.slice_len < 8 || L.slice_len % 8)
+        return hipErrorInvalidValue;
+    switch (L.ni) {
+        case 1: return soft ? launch_own<1, true>(L, P, s) : launch_own<1, false>(L, P, s);
+        case 2: return soft ? launch_own<2, true>(L, P, s) : launch_own<2, false>(L, P, s);
+        case 4: return soft ? launch_own<4, true>(L, P, s) : launch_own<4, false>(L, P, s);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_mass_check(const float4* posm, const BatchInst* insts, int n_inst, int n, float* umass,
@@ -274,12 +372,12 @@ hipError_t launch_reset_queue(int* queue, int n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_batch_sweep(const BatchSweepLaunch& L, const DevParams& P, hipStream_t s)
+hipError_t launch_batch_sweep(const BatchSweepLaunch& L, hipStream_t s)
 {
     if (L.n_items <= 0) return hipSuccess;
     if (L.waves_per_block < 1 || L.waves_per_block > kBlock / 64) return hipErrorInvalidValue;
     if (L.ni_max != 1 && L.ni_max != 2) return hipErrorInvalidValue;
-    return L.soft ? launch_b<true>(L, P, s) : launch_b<false>(L, P, s);
+    return L.soft ? launch_b<true>(L, s) : launch_b<false>(L, s);
 }
 
 }  // namespace grasph

@@ -4,8 +4,7 @@
 // Same results as the sweep of sweep.hip (softened gravity of
 // calcAcceleration, src/computeDerivatives.h:229-235), organised by groups
 // of 1024 consecutive slots:
-//  - in-group gravity, one wavefront per block of 64 slots (and share of the
-//    group's partners), one-sided through the pair loop of sweep_core.hpp;
+//  - in-group gravity, one-sided (own_block.hpp);
 //  - far field: every pair of slots in different groups is computed once,
 //    for both sides (Newton's third law).  One wavefront owns a group (16
 //    slots per lane).  The later groups' particles come 16 at a time, one
@@ -28,12 +27,13 @@
 #include <vector>
 
 #include "far_rotation.hpp"
-#include "sweep_core.hpp"
+#include "own_block.hpp"
 #include "sym_geometry.hpp"
 
 namespace grasph {
 namespace {
 
+constexpr int kBlock = 256;
 constexpr int kFarThreads = 64;  // one wavefront owns a group
 static_assert(kGroupSB == 1 && kSB == kGroup, "the far field assumes one wavefront per group");
 
@@ -51,51 +51,34 @@ __device__ __forceinline__ float swap16_sum(float p, float q)
 }
 // ------------------------------------------------------------------ kernels
 
-// In-group gravity of the 64 slots of block I of the instance whose slots are
-// [base, base + n), share `sl` of `ns`: the blocks of its group are cut into
-// ns runs of equal count, and this wavefront takes run sl.  Writes the slot's
-// compensated gravity partial (slot-indexed, two float4) in the plane of
-// share sl; the combine folds the planes in share order.
-template <bool SOFT, bool UM>
-__device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, const int base, const int n, const int nb,
-                                              const int I, const int sl, const int ns, const int lane,
-                                              float4* __restrict__ near_part, const float H2, const float m)
+// In-group gravity: a workgroup takes 64 NI slots of a group, its wavefronts
+// an equal share of the group's slots as partners each (whole shares of
+// kGroup / waves, whatever the group holds).  Writes the slot's compensated
+// sums (slot-indexed, two float4).
+template <int NI, bool SOFT>
+__device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, const int o0, const int g0, const int g1,
+                                              float4* __restrict__ near_part, const float h2,
+                                              const float* __restrict__ um, float* lds)
 {
-    constexpr int kGroupBlocks = kGroup / 64;  // 16
-    const int t = base + 64 * I + lane;  // slots of the instance: [base, base + n)
-    const bool act = 64 * I + lane < n;
-    float xi[1], yi[1], zi[1];
-    xi[0] = yi[0] = zi[0] = 0.0f;
-    if (act) {
-        const float4 p = xs[t];
-        xi[0] = p.x; yi[0] = p.y; zi[0] = p.z;
-    }
-    Acc<1> a;
-    a.ax[0] = a.ay[0] = a.az[0] = a.phi[0] = 0.0f;
-    a.sx[0] = a.sy[0] = a.sz[0] = a.sphi[0] = CSum{0.0f, 0.0f};
-    const int G0 = (I / kGroupBlocks) * kGroupBlocks, total = min(nb, G0 + kGroupBlocks) - G0;  // own group's blocks
-    const int r0 = G0 + sl * total / ns, r1 = G0 + (sl + 1) * total / ns;
-    if (r0 < r1)
-        sweep_range<1, true, false, SOFT, UM>(xs, base + 64 * r0, base + min(n, 64 * r1), xi, yi, zi, a, H2, 0.0f, m);
-    if (!act) return;
-    near_part[2 * (size_t)t] = make_float4(a.sx[0].s, a.sy[0].s, a.sz[0].s, 0.0f);
-    near_part[2 * (size_t)t + 1] = make_float4(a.sx[0].c, a.sy[0].c, a.sz[0].c, 0.0f);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
+    auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
+        near_part[2 * (size_t)t] = make_float4(x.s, y.s, z.s, 0.0f);
+        near_part[2 * (size_t)t + 1] = make_float4(x.c, y.c, z.c, 0.0f);
+    };
+    if (um[0] != 0.0f)
+        own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
+    else
+        own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
 }
 
 template <bool SOFT>
-__global__ __launch_bounds__(kBlock) void ingroup_kernel(const float4* __restrict__ xs, const int n, const int nb,
-                                                         float4* __restrict__ near_part, const float H2,
-                                                         const float* __restrict__ umass)
+__global__ __launch_bounds__(64 * kOwnMaxWaves) void ingroup_kernel(const float4* __restrict__ xs, const int n,
+                                                                    float4* __restrict__ near_part, const float h2,
+                                                                    const float* __restrict__ umass)
 {
-    const int I = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kBlock + threadIdx.x) >> 6));
-    const int lane = threadIdx.x & 63;
-    if (I >= nb) return;
-    const int sl = blockIdx.y, ns = gridDim.y;  // share sl of ns
-    float4* const part = near_part + 2 * (size_t)sl * n;
-    if (umass[0] != 0.0f)
-        ingroup_block<SOFT, true>(xs, 0, n, nb, I, sl, ns, lane, part, H2, umass[1]);
-    else
-        ingroup_block<SOFT, false>(xs, 0, n, nb, I, sl, ns, lane, part, H2, 1.0f);
+    extern __shared__ float lds[];
+    const int o0 = 64 * blockIdx.x, g0 = o0 / kGroup * kGroup;
+    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), near_part, h2, umass, lds);
 }
 
 // One chunk of 16 partners (pj: row lane l holds partner l) against the
@@ -368,7 +351,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
     far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, apart, plain, bpart, H2, umass, lsum);
 }
 
-// Per slot, in a fixed order: the near partials (share order), the far own-side fragments
+// Per slot, in a fixed order: the in-group sums, the far own-side fragments
 // (workgroup order), the far partner-side partials (group order, negated:
 // they were summed as seen from the other side), compensated; then the
 // acceleration is finished as the one-range sweep does.  With PARTS > 1
@@ -380,7 +363,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
 template <int PARTS, bool PLAIN>
 __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
-    const int n, const int nshares, const int64_t nsb, const int64_t U, const int W, const int Q, const int grav,
+    const int n, const int64_t nsb, const int64_t U, const int W, const int Q, const int grav,
     const int* __restrict__ perm,
     const float4* __restrict__ xs, float4* __restrict__ acc, const int finish, const int add_acc,
     const float4* __restrict__ vel, float4* __restrict__ xvel, float* __restrict__ maxvsig, const DevParams P)
@@ -390,11 +373,9 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
     const int t = blockIdx.x * kSlots + ((int)threadIdx.x - p * kSlots);
     CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
     if (grav && t < n) {
-        for (int sl = p; sl < nshares; sl += PARTS) {
-            const size_t e = 2 * ((size_t)sl * n + t);
-            const float4 a = near_part[e], c = near_part[e + 1];
-            x.add(a.x); y.add(a.y); z.add(a.z);
-            x.c += c.x; y.c += c.y; z.c += c.z;
+        if (p == 0) {
+            const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
+            x = CSum{a.x, c.x}; y = CSum{a.y, c.y}; z = CSum{a.z, c.z};
         }
         const int64_t g = t / kGroup, local = t - g * kGroup;
         if (U > 0 && g < rows_with_units(nsb)) {
@@ -491,7 +472,7 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
 // partials join them and the acceleration is finished as in the combine.
 __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
-    float4* __restrict__ accsum, const int n, const int nshares, const int c0, const int c1, const int64_t U,
+    float4* __restrict__ accsum, const int n, const int c0, const int c1, const int64_t U,
     const int W, const int Q, const int plain, const int first, const int last, const int* __restrict__ perm,
     float4* __restrict__ acc, const int finish, const int add_acc, float4* __restrict__ xvel,
     float* __restrict__ maxvsig, const DevParams P)
@@ -544,9 +525,8 @@ __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
         accsum[2 * (size_t)t + 1] = make_float4(x.c, y.c, z.c, 0.0f);
         return;
     }
-    for (int sl = 0; sl < nshares; ++sl) {
-        const size_t e = 2 * ((size_t)sl * n + t);
-        const float4 a = near_part[e], c = near_part[e + 1];
+    {
+        const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
         x.add(a.x); y.add(a.y); z.add(a.z);
         x.c += c.x; y.c += c.y; z.c += c.z;
     }
@@ -580,18 +560,12 @@ __global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4*
                                                                    float4* __restrict__ near_part,
                                                                    const float* __restrict__ umass)
 {
+    __shared__ float lds[own_lds_floats(4, kBlock / 64)];
     const int4 bl = blk[xcd_block((int)blockIdx.x, (int)gridDim.x)];  // XCD-contiguous (xcd_block)
-    const int lane = threadIdx.x & 63;
-    const int first = __builtin_amdgcn_readfirstlane(bl.y + 64 * (int)(threadIdx.x >> 6));
-    if (first >= bl.z) return;
-    const int k = bl.x;
-    const SymInst S = sinst[k];
-    const int I = (first - S.off) >> 6;
-    const float H2 = insts[k].H2;
-    if (umass[2 * k] != 0.0f)
-        ingroup_block<SOFT, true>(xs, S.off, S.n, S.nb, I, 0, 1, lane, near_part, H2, umass[2 * k + 1]);
-    else
-        ingroup_block<SOFT, false>(xs, S.off, S.n, S.nb, I, 0, 1, lane, near_part, H2, 1.0f);
+    const SymInst S = sinst[bl.x];
+    const int g0 = S.off + (bl.y - S.off) / kGroup * kGroup;
+    ingroup_block<4, SOFT>(xs, bl.y, g0, min(S.off + S.n, g0 + kGroup), near_part, insts[bl.x].H2, umass + 2 * bl.x,
+                           lds);
 }
 
 // one piece of a far row of an instance of the batch: group R.g against
@@ -729,16 +703,15 @@ SymCol sym_column(int64_t nsb, int split, int wanted, int c0, int c1)
     return C;
 }
 
-SymGeom sym_geometry(int64_t n, int wgs, int nshares, int64_t col_elems)
+SymGeom sym_geometry(int64_t n, int wgs, int64_t col_elems)
 {
     SymGeom G;
-    G.nb = (int)((n + 63) / 64);
     G.nsb = (n + kSB - 1) / kSB;
     G.groups = (int)((G.nsb + kGroupSB - 1) / kGroupSB);
     G.split = far_split(n, wgs);
     G.units = row_prefix(rows_with_units(G.nsb), G.nsb, G.split);
     G.wgs = far_workgroups(wgs, G.units);
-    G.near_elems = 2 * n * nshares;
+    G.near_elems = 2 * n;
     G.apart_elems = (int64_t)kFragElems * (G.groups + wgs);
     G.plain = fragments_plain((G.units + G.wgs - 1) / G.wgs);
     G.bpart_elems = 3 * bpart_group_base(G.groups);
@@ -752,21 +725,22 @@ SymGeom sym_geometry(int64_t n, int wgs, int nshares, int64_t col_elems)
     return G;
 }
 
-// gravity inside the groups (the partials of the combine)
+// gravity inside the groups
 hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0 || !L.grav) return hipSuccess;
-    if (L.nshares < 1) return hipErrorInvalidValue;
-    const int nb = (L.n + 63) / 64;
-    const dim3 grid((nb + kBlock / 64 - 1) / (kBlock / 64), L.nshares);
+    const int w = L.near_waves;  // a power of two: the shares cover the group exactly
+    if (w < 1 || w > kOwnMaxWaves || (w & (w - 1))) return hipErrorInvalidValue;
+    const dim3 grid((L.n + 63) / 64), block(64 * w);
+    const size_t lds = sizeof(float) * own_lds_floats(1, w);
     if (P.H2 > 0.0f)
-        hipLaunchKernelGGL(ingroup_kernel<true>, grid, dim3(kBlock), 0, s, L.xs, L.n, nb, L.near_part, P.H2, L.umass);
+        hipLaunchKernelGGL(ingroup_kernel<true>, grid, block, lds, s, L.xs, L.n, L.near_part, P.H2, L.umass);
     else
-        hipLaunchKernelGGL(ingroup_kernel<false>, grid, dim3(kBlock), 0, s, L.xs, L.n, nb, L.near_part, P.H2, L.umass);
+        hipLaunchKernelGGL(ingroup_kernel<false>, grid, block, lds, s, L.xs, L.n, L.near_part, P.H2, L.umass);
     return hipGetLastError();
 }
 
-bool sym_has_far(const SymLaunch& L) { return L.n > 0 && L.grav && sym_geometry(L.n, L.wgs, 1).units > 0; }
+bool sym_has_far(const SymLaunch& L) { return L.n > 0 && L.grav && sym_geometry(L.n, L.wgs).units > 0; }
 
 template <bool SOFT>
 void launch_far_column(const SymLaunch& L, const SymCol& C, const int split, const DevParams& P, hipStream_t s)
@@ -779,7 +753,7 @@ void launch_column_combine(const SymLaunch& L, const SymCol& C, const int split,
                            const DevParams& P, hipStream_t s)
 {
     hipLaunchKernelGGL(sym_column_combine_kernel, dim3((L.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, L.near_part,
-                       L.apart, L.bpart, L.accsum, L.n, L.nshares, C.c0, C.c1, C.units, C.wgs, split, C.plain ? 1 : 0,
+                       L.apart, L.bpart, L.accsum, L.n, C.c0, C.c1, C.units, C.wgs, split, C.plain ? 1 : 0,
                        first ? 1 : 0, last ? 1 : 0, L.perm, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0, L.xvel,
                        L.maxvsig, P);
 }
@@ -790,7 +764,7 @@ void launch_column_combine(const SymLaunch& L, const SymCol& C, const int split,
 hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (!sym_has_far(L)) return hipSuccess;
-    const SymGeom G = sym_geometry(L.n, L.wgs, L.nshares, L.col_elems);
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     if (G.ncols == 1) {
         if (P.H2 > 0.0f)
             hipLaunchKernelGGL((far_kernel<true>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
@@ -813,7 +787,7 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0 || !(L.grav || L.finish)) return hipSuccess;
-    const SymGeom G = sym_geometry(L.n, L.wgs, L.nshares, L.col_elems);
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     if (G.ncols > 1 && sym_has_far(L)) {
         // the last column batch's combine, which finishes
         const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
@@ -825,7 +799,7 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
     const int parts = L.n >= 98304 ? 1 : L.n >= 49152 ? 2 : L.n >= 24576 ? 4 : 8;
 #define GRASPH_COMBINE(PARTS, PLAIN)                                                                                  \
     hipLaunchKernelGGL((sym_combine_kernel<PARTS, PLAIN>), dim3((L.n + kBlock / PARTS - 1) / (kBlock / PARTS)),        \
-                       dim3(kBlock), 0, s, L.near_part, L.apart, L.bpart, L.n, L.nshares, G.nsb, G.units, L.wgs,       \
+                       dim3(kBlock), 0, s, L.near_part, L.apart, L.bpart, L.n, G.nsb, G.units, L.wgs,       \
                        G.split, L.grav ? 1 : 0, L.perm, L.xs, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0, L.vel,       \
                        L.xvel, L.maxvsig, P)
     if (G.plain) {
@@ -857,7 +831,6 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
         if (sym)
             for (int64_t s = offsets[k]; s < offsets[k + 1]; s += 256)
                 T.blk.push_back(make_int4(k, (int)s, (int)std::min<int64_t>(s + 256, offsets[k + 1]), 0));
-        S.nb = (int)((S.n + 63) / 64);
         S.nsb = (int)((S.n + kSB - 1) / kSB);
         S.nrows = (int)rows_with_units(S.nsb);
         S.row0 = row0;

@@ -161,7 +161,10 @@ int grasph_destroy(grasph_ctx* ctx);
  * and an array allocated at a freed one's address counts as the same
  * particles until the next re-sort: slower, never wrong),
  * "profile" (1 = record HIP events around each kernel), "sweep_i_per_lane"
- * (1 or 2), "sweep_slices" (j-split of the sweep, 0 = automatic),
+ * (particles per lane of the one-sided sweep: 2, or 1 = chosen from the
+ * count, the default; the results are the same bit for bit), "sweep_slices"
+ * (j-split of the sweep, 0 = automatic; past a workgroup's 8 or 16 wavefronts
+ * rounded up to whole workgroups),
  * "batch_waves_per_block", "batch_blocks_per_cu" (batched sweep launch
  * shape), "sweep_symmetric" (single
  * instance: 1 = gravity between groups of 1024 particles evaluated once per
@@ -176,7 +179,7 @@ int grasph_destroy(grasph_ctx* ctx);
  * the partials, the running sums kept between batches in 32 B per particle;
  * results agree with the unbatched far field to FP32 rounding),
  * "sym_near_shares" (wavefronts per 64 particles in its in-group gravity, 1-16,
- * 0 = chosen from the occupancy), "sym_list_priority" (0, 1 or 2: kept for
+ * rounded down to a power of two; 0 = chosen from the count), "sym_list_priority" (0, 1 or 2: kept for
  * callers that set it; without effect, as the lists no longer run beside the
  * far field), "batch_symmetric" (1 = batches use the
  * symmetric sweep for their instances of at least "batch_symmetric_min"
