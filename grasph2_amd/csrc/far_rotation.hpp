@@ -39,10 +39,10 @@ namespace {
 constexpr int kRow = 16;  // partners per rotated chunk (one DPP row)
 
 // Own slots of a lane in the far field: position, mass and the plain
-// gravity sums of the current unit.  At the end of a unit those go into
-// the wavefront's LDS sums (lsum[1024 c + slot], component c: plain sums of
-// at most kFoldsPerFlush units), and every kFoldsPerFlush units and at the
-// end of the row the LDS sums go into the row's own-side fragment in global
+// gravity sums since the last fold.  A fold adds those to the wavefront's
+// LDS sums (lsum[1024 c + slot], component c: plain sums of at most
+// kFoldsPerFlush folds), and every kFoldsPerFlush folds and at the end of
+// the row the LDS sums go into the row's own-side fragment in global
 // memory (float4 sums at frag[frag_elem(slot)], their corrections 64
 // further), compensated.  Neither level takes registers from the pair loop,
 // and the fragment is written about once per row.
@@ -51,7 +51,7 @@ struct FarOwn {
     float ax[kNI], ay[kNI], az[kNI];
     float* lsum;
     float4* frag;
-    int folds;   // units in lsum since the last flush (0: lsum holds nothing)
+    int folds;   // folds in lsum since the last flush (0: lsum holds nothing)
     bool fresh;  // nothing flushed into the fragment yet: the first flush writes it
     bool plain;  // every fragment is flushed once: no correction planes
 };

@@ -183,7 +183,7 @@ hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 struct SymGeom {
     int groups, wgs;
     int64_t nsb, units;   // super-blocks; far work units
-    int split;            // pieces per partner super-block in a far unit (1, 2 or 4)
+    int split;            // pieces a partner group is cut into for the far work's split
     int64_t near_elems;   // float4: in-group sums and their corrections per slot
     int64_t apart_elems;  // float4: far own-side fragments (kFragElems each)
     bool plain;           // no far workgroup flushes a fragment twice: no correction planes
@@ -198,7 +198,7 @@ struct SymCol {
     int wgs;
     bool plain;
 };
-SymCol sym_column(int64_t nsb, int split, int wanted, int c0, int c1);
+SymCol sym_column(int split, int fold, int wanted, int c0, int c1);
 int sym_default_workgroups(int cus);  // far-field workgroups for 2 wavefronts per SIMD
 struct SymLaunch {
     const float4* xs;   // slot-ordered positions + masses

@@ -84,8 +84,8 @@ __host__ inline std::vector<int> sym_columns(int64_t nsb, int64_t max_elems)
 }
 
 // far units of row g: each partner super-block of [kGroupSB (g + 1), nsb)
-// cut into Q pieces of kSB / Q partners (Q = 1, 2, 4, 8 or 16; more pieces
-// give small particle counts enough units to fill the GPU)
+// cut into Q pieces of kSB / Q partners (Q = 1 to 64; more pieces spread the
+// work more evenly)
 __device__ __host__ inline int64_t row_units(int64_t g, int64_t nsb, int Q = 1)
 {
     const int64_t u = nsb - (int64_t)kGroupSB * (g + 1);
@@ -111,11 +111,12 @@ __device__ __host__ inline int64_t row_of_unit(int64_t u, int64_t nsb, int Q = 1
 // pieces per partner super-block for n particles and `wanted` far
 // workgroups (as many as run at once): the kernel lasts as long as its
 // fullest share, ceil(U / W) units of kSB / Q partners with W = min(wanted,
-// U); the Q of 2, 4, 8, 16 that makes that shortest, the fewest pieces on
-// a tie (smaller units cost more per partner)
-// a piece has at most 512 partners (a slot's plain FP32 own-side sum takes
-// at most that many terms) and at least 64 (4 chunks of 16)
-constexpr int kMinSplit = 2, kMaxSplit = 16;
+// U); the Q of 2 to 64 (a piece is at least one chunk of 16 partners) that
+// makes that shortest, the fewest pieces on a tie.  A share is one run of
+// partners per row whatever Q is, so pieces cost nothing by themselves
+// (N = 50021: 8 pieces leave the fullest of 2048 shares 9% above the mean,
+// 64 pieces 0.7%; Plummer step 419 -> 391 us, N = 17000 111 -> 83).
+constexpr int kMinSplit = 2, kMaxSplit = 64;
 __device__ __host__ inline int far_split(int64_t n, int64_t wanted)
 {
     const int64_t nsb = (n + kSB - 1) / kSB;
@@ -161,19 +162,19 @@ __device__ __host__ inline int64_t bpart_group_base(int64_t h) { return (int64_t
 // Own-side fragments: one per (row, wavefront that worked on the row), in
 // float4 elements, 2 kGroup of them: for each 64 slots of the group, their
 // 64 sums (x y z, w unused), then those sums' 64 corrections (slot s: sums
-// at frag_elem(s), corrections 64 further).  A wavefront adds a unit's
-// own-side sums to LDS sums and those to the fragment every kFoldsPerFlush
-// units and at the end of its stay on the row.  The first flush writes the
-// sums (their corrections are exactly zero).  When no wavefront stays longer
-// than kFoldsPerFlush units on a row, every fragment is flushed once: it is
+// at frag_elem(s), corrections 64 further).  A wavefront folds its own-side
+// sums into LDS sums every so many partners and those into the fragment every
+// kFoldsPerFlush folds and at the end of its stay on the row.  The first flush
+// writes the sums (their corrections are exactly zero).  When no stay has more
+// than kFoldsPerFlush folds, every fragment is flushed once: it is
 // plain, and neither the far field nor the combine touch its corrections;
 // otherwise the first flush writes zero corrections too.
 constexpr int kFoldsPerFlush = 16;
 constexpr int kFragElems = 2 * kGroup;
 __device__ __host__ inline int frag_elem(int slot) { return 128 * (slot >> 6) + (slot & 63); }
-__device__ __host__ inline bool fragments_plain(int64_t max_units_per_visit)
+__device__ __host__ inline bool fragments_plain(int64_t max_folds_per_visit)
 {
-    return max_units_per_visit <= kFoldsPerFlush;
+    return max_folds_per_visit <= kFoldsPerFlush;
 }
 
 }  // namespace grasph

@@ -120,13 +120,11 @@ __device__ __forceinline__ float4 load_partner_row(const float4* __restrict__ xs
     }
     return xs[jc];
 }
-// BOUNDED: partners at or past n are far away and massless (applied where
-// the chunk is used, so the load's wait stays there)
-template <bool BOUNDED>
+// partners at or past n: far away and massless (applied where the chunk is
+// used, so the load's wait stays there)
 __device__ __forceinline__ float4 bound_partner_row(const float4 v, const int b, const int n, const int lane)
 {
-    if (BOUNDED && b + (lane & (kRow - 1)) >= n) return make_float4(3.0e18f, 3.0e18f, 3.0e18f, 0.0f);
-    return v;
+    return b + (lane & (kRow - 1)) >= n ? make_float4(3.0e18f, 3.0e18f, 3.0e18f, 0.0f) : v;
 }
 
 // component of the partner side this lane holds after far_chunk_rot: row 0
@@ -137,30 +135,6 @@ __device__ __forceinline__ int partner_comp_rot(const int lane)
 {
     const int row = lane >> 4;
     return row == 0 ? 0 : row == 2 ? 1 : 2;
-}
-
-// Partners [b0, b0 + 16 nchunks) of group J against the wavefront's slots;
-// each chunk's partner side (summed over the whole group: one wavefront
-// owns it) goes straight to row g's partials bp (bp[3 p + c]: partner p of
-// group J, component c; UM: times the common mass m).  The store has no
-// condition: partners past n (only in the instance's last group, whose
-// partials are allocated whole) get values nobody reads, and a store behind
-// a branch makes the compiler spill the chunk's registers.
-template <bool UM, bool SOFT, bool BOUNDED>
-__device__ __forceinline__ void far_segment_rot(const float4* __restrict__ xs, const int n, const int b0,
-                                                const int nchunks, const int J, FarOwn& o, const float H2,
-                                                const int lane, float* __restrict__ bp, const float m)
-{
-    const int comp = partner_comp_rot(lane);
-    const int p0 = b0 - kGroup * J + (lane & (kRow - 1));  // this lane's partner within group J, chunk 0
-    float4 A = load_partner_row<UM>(xs, b0, n, lane);
-    for (int q = 0; q < nchunks; ++q) {
-        const float4 B = load_partner_row<UM>(xs, b0 + kRow * (q + 1), n, lane);  // unused after the last
-        const float v = far_chunk_rot<UM, SOFT>(bound_partner_row<BOUNDED>(A, b0 + kRow * q, n, lane), o, H2);
-        const int p = p0 + kRow * q;
-        bp[3 * p + comp] = UM ? v * m : v;  // p past n: in the last group's partials, never read
-        A = B;
-    }
 }
 
 // The own slots of row g (slots 1024 g + 64 q + lane, q < kNI) of an
@@ -190,7 +164,7 @@ __device__ __forceinline__ void far_load_row(const float4* __restrict__ xs, cons
 
 // The lane's slot of own slot q, through an empty asm statement: indexed
 // by it, the LDS sums and the fragment are never kept in registers across
-// a row's units by the compiler (96 more live values, which the pair loop
+// a row's folds by the compiler (96 more live values, which the pair loop
 // cannot spare).
 __device__ __forceinline__ int own_lane(const int lane)
 {
@@ -226,8 +200,8 @@ __device__ __forceinline__ void far_flush_own(FarOwn& o, const int lane)
     o.folds = 0;
 }
 
-// The lane's plain own-side sums of a unit added to its LDS sums, then
-// cleared; every kFoldsPerFlush units the LDS sums go to the fragment.
+// The lane's plain own-side sums added to its LDS sums, then cleared;
+// every kFoldsPerFlush folds the LDS sums go to the fragment.
 template <bool UM>
 __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int lane)
 {
@@ -247,108 +221,121 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
     if (++o.folds == kFoldsPerFlush) far_flush_own(o, lane);
 }
 
-// One far unit of row g: piece `piece` of Q (kSB / Q partners, Q >= 2) of
-// partner group J against the wavefront's 1024 slots; the partials of group
-// J start at element 3 (bpart_group_base(J) - boff) of bpart (boff: the
-// groups before the column batch).  The partner side is
-// stored per chunk as row g's partials; the own side is folded at the end,
-// so a slot adds at most 512 terms in plain FP32 before they join its LDS
-// sum (and at most kFoldsPerFlush such sums before they join the
-// compensated fragment).
-template <bool UM, bool SOFT, int QC = 0>
-__device__ __forceinline__ void far_unit(const float4* __restrict__ xs, const int n, const int64_t g, const int J,
-                                         const int piece, const int Qr, FarOwn& o, float* __restrict__ bpart,
-                                         const int64_t boff, const float H2, const float m, const int lane)
+// Partners [b0, b1) (multiples of 16; those past n are left out) against the
+// slots of row g, a chunk of 16 at a time; each chunk's partner side (summed
+// over the whole group: one wavefront owns it) goes straight to row g's
+// partials of its group (element 3 (bpart_group_base(J) - boff) on holds
+// group J's; boff: the groups before the column batch; UM: times the common
+// mass m).  The store has no condition: partners of the last chunk past n
+// (their group's partials are allocated whole) get values nobody reads, and
+// a store behind a branch makes the compiler spill the chunk's registers.
+// The own side is folded every `fold` partners and at the end, so a slot
+// adds at most that many terms in plain FP32 before they join its LDS sum
+// (and at most kFoldsPerFlush such sums before they join the compensated
+// fragment): 512 from 131072 particles on, where a fold every 128 costs 1.3%
+// of the step and the sums of many workgroups average their rounding; 128
+// below (N = 50021: error against FP64 5.3e-8 of the norm, 6.8e-8 with 512,
+// for 1.4% of the step) and 512 in batches.
+constexpr int kFarFoldLarge = 512, kFarFoldSmall = 128, kFarFoldMin = 131072;
+static int far_fold(int64_t n) { return n >= kFarFoldMin ? kFarFoldLarge : kFarFoldSmall; }
+template <bool UM, bool SOFT>
+__device__ __forceinline__ void far_range(const float4* __restrict__ xs, const int n, const int64_t g, const int b0,
+                                          const int b1, const int fold, FarOwn& o, float* __restrict__ bpart,
+                                          const int64_t boff, const float H2, const float m, const int lane)
 {
-    const int Q = QC ? QC : Qr;  // QC: the split known at compile time (2 for the largest counts)
-    const int len = kSB / Q, b0 = kSB * J + len * piece, nchunks = len / kRow;
-    float* const bp = bpart + 3 * (bpart_group_base(J) - boff + g * kGroup);
-    if (b0 + len > n)
-        far_segment_rot<UM, SOFT, true>(xs, n, b0, nchunks, J, o, H2, lane, bp, m);
-    else
-        far_segment_rot<UM, SOFT, false>(xs, n, b0, nchunks, J, o, H2, lane, bp, m);
-    far_fold_own<UM>(o, m, lane);
+    const int end = min(b1, n);
+    if (b0 >= end) {  // a share of the last group past n: zeros in its fragment
+        far_fold_own<UM>(o, m, lane);
+        return;
+    }
+    float* bp = nullptr;  // row g's partials of the chunk's first partner, for this lane
+    int terms = 0;
+    float4 A = load_partner_row<UM>(xs, b0, n, lane);
+    for (int b = b0; b < end; b += kRow) {
+        if (b == b0 || b % kGroup == 0)
+            bp = bpart + 3 * (bpart_group_base(b / kGroup) - boff + g * kGroup + b % kGroup) +
+                 3 * (lane & (kRow - 1)) + partner_comp_rot(lane);
+        const float4 B = load_partner_row<UM>(xs, b + kRow, n, lane);  // unused after the last
+        if (b + kRow > end) A = bound_partner_row(A, b, n, lane);
+        const float v = far_chunk_rot<UM, SOFT>(A, o, H2);
+        *bp = UM ? v * m : v;
+        bp += 3 * kRow;
+        A = B;
+        terms += kRow;
+        if (terms == fold || b + kRow >= end) {
+            far_fold_own<UM>(o, m, lane);
+            terms = 0;
+        }
+    }
 }
 
 // Far field of one instance, or (COL) column batch [c0, c1) of its partner
 // groups.  Workgroup k of W takes the units [k U / W, (k + 1) U / W) of the
 // rows g (group g against its later groups, or those in the batch, each cut
-// into Q pieces) laid end to end; its own-side sums of row g go to fragment
-// g + k (plain: no workgroup has more than kFoldsPerFlush units).  The
-// whole far field keeps a kernel of its own (far_kernel), so the row
-// arithmetic of the batches does not change its code.
-template <bool UM, bool SOFT, int QC, bool COL>
+// into Q pieces) laid end to end: consecutive partners, row by row.  Its
+// own-side sums of row g go to fragment g + k (plain: every fragment is
+// flushed once).  The whole far field keeps a kernel of its own (far_kernel),
+// so the row arithmetic of the batches does not change its code.
+template <bool UM, bool SOFT, bool COL>
 __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const int n, const int64_t nsb, const int c0,
-                                         const int c1, const int64_t U, const int W, const int Qr,
+                                         const int c1, const int64_t U, const int W, const int Q, const int fold,
                                          float4* __restrict__ apart, const bool plain, float* __restrict__ bpart,
                                          const float H2, const float m, float* lsum)
 {
-    const int Q = QC ? QC : Qr;
-    const int k = blockIdx.x, lane = threadIdx.x;
-    const int64_t u0 = (int64_t)k * U / W, u1 = (int64_t)(k + 1) * U / W;
-    if (u0 >= u1) return;
+    const int k = blockIdx.x, lane = threadIdx.x, len = kSB / Q;
+    int64_t u = (int64_t)k * U / W;
+    const int64_t u1 = (int64_t)(k + 1) * U / W;
+    if (u >= u1) return;
     const int64_t boff = COL ? bpart_group_base(c0) : 0;
-    int64_t g = COL ? col_row_of_unit(u0, c0, c1, Q) : row_of_unit(u0, nsb, Q);
-    int64_t s = u0 - (COL ? col_row_prefix(g, c0, c1, Q) : row_prefix(g, nsb, Q));
+    int64_t g = COL ? col_row_of_unit(u, c0, c1, Q) : row_of_unit(u, nsb, Q);
+    int64_t s = u - (COL ? col_row_prefix(g, c0, c1, Q) : row_prefix(g, nsb, Q));  // first unit within row g
     FarOwn o;
-    far_load_row(xs, n, g, lane, lsum, apart + (size_t)kFragElems * (g + k), plain, o);
-    for (int64_t u = u0; u < u1; ++u) {
-        if (s == (COL ? col_row_units(g, c0, c1, Q) : row_units(g, nsb, Q))) {
-            far_flush_own(o, lane);
-            ++g;
-            s = 0;
-            far_load_row(xs, n, g, lane, lsum, apart + (size_t)kFragElems * (g + k), plain, o);
-        }
-        const int J = (int)((COL ? col_first_group(g, c0) : g + 1) + s / Q);
-        far_unit<UM, SOFT, QC>(xs, n, g, J, (int)(s % Q), Q, o, bpart, boff, H2, m, lane);
-        ++s;
+    for (; u < u1; ++g, s = 0) {
+        const int64_t row = COL ? col_row_units(g, c0, c1, Q) : row_units(g, nsb, Q);
+        const int64_t cnt = min(row - s, u1 - u);
+        const int first = kSB * (int)(COL ? col_first_group(g, c0) : g + 1) + len * (int)s;
+        far_load_row(xs, n, g, lane, lsum, apart + (size_t)kFragElems * (g + k), plain, o);
+        far_range<UM, SOFT>(xs, n, g, first, first + len * (int)cnt, fold, o, bpart, boff, H2, m, lane);
+        far_flush_own(o, lane);
+        u += cnt;
     }
-    far_flush_own(o, lane);
 }
 
 template <bool SOFT, bool COL>
 __device__ __forceinline__ void far_dispatch(const float4* __restrict__ xs, const int n, const int64_t nsb,
                                              const int c0, const int c1, const int64_t U, const int W, const int Q,
-                                             float4* __restrict__ apart, const int plain,
+                                             const int fold, float4* __restrict__ apart, const int plain,
                                              float* __restrict__ bpart, const float H2,
                                              const float* __restrict__ umass, float* lsum)
 {
-    const bool um = umass[0] != 0.0f;
-    if (Q == 2) {
-        if (um)
-            far_work<true, SOFT, 2, COL>(xs, n, nsb, c0, c1, U, W, 2, apart, plain, bpart, H2, umass[1], lsum);
-        else
-            far_work<false, SOFT, 2, COL>(xs, n, nsb, c0, c1, U, W, 2, apart, plain, bpart, H2, 1.0f, lsum);
-    } else {
-        if (um)
-            far_work<true, SOFT, 0, COL>(xs, n, nsb, c0, c1, U, W, Q, apart, plain, bpart, H2, umass[1], lsum);
-        else
-            far_work<false, SOFT, 0, COL>(xs, n, nsb, c0, c1, U, W, Q, apart, plain, bpart, H2, 1.0f, lsum);
-    }
+    if (umass[0] != 0.0f)
+        far_work<true, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, umass[1], lsum);
+    else
+        far_work<false, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, 1.0f, lsum);
 }
 
 template <bool SOFT>
 __global__ __launch_bounds__(kFarThreads, 2) void far_kernel(const float4* __restrict__ xs, const int n,
                                                             const int64_t nsb, const int64_t U, const int W,
-                                                            const int Q, float4* __restrict__ apart,
-                                                            const int plain, float* __restrict__ bpart,
-                                                            const float H2, const float* __restrict__ umass)
+                                                            const int Q, const int fold,
+                                                            float4* __restrict__ apart, const int plain,
+                                                            float* __restrict__ bpart, const float H2, const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
-    far_dispatch<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, apart, plain, bpart, H2, umass, lsum);
+    far_dispatch<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, bpart, H2, umass, lsum);
 }
 
 // one column batch [c0, c1) of the far field
 template <bool SOFT>
 __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4* __restrict__ xs, const int n,
                                                                    const int c0, const int c1, const int64_t U,
-                                                                   const int W, const int Q,
+                                                                   const int W, const int Q, const int fold,
                                                                    float4* __restrict__ apart, const int plain,
                                                                    float* __restrict__ bpart, const float H2,
                                                                    const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
-    far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, apart, plain, bpart, H2, umass, lsum);
+    far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, umass, lsum);
 }
 
 // Per slot, in a fixed order: the in-group sums, the far own-side fragments
@@ -569,7 +556,7 @@ __global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4*
 }
 
 // one piece of a far row of an instance of the batch: group R.g against
-// R.units partner groups from j0 on, two pieces of 512 partners each
+// R.units partner groups from j0 on
 template <bool UM, bool SOFT>
 __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, const int n, const SymRow R, const int j0,
                                               float* lsum, float4* frag, const bool plain, float* __restrict__ bk,
@@ -577,8 +564,7 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
 {
     FarOwn o;
     far_load_row(xk, n, R.g, lane, lsum, frag, plain, o);
-    for (int s = 0; s < 2 * R.units; ++s)
-        far_unit<UM, SOFT, 2>(xk, n, R.g, j0 + (s >> 1), s & 1, 2, o, bk, 0, H2, m, lane);
+    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kFarFoldLarge, o, bk, 0, H2, m, lane);
     far_flush_own(o, lane);
 }
 
@@ -690,16 +676,22 @@ int sym_default_workgroups(int cus)
     return std::max(1, 8 * cus / kGroupSB);  // 2 wavefronts per SIMD
 }
 
+// the most folds a workgroup makes in one row of `units` units cut among wgs
+// workgroups (far_range: one for every `fold` partners)
+static int64_t far_folds(int64_t units, int wgs, int split, int fold)
+{
+    return ((units + wgs - 1) / wgs * (kSB / split) + fold - 1) / fold;
+}
+
 // one column batch's units, far workgroups (of `wanted`) and fragment kind
-SymCol sym_column(int64_t nsb, int split, int wanted, int c0, int c1)
+SymCol sym_column(int split, int fold, int wanted, int c0, int c1)
 {
     SymCol C;
     C.c0 = c0;
     C.c1 = c1;
     C.units = col_row_prefix(col_rows(c1), c0, c1, split);
     C.wgs = far_workgroups(wanted, C.units);
-    C.plain = fragments_plain((C.units + C.wgs - 1) / C.wgs);
-    (void)nsb;
+    C.plain = fragments_plain(far_folds(C.units, C.wgs, split, fold));
     return C;
 }
 
@@ -713,7 +705,7 @@ SymGeom sym_geometry(int64_t n, int wgs, int64_t col_elems)
     G.wgs = far_workgroups(wgs, G.units);
     G.near_elems = 2 * n;
     G.apart_elems = (int64_t)kFragElems * (G.groups + wgs);
-    G.plain = fragments_plain((G.units + G.wgs - 1) / G.wgs);
+    G.plain = fragments_plain(far_folds(G.units, G.wgs, G.split, far_fold(n)));
     G.bpart_elems = 3 * bpart_group_base(G.groups);
     G.ncols = 1;
     if (G.bpart_elems > col_elems) {
@@ -746,7 +738,7 @@ template <bool SOFT>
 void launch_far_column(const SymLaunch& L, const SymCol& C, const int split, const DevParams& P, hipStream_t s)
 {
     hipLaunchKernelGGL((far_column_kernel<SOFT>), dim3(C.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, C.c0, C.c1,
-                       C.units, C.wgs, split, L.apart, C.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                       C.units, C.wgs, split, far_fold(L.n), L.apart, C.plain ? 1 : 0, L.bpart, P.H2, L.umass);
 }
 
 void launch_column_combine(const SymLaunch& L, const SymCol& C, const int split, const bool first, const bool last,
@@ -768,15 +760,15 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
     if (G.ncols == 1) {
         if (P.H2 > 0.0f)
             hipLaunchKernelGGL((far_kernel<true>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                               L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         else
             hipLaunchKernelGGL((far_kernel<false>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                               L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         return hipGetLastError();
     }
     const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
     for (int b = 0; b < G.ncols; ++b) {
-        const SymCol C = sym_column(G.nsb, G.split, L.wgs, c[b], c[b + 1]);
+        const SymCol C = sym_column(G.split, far_fold(L.n), L.wgs, c[b], c[b + 1]);
         if (P.H2 > 0.0f) launch_far_column<true>(L, C, G.split, P, s); else launch_far_column<false>(L, C, G.split, P, s);
         if (b + 1 < G.ncols) launch_column_combine(L, C, G.split, b == 0, false, P, s);
     }
@@ -791,7 +783,7 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
     if (G.ncols > 1 && sym_has_far(L)) {
         // the last column batch's combine, which finishes
         const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
-        const SymCol C = sym_column(G.nsb, G.split, L.wgs, c[G.ncols - 1], c[G.ncols]);
+        const SymCol C = sym_column(G.split, far_fold(L.n), L.wgs, c[G.ncols - 1], c[G.ncols]);
         launch_column_combine(L, C, G.split, false, true, P, s);
         return hipGetLastError();
     }
@@ -840,7 +832,7 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
             for (int h = 0; h < batch_row_pieces(u); ++h) {
                 const int units = (int)(batch_piece_begin(u, h + 1) - batch_piece_begin(u, h));
                 T.rows.push_back(SymRow{k, g, h, units});
-                T.plain = T.plain && fragments_plain(2 * (int64_t)units);  // two far units per partner group
+                T.plain = T.plain && fragments_plain((int64_t)units * kGroup / kFarFoldLarge);
             }
         }
         row0 += S.nrows;

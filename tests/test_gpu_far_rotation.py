@@ -33,3 +33,27 @@ def test_far_pairs_match_fp64(n, uniform):
     # a slot adds at most 512 terms in plain FP32 before they are compensated: random-walk rounding of
     # sqrt(512) half-ulps is 7e-7 of the partial sums, a tenth of that norm-wise over ~10 partials
     assert mx < 1e-5 and norm < 1e-6, (mx, norm)
+
+
+# Rows cut into shares of 16 partners: a last group of one particle (all its
+# shares but one lie past the end), of one whole chunk, of one particle more;
+# folds every 128 partners (below 131072 particles) and every 512 (from there),
+# against the one-sided sweep, which is compensated.
+@pytest.mark.parametrize("n", [17 * 1024 + 1, 18 * 1024 + 16, 18 * 1024 + 17, 131071, 128 * 1024 + 1])
+def test_far_shares(n):
+    print("far shares n=%d" % n, flush=True)
+    h, prm = ics.plummer(n, seed=n)
+    h["posm"][:, 3] *= np.random.default_rng(n).uniform(0.5, 2.0, size=n).astype(np.float32)
+    out = []
+    for symmetric in (1, 0):
+        ctx = g.Context(0)
+        ctx.set_option("sweep_symmetric", symmetric)
+        d = g.DeviceParticles.from_host(h)
+        ctx.compute_derivatives(d, prm)
+        g.hip.synchronize()
+        out.append(d.download(["acc"])["acc"])
+        d.free()
+        ctx.close()
+    mx, norm = vec_errors(out[0], out[1])
+    # both sides within the bound above of the exact sums
+    assert mx < 2e-5 and norm < 1e-6, (mx, norm)
