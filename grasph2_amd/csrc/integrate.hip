@@ -172,9 +172,9 @@ __global__ __launch_bounds__(kBlock) void vts_kick_kernel(float4* __restrict__ v
         v.y = v.y + a.y * h;
         v.z = v.z + a.z * h;
         vel[i] = make_float4(v.x, v.y, v.z, 0.0f);
-        if (P.flags & GRASPH_ACCELERATION_CRITERION) {  // :149-151
-            const float la = __fsqrt_rn(dist2_exact(a.x, a.y, a.z));  // length(acc), products and sums unfused
-            mindt = fminf(mindt, __fsqrt_rn(__fdiv_rn(mul_exact(P.acc_acc, P.H), la)));
+        if (P.flags & GRASPH_ACCELERATION_CRITERION) {  // :149-151; sqrtf rounds correctly, __fsqrt_rn does not
+            const float la = sqrtf(dist2_exact(a.x, a.y, a.z));  // length(acc), products and sums unfused
+            mindt = fminf(mindt, sqrtf(__fdiv_rn(mul_exact(P.acc_acc, P.H), la)));
         }
         if (P.flags & GRASPH_VELOCITY_CRITERION)  // :152-154
             mindt = fminf(mindt, __fdiv_rn(mul_exact(P.vel_acc, P.H), maxvsig[i]));
