@@ -561,6 +561,7 @@ int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
     N.nbr = b.d_nbr;
     N.nbr_cnt = b.d_cnt;
     N.n = (int)b.ntotal;
+    N.lanes = 4;
     N.kmax = b.kmax;
     N.balsara = p->balsara;
     N.density_dt = p->density_dt;

@@ -238,6 +238,15 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
     return L;
 }
 
+// Lanes per particle of the passes: 16 while the particles' 4 would leave the
+// GPU's SIMDs idle, 4 from there (16 lanes walk short lists in few, partly
+// empty steps).  Passes called one by one / SPH without gravity, 16 against 4
+// lanes: 4096 particles 119 against 139 us / 47 against 57, 8192 144 against
+// 159 / 54 against 59, 11000 198 against 209 / 63 against 59, 16384 213
+// against 222 / 64 against 60.
+constexpr int64_t kPassLanes16Max = 10240;
+int pass_lanes(int64_t n) { return n <= kPassLanes16Max ? 16 : 4; }
+
 NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
 {
     NbrLaunch L;
@@ -251,9 +260,7 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
     L.nbr = c.nbr;
     L.nbr_cnt = c.nbr_cnt;
     L.n = (int)p->n;
-    // long lists (a capacity grown past 512 after contact): 4 lanes per
-    // particle, 4 times the wavefronts to hide the gathers' latency
-    L.sub = c.max_neighbours > 512 ? 4 : 1;
+    L.lanes = pass_lanes(L.n);
     L.kmax = c.max_neighbours;
     L.balsara = p->balsara;
     L.density_dt = p->density_dt;

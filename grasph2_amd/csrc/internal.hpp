@@ -356,10 +356,11 @@ __device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_bl
     SlotMap m;
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
     if (BATCH) {
-        const int4 b = T.blk[blk];
+        const int parts = 256 / slots_per_block;  // blocks per entry of the table
+        const int4 b = T.blk[blk / parts];
         const BatchInst I = T.insts[b.x];
         m.inst = b.x;
-        m.slot0 = b.y;
+        m.slot0 = b.y + blk % parts * slots_per_block;
         m.slot_end = b.z;
         m.off = I.off;
         m.n = I.n;
@@ -478,7 +479,7 @@ struct NbrLaunch {
     float4* xvel;
     float* maxvsig;
     bool acc_has_gravity;
-    int sub;        // lanes per particle in the passes (one instance only): 1 or 4
+    int lanes;      // lanes per particle in the list passes: 4 or, in one instance, 16
     BlockTables T;  // batch tables (T.nblocks == 0 for one instance)
 };
 hipError_t launch_density(const NbrLaunch& L, float* density, const DevParams& P, hipStream_t s);

@@ -11,16 +11,25 @@
 //          environmentAcceleration (:300-312), added to the gravity the
 //          sweep left in acc with compensated (TwoSum) accumulation.
 //
-// One particle per lane in Morton order (slot t -> i = perm[t]).  Every
-// input a pass reads for a neighbour sits in one 64-byte slot record,
-// rec[j] = {x y z m, vx vy vz rho, sigma/rho^2 (6) balsara rho}, in slot
-// order: one neighbour costs one contiguous gather, and a particle's
+// Several lanes share a particle, particles in slot order (slot t ->
+// i = perm[t]).  Every input a pass reads for a neighbour sits in one 64-byte
+// slot record, rec[j] = {x y z m, vx vy vz rho, sigma/rho^2 (6) balsara rho},
+// in slot order: one neighbour costs one contiguous gather, and a particle's
 // neighbours' records are close together in memory.  Outputs go to
 // particle i of the caller's arrays.  The list is stored in tiles of 64
-// slots (list_entry), so a wavefront's loads of its k-th neighbours are
-// contiguous, and holds slot indices in increasing order.  A particle whose
-// count exceeds the list capacity falls back to a scan over its instance's
-// slots with the exact neighbour test, so a full list never loses partners.
+// slots (list_entry) and holds slot indices in increasing order.  A particle
+// whose count exceeds the list capacity falls back to a scan over its
+// instance's slots with the exact neighbour test, so a full list never loses
+// partners.
+//
+// What bounds them: a pass mixes FP64 and FP32 work, so every vector
+// instruction takes about 4 clocks, and the acceleration pass's gathers look
+// up 4 lines of the vector cache per pair, a line per clock and CU: at 200003
+// particles 188000 of its 200000 clocks (fetching each record by 4 lanes
+// together and exchanging the pieces through LDS halves the look-ups, but the
+// exchange's instructions cost what that gives).  Density and strain are
+// bound by their instructions.  At small counts a wavefront is alone on its
+// SIMD (5.5 clocks per instruction) and the lanes per particle decide.
 //
 // Every kernel serves one instance (SlotMap from the kernel arguments) or a
 // batch (SlotMap and parameters of the block's instance from tables).
@@ -28,15 +37,23 @@
 
 // No multiply-add contraction in this file: the pair arithmetic is inlined
 // into the list walk and into the overflow scan, and contraction decided per
-// call site could round the two differently.  Every product and sum rounds
-// as written, as in the FP32 oracle; the passes are bound by their gathers,
-// not by arithmetic.
+// call site could round the two differently.  Products and sums round as
+// written, and fused ones are written as such.
 #pragma clang fp contract(off)
 
 namespace grasph {
 namespace {
 
-constexpr int kBlock = 256;
+constexpr int kBlock = 256, kWaves = kBlock / 64;
+// steps in flight of each pass's walk (for_each_neighbour's D): what hides
+// their latency is wavefronts, and a deeper ring costs them registers
+// (density 48 -> 38 us, strain 101 -> 74, acceleration 101 -> 89 at 200003
+// particles, half of it from dropping 4, 2 and 2 steps to these)
+constexpr int kDeepDensity = 2, kDeepStrain = 1, kDeepAccel = 1;
+
+// lambdas are inlined by force: called from the list walk and the overflow
+// scan, they would otherwise stay calls and pass the records through scratch
+#define GRASPH_INLINE __attribute__((always_inline))
 
 struct Tens {  // full 3x3, row-major, as mpu::Mat<float,3,3>
     float m[3][3];
@@ -70,103 +87,170 @@ struct Lists {
     const int* cnt;
 };
 
+// LPP lanes share a particle (4 or 16): lane l of a wavefront serves
+// particle l / LPP of the wavefront's 64 / LPP, and in step e of the walk
+// neighbour e LPP + l % LPP of its list.  The terms are then added in the
+// list's order whatever LPP is (OrderedSums), so the sums do not depend on
+// it: a batch's equal the single instance's bit for bit, and a list's those
+// of its overflow scan.  Against one lane per particle: 4 to 16 times the
+// wavefronts for small counts (8192 particles: density, strain and
+// acceleration 76 -> 27 us), lists of 16 or 4 particles instead of 64 to wait
+// for, and neighbouring lanes read neighbouring records (512 instances:
+// 4.7 -> 3.9 ms).
+template <int LPP>
+__device__ __forceinline__ int pass_slot(const SlotMap& m)
+{
+    return m.slot0 + (int)threadIdx.x / LPP;
+}
+
+// Orders the wavefront's LDS accesses around it (the hardware executes one
+// wavefront's in order; the compiler must not move them).
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ void acc_add(CSum& a, float v) { a.add(v); }
+__device__ __forceinline__ void acc_add(float& a, float v) { a += v; }
+__device__ __forceinline__ void acc_add(double& a, double v) { a += v; }
+__device__ __forceinline__ float acc_value(const CSum& a) { return a.value(); }
+__device__ __forceinline__ float acc_value(float a) { return a; }
+__device__ __forceinline__ double acc_value(double a) { return a; }
+
+// NC running sums of a particle (A: the accumulator of terms of type T), the
+// terms added in the order of the neighbours: the lanes of a particle write
+// their terms to LDS (kRow apart, so the components' rows start in different
+// banks) and lane s adds all LPP terms of the components s, s + LPP, ....
+template <int LPP, int NC, typename T, typename A>
+struct OrderedSums {
+    static constexpr int K = (NC + LPP - 1) / LPP;
+    static constexpr int kRow = 64 + 16 / (int)sizeof(T);
+    static constexpr int kLds = NC * kRow;  // elements of T per wavefront
+    A a[K];
+
+    // the component of accumulator k (lanes without one repeat the last)
+    __device__ __forceinline__ static int comp(int sub, int k) { return min(sub + k * LPP, NC - 1); }
+    // the step's terms (this lane's in v) of the group's first `rem` lanes
+    __device__ __forceinline__ void add(const T (&v)[NC], const int rem, T* lds, const int lane)
+    {
+        const int sub = lane % LPP;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) lds[c * kRow + lane] = v[c];
+        wave_lds_order();
+        T w[K][LPP];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const T* row = (const T*)__builtin_assume_aligned(lds + comp(sub, k) * kRow + (lane - sub), 16);
+#pragma unroll
+            for (int u = 0; u < LPP; ++u) w[k][u] = row[u];
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int u = 0; u < LPP; ++u)
+            if (u < rem) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) acc_add(a[k], w[k][u]);
+            }
+    }
+    // one neighbour's terms, the same in every lane of the group
+    __device__ __forceinline__ void add_one(const T (&v)[NC], T* lds, const int lane)
+    {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) lds[c * kRow + lane] = v[c];
+#pragma unroll
+        for (int k = 0; k < K; ++k) acc_add(a[k], lds[comp(lane % LPP, k) * kRow + lane]);
+    }
+    // sum c, in every lane of the group (all lanes of the wavefront take part)
+    __device__ __forceinline__ T value(const int c, const int lane) const
+    {
+        return __shfl(acc_value(a[c / LPP]), lane - lane % LPP + c % LPP, 64);
+    }
+};
+
+// four floats that the compiler keeps in registers through the walk's rings
+// (float4, a class, it copies as 16 bytes of memory, through scratch)
+typedef float vec4 __attribute__((ext_vector_type(4)));
+
 // Walk slot t's neighbours: the list, or when it overflowed, a scan of the
 // instance's slots with the exact test (same partners, same order).
-// load(j) fetches what body(j, data) needs; the walk is software-pipelined
-// D deep: while partner e is computed, the data of partners e+1 .. e+D-1
-// and the indices up to e+2D-1 are in flight (slot u of the rings holds
-// the partners e with e mod D = u).  The look-ahead past the end reloads
-// the last partner (always in range).  Deeper rings hide more of the gather
-// latency where few wavefronts share a SIMD (one instance: 2048 wavefronts
-// at 131072 particles), shallower ones keep the registers low where many
-// do (batches).
-template <int D, int SUB, typename L, typename F>
-__device__ __forceinline__ void for_each_neighbour(const float4* __restrict__ xs, const Lists& Ls,
-                                                   const size_t nstride, const int t, const int kmax,
-                                                   const float4 pi, const SlotMap& m, const float H2, const int sub,
-                                                   L&& load, F&& body)
+// step(q, rem): q holds the first PIECES float4 of the neighbour's record (of
+// STRIDE float4 at src); lane sub has one if sub < rem (the others repeat the
+// last).  one(q): a neighbour found by the scan, the same for the whole group.
+//
+// The walk is software-pipelined D deep: while step e is computed, the
+// records of steps e + 1 .. e + D and the indices up to e + 2 D are in
+// flight.  A group past its list's end is masked off; within its last steps
+// its lanes repeat the last neighbour.
+template <int D, int LPP, int PIECES, int STRIDE, typename S, typename O>
+__device__ __forceinline__ void for_each_neighbour(const vec4* __restrict__ src, const float4* __restrict__ xs,
+                                                   const Lists& Ls, const int t, const bool act, const int kmax,
+                                                   const float4 pi, const SlotMap& m, const float H2, S&& step,
+                                                   O&& one)
 {
+    const int lane = threadIdx.x & 63, sub = lane % LPP;
     const int cnt = Ls.cnt[t];
-    if (cnt <= kmax) {
-        // this lane's share of the list: entries sub, sub + SUB, ...
-        const int cl = cnt > sub ? (cnt - 1 - sub) / SUB + 1 : 0;
-        if (cl <= 0) return;
-        const int* list = Ls.nbr + list_entry(t, sub, kmax);
-        constexpr size_t kStride = 64 * SUB;
-        const int last = cl - 1;
-        int jcur[D], jnx[D];
-        decltype(load(0)) dd[D];
+    const int c = act && cnt <= kmax ? cnt : 0;
+    // what a lane reads past its list's end is some slot of the instance: the
+    // list's last entry (a lane without a list walks entry 0 of slot t's
+    // overflowed one, or reads slot 0 from a count of 0)
+    const int* list = cnt > 0 ? Ls.nbr + list_entry(t, 0, kmax) : Ls.cnt + t;
+    const int last = max(c - 1, 0);
+    const auto index = [&](int e) GRASPH_INLINE { return list[64 * (uint64_t)(uint32_t)min(e * LPP + sub, last)]; };
+    const auto fetch = [&](int j, vec4 (&r)[PIECES]) GRASPH_INLINE {
 #pragma unroll
-        for (int u = 0; u < D; ++u) jcur[u] = list[kStride * min(u, last)];
+        for (int q = 0; q < PIECES; ++q) r[q] = src[STRIDE * (uint64_t)(uint32_t)j + q];
+    };
+    int jn[D];
+    vec4 r[D][PIECES];
+    const auto turn = [&](int e, int& j, vec4 (&rr)[PIECES]) GRASPH_INLINE {
+        vec4 q[PIECES];
 #pragma unroll
-        for (int u = 0; u < D; ++u) jnx[u] = list[kStride * min(u + D, last)];
+        for (int p = 0; p < PIECES; ++p) q[p] = rr[p];
+        fetch(j, rr);  // step e + D (its indices came D steps ago)
+        j = index(e + 2 * D);
+        step(q, c - e * LPP);
+    };
 #pragma unroll
-        for (int u = 0; u < D; ++u) dd[u] = load(jcur[u]);
-        for (int k = 0; k < cl; k += D) {
+    for (int u = 0; u < D; ++u) jn[u] = index(u);
 #pragma unroll
-            for (int u = 0; u < D; ++u) {
-                const int e = k + u;
-                if (e < cl) body(jcur[u], dd[u]);
-                jcur[u] = jnx[u];
-                dd[u] = load(jcur[u]);  // partner e + D (its index came D partners ago)
-                jnx[u] = list[kStride * min(e + 2 * D, last)];
-            }
-        }
-    } else {
-        // the same share of the partners in slot order: the partner count
-        // picks the lane, so the sums split as over the list
-        int idx = 0;
-        for (int j = m.off; j < m.off + m.n; ++j) {
-            const float4 pj = xs[j];
-            if (is_neighbour(dist2_exact(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z), H2)) {
-                if (SUB == 1 || idx % SUB == sub) body(j, load(j));
-                ++idx;
-            }
+    for (int u = 0; u < D; ++u) {
+        fetch(jn[u], r[u]);
+        jn[u] = index(u + D);
+    }
+    for (int e = 0; e * LPP < c; e += D) {
+        turn(e, jn[0], r[0]);
+        if constexpr (D > 1) turn(e + 1, jn[1], r[1]);
+        if constexpr (D > 2) turn(e + 2, jn[2], r[2]);
+        if constexpr (D > 3) turn(e + 3, jn[3], r[3]);
+    }
+    if (act && cnt > kmax) {
+        const int end = m.off + m.n;
+        for (int j0 = m.off; j0 < end; j0 += LPP) {
+            const float4 pj = xs[min(j0 + sub, end - 1)];
+            const bool is = j0 + sub < end && is_neighbour(dist2_exact(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z), H2);
+            const auto found = [&](int j) GRASPH_INLINE {
+                vec4 q[PIECES];
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) q[p] = src[STRIDE * (size_t)j + p];
+                one(q);
+            };
+            // the group's lanes test LPP slots at once
+            unsigned b = (unsigned)(__ballot(is) >> (lane - sub)) & ((1u << LPP) - 1u);
+            for (; b != 0u; b &= b - 1u) found(j0 + __ffs(b) - 1);
         }
     }
 }
 
-// SUB lanes share a particle when its list is long (one instance, SUB = 4):
-// lane l of a wavefront serves particle l mod (64 / SUB) of the wavefront's
-// 64 / SUB and walks its neighbours sub, sub + SUB, ... (sub = l div (64 /
-// SUB)); the lanes' sums are then added in a fixed order (the lane with
-// sub = 0 adds sub 1's, then the sum of subs 2 and 3) and that lane writes.
-template <int SUB>
-__device__ __forceinline__ int pass_sub() { return (int)(threadIdx.x & 63) / (64 / SUB); }
-template <int SUB>
-__device__ __forceinline__ int pass_slot(const SlotMap& m)
-{
-    constexpr int kPPW = 64 / SUB;
-    return m.slot0 + (int)(threadIdx.x >> 6) * kPPW + (int)(threadIdx.x & 63) % kPPW;
-}
-template <int SUB>
-__device__ __forceinline__ void merge_subs(CSum& a)
-{
-#pragma unroll
-    for (int o = 64 / SUB; o < 64; o <<= 1) {
-        const float s = __shfl_xor(a.s, o, 64), c = __shfl_xor(a.c, o, 64);
-        a.add(s);
-        a.c += c;
-    }
-}
-template <int SUB, typename T>
-__device__ __forceinline__ void sum_subs(T& a)
-{
-#pragma unroll
-    for (int o = 64 / SUB; o < 64; o <<= 1) a = a + __shfl_xor(a, o, 64);
-}
-template <int SUB>
+template <int LPP>
 __device__ __forceinline__ void max_subs(float& a)
 {
 #pragma unroll
-    for (int o = 64 / SUB; o < 64; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
+    for (int o = 1; o < LPP; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
 }
 
-struct PV {  // position/mass and velocity/density of a partner
-    float4 pm, vr;
-};
-
-template <bool BATCH, int SUB>
+template <bool BATCH, int LPP>
 __global__ __launch_bounds__(kBlock) void density_kernel(const float4* __restrict__ xs, SlotRec* __restrict__ rec,
                                                          const int* __restrict__ perm,
                                                          const Lists Ls,
@@ -174,103 +258,117 @@ __global__ __launch_bounds__(kBlock) void density_kernel(const float4* __restric
                                                          float* __restrict__ density, const BlockTables T,
                                                          const DevParams P0)
 {
-    // batches, and the long lists of bodies in contact (SUB > 1): issue
-    // ahead of the far field's wavefronts that run beside (ensemble of 512:
-    // 16.25-16.30 -> 15.98-16.16 ms per step; collision N = 131072 after
-    // impact: 5.59-5.62 -> 5.03-5.23)
-    if (BATCH || SUB > 1) __builtin_amdgcn_s_setprio(3);
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / SUB);
-    const int t = pass_slot<SUB>(m), sub = pass_sub<SUB>();
-    const bool act = t < m.slot_end;
-    if (SUB == 1 && !act) return;
-    const int tc = act ? t : m.slot0;  // lanes past the end take part in the lanes' sums only
+    using Rho = OrderedSums<LPP, 1, float, CSum>;
+    __shared__ __attribute__((aligned(16))) float terms[kWaves][Rho::kLds];
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
+    const bool act = t0 < m.slot_end;
+    const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges
+    float* const lt = terms[threadIdx.x >> 6];
     const DevParams P = BATCH ? T.prm[m.inst] : P0;
-    const int i = perm ? perm[tc] : tc;
-    const float4 pi = xs[tc];  // positions from the compact slot-ordered array (16 B per partner)
-    CSum rho{0.0f, 0.0f};
-    if (act)
-        for_each_neighbour<SUB == 1 && !BATCH ? 4 : 2, SUB>(xs, Ls, nstride, t, kmax, pi, m, P.H2, sub,
-                                                           [&](int j) { return xs[j]; }, [&](int, const float4 pj) {
-            rho.add(pj.w * kernel_w_f64(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z, P));
+    const float4 pi = xs[t];  // positions from the compact slot-ordered array (16 B per partner)
+    Rho rho{};
+    const auto term = [&](const vec4 (&q)[1], float (&v)[1]) GRASPH_INLINE {
+        v[0] = q[0].w * kernel_w_f64(pi.x - q[0].x, pi.y - q[0].y, pi.z - q[0].z, P);
+    };
+    for_each_neighbour<kDeepDensity, LPP, 1, 1>(
+        (const vec4*)xs, xs, Ls, t, act, kmax, pi, m, P.H2,
+        [&](const vec4 (&q)[1], int rem) GRASPH_INLINE {
+            float v[1];
+            term(q, v);
+            rho.add(v, rem, lt, lane);
+        },
+        [&](const vec4 (&q)[1]) GRASPH_INLINE {
+            float v[1];
+            term(q, v);
+            rho.add_one(v, lt, lane);
         });
-    if (SUB > 1) {
-        merge_subs<SUB>(rho);
-        if (!act || sub != 0) return;
-    }
-    float r = rho.value();
+    float r = rho.value(0, lane);
+    if (!act || lane % LPP != 0) return;
     if ((P.flags & GRASPH_DEAL_WITH_NO_PARTNERS) && r < 0.001f) r = P.rho0 * 0.01f;  // :85-88
-    density[i] = r;
+    density[perm ? perm[t] : t] = r;
     rec[t].vr.w = r;  // the strain / record passes read densities from the slot records
 }
 
-template <bool BATCH, int SUB, bool SOLIDS, bool BALS, bool INTD>
+template <bool BATCH, int LPP, bool SOLIDS, bool BALS, bool INTD>
 __global__ __launch_bounds__(kBlock) void strain_kernel(
     const float4* __restrict__ xs, SlotRec* __restrict__ rec, const float* __restrict__ dstress,
     const int* __restrict__ perm, const Lists Ls, const size_t nstride, const int kmax, float* __restrict__ balsara,
     float* __restrict__ density_dt, float* __restrict__ dstress_dt, const BlockTables T, const DevParams P0)
 {
-    // batches, and the long lists of bodies in contact (SUB > 1): issue
-    // ahead of the far field's wavefronts that run beside (ensemble of 512:
-    // 16.25-16.30 -> 15.98-16.16 ms per step; collision N = 131072 after
-    // impact: 5.59-5.62 -> 5.03-5.23)
-    if (BATCH || SUB > 1) __builtin_amdgcn_s_setprio(3);
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / SUB);
-    const int t0 = pass_slot<SUB>(m), sub = pass_sub<SUB>();
-    const bool act = t0 < m.slot_end;
-    if (SUB == 1 && !act) return;
-    const int t = act ? t0 : m.slot0;  // lanes past the end take part in the lanes' sums only
-    const DevParams P = BATCH ? T.prm[m.inst] : P0;
-    const int i = perm ? perm[t] : t;
-    const float4 pi = rec[t].pm;
-    const float4 vi = rec[t].vr;
-    const float rhoi = vi.w;
-
     // Sums and terms in FP64 from the FP32 inputs: the velocity divergence
     // and curl cancel strongly where bodies meet, and the Balsara factor
     // built from them scales the artificial viscosity of the acceleration
-    // pass, where FP32 rounding here showed up amplified.
+    // pass, where FP32 rounding here showed up amplified.  Solids: the nine
+    // sums M_ab of vol v_a g_b, which hold the strain rate (-M's symmetric
+    // part, models.h:225-248), the rotation rate (-M's antisymmetric part)
+    // and div v (-M's trace); liquids: curl v with a Balsara switch, and div v
+    // where it is used.
+    constexpr int kRot = SOLIDS ? 9 : BALS ? 3 : 0;
+    constexpr int NC = kRot + (!SOLIDS && (BALS || INTD) ? 1 : 0);
+    constexpr int kTerms = NC > 0 ? NC : 1;
+    using Rates = OrderedSums<LPP, kTerms, double, double>;
+    __shared__ __attribute__((aligned(16))) double terms[kWaves][Rates::kLds];
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
+    const bool act = t0 < m.slot_end;
+    const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges
+    double* const lt = terms[threadIdx.x >> 6];
+    const DevParams P = BATCH ? T.prm[m.inst] : P0;
+    const int i = perm ? perm[t] : t;
+    const float4 pi = rec[t].pm;
+    const float4 vr = rec[t].vr;
+    const float rhoi = vr.w;
+    const struct { double x, y, z; } vi = {vr.x, vr.y, vr.z};
+
+    Rates R{};
+    const auto term = [&](const vec4 (&q)[2], double (&v)[kTerms]) GRASPH_INLINE {
+        const vec4 pj = q[0], vj = q[1];
+        const double rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
+        const double s = dw_over_r_f64(pair_sep(rx, ry, rz, P), P) * div_f64(pj.w, vj.w);  // vol = m_j / rho_j
+        const double gx = s * rx, gy = s * ry, gz = s * rz;
+        const double vx = vi.x - (double)vj.x, vy = vi.y - (double)vj.y, vz = vi.z - (double)vj.z;
+        if constexpr (SOLIDS) {
+            v[0] = vx * gx; v[1] = vx * gy; v[2] = vx * gz;
+            v[3] = vy * gx; v[4] = vy * gy; v[5] = vy * gz;
+            v[6] = vz * gx; v[7] = vz * gy; v[8] = vz * gz;
+        } else {
+            if constexpr (BALS) {  // curl v, computeDerivatives.h:134
+                v[0] = __builtin_fma(vy, gz, -(vz * gy));
+                v[1] = __builtin_fma(vz, gx, -(vx * gz));
+                v[2] = __builtin_fma(vx, gy, -(vy * gx));
+            }
+            if constexpr (BALS || INTD) v[NC - 1] = -__builtin_fma(vz, gz, __builtin_fma(vy, gy, vx * gx));  // :137
+        }
+        if constexpr (NC == 0) v[0] = 0.0;
+    };
+    for_each_neighbour<kDeepStrain, LPP, 2, 4>(
+        (const vec4*)rec, xs, Ls, t, act, kmax, pi, m, P.H2,
+        [&](const vec4 (&q)[2], int rem) GRASPH_INLINE {
+            double v[kTerms];
+            term(q, v);
+            R.add(v, rem, lt, lane);
+        },
+        [&](const vec4 (&q)[2]) GRASPH_INLINE {
+            double v[kTerms];
+            term(q, v);
+            R.add_one(v, lt, lane);
+        });
     double exx = 0, eyy = 0, ezz = 0, exy = 0, exz = 0, eyz = 0;  // strain rate (symmetric)
     double rxy = 0, rxz = 0, ryz = 0;                              // rotation rate (antisymmetric)
     double divv = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-
-    if (act)
-    for_each_neighbour<SUB == 1 && !BATCH ? 4 : 2, SUB>(xs, Ls, nstride, t, kmax, pi, m, P.H2, sub,
-                                                       [&](int j) { return PV{rec[j].pm, rec[j].vr}; },
-                                                       [&](int, const PV& q) {
-        const float4 pj = q.pm;
-        const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-        const double s = dw_over_r_f64(rx, ry, rz, P);
-        const double gx = s * (double)rx, gy = s * (double)ry, gz = s * (double)rz;
-        const float4 vj = q.vr;
-        const double vx = (double)vi.x - (double)vj.x, vy = (double)vi.y - (double)vj.y,
-                     vz = (double)vi.z - (double)vj.z;
-        const double vol = (double)pj.w / (double)vj.w;  // one division per pair, shared by the terms below
-        if (SOLIDS) {  // models.h:225-248
-            const double tmp = -0.5 * vol;
-            exx += tmp * (vx * gx + vx * gx);
-            exy += tmp * (vx * gy + vy * gx);
-            exz += tmp * (vx * gz + vz * gx);
-            eyy += tmp * (vy * gy + vy * gy);
-            eyz += tmp * (vy * gz + vz * gy);
-            ezz += tmp * (vz * gz + vz * gz);
-            rxy += tmp * (vx * gy - vy * gx);
-            rxz += tmp * (vx * gz - vz * gx);
-            ryz += tmp * (vy * gz - vz * gy);
-        } else if (BALS) {  // curl v, computeDerivatives.h:134
-            const double f = vol;
-            cx += f * (vy * gz - vz * gy);
-            cy += f * (vz * gx - vx * gz);
-            cz += f * (vx * gy - vy * gx);
-        }
-        if (BALS || INTD) divv -= vol * (vx * gx + vy * gy + vz * gz);  // :137
-    });
-    if (SUB > 1) {
-        sum_subs<SUB>(exx); sum_subs<SUB>(eyy); sum_subs<SUB>(ezz);
-        sum_subs<SUB>(exy); sum_subs<SUB>(exz); sum_subs<SUB>(eyz);
-        sum_subs<SUB>(rxy); sum_subs<SUB>(rxz); sum_subs<SUB>(ryz);
-        sum_subs<SUB>(divv); sum_subs<SUB>(cx); sum_subs<SUB>(cy); sum_subs<SUB>(cz);
-        if (!act || sub != 0) return;
+    if constexpr (SOLIDS) {
+        const double xy = R.value(1, lane), yx = R.value(3, lane), xz = R.value(2, lane), zx = R.value(6, lane),
+                     yz = R.value(5, lane), zy = R.value(7, lane);
+        exx = -R.value(0, lane); eyy = -R.value(4, lane); ezz = -R.value(8, lane);
+        exy = -0.5 * (xy + yx); exz = -0.5 * (xz + zx); eyz = -0.5 * (yz + zy);
+        rxy = -0.5 * (xy - yx); rxz = -0.5 * (xz - zx); ryz = -0.5 * (yz - zy);
+        if (BALS || INTD) divv = exx + eyy + ezz;
+    } else {
+        if constexpr (BALS) { cx = R.value(0, lane); cy = R.value(1, lane); cz = R.value(2, lane); }
+        if constexpr (BALS || INTD) divv = R.value(NC - 1, lane);
     }
+    if (!act || lane % LPP != 0) return;
 
     // do_after, computeDerivatives.h:144-161
     Tens S = sym_to_full(0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
@@ -345,23 +443,21 @@ __global__ __launch_bounds__(kBlock) void prep_kernel(SlotRec* __restrict__ rec,
     }
 }
 
-template <bool BATCH, int SUB, bool SOLIDS, bool BALS, bool AV, bool XSPH, bool ARTS>
+template <bool BATCH, int LPP, bool SOLIDS, bool BALS, bool AV, bool XSPH, bool ARTS>
 __global__ __launch_bounds__(kBlock) void accel_kernel(
     const float4* __restrict__ xs, const SlotRec* __restrict__ rec, const int* __restrict__ perm, const Lists Ls,
     const size_t nstride,
     const int kmax, float4* __restrict__ acc, float4* __restrict__ xvel, float* __restrict__ maxvsig,
     const int acc_has_gravity, const BlockTables T, const DevParams P0)
 {
-    // batches, and the long lists of bodies in contact (SUB > 1): issue
-    // ahead of the far field's wavefronts that run beside (ensemble of 512:
-    // 16.25-16.30 -> 15.98-16.16 ms per step; collision N = 131072 after
-    // impact: 5.59-5.62 -> 5.03-5.23)
-    if (BATCH || SUB > 1) __builtin_amdgcn_s_setprio(3);
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / SUB);
-    const int t0 = pass_slot<SUB>(m), sub = pass_sub<SUB>();
+    using Acc = OrderedSums<LPP, 3, float, CSum>;
+    using Xv = OrderedSums<LPP, 3, float, float>;
+    __shared__ __attribute__((aligned(16))) float terms[kWaves][(XSPH ? 2 : 1) * Acc::kLds];
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63, sub = lane % LPP;
     const bool act = t0 < m.slot_end;
-    if (SUB == 1 && !act) return;
-    const int t = act ? t0 : m.slot0;  // lanes past the end take part in the lanes' sums only
+    const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges
+    float* const lt = terms[threadIdx.x >> 6];
     const DevParams P = BATCH ? T.prm[m.inst] : P0;
     const int i = perm ? perm[t] : t;
     const float4 pi = rec[t].pm;
@@ -372,74 +468,89 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
     const float sxx = ra.x, syy = ra.y, szz = ra.z, sxy = ra.w, sxz = rb.x, syz = rb.y;
     const float arts_i = (ARTS && !SOLIDS) ? ((sxx > 0) ? (-P.mateps * sxx) : 0.0f) : 0.0f;
 
-    CSum ax{0.0f, 0.0f}, ay{0.0f, 0.0f}, az{0.0f, 0.0f};
-    if (acc_has_gravity && sub == 0) {
+    Acc A{};
+    Xv X{};
+    if (acc_has_gravity) {
         const float4 g = acc[i];
-        ax.s = g.x; ay.s = g.y; az.s = g.z;
+        A.a[0].s = sub == 0 ? g.x : sub == 1 ? g.y : g.z;
     }
     float mv = 0.0f;
-    float xvx = 0.0f, xvy = 0.0f, xvz = 0.0f;
 
-    if (act)
-    for_each_neighbour<SUB == 1 && !BATCH ? 4 : 2, SUB>(xs, Ls, nstride, t, kmax, pi, m, P.H2, sub,
-                                                       [&](int j) { return rec[j]; },
-                                                       [&](int, const SlotRec& q) {
-        const float4 pj = q.pm;
+    const auto term = [&](const vec4 (&q)[4], float (&f)[3], float (&x)[3], const bool counts) GRASPH_INLINE {
+        const vec4 pj = q[0], vj = q[1], qa = q[2], qb = q[3];
         const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-        const float r2 = dist2_exact(rx, ry, rz);
-        const float r = sqrtf(r2);
-        float gx, gy, gz;  // dW/r r_ij: FP64, rounded once (the pair terms cancel where the stresses are large)
-        kernel_gradient_f64(rx, ry, rz, P, gx, gy, gz);
-        const float4 qa = q.ra, qb = q.rb;
-        const float rhoj = qb.w;
+        // dW/r r_ij: FP64, rounded once (the pair terms cancel where the stresses are large)
+        const PairSep sep = pair_sep(rx, ry, rz, P);
+        const double s = dw_over_r_f64(sep, P);
+        const float gx = (float)(s * (double)rx), gy = (float)(s * (double)ry), gz = (float)(s * (double)rz);
+        const float rho2 = rhoi + qb.w, irho2 = AV || XSPH ? rcp_f32(rho2) : 0.0f;  // twice the mean density
         const float mj = pj.w;
-        float fx, fy, fz;
+        const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+        float II = 0.0f;
+        if (AV) {  // :277-289 (models.h:158-185)
+            const float wij = __builtin_fmaf(rz, vz, __builtin_fmaf(ry, vy, rx * vx)) * (float)sep.ir;
+            const float vsig = __builtin_fmaf(-3.0f, wij, P.c + P.c);
+            const float b = BALS ? bi + qb.z : 2.0f;
+            const float II0 = div_f32(-0.5f * P.alpha * b * wij * vsig, rho2, irho2);
+            II = wij < 0.0f ? II0 : 0.0f;
+            if (BALS && counts && wij < 0.0f) mv = fmaxf(mv, vsig);
+        }
         if (SOLIDS) {  // acc += m_j (stress . gradw), stress = sOR_i + sOR_j  (:260, :275)
             const float txx = sxx + qa.x, tyy = syy + qa.y, tzz = szz + qa.z;
             const float txy = sxy + qa.w, txz = sxz + qb.x, tyz = syz + qb.y;
-            fx = mj * (txx * gx + txy * gy + txz * gz);
-            fy = mj * (txy * gx + tyy * gy + tyz * gz);
-            fz = mj * (txz * gx + tyz * gy + tzz * gz);
+            f[0] = __builtin_fmaf(txz, gz, __builtin_fmaf(txy, gy, txx * gx));
+            f[1] = __builtin_fmaf(tyz, gz, __builtin_fmaf(tyy, gy, txy * gx));
+            f[2] = __builtin_fmaf(tzz, gz, __builtin_fmaf(tyz, gy, txz * gx));
         } else {
             float st = sxx + qa.x;
             if (ARTS) {  // :263-272 (liquid artificial pressure)
-                const float f = powf(w_spline(r, P.H, P.Wpref) / P.Wnorm, P.matexp);
+                const float r = sqrtf(dist2_exact(rx, ry, rz));
+                const float fa = powf(w_spline(r, P.H, P.Wpref) / P.Wnorm, P.matexp);
                 const float arts_j = (qa.x > 0) ? (-P.mateps * qa.x) : 0.0f;
-                st += f * (arts_i + arts_j);
+                st += fa * (arts_i + arts_j);
             }
-            fx = mj * (st * gx);
-            fy = mj * (st * gy);
-            fz = mj * (st * gz);
+            f[0] = st * gx;
+            f[1] = st * gy;
+            f[2] = st * gz;
         }
-        const float4 vj = q.vr;
-        const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-        if (AV) {  // :277-289
-            const float II = artificial_viscosity(BALS ? &mv : nullptr, P.alpha, rhoi, rhoj, vx, vy, vz, rx, ry, rz, r,
-                                                  P.c, P.c, bi, BALS ? qb.z : 1.0f);
-            const float mII = mj * II;
-            fx -= mII * gx;
-            fy -= mII * gy;
-            fz -= mII * gz;
+        if (AV) {
+            f[0] = __builtin_fmaf(-II, gx, f[0]);
+            f[1] = __builtin_fmaf(-II, gy, f[1]);
+            f[2] = __builtin_fmaf(-II, gz, f[2]);
         }
-        ax.add(fx);
-        ay.add(fy);
-        az.add(fz);
+        f[0] *= mj;
+        f[1] *= mj;
+        f[2] *= mj;
         if (XSPH) {  // :291-294
-            const float w = w_spline(r, P.H, P.Wpref);
-            const float f = 2.0f * mj / (rhoi + rhoj);
-            xvx += f * (vj.x - vi.x) * w;
-            xvy += f * (vj.y - vi.y) * w;
-            xvz += f * (vj.z - vi.z) * w;
+            const float qf = (float)sep.q, om = 1.0f - qf;
+            const float w = P.Wpref * (qf < 0.5f ? __builtin_fmaf(-6.0f * qf * qf, om, 1.0f) : 2.0f * om * om * om);
+            const float fx = div_f32(2.0f * mj, rho2, irho2) * w;
+            x[0] = -fx * vx;
+            x[1] = -fx * vy;
+            x[2] = -fx * vz;
         }
-    });
-    if (SUB > 1) {
-        merge_subs<SUB>(ax); merge_subs<SUB>(ay); merge_subs<SUB>(az);
-        if (BALS && AV) max_subs<SUB>(mv);
-        if (XSPH) { sum_subs<SUB>(xvx); sum_subs<SUB>(xvy); sum_subs<SUB>(xvz); }
-        if (!act || sub != 0) return;
+    };
+    for_each_neighbour<kDeepAccel, LPP, 4, 4>(
+        (const vec4*)rec, xs, Ls, t, act, kmax, pi, m, P.H2,
+        [&](const vec4 (&q)[4], int rem) GRASPH_INLINE {
+            float f[3], x[3];
+            term(q, f, x, sub < rem);
+            A.add(f, rem, lt, lane);
+            if constexpr (XSPH) X.add(x, rem, lt + Acc::kLds, lane);
+        },
+        [&](const vec4 (&q)[4]) GRASPH_INLINE {
+            float f[3], x[3];
+            term(q, f, x, true);
+            A.add_one(f, lt, lane);
+            if constexpr (XSPH) X.add_one(x, lt + Acc::kLds, lane);
+        });
+    float fx = A.value(0, lane), fy = A.value(1, lane), fz = A.value(2, lane);
+    float xvx = 0.0f, xvy = 0.0f, xvz = 0.0f;
+    if constexpr (XSPH) {
+        xvx = X.value(0, lane); xvy = X.value(1, lane); xvz = X.value(2, lane);
     }
-
-    float fx = ax.value(), fy = ay.value(), fz = az.value();
+    if (BALS && AV) max_subs<LPP>(mv);
+    if (!act || sub != 0) return;
     environment_acceleration(P, fx, fy, fz);
     acc[i] = make_float4(fx, fy, fz, 0.0f);
     if (maxvsig) maxvsig[i] = mv;
@@ -470,24 +581,23 @@ __global__ __launch_bounds__(kBlock) void finish_kernel(const float4* __restrict
 
 inline Lists lists_of(const NbrLaunch& L) { return Lists{L.nbr, L.nbr_cnt}; }
 
-inline int sub_of(const NbrLaunch& L) { return L.T.nblocks > 0 || L.sub <= 1 ? 1 : 4; }
 inline dim3 grid_plain(const NbrLaunch& L)  // per-particle kernels without a list walk
 {
     return dim3(L.T.nblocks > 0 ? L.T.nblocks : (L.n + kBlock - 1) / kBlock);
 }
 inline dim3 grid_of(const NbrLaunch& L)
 {
-    const int per = kBlock / sub_of(L);  // particles per block
-    return dim3(L.T.nblocks > 0 ? L.T.nblocks : (L.n + per - 1) / per);
+    const int per = kBlock / L.lanes;  // particles per block
+    return dim3(L.T.nblocks > 0 ? L.T.nblocks * L.lanes : (L.n + per - 1) / per);
 }
 
-template <bool BATCH, int SUB>
+template <bool BATCH, int LPP>
 hipError_t strain_b(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 {
     const bool so = P.flags & GRASPH_SOLIDS, ba = P.flags & GRASPH_BALSARA_SWITCH,
                in = P.flags & GRASPH_INTEGRATE_DENSITY;
 #define GRASPH_STRAIN(A, B, C)                                                                                     \
-    hipLaunchKernelGGL((strain_kernel<BATCH, SUB, A, B, C>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.dstress, \
+    hipLaunchKernelGGL((strain_kernel<BATCH, LPP, A, B, C>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.dstress, \
                        L.perm, lists_of(L), (size_t)L.n, L.kmax, L.balsara, L.density_dt, L.dstress_dt, L.T, P)
     const int key = (so ? 4 : 0) | (ba ? 2 : 0) | (in ? 1 : 0);
     switch (key) {
@@ -504,14 +614,14 @@ hipError_t strain_b(const NbrLaunch& L, const DevParams& P, hipStream_t s)
     return hipGetLastError();
 }
 
-template <bool BATCH, int SUB>
+template <bool BATCH, int LPP>
 hipError_t accel_b(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 {
     const bool so = P.flags & GRASPH_SOLIDS, ba = P.flags & GRASPH_BALSARA_SWITCH,
                av = P.flags & GRASPH_ARTIFICIAL_VISCOSITY, xs = P.flags & GRASPH_XSPH,
                ar = P.flags & GRASPH_ARTIFICIAL_STRESS;
 #define GRASPH_ACCEL(A, B, C, D, E)                                                                                  \
-    hipLaunchKernelGGL((accel_kernel<BATCH, SUB, A, B, C, D, E>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec,    \
+    hipLaunchKernelGGL((accel_kernel<BATCH, LPP, A, B, C, D, E>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec,    \
                        L.perm,                                                                                     \
                        lists_of(L), (size_t)L.n, L.kmax, L.acc, L.xvel, L.maxvsig, L.acc_has_gravity ? 1 : 0,  \
                        L.T, P)
@@ -553,23 +663,21 @@ hipError_t accel_b(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 hipError_t launch_density(const NbrLaunch& L, float* density, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0) return hipSuccess;
-    if (L.T.nblocks > 0)
-        hipLaunchKernelGGL((density_kernel<true, 1>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.perm, lists_of(L),
-                           (size_t)L.n, L.kmax, density, L.T, P);
-    else if (sub_of(L) == 4)
-        hipLaunchKernelGGL((density_kernel<false, 4>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.perm,
-                           lists_of(L), (size_t)L.n, L.kmax, density, L.T, P);
-    else
-        hipLaunchKernelGGL((density_kernel<false, 1>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.perm,
-                           lists_of(L), (size_t)L.n, L.kmax, density, L.T, P);
+#define GRASPH_DENSITY(BATCH, LPP)                                                                               \
+    hipLaunchKernelGGL((density_kernel<BATCH, LPP>), grid_of(L), dim3(kBlock), 0, s, L.xs, L.rec, L.perm, lists_of(L), \
+                       (size_t)L.n, L.kmax, density, L.T, P)
+    if (L.T.nblocks > 0) GRASPH_DENSITY(true, 4);
+    else if (L.lanes == 16) GRASPH_DENSITY(false, 16);
+    else GRASPH_DENSITY(false, 4);
+#undef GRASPH_DENSITY
     return hipGetLastError();
 }
 
 hipError_t launch_strain(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0) return hipSuccess;
-    if (L.T.nblocks > 0) return strain_b<true, 1>(L, P, s);
-    return sub_of(L) == 4 ? strain_b<false, 4>(L, P, s) : strain_b<false, 1>(L, P, s);
+    if (L.T.nblocks > 0) return strain_b<true, 4>(L, P, s);
+    return L.lanes == 16 ? strain_b<false, 16>(L, P, s) : strain_b<false, 4>(L, P, s);
 }
 
 hipError_t launch_prep(const NbrLaunch& L, const DevParams& P, hipStream_t s)
@@ -587,8 +695,8 @@ hipError_t launch_prep(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 hipError_t launch_accel(const NbrLaunch& L, const DevParams& P, hipStream_t s)
 {
     if (L.n <= 0) return hipSuccess;
-    if (L.T.nblocks > 0) return accel_b<true, 1>(L, P, s);
-    return sub_of(L) == 4 ? accel_b<false, 4>(L, P, s) : accel_b<false, 1>(L, P, s);
+    if (L.T.nblocks > 0) return accel_b<true, 4>(L, P, s);
+    return L.lanes == 16 ? accel_b<false, 16>(L, P, s) : accel_b<false, 4>(L, P, s);
 }
 
 hipError_t launch_finish(const NbrLaunch& L, const DevParams& P, hipStream_t s)

@@ -25,9 +25,10 @@ struct DevParams {
     float cand;  // d2 = r2 + H2 threshold that admits every pair with r2 <= H2
     // variable-step leapfrog, settings/settings.h:56-62
     float ts_init, ts_min, ts_max, acc_acc, vel_acc;
-    // FP64 constants of the passes' kernel and gradient: 1/H, the W and dW
-    // prefactors and the dW prefactor over H (SPH only, H > 0)
-    double invH64, Wpref64, dWpref64, dWprefH64;
+    // FP64 constants of the passes' kernel and gradient (SPH only, H > 0):
+    // 1/H; the W prefactor, times -6 and times 2; the dW prefactor over H
+    // times 3 and times -2, and the dW prefactor times -1
+    double invH64, Wpref64, Wi64, Wo64, dWq64, dW064, dWm64;
 };
 
 // Everything below rounds each product and sum as written, wherever it is
@@ -69,41 +70,74 @@ __host__ __device__ inline float dw_spline(float r, float h, float factor)
                                  : 0.0f);
 }
 
-// The kernel gradient g = dW(r)/r * r_ij (src/sph/kernel.h:169-175 over r)
-// of a pair at the FP32 separation (rx, ry, rz), evaluated in FP64 and
-// rounded once per component.  Where a particle's pair terms cancel (the
-// compressed zone of a contact), the half-dozen FP32 roundings of this
-// factor, amplified by the cancellation, dominated the acceleration error
-// against FP64; rounded once they leave a fifth of it.  For q < 1/2 the
-// factor is prefactor (3 q - 2) / H (q / r = 1 / H), for q >= 1/2
-// -prefactor (1 - q)^2 / r; both pieces meet at q = 1/2.
-__device__ inline double dw_over_r_f64(float rx, float ry, float rz, const DevParams& P)
+// 1 / sqrt(x) in FP64 to an ulp or two: the hardware's estimate (2^-23) and
+// one third-order step.  x > 0 (a neighbour's distance); 0 gives NaN.
+__device__ inline double rsqrt_f64(double x)
 {
-    const double x = rx, y = ry, z = rz;
-    const double r2 = (x * x + y * y) + z * z;
-    const double ir = rsqrt(r2);
-    const double q = r2 * ir * P.invH64;
-    const double om = 1.0 - q;
-    return (q < 0.5) ? P.dWprefH64 * (3.0 * q - 2.0) : -P.dWpref64 * (om * om) * ir;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-x * y, y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
 }
-__device__ inline void kernel_gradient_f64(float rx, float ry, float rz, const DevParams& P, float& gx, float& gy,
-                                           float& gz)
+// a / b in FP64 to an ulp or two for quotients of FP32 values (whose range
+// needs no scaling), zeros, infinities and NaN as in IEEE division
+__device__ inline double div_f64(double a, double b)
 {
-    const double s = dw_over_r_f64(rx, ry, rz, P);
-    gx = (float)(s * (double)rx);
-    gy = (float)(s * (double)ry);
-    gz = (float)(s * (double)rz);
+    const double y = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, y, 1.0);
+    return __builtin_amdgcn_div_fixup(a * __builtin_fma(y, __builtin_fma(e, e, e), y), b, a);
+}
+// 1 / b for div_f32 below (b's exponent well inside FP32's range)
+__device__ inline float rcp_f32(float b)
+{
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+// a / b, y = rcp_f32(b): rounded once (an error of at most half an ulp and
+// 2^-20 of one), zeros, infinities and NaN as in IEEE division
+__device__ inline float div_f32(float a, float b, float y)
+{
+    const float q = a * y;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
+}
+
+// A pair's separation in FP64 from the FP32 coordinate differences: 1 / r and
+// q = r / H.
+struct PairSep {
+    double ir, q;
+};
+__device__ inline PairSep pair_sep(double x, double y, double z, const DevParams& P)
+{
+    const double r2 = __builtin_fma(z, z, __builtin_fma(y, y, x * x));
+    PairSep s;
+    s.ir = rsqrt_f64(r2);
+    s.q = r2 * s.ir * P.invH64;
+    return s;
+}
+// The kernel gradient is g = dW(r)/r * r_ij (src/sph/kernel.h:169-175 over r);
+// this is its factor dW(r)/r, in FP64.  The passes round g once per component:
+// where a particle's pair terms cancel (the compressed zone of a contact), the
+// half-dozen FP32 roundings of the factor, amplified by the cancellation,
+// dominated the acceleration error against FP64; rounded once they leave a
+// fifth of it.  For q < 1/2 the factor is prefactor (3 q - 2) / H (q / r =
+// 1 / H), for q >= 1/2 -prefactor (1 - q)^2 / r; both pieces meet at q = 1/2.
+__device__ inline double dw_over_r_f64(const PairSep& s, const DevParams& P)
+{
+    const double om = 1.0 - s.q;
+    const double in = __builtin_fma(s.q, P.dWq64, P.dW064);
+    const double out = om * om * s.ir * P.dWm64;
+    return s.q < 0.5 ? in : out;
 }
 // W(r) (src/sph/kernel.h:130-136) in FP64 at the FP32 separation, rounded
 // once: the density sum then carries about half an ulp per particle, which
-// the pressures of a strongly compressed zone would otherwise amplify
+// the pressures of a strongly compressed zone would otherwise amplify.
+// 1 - 6 q^2 (1 - q) for q < 1/2, 2 (1 - q)^3 from there.
 __device__ inline float kernel_w_f64(float rx, float ry, float rz, const DevParams& P)
 {
-    const double x = rx, y = ry, z = rz;
-    const double q = sqrt((x * x + y * y) + z * z) * P.invH64;
+    const double q = pair_sep(rx, ry, rz, P).q;
     const double om = 1.0 - q;
-    const double w = (q < 0.5) ? (6.0 * q * q * q - 6.0 * q * q + 1.0) : 2.0 * (om * om * om);
-    return (float)(P.Wpref64 * w);
+    const bool in = q < 0.5;
+    const double x = in ? q : om;
+    return (float)__builtin_fma(in ? P.Wi64 : P.Wo64, x * x * om, in ? P.Wpref64 : 0.0);
 }
 
 // src/sph/eos.h:88-96
@@ -149,22 +183,6 @@ struct CSum {
     }
     __device__ inline float value() const { return s + c; }
 };
-
-// src/sph/models.h:172-185 (with maxVsig) / :158-170 (without)
-__device__ inline float artificial_viscosity(float* maxvsig, float alpha, float di, float dj, float vx, float vy,
-                                             float vz, float rx, float ry, float rz, float r, float ci, float cj,
-                                             float bi, float bj)
-{
-    const float wij = (rx * vx + ry * vy + rz * vz) / r;
-    float II = 0.0f;
-    if (wij < 0.0f) {
-        const float vsig = ci + cj - 3.0f * wij;
-        const float rhoij = (di + dj) * 0.5f;
-        II = -0.25f * (bi + bj) * alpha * wij * vsig / rhoij;
-        if (maxvsig) *maxvsig = fmaxf(*maxvsig, vsig);
-    }
-    return II;
-}
 
 // src/sph/models.h:187-192
 __device__ inline float balsara_switch(float divv, float cx, float cy, float cz, float c, float h)
@@ -229,9 +247,13 @@ __host__ inline DevParams make_dev_params(const grasph_params* p)
     const double h = p->H;
     d.invH64 = h > 0.0 ? 1.0 / h : 0.0;
     d.Wpref64 = d.dim == 1 ? 4.0 / (3.0 * h) : d.dim == 2 ? 40.0 / (7.0 * M_PI * h * h) : 8.0 / (M_PI * h * h * h);
-    d.dWpref64 = d.dim == 1 ? 24.0 / (3.0 * h * h) : d.dim == 2 ? 240.0 / (7.0 * M_PI * h * h * h)
-                                                                : 48.0 / (M_PI * h * h * h * h);
-    d.dWprefH64 = h > 0.0 ? d.dWpref64 / h : 0.0;
+    const double dW = d.dim == 1 ? 24.0 / (3.0 * h * h) : d.dim == 2 ? 240.0 / (7.0 * M_PI * h * h * h)
+                                                                     : 48.0 / (M_PI * h * h * h * h);
+    d.Wi64 = -6.0 * d.Wpref64;
+    d.Wo64 = 2.0 * d.Wpref64;
+    d.dWq64 = h > 0.0 ? 3.0 * dW / h : 0.0;
+    d.dW064 = h > 0.0 ? -2.0 * dW / h : 0.0;
+    d.dWm64 = -dW;
     return d;
 }
 

@@ -1,0 +1,67 @@
+"""The list passes (csrc/nbr_passes.hip) with 16 and with 4 lanes per
+particle: the sums are taken in the list's order, so lists, overflow scans,
+single instances and batches agree bit for bit, at counts that leave a
+wavefront's groups and a group's lanes partly empty."""
+import numpy as np
+import pytest
+
+import grasph2_amd as g
+from grasph2_amd import ics
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("density", "dstress_dt", "density_dt", "balsara", "acc", "xvel", "maxvsig")
+
+
+def workload(kind, n):
+    if kind == "solid":
+        return ics.collision(n, seed=n, gap=-2.0, gravity=False)
+    h, prm = ics.liquid_blob(n, seed=n, gravity=False,
+                             fields=("posm", "pos64", "vel", "acc", "density", "density_dt", "balsara", "maxvsig", "xvel"))
+    h["vel"][:, :3] = np.random.default_rng(n).normal(0.0, 0.1, size=(n, 3))
+    if kind == "xsph":
+        prm.flags |= g.XSPH
+        prm.xsph_factor = 0.5
+    else:  # artificial pressure, no Balsara switch
+        prm.flags |= g.ARTIFICIAL_STRESS
+        prm.flags &= ~g.BALSARA_SWITCH
+    return h, prm
+
+
+def run(h, prm, capacity):
+    ctx = g.Context(0)
+    if capacity:
+        ctx.set_option("max_neighbours_grow", 0)
+        ctx.set_option("max_neighbours", capacity)
+    d = g.DeviceParticles.from_host(h)
+    ctx.compute_derivatives(d, prm)
+    g.hip.synchronize()
+    out = d.download([f for f in FIELDS if f in h])
+    d.free()
+    ctx.close()
+    return out
+
+
+@pytest.mark.parametrize("kind", ["solid", "xsph", "pressure"])
+@pytest.mark.parametrize("n", [2, 5, 17, 333, 10240, 10241])
+def test_lists_scans_and_batches_agree(kind, n):
+    print("passes kind=%s n=%d" % (kind, n), flush=True)
+    h, prm = workload(kind, n)
+    a = run(h, prm, 0)
+    assert np.all(np.isfinite(a["acc"]))
+    b = run(h, prm, 33)  # the particles inside overflow, those at the surface don't
+    for f in a:
+        assert np.array_equal(a[f], b[f]), f
+    if n > 400:
+        h2, prm2 = workload(kind, 37)  # a batch walks with 4 lanes: against 16 of the single instance
+        host, offsets = g.pack_batch([h2, h, h2])
+        ctx = g.Context(0)
+        d = g.DeviceParticles.from_host(host)
+        ctx.batch_compute_derivatives(d, ctx.batch(offsets, [prm2, prm, prm2]))
+        g.hip.synchronize()
+        got = g.unpack_batch(d.download(list(a)), offsets)
+        d.free()
+        ctx.close()
+        for f in a:
+            assert np.array_equal(got[1][f], a[f]), f
+            assert np.array_equal(got[0][f], got[2][f]), f
