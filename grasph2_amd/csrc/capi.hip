@@ -47,28 +47,57 @@ ProfScope::~ProfScope()
     c->ev_pending.push_back(Ctx::Ev{a, b, cls});
 }
 
-// The one-sided sweep's shape: one slot per lane below kOwnFour particles,
-// four from there on (Plummer steps at 6000: 26.9 us with one, 27.4 with
-// four; at 8192: 47 and 31), and as many shares of the partners as give ~16
-// (four slots per lane: 8) wavefronts per compute unit, of 32 partners or
-// more (1000 particles: 28 us with one share per slot block, 14 with 16).
-constexpr int64_t kOwnFour = 6144;
+// The one-sided sweep's shape for a number of shares of the partners: one or
+// four slots per lane, a share to each of a workgroup's wavefronts (16, with
+// four slots 8: what a compute unit runs at once; or half as many) and
+// `planes` workgroups to cover them, whose sums a second kernel adds.  Half
+// workgroups come in odd numbers only, so the shares alone tell the shape.
+// Both forms keep the same pace, so the one that takes fewer rounds of
+// workgroups over the compute units, times (a share's partners + a
+// wavefront's start), and the second kernel least, is taken (Plummer steps with one / four slots: 6144
+// particles 20.4 / 24.2 us, 9500 37.8 / 38.0, 11000 52.7 / 46.6; allocation-
+// free SPH at 40000 597 / 839; 1000 particles with one workgroup's shares 11.0,
+// with two 12.6, 1500 13.7 and 12.5).
+constexpr int64_t kOwnStart = 32, kOwnShare = 32;  // a start's cost and the least share, in partners
+constexpr int kOwnSlicesMax = 64;
 
-OwnPlan own_plan(const Ctx& c, int64_t n, int slices)
+static int64_t own_shape(const Ctx& c, int64_t n, int slices, int ni, OwnPlan& p)
 {
-    OwnPlan p;
-    p.ni = c.sweep_ni == 2 ? 2 : n >= kOwnFour ? 4 : 1;
-    const int max_waves = p.ni == 4 ? 8 : 16;  // LDS: the wavefronts' sums in 64 KiB
-    if (slices <= 0) {
-        const int64_t blocks = (n + 64 * p.ni - 1) / (64 * p.ni), target = (p.ni == 4 ? 8 : 16) * (int64_t)c.cus;
-        slices = (int)std::max<int64_t>(1, std::min<int64_t>((target + blocks - 1) / blocks, n / 32));
-        if (slices > max_waves) slices = slices / max_waves * max_waves;  // whole workgroups
-        slices = std::min(slices, 64);
-    }
-    p.waves = std::min(slices, max_waves);
+    const int full = ni == 4 ? 8 : 16, half = full / 2;  // LDS: the wavefronts' sums in 64 KiB
+    p.ni = ni;
+    p.waves = slices > half && slices % full && slices % half == 0 ? half : std::min(slices, full);
     p.planes = (slices + p.waves - 1) / p.waves;
     p.len = (int)(((n + p.slices() - 1) / p.slices() + 7) / 8 * 8);
-    return p;
+    const int64_t groups = (n + 64 * ni - 1) / (64 * ni) * p.planes, room = (int64_t)c.cus * (full / p.waves);
+    return (ni == 4 ? 2 : 1) * ((groups + room - 1) / room) * (p.len + kOwnStart) +
+           (p.planes > 1 ? 36 + 4 * p.planes : 0);
+}
+
+// slices 0: the number of shares (of 32 partners or more) that costs least.
+// As many as give 8 (16) wavefronts per compute unit, whatever that leaves
+// of a last round, took 28.8 us at 5500 particles (now 20.3), 76.6 at 11000.
+OwnPlan own_plan(const Ctx& c, int64_t n, int slices, int max_planes)
+{
+    const auto shape = [&](int s, OwnPlan& p) {
+        if (c.sweep_ni == 2) return own_shape(c, n, s, 2, p);
+        OwnPlan one;
+        const int64_t cost = own_shape(c, n, s, 4, p), cost1 = own_shape(c, n, s, 1, one);
+        if (cost1 < cost) p = one;
+        return std::min(cost, cost1);
+    };
+    OwnPlan best, p;
+    if (slices > 0 || n < 16 * kOwnShare) {
+        shape(slices > 0 ? slices : (int)std::max<int64_t>(1, n / kOwnShare), best);
+        return best;
+    }
+    int64_t least = shape(4, best);
+    for (int s = 8; s <= kOwnSlicesMax && n / s >= kOwnShare; s += 4) {
+        const int64_t cost = shape(s, p);
+        if (cost >= least || p.planes > max_planes) continue;
+        least = cost;
+        best = p;
+    }
+    return best;
 }
 
 namespace {
@@ -272,12 +301,12 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
 }
 
 // The symmetric sweep's default thresholds (option sweep_symmetric = 2),
-// measured step times against the one-sided sweep: with neighbour lists
-// (collision) 0.319 against 0.322 ms at 16384 particles, 0.269 against
-// 0.221 at 8192; gravity alone (Plummer) 0.106 against 0.116 ms at 16384,
-// 0.216 against 0.222 at 24576, 0.268 against 0.369 at 32768.
-constexpr int64_t kSymAutoMinLists = 16384;
-constexpr int64_t kSymAutoMinGravity = 16384;
+// measured step times, symmetric against one-sided: with neighbour lists
+// (default solids / collision) 106 / 119 against 105 / 113 us at 12500
+// particles, 112 / 124 against 115 / 127 at 14000; gravity alone (Plummer) 69
+// against 66 at 14000, 77 against 76 at 15500, 82 against 94 at 16500.
+constexpr int64_t kSymAutoMinLists = 13312;
+constexpr int64_t kSymAutoMinGravity = 15360;
 
 int sym_wgs(const Ctx& c) { return c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(c.cus); }
 
@@ -427,7 +456,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     const bool sym = sweep_grav &&
                      (c.sweep_symmetric == 1 ||
                       (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity)));
-    const OwnPlan plan = own_plan(c, n, c.sweep_slices);
+    const OwnPlan plan = own_plan(c, n, c.sweep_slices, kOwnSlicesMax);
     const bool masses = sweep_grav && (sym || n >= kMassCheckMin);  // the equal-mass check
     if (need_list) {
         grow_list_capacity(c, n, s);
@@ -623,15 +652,15 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
 
     // the j-split: as the allocating path would take it, fewer planes until
     // the arrays fit
-    OwnPlan plan = own_plan(sh, n, c.sweep_slices);
-    if (!grav) plan = own_plan(sh, n, 1);
+    OwnPlan plan = own_plan(sh, n, grav ? c.sweep_slices : 1, kOwnSlicesMax);
     size_t need = 0;
     for (;;) {
         Carve m{nullptr, 0};
         carve_derivative_arrays(sh, m, n, lists, grav, plan.planes);
         need = m.used;
         if (need <= (size_t)GRASPH_NOALLOC_SCRATCH_BYTES || plan.planes == 1) break;
-        plan = own_plan(sh, n, plan.waves * (plan.planes - 1));
+        plan = c.sweep_slices > 0 ? own_plan(sh, n, plan.waves * (plan.planes - 1), kOwnSlicesMax)
+                                  : own_plan(sh, n, 0, plan.planes - 1);
     }
     if (need > (size_t)GRASPH_NOALLOC_SCRATCH_BYTES)
         return fail(c, GRASPH_E_INVALID,

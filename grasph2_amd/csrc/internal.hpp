@@ -631,11 +631,14 @@ struct OwnPlan {
     int ni, waves, planes, len;
     int slices() const { return waves * planes; }
 };
-OwnPlan own_plan(const Ctx& c, int64_t n, int slices);
+// slices: the option sweep_slices, 0 for the automatic choice (of at most
+// max_planes planes)
+OwnPlan own_plan(const Ctx& c, int64_t n, int slices, int max_planes);
 // particles from which the one-sided sweep looks whether all masses are equal
-// (the check's launch costs more than the multiply per pair it saves: Plummer
-// 1000 14.2 -> 10 us per step without it)
-constexpr int64_t kMassCheckMin = 6144;
+// (the check's launch costs more than the multiply per pair it saves: without
+// it Plummer 1000 14.2 -> 10 us per step, 9500 42.4 -> 38, allocation-free SPH
+// at 20000 240 -> 236; at 24000 271 -> 274)
+constexpr int64_t kMassCheckMin = 24576;
 
 // arrays each pass needs, by configuration; 0 or a GRASPH_E_INVALID code
 int check_derivative_arrays(Ctx& c, const grasph_particles* p, uint32_t f, int which);
