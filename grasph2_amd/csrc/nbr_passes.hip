@@ -321,6 +321,11 @@ __global__ __launch_bounds__(kBlock) void strain_kernel(
     const float rhoi = vr.w;
     const struct { double x, y, z; } vi = {vr.x, vr.y, vr.z};
 
+    float st[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // the stress used after the walk, on its way during it
+    if (SOLIDS) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) st[c] = dstress[m.plane6(c, i)];
+    }
     Rates R{};
     const auto term = [&](const vec4 (&q)[2], double (&v)[kTerms]) GRASPH_INLINE {
         const vec4 pj = q[0], vj = q[1];
@@ -371,10 +376,7 @@ __global__ __launch_bounds__(kBlock) void strain_kernel(
     if (!act || lane % LPP != 0) return;
 
     // do_after, computeDerivatives.h:144-161
-    Tens S = sym_to_full(0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
-    if (SOLIDS)
-        S = sym_to_full(dstress[m.plane6(0, i)], dstress[m.plane6(1, i)], dstress[m.plane6(2, i)],
-                        dstress[m.plane6(3, i)], dstress[m.plane6(4, i)], dstress[m.plane6(5, i)]);
+    Tens S = sym_to_full(st[0], st[1], st[2], st[3], st[4], st[5]);
     float sdt[6] = {0, 0, 0, 0, 0, 0};
     if (SOLIDS) {
         const Tens ed = sym_to_full((float)exx, (float)eyy, (float)ezz, (float)exy, (float)exz, (float)eyz);

@@ -22,6 +22,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kBoxBlocks = 256;
+// counts up to this are ordered by rank (rank_kernel), larger ones by a sort
+constexpr int kRankMax = 16384;
 
 __global__ __launch_bounds__(kBlock) void bbox_partial(const float4* __restrict__ posm, const int n,
                                                        float* __restrict__ part)
@@ -49,30 +51,26 @@ __global__ __launch_bounds__(kBlock) void bbox_partial(const float4* __restrict_
     if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-// one block of kBlock threads folds the nparts (<= kBlock) block boxes
-__global__ __launch_bounds__(kBlock) void bbox_final(float* __restrict__ part, const int nparts)
+// the boxes of a block's threads folded into one, in every thread
+template <int THREADS>
+__device__ __forceinline__ void bbox_fold(float (&box)[6])
 {
-    __shared__ float sh[6][kBlock / 64];
-    const int b = threadIdx.x, lane = b & 63, w = b >> 6;
-    float v[6];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) v[d] = (b < nparts) ? part[b * 6 + d] : ((d < 3) ? INFINITY : -INFINITY);
+    __shared__ float sh[6][THREADS / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1)
 #pragma unroll
         for (int d = 0; d < 6; ++d) {
-            const float o = __shfl_xor(v[d], off, 64);
-            v[d] = (d < 3) ? fminf(v[d], o) : fmaxf(v[d], o);
+            const float o = __shfl_xor(box[d], off, 64);
+            box[d] = (d < 3) ? fminf(box[d], o) : fmaxf(box[d], o);
         }
     if (lane == 0)
 #pragma unroll
-        for (int d = 0; d < 6; ++d) sh[d][w] = v[d];
+        for (int d = 0; d < 6; ++d) sh[d][w] = box[d];
     __syncthreads();
-    if (b < 6) {
-        float r = sh[b][0];
-        for (int q = 1; q < kBlock / 64; ++q) r = (b < 3) ? fminf(r, sh[b][q]) : fmaxf(r, sh[b][q]);
-        part[nparts * 6 + b] = r;
-    }
+#pragma unroll
+    for (int d = 0; d < 6; ++d)
+        for (int q = 0; q < THREADS / 64; ++q) box[d] = (d < 3) ? fminf(box[d], sh[d][q]) : fmaxf(box[d], sh[d][q]);
 }
 
 __device__ inline uint32_t spread10(uint32_t v)
@@ -116,7 +114,7 @@ __device__ inline uint32_t hilbert_index(uint32_t x, uint32_t y, uint32_t z)
 // cubes of a 1024th of the longest side; across a side less than an eighth of
 // it they are finer (bodies far apart keep their resolution across the line
 // between them).
-__device__ inline uint32_t curve_key(const float4 p, const float* __restrict__ box)
+__device__ inline uint32_t curve_key(const float4 p, const float* box)
 {
     const float c[3] = {p.x, p.y, p.z};
     float ext[3], longest = 0.0f;
@@ -137,14 +135,98 @@ __device__ inline uint32_t curve_key(const float4 p, const float* __restrict__ b
     return hilbert_index(q[0], q[1], q[2]);
 }
 
+// keys of the particles from the nparts (<= kBlock) block boxes
 __global__ __launch_bounds__(kBlock) void curve_keys(const float4* __restrict__ posm, const int n,
-                                                     const float* __restrict__ box, uint32_t* __restrict__ keys,
-                                                     int* __restrict__ vals)
+                                                     const float* __restrict__ part, const int nparts,
+                                                     uint32_t* __restrict__ keys, int* __restrict__ vals)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int i = blockIdx.x * kBlock + threadIdx.x, b = threadIdx.x;
+    const float4 p = posm[min(i, n - 1)];
+    float box[6];
+#pragma unroll
+    for (int d = 0; d < 6; ++d) box[d] = (b < nparts) ? part[b * 6 + d] : ((d < 3) ? INFINITY : -INFINITY);
+    bbox_fold<kBlock>(box);
     if (i >= n) return;
-    keys[i] = curve_key(posm[i], box);
+    keys[i] = curve_key(p, box);
     vals[i] = i;
+}
+
+// keys of up to kRankMax particles in one launch: every workgroup finds the
+// whole bounding box for itself (256 KiB of positions from L2 at most)
+constexpr int kRankThreads = 1024;
+__global__ __launch_bounds__(kRankThreads) void rank_keys(const float4* __restrict__ posm, const int n,
+                                                          uint32_t* __restrict__ keys)
+{
+    const int i = blockIdx.x * kRankThreads + threadIdx.x;
+    float box[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll 4
+    for (int j = threadIdx.x; j < n; j += kRankThreads) {
+        const float4 p = posm[j];
+        box[0] = fminf(box[0], p.x); box[1] = fminf(box[1], p.y); box[2] = fminf(box[2], p.z);
+        box[3] = fmaxf(box[3], p.x); box[4] = fmaxf(box[4], p.y); box[5] = fmaxf(box[5], p.z);
+    }
+    const float4 p = posm[min(i, n - 1)];
+    bbox_fold<kRankThreads>(box);
+    if (i < n) keys[i] = curve_key(p, box);
+}
+
+// The order of up to kRankMax particles, without a sort: particle i's slot is
+// the number of particles before it on the curve, those with a smaller key
+// and, of its own key, those with a smaller index.  A workgroup counts for 32
+// particles: its half wavefronts 1/32 of the keys each, a particle per lane,
+// all lanes of a half reading the same keys from LDS, four at a time.  The
+// sign of (key j - limit) is shifted into a word that a population count
+// adds up every 32 keys: two plain vector instructions a pair (a compare and
+// an add with its carry take twice the clocks).  Rank, keys and bounding box
+// in two launches: allocation-free SPH step at 1000 particles 61.9 -> 56.2 us,
+// 8192 108 -> 92, 16384 167 -> 164; past kRankMax the sort is the faster one.
+constexpr int kRankWaves = 16, kRankOwn = 32;              // particles of a workgroup
+constexpr int kRankShares = 64 / kRankOwn * kRankWaves;    // shares of the keys
+__global__ __launch_bounds__(64 * kRankWaves) void rank_kernel(const uint32_t* __restrict__ keys, const int n,
+                                                               int* __restrict__ perm)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t all[kRankMax];
+    __shared__ int part[kRankShares][kRankOwn];
+    const int own = threadIdx.x % kRankOwn, share = threadIdx.x / kRankOwn;
+    const int i0 = kRankOwn * blockIdx.x, i = i0 + own;
+    const uint32_t key = keys[min(i, n - 1)];
+    const int blocks = (n + kRankOwn - 1) / kRankOwn;  // of as many keys; the shares take whole ones
+    for (int j = threadIdx.x; j < blocks * kRankOwn; j += 64 * kRankWaves)
+        all[j] = j < n ? keys[j] : 0x40000000u;  // past the end: after every key of 30 bits
+    __syncthreads();
+    const int b0 = blocks * share / kRankShares, b1 = blocks * (share + 1) / kRankShares;
+    int before = 0;
+    for (int b = b0; b < b1; ++b) {
+        uint32_t less = 0;
+        const uint4* const k4 = reinterpret_cast<const uint4*>(all + kRankOwn * b);
+        if (b == (int)blockIdx.x) {  // its own block
+#pragma unroll
+            for (int u = 0; u < kRankOwn / 4; ++u) {
+                const uint4 k = k4[u];
+                less = __builtin_amdgcn_alignbit(less, k.x - key - (4 * u + 0 < own ? 1u : 0u), 31);
+                less = __builtin_amdgcn_alignbit(less, k.y - key - (4 * u + 1 < own ? 1u : 0u), 31);
+                less = __builtin_amdgcn_alignbit(less, k.z - key - (4 * u + 2 < own ? 1u : 0u), 31);
+                less = __builtin_amdgcn_alignbit(less, k.w - key - (4 * u + 3 < own ? 1u : 0u), 31);
+            }
+        } else {
+            const uint32_t limit = key + (b < (int)blockIdx.x ? 1u : 0u);
+#pragma unroll
+            for (int u = 0; u < kRankOwn / 4; ++u) {
+                const uint4 k = k4[u];
+                less = __builtin_amdgcn_alignbit(less, k.x - limit, 31);
+                less = __builtin_amdgcn_alignbit(less, k.y - limit, 31);
+                less = __builtin_amdgcn_alignbit(less, k.z - limit, 31);
+                less = __builtin_amdgcn_alignbit(less, k.w - limit, 31);
+            }
+        }
+        before += __builtin_popcount(less);
+    }
+    part[share][own] = before;
+    __syncthreads();
+    if (share != 0 || i >= n) return;
+#pragma unroll
+    for (int w = 1; w < kRankShares; ++w) before += part[w][own];
+    perm[before] = i;
 }
 
 // one block per instance: bounding box of its particles
@@ -264,12 +346,17 @@ size_t reorder_tmp_bytes(int n)
 hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(bbox_partial, dim3(kBoxBlocks), dim3(kBlock), 0, s, posm, n, c.bbox);
-    static_assert(kBoxBlocks <= kBlock, "bbox_final folds at most one box per thread");
-    hipLaunchKernelGGL(bbox_final, dim3(1), dim3(kBlock), 0, s, c.bbox, kBoxBlocks);
-    const int blocks = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(curve_keys, dim3(blocks), dim3(kBlock), 0, s, posm, n, c.bbox + kBoxBlocks * 6, c.keys,
-                       c.vals);
+    if (n <= kRankMax) {
+        hipLaunchKernelGGL(rank_keys, dim3((n + kRankThreads - 1) / kRankThreads), dim3(kRankThreads), 0, s, posm, n,
+                           c.keys);
+        hipLaunchKernelGGL(rank_kernel, dim3((n + kRankOwn - 1) / kRankOwn), dim3(64 * kRankWaves), 0, s, c.keys, n,
+                           c.perm);
+        return hipGetLastError();
+    }
+    const int blocks = (n + kBlock - 1) / kBlock, parts = std::min(blocks, kBoxBlocks);
+    static_assert(kBoxBlocks <= kBlock, "curve_keys folds at most one box per thread");
+    hipLaunchKernelGGL(bbox_partial, dim3(parts), dim3(kBlock), 0, s, posm, n, c.bbox);
+    hipLaunchKernelGGL(curve_keys, dim3(blocks), dim3(kBlock), 0, s, posm, n, c.bbox, parts, c.keys, c.vals);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     size_t bytes = c.sort_tmp_bytes;

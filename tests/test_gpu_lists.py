@@ -88,3 +88,21 @@ def test_batch_counts_equal_single_instances(sizes):
         assert np.array_equal(got[k]["acc"], ref["acc"])
     ctx.close()
     one.close()
+
+
+@pytest.mark.parametrize("kind", ["ball", "coincident"])  # all keys differ; many are the same
+@pytest.mark.parametrize("n", [31, 33, 1025, 16384, 16385])
+def test_order_by_rank_and_by_sort(kind, n):
+    """Slots from the rank kernel (up to 16384 particles) and from the sort: a
+    slot left out or filled twice would change the counts."""
+    print("order kind=%s n=%d" % (kind, n), flush=True)
+    h, prm = particles(kind, n, np.random.default_rng(n))
+    prm.H = min(prm.H, 2.5 * (4.2 / n) ** (1.0 / 3.0))
+    ctx = g.Context(0)
+    d = g.DeviceParticles.from_host(h)
+    ctx.calc_density(d, prm)
+    pairs, mx, _ = ctx.neighbour_stats()
+    d.free()
+    ctx.close()
+    want = brute_counts(h["posm"][:, :3], prm.H)
+    assert (pairs, mx) == (int(want.sum()), int(want.max()))
