@@ -9,32 +9,43 @@
 //
 // One wavefront makes the lists of 8 slots.  Lane l tests box l of 64 boxes
 // of 512 against the 8 slots' own box, then lane l box l of the 64 boxes of 8
-// in each that is near; every near one is 8 partners j, and lane l = 8 i + j
-// takes the pair (i, j).  The 64 lanes' hits in one ballot give slot i its
-// partners as a byte in slot order, so a partner's place in the list is the
-// count so far plus the bits below it: the lists come out in increasing slot
-// order, complete and one to a slot, whatever the launch shape.
+// in each that is near, then the particles of the near ones, 64 at a time:
+// those within H of the own box are collected in LDS, in slot order.  Lane
+// l = 8 i + j takes slot i against every eighth of them from the j-th on; the
+// 64 lanes' hits in one ballot give slot i its partners as a byte in slot
+// order, so a partner's place in the list is the count so far plus the bits
+// below it: the lists come out in increasing slot order, complete and one to a
+// slot, whatever the launch shape.
 //
-// What bounds it: the vector issue, ~25 instructions per 64 pairs.  A box of
-// 8 slots meets ~70 boxes within H = 2.5 spacings, so a slot is tested
-// against ~560 partners for its ~65 neighbours; blocks of 64 slots against
-// blocks of 64 partners, one slot per lane, tested ~1900 and appended lane by
-// lane in branches.  Partners are read into vector registers (the 8 rows of
-// lanes share a 128-byte line): a scalar operand would halve the issue rate
-// (far_rotation.hpp).  Measured: N = 131072 collision 115 us, where blocks of
-// 64 with their shares, merge and count maximum took 300; 20011 particles
-// 50 us instead of 135; 65536 squeezed ones (430 partners each) 253
-// instead of 640.
+// What bounds it: instructions, 1150 vector ones per wavefront, and the
+// stores (each 4 bytes of a line of its own).  8 slots meet ~70 boxes within
+// H = 2.5 spacings, 560 particles, for ~65 neighbours each, of which ~250 come
+// within H of their box: testing the slots against those instead of all 560
+// took N = 200003 from 126 to 92 us, 65536 squeezed ones (430 partners each)
+// from 190 to 137, 512 instances from 1.63 to 1.15 ms.
 #include "internal.hpp"
 
 namespace grasph {
 namespace {
 
 constexpr int kBoxThreads = kBoxCoarse;  // slots of a coarse box: one workgroup
-constexpr int kTile = 64;                // slots per workgroup of the list kernel
+constexpr int kTile = 32;                // slots per workgroup of the list kernel
 constexpr int kListThreads = 8 * kTile;
 constexpr int kBoxList = 384;            // near fine boxes a wavefront collects before it tests them
-constexpr int kAhead = 4;                // boxes' partners in flight
+constexpr int kAhead = 2;                // loads of 8 boxes' partners in flight
+constexpr int kPartners = 256;           // close partners a wavefront collects before it tests them
+
+#define GRASPH_INLINE __attribute__((always_inline))
+typedef float vec4 __attribute__((ext_vector_type(4)));
+
+// Orders the wavefront's LDS accesses around it (the hardware executes one
+// wavefront's in order; the compiler must not move them).
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // whether two boxes come within H of each other
 __device__ __forceinline__ bool boxes_near(const float4 lo, const float4 hi, const float4 l2, const float4 h2,
@@ -78,7 +89,9 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
                                                             const BatchInst* __restrict__ insts,
                                                             int* __restrict__ max_dev, int* __restrict__ max_host)
 {
-    __shared__ int boxes[kTile / kBoxFine][kBoxList];  // one wavefront's row is its own: no barrier
+    // one wavefront's rows are its own: no barrier
+    __shared__ int boxes[kTile / kBoxFine][kBoxList];
+    __shared__ vec4 partners[kTile / kBoxFine][kPartners];
     // XCD-contiguous (xcd_block): neighbouring tiles read the same partners
     const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
@@ -86,14 +99,14 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     float H2 = h2;
     const float4 *fine = fine0, *coarse = coarse0;
     if (BATCH) {
-        const int4 bl = blk[tile / 4];  // 256 slots: four tiles
+        const int4 bl = blk[tile / (256 / kTile)];  // of 256 slots
         const BatchInst I = insts[bl.x];
         off = I.off;
         n = I.n;
         H2 = I.H2;
         fine += 2 * (size_t)I.fine0;
         coarse += 2 * (size_t)I.coarse0;
-        first = bl.y - off + kTile * (tile % 4) + kBoxFine * wave;
+        first = bl.y - off + kTile * (tile % (256 / kTile)) + kBoxFine * wave;
     } else {
         first = kTile * tile + kBoxFine * wave;
     }
@@ -125,43 +138,61 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         }
         return any;
     };
-    int* const list = nbr + list_entry(off + t, 0, kmax);
+    // entry k of this lane's slot, in bytes from the wavefront's first tile of
+    // the lists (which its 8 slots may leave, in a batch)
+    char* const lists = reinterpret_cast<char*>(nbr + list_entry(off + first, 0, kmax) - ((off + first) & 63));
+    const uint32_t column = 4u * (uint32_t)(((off + t) >> 6 != (off + first) >> 6 ? kmax * 64 : 0) + ((off + t) & 63));
     const uint32_t bit = 1u << j, below = bit - 1u;
     const int shift = 8 * (i & 3);
-    // the instance's last fine box may be short: its bits, the same in every byte
-    const uint64_t tail = n % kBoxFine ? 0x0101010101010101ull * ((1u << (n % kBoxFine)) - 1u) : ~0ull;
     const float4* const xj = xs + off;
-    int cnt = 0;
-    // The pairs of this wavefront's slots with the partners of the m boxes in
-    // box[]: kAhead boxes' partners in flight while one is tested.
+    vec4* const part = partners[wave];
+    int cnt = 0, np = 0;  // partners found for this lane's slot; partners collected
+    // The pairs of this wavefront's slots with the partners collected.
+    auto test_partners = [&]() {
+        if (lane < 8) part[np + lane] = __int_as_float(0x7fc00000);  // NaN hits nothing
+        wave_lds_order();
+        for (int b = 0; b < np; b += 8) {
+            const vec4 q = part[b + j];
+            const bool hit = is_neighbour(dist2_exact(xi - q.x, yi - q.y, zi - q.z), H2);
+            const uint64_t hits = __builtin_amdgcn_ballot_w64(hit);
+            const uint32_t half = lane < 32 ? (uint32_t)hits : (uint32_t)(hits >> 32);
+            const uint32_t mine = (half >> shift) & 0xffu;
+            const int k = cnt + __builtin_popcount(mine & below);
+            if (hit && k < kmax) *reinterpret_cast<int*>(lists + (column + 256u * (uint32_t)k)) = __float_as_int(q.w);
+            cnt += __builtin_popcount(mine);
+        }
+        wave_lds_order();
+        np = 0;
+    };
+    // The partners in the m boxes of box[] within H of this wavefront's own
+    // box, collected: 8 boxes at a time, kAhead times as many on their way.
     auto test_boxes = [&](const int m) {
-        for (int b0 = 0; b0 < m; b0 += 64) {
-            const int mb = min(64, m - b0);
-            const int mine64 = box[b0 + min(lane, mb - 1)];
-            float3 q[kAhead];
-            int f[kAhead];
+        wave_lds_order();
+        int at[kAhead];
+        vec4 q[kAhead];
+        const auto fetch = [&](const int b, int& a, vec4& v) GRASPH_INLINE {
+            const int u = b + i;
+            a = u < m ? kBoxFine * box[min(u, m - 1)] + j : n;
+            v = *reinterpret_cast<const vec4*>(xj + min(a, n - 1));
+        };
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) fetch(8 * u, at[u], q[u]);
+        for (int b0 = 0; b0 < m; b0 += 8 * kAhead) {
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
-                f[u] = __builtin_amdgcn_readlane(mine64, min(u, mb - 1));
-                q[u] = *reinterpret_cast<const float3*>(xj + min(kBoxFine * f[u] + j, n - 1));
-            }
-            for (int k0 = 0; k0 < mb; k0 += kAhead) {
-#pragma unroll
-                for (int u = 0; u < kAhead; ++u) {
-                    const int fb = f[u];
-                    const float r2 = dist2_exact(xi - q[u].x, yi - q[u].y, zi - q[u].z);
-                    uint64_t hits = __builtin_amdgcn_ballot_w64(is_neighbour(r2, H2));
-                    f[u] = __builtin_amdgcn_readlane(mine64, min(k0 + u + kAhead, mb - 1));
-                    q[u] = *reinterpret_cast<const float3*>(xj + min(kBoxFine * f[u] + j, n - 1));
-                    if (k0 + u >= mb) hits = 0;
-                    if (fb == nf - 1) hits &= tail;
-                    if (!hits) continue;
-                    const uint32_t half = lane < 32 ? (uint32_t)hits : (uint32_t)(hits >> 32);
-                    const uint32_t mine = (half >> shift) & 0xffu;
-                    const int k = cnt + __builtin_popcount(mine & below);
-                    if ((mine & bit) && k < kmax) list[64 * (size_t)k] = off + kBoxFine * fb + j;
-                    cnt += __builtin_popcount(mine);
-                }
+                const int a = at[u];
+                vec4 p = q[u];
+                fetch(b0 + 8 * (u + kAhead), at[u], q[u]);
+                const float gx = fmaxf(0.0f, fmaxf(lo.x - p.x, p.x - hi.x));
+                const float gy = fmaxf(0.0f, fmaxf(lo.y - p.y, p.y - hi.y));
+                const float gz = fmaxf(0.0f, fmaxf(lo.z - p.z, p.z - hi.z));
+                const bool close = a < n && dist2_exact(gx, gy, gz) <= H2;
+                const uint64_t all = __builtin_amdgcn_ballot_w64(close);
+                p.w = __int_as_float(off + a);
+                if (close)
+                    part[np + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0))] = p;
+                np += __builtin_popcountll(all);
+                if (np > kPartners - 72) test_partners();
             }
         }
     };
@@ -191,6 +222,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         }
     }
     test_boxes(m);
+    test_partners();
     if (j == 0 && t < n) nbr_cnt[off + t] = cnt;
     // a list that overflowed reports the largest count: to the device's
     // maximum of this evaluation, and to the host's when it raises that one
@@ -219,7 +251,7 @@ hipError_t launch_batch_lists(const ListLaunch& L, hipStream_t s)
     if (L.n <= 0 || L.n_blk <= 0) return hipSuccess;
     hipLaunchKernelGGL(batch_box_kernel, dim3(L.n_blk), dim3(kBoxThreads), 0, s, L.xs, L.blk, L.insts, L.fine,
                        L.coarse);
-    hipLaunchKernelGGL(list_kernel<true>, dim3(4 * L.n_blk), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
+    hipLaunchKernelGGL(list_kernel<true>, dim3(256 / kTile * L.n_blk), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
                        L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk, L.insts, nullptr, nullptr);
     return hipGetLastError();
 }
