@@ -288,6 +288,7 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
     L.perm = order_of(c);
     L.nbr = c.nbr;
     L.nbr_cnt = c.nbr_cnt;
+    L.coarse = c.box + 2 * fine_boxes(p->n);
     L.n = (int)p->n;
     L.lanes = pass_lanes(L.n);
     L.kmax = c.max_neighbours;

@@ -344,7 +344,7 @@ __device__ inline int xcd_block(int b, int nb)
 
 // What one block of a per-particle pass works on.
 struct SlotMap {
-    int slot0, slot_end, off, n, inst;
+    int slot0, slot_end, off, n, inst, coarse0;
     // element c of particle i in an array of 6 (resp. 3) planes per instance
     __device__ size_t plane6(int c, int i) const { return 6 * (size_t)off + (size_t)c * n + (size_t)(i - off); }
     __device__ size_t plane3(int c, int i) const { return 3 * (size_t)off + (size_t)c * n + (size_t)(i - off); }
@@ -364,12 +364,14 @@ __device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_bl
         m.slot_end = b.z;
         m.off = I.off;
         m.n = I.n;
+        m.coarse0 = I.coarse0;
     } else {
         m.inst = 0;
         m.slot0 = blk * slots_per_block;
         m.slot_end = n;
         m.off = 0;
         m.n = n;
+        m.coarse0 = 0;
     }
     return m;
 }
@@ -470,6 +472,7 @@ struct NbrLaunch {
     const int* perm;
     const int* nbr;
     const int* nbr_cnt;
+    const float4* coarse;  // the lists' boxes of 512 slots
     int n;
     int kmax;
     float* balsara;

@@ -85,6 +85,7 @@ __device__ inline float dsdt_entry(const Tens& ed, const Tens& rd, const Tens& S
 struct Lists {
     const int* nbr;
     const int* cnt;
+    const float4* coarse;  // boxes of 512 slots
 };
 
 // LPP lanes share a particle (4 or 16): lane l of a wavefront serves
@@ -174,7 +175,8 @@ struct OrderedSums {
 typedef float vec4 __attribute__((ext_vector_type(4)));
 
 // Walk slot t's neighbours: the list, or when it overflowed, a scan of the
-// instance's slots with the exact test (same partners, same order).
+// instance's slots, in the boxes of 512 within H, with the exact test (same
+// partners, same order).
 // step(q, rem): q holds the first PIECES float4 of the neighbour's record (of
 // STRIDE float4 at src); lane sub has one if sub < rem (the others repeat the
 // last).  one(q): a neighbour found by the scan, the same for the whole group.
@@ -226,19 +228,29 @@ __device__ __forceinline__ void for_each_neighbour(const vec4* __restrict__ src,
         if constexpr (D > 3) turn(e + 3, jn[3], r[3]);
     }
     if (act && cnt > kmax) {
-        const int end = m.off + m.n;
-        for (int j0 = m.off; j0 < end; j0 += LPP) {
-            const float4 pj = xs[min(j0 + sub, end - 1)];
-            const bool is = j0 + sub < end && is_neighbour(dist2_exact(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z), H2);
-            const auto found = [&](int j) GRASPH_INLINE {
-                vec4 q[PIECES];
+        const float4* const coarse = Ls.coarse + 2 * (size_t)m.coarse0;
+        for (int first = 0; first < m.n; first += kBoxCoarse) {
+            // a box farther than H holds none of the partners (lists.hip)
+            const float4 lo = coarse[2 * (first / kBoxCoarse)], hi = coarse[2 * (first / kBoxCoarse) + 1];
+            const float bx = fmaxf(0.0f, fmaxf(lo.x - pi.x, pi.x - hi.x));
+            const float by = fmaxf(0.0f, fmaxf(lo.y - pi.y, pi.y - hi.y));
+            const float bz = fmaxf(0.0f, fmaxf(lo.z - pi.z, pi.z - hi.z));
+            if (!(dist2_exact(bx, by, bz) <= H2)) continue;
+            const int end = m.off + min(first + kBoxCoarse, m.n);
+            for (int j0 = m.off + first; j0 < end; j0 += LPP) {
+                const float4 pj = xs[min(j0 + sub, end - 1)];
+                const bool is =
+                    j0 + sub < end && is_neighbour(dist2_exact(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z), H2);
+                const auto found = [&](int j) GRASPH_INLINE {
+                    vec4 q[PIECES];
 #pragma unroll
-                for (int p = 0; p < PIECES; ++p) q[p] = src[STRIDE * (size_t)j + p];
-                one(q);
-            };
-            // the group's lanes test LPP slots at once
-            unsigned b = (unsigned)(__ballot(is) >> (lane - sub)) & ((1u << LPP) - 1u);
-            for (; b != 0u; b &= b - 1u) found(j0 + __ffs(b) - 1);
+                    for (int p = 0; p < PIECES; ++p) q[p] = src[STRIDE * (size_t)j + p];
+                    one(q);
+                };
+                // the group's lanes test LPP slots at once
+                unsigned b = (unsigned)(__ballot(is) >> (lane - sub)) & ((1u << LPP) - 1u);
+                for (; b != 0u; b &= b - 1u) found(j0 + __ffs(b) - 1);
+            }
         }
     }
 }
@@ -581,7 +593,7 @@ __global__ __launch_bounds__(kBlock) void finish_kernel(const float4* __restrict
     if (maxvsig) maxvsig[i] = 0.0f;
 }
 
-inline Lists lists_of(const NbrLaunch& L) { return Lists{L.nbr, L.nbr_cnt}; }
+inline Lists lists_of(const NbrLaunch& L) { return Lists{L.nbr, L.nbr_cnt, L.coarse}; }
 
 inline dim3 grid_plain(const NbrLaunch& L)  // per-particle kernels without a list walk
 {

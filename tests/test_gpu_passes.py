@@ -65,3 +65,25 @@ def test_lists_scans_and_batches_agree(kind, n):
         for f in a:
             assert np.array_equal(got[1][f], a[f]), f
             assert np.array_equal(got[0][f], got[2][f]), f
+
+
+@pytest.mark.parametrize("kind", ["solid", "xsph"])
+def test_overflow_scans_in_a_batch(kind):
+    """Scans of the second and third instance's own boxes of 512 slots."""
+    print("passes batch overflow kind=%s" % kind, flush=True)
+    sizes = (700, 1025, 2500)
+    inst = [workload(kind, n) for n in sizes]
+    host, offsets = g.pack_batch([h for h, _ in inst])
+    ctx = g.Context(0)
+    ctx.set_option("max_neighbours_grow", 0)
+    ctx.set_option("max_neighbours", 33)
+    d = g.DeviceParticles.from_host(host)
+    ctx.batch_compute_derivatives(d, ctx.batch(offsets, [p for _, p in inst]))
+    g.hip.synchronize()
+    a = [run(h, p, 0) for h, p in inst]
+    got = g.unpack_batch(d.download(list(a[0])), offsets)
+    d.free()
+    ctx.close()
+    for k in range(len(sizes)):
+        for f in a[k]:
+            assert np.array_equal(got[k][f], a[k][f]), (k, f)
