@@ -120,20 +120,55 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         xi = p.x; yi = p.y; zi = p.z;
     }
     const int nf = (n + kBoxFine - 1) / kBoxFine, nc = (n + kBoxCoarse - 1) / kBoxCoarse;
-    const float4 lo = fine[2 * (first / kBoxFine)], hi = fine[2 * (first / kBoxFine) + 1];
-    // eight slots that span a jump of the slot order have a box that says
-    // little: there (wider than H^2's reach both ways) the boxes are tested
-    // against the particles one by one (without it one such wavefront tested
-    // every particle: N = 200003, 1736 us instead of 207)
-    const float wide = fmaxf(hi.x - lo.x, fmaxf(hi.y - lo.y, hi.z - lo.z));
-    const bool jump = __builtin_amdgcn_readfirstlane(wide * wide > 4.0f * H2);
+    float4 lo = fine[2 * (first / kBoxFine)], hi = fine[2 * (first / kBoxFine) + 1];
+    // Eight slots that span a jump of the slot order (where the curve leaves
+    // the particles and comes back) have a box that says little.  Where it is
+    // wider than H^2's reach both ways, it is cut in two at the longest step
+    // between its slots, and if a part still is, boxes are tested against the
+    // slots one by one.  (With the wide box one such wavefront tested every
+    // particle: N = 200003, 1736 us instead of 207; with all of them slot by
+    // slot those wavefronts were the last by far: liquid of 8192 TBD us.)
+    const auto wide = [&](const float4 l, const float4 h) {
+        const float w = fmaxf(h.x - l.x, fmaxf(h.y - l.y, h.z - l.z));
+        return (bool)__builtin_amdgcn_readfirstlane(w * w > 4.0f * H2);
+    };
     const int own = min(kBoxFine, n - first);
+    const auto slot = [&](const int q) {
+        return make_float4(lane_value(xi, 8 * q), lane_value(yi, 8 * q), lane_value(zi, 8 * q), 0.0f);
+    };
+    const bool jump = wide(lo, hi);
+    bool each = false;
+    float4 lo2 = lo, hi2 = hi;  // the second part's box
+    if (jump) {
+        int cut = 1;
+        float longest = -1.0f;
+        for (int q = 1; q < own; ++q) {
+            const float4 p = slot(q), o = slot(q - 1);
+            const float d = dist2_exact(p.x - o.x, p.y - o.y, p.z - o.z);
+            if (d > longest) {
+                longest = d;
+                cut = q;
+            }
+        }
+        lo = hi = slot(0);
+        lo2 = hi2 = slot(own - 1);
+        for (int q = 0; q < own; ++q) {
+            const float4 p = slot(q);
+            float4 &l = q < cut ? lo : lo2, &h = q < cut ? hi : hi2;
+            l.x = fminf(l.x, p.x); l.y = fminf(l.y, p.y); l.z = fminf(l.z, p.z);
+            h.x = fmaxf(h.x, p.x); h.y = fmaxf(h.y, p.y); h.z = fmaxf(h.z, p.z);
+        }
+        each = wide(lo, hi) || wide(lo2, hi2);
+    }
     auto near = [&](const float4 l2, const float4 h2) -> bool {
-        if (!jump) return boxes_near(lo, hi, l2, h2, H2);
+        if (!each) {
+            bool any = boxes_near(lo, hi, l2, h2, H2);
+            if (jump) any = any || boxes_near(lo2, hi2, l2, h2, H2);
+            return any;
+        }
         bool any = false;
         for (int q = 0; q < own; ++q) {
-            const float x = lane_value(xi, 8 * q), y = lane_value(yi, 8 * q), z = lane_value(zi, 8 * q);
-            const float4 p = make_float4(x, y, z, 0.0f);
+            const float4 p = slot(q);
             any = any || boxes_near(p, p, l2, h2, H2);
         }
         return any;
@@ -183,10 +218,10 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
                 const int a = at[u];
                 vec4 p = q[u];
                 fetch(b0 + 8 * (u + kAhead), at[u], q[u]);
-                const float gx = fmaxf(0.0f, fmaxf(lo.x - p.x, p.x - hi.x));
-                const float gy = fmaxf(0.0f, fmaxf(lo.y - p.y, p.y - hi.y));
-                const float gz = fmaxf(0.0f, fmaxf(lo.z - p.z, p.z - hi.z));
-                const bool close = a < n && dist2_exact(gx, gy, gz) <= H2;
+                const float4 at4 = make_float4(p.x, p.y, p.z, 0.0f);
+                bool close = boxes_near(lo, hi, at4, at4, H2);
+                if (jump) close = close || boxes_near(lo2, hi2, at4, at4, H2);
+                close = close && a < n;
                 const uint64_t all = __builtin_amdgcn_ballot_w64(close);
                 p.w = __int_as_float(off + a);
                 if (close)
