@@ -137,6 +137,43 @@ __device__ __host__ inline int far_split(int64_t n, int64_t wanted)
 }
 // the workgroup whose share [k U / W, (k + 1) U / W) holds unit u
 __device__ __host__ inline int64_t wg_of_unit(int64_t u, int64_t U, int64_t W) { return ((u + 1) * W - 1) / U; }
+// Wavefronts of the whole far field's workgroups: workgroup K's are k =
+// kFarMerge K and the next.  Where all of them are there and work on one row,
+// their own-side sums leave as one fragment, wavefront kFarMerge K's
+// (far_merged_row: that row, else -1).  Only plain fragments are merged.
+constexpr int kFarMerge = 4;
+__device__ __host__ inline int64_t far_merged_row(int64_t k0, int64_t U, int64_t W, int64_t nsb, int Q)
+{
+    if (k0 + kFarMerge > W) return -1;
+    const int64_t g = row_of_unit(k0 * U / W, nsb, Q);
+    return (k0 + kFarMerge) * U / W <= row_prefix(g + 1, nsb, Q) ? g : -1;
+}
+// The fragments of a row whose units are [u0, u1): those of wavefronts k0 ..
+// k0 + lead - 1, `merged` of whole workgroups, and the wavefronts' after them.
+struct RowFragments {
+    int64_t k0, lead, merged, count;
+    __device__ __host__ int64_t wavefront(int64_t e) const  // whose the e-th is
+    {
+        return k0 + e + (e < lead ? 0 : e < lead + merged ? (kFarMerge - 1) * (e - lead) : (kFarMerge - 1) * merged);
+    }
+};
+__device__ __host__ inline RowFragments row_fragments(int64_t u0, int64_t u1, int64_t U, int64_t W, bool merge)
+{
+    RowFragments R;
+    R.k0 = wg_of_unit(u0, U, W);
+    const int64_t k1 = wg_of_unit(u1 - 1, U, W) + 1;  // wavefronts [k0, k1)
+    R.lead = R.count = k1 - R.k0;
+    R.merged = 0;
+    if (!merge) return R;
+    const int64_t first = (R.k0 + (R.k0 * U / W < u0) + kFarMerge - 1) / kFarMerge;  // workgroups [first, last)
+    const int64_t last = (k1 - (k1 * U / W > u1)) / kFarMerge;
+    if (first < last) {
+        R.lead = kFarMerge * first - R.k0;
+        R.merged = last - first;
+        R.count -= (kFarMerge - 1) * R.merged;
+    }
+    return R;
+}
 // workgroups of the far kernel: at most the units, so every one has a share and a row's
 // fragments come from consecutive workgroups
 __host__ inline int far_workgroups(int64_t wanted, int64_t units)

@@ -205,6 +205,7 @@ __device__ __forceinline__ void far_flush_own(FarOwn& o, const int lane)
 template <bool UM>
 __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int lane)
 {
+    if (o.folds == kFoldsPerFlush) far_flush_own(o, lane);
     const int l = own_lane(lane);
     const bool first = o.folds == 0;
 #pragma unroll
@@ -218,7 +219,7 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
         o.lsum[2 * kGroup + slot] = first ? az : o.lsum[2 * kGroup + slot] + az;
         o.ax[q] = o.ay[q] = o.az[q] = 0.0f;
     }
-    if (++o.folds == kFoldsPerFlush) far_flush_own(o, lane);
+    ++o.folds;
 }
 
 // Partners [b0, b1) (multiples of 16; those past n are left out) against the
@@ -279,10 +280,11 @@ __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const i
 template <bool UM, bool SOFT, bool COL>
 __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const int n, const int64_t nsb, const int c0,
                                          const int c1, const int64_t U, const int W, const int Q, const int fold,
-                                         float4* __restrict__ apart, const bool plain, float* __restrict__ bpart,
-                                         const float H2, const float m, float* lsum)
+                                         float4* __restrict__ apart, const bool plain, const int k, const bool merge,
+                                         float* __restrict__ bpart, const float H2, const float m, float* lsum)
 {
-    const int k = blockIdx.x, lane = threadIdx.x, len = kSB / Q;
+    if (k >= W) return;
+    const int lane = threadIdx.x & 63, len = kSB / Q;
     int64_t u = (int64_t)k * U / W;
     const int64_t u1 = (int64_t)(k + 1) * U / W;
     if (u >= u1) return;
@@ -296,7 +298,7 @@ __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const in
         const int first = kSB * (int)(COL ? col_first_group(g, c0) : g + 1) + len * (int)s;
         far_load_row(xs, n, g, lane, lsum, apart + (size_t)kFragElems * (g + k), plain, o);
         far_range<UM, SOFT>(xs, n, g, first, first + len * (int)cnt, fold, o, bpart, boff, H2, m, lane);
-        far_flush_own(o, lane);
+        if (!merge) far_flush_own(o, lane);
         u += cnt;
     }
 }
@@ -305,24 +307,48 @@ template <bool SOFT, bool COL>
 __device__ __forceinline__ void far_dispatch(const float4* __restrict__ xs, const int n, const int64_t nsb,
                                              const int c0, const int c1, const int64_t U, const int W, const int Q,
                                              const int fold, float4* __restrict__ apart, const int plain,
-                                             float* __restrict__ bpart, const float H2,
-                                             const float* __restrict__ umass, float* lsum)
+                                             const int k, const bool merge, float* __restrict__ bpart,
+                                             const float H2, const float* __restrict__ umass, float* lsum)
 {
     if (umass[0] != 0.0f)
-        far_work<true, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, umass[1], lsum);
+        far_work<true, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, k, merge, bpart, H2, umass[1], lsum);
     else
-        far_work<false, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, 1.0f, lsum);
+        far_work<false, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, k, merge, bpart, H2, 1.0f, lsum);
 }
 
+// Wavefronts share a workgroup so that, when their ranges lie in one row (all
+// but two a row), their own-side sums leave as one fragment: a fragment per
+// wavefront was 34 MB written and read again, whatever the count (Plummer
+// N = 16384: 69.6 -> 66.6 us per step, 50021: 441 -> 434).
 template <bool SOFT>
-__global__ __launch_bounds__(kFarThreads, 2) void far_kernel(const float4* __restrict__ xs, const int n,
-                                                            const int64_t nsb, const int64_t U, const int W,
-                                                            const int Q, const int fold,
-                                                            float4* __restrict__ apart, const int plain,
-                                                            float* __restrict__ bpart, const float H2, const float* __restrict__ umass)
+__global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __restrict__ xs, const int n,
+                                                               const int64_t nsb, const int64_t U, const int W,
+                                                               const int Q, const int fold,
+                                                               float4* __restrict__ apart, const int plain,
+                                                               float* __restrict__ bpart, const float H2,
+                                                               const float* __restrict__ umass)
 {
-    __shared__ float lsum[3 * kGroup];
-    far_dispatch<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, bpart, H2, umass, lsum);
+    __shared__ float lsum[kFarMerge][3 * kGroup];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int k0 = kFarMerge * (int)blockIdx.x;
+    const int64_t g = plain ? far_merged_row(k0, U, W, nsb, Q) : -1;
+    const bool merge = g >= 0;  // the same for the whole workgroup
+    far_dispatch<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, k0 + wave, merge, bpart, H2, umass,
+                              lsum[wave]);
+    if (!merge) return;
+    __syncthreads();
+    float4* const fr = apart + (size_t)kFragElems * (g + k0);
+    for (int q = wave; q < kNI; q += kFarMerge) {
+        const int slot = 64 * q + lane;
+        CSum v[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            v[c] = CSum{lsum[0][kGroup * c + slot], 0.0f};
+#pragma unroll
+            for (int w = 1; w < kFarMerge; ++w) v[c].add(lsum[w][kGroup * c + slot]);
+        }
+        fr[128 * q + lane] = make_float4(v[0].value(), v[1].value(), v[2].value(), 0.0f);  // frag_elem(slot)
+    }
 }
 
 // one column batch [c0, c1) of the far field
@@ -335,7 +361,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
                                                                    const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
-    far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, bpart, H2, umass, lsum);
+    far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
 }
 
 // Per slot, in a fixed order: the in-group sums, the far own-side fragments
@@ -366,18 +392,18 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
         }
         const int64_t g = t / kGroup, local = t - g * kGroup;
         if (U > 0 && g < rows_with_units(nsb)) {
-            // one fragment per workgroup that touched the row (every workgroup
-            // has a share: W <= U); eight fragments' loads in flight before
-            // their ordered adds
-            const int64_t k0 = wg_of_unit(row_prefix(g, nsb, Q), U, W);
-            const int64_t k1 = wg_of_unit(row_prefix(g + 1, nsb, Q) - 1, U, W);
-            int64_t k = k0 + p;
-            const int el = frag_elem((int)local);
-            for (; k + 7 * PARTS <= k1; k += 8 * PARTS) {
+            // one fragment per wavefront that touched the row (every wavefront
+            // has a share: W <= U), or per workgroup of them; eight fragments'
+            // loads in flight before their ordered adds
+            const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
+            const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
+            const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
+            int64_t k = p;
+            for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
                 float4 f[8], fc[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const float4* fr = apart + (size_t)kFragElems * (g + k + u * PARTS) + el;
+                    const float4* fr = fragment(k + u * PARTS);
                     f[u] = fr[0];
                     if (!PLAIN) fc[u] = fr[64];
                 }
@@ -387,8 +413,8 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
                     if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
                 }
             }
-            for (; k <= k1; k += PARTS) {
-                const float4* fr = apart + (size_t)kFragElems * (g + k) + el;
+            for (; k < R.count; k += PARTS) {
+                const float4* fr = fragment(k);
                 const float4 f = fr[0];
                 x.add(f.x); y.add(f.y); z.add(f.z);
                 if (!PLAIN) {
@@ -758,11 +784,12 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
     if (!sym_has_far(L)) return hipSuccess;
     const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     if (G.ncols == 1) {
+        const int far_groups = (L.wgs + kFarMerge - 1) / kFarMerge;
         if (P.H2 > 0.0f)
-            hipLaunchKernelGGL((far_kernel<true>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
+            hipLaunchKernelGGL((far_kernel<true>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
                                L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         else
-            hipLaunchKernelGGL((far_kernel<false>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, G.nsb, G.units,
+            hipLaunchKernelGGL((far_kernel<false>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
                                L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         return hipGetLastError();
     }
