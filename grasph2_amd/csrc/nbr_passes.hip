@@ -502,7 +502,9 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
         const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
         float II = 0.0f;
         if (AV) {  // :277-289 (models.h:158-185)
-            const float wij = __builtin_fmaf(rz, vz, __builtin_fmaf(ry, vy, rx * vx)) * (float)sep.ir;
+            // unfused, as the reference rounds it: in a rigid rotation every v . r is rounding alone, and its sign
+            // decides whether the pair counts for maxvsig
+            const float wij = (rx * vx + ry * vy + rz * vz) * (float)sep.ir;
             const float vsig = __builtin_fmaf(-3.0f, wij, P.c + P.c);
             const float b = BALS ? bi + qb.z : 2.0f;
             const float II0 = div_f32(-0.5f * P.alpha * b * wij * vsig, rho2, irho2);

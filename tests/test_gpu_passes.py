@@ -7,6 +7,7 @@ import pytest
 
 import grasph2_amd as g
 from grasph2_amd import ics
+from oracle import pyoracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +88,18 @@ def test_overflow_scans_in_a_batch(kind):
     for k in range(len(sizes)):
         for f in a[k]:
             assert np.array_equal(got[k][f], a[k][f]), (k, f)
+
+
+def test_rigid_rotation_counts_the_same_pairs():
+    """In a rigid rotation v . r of every pair is FP32 rounding, whose sign
+    decides whether the pair counts for maxvsig: evaluated as the FP32 oracle
+    rounds it, the same particles have none."""
+    n = 4000
+    print("passes rigid rotation n=%d" % n, flush=True)
+    h, prm = ics.large_sphere(n, seed=3, noise=0.0, spin=0.3)
+    prm.flags &= ~g.SELF_GRAVITY
+    got = run(h, prm, 0)["maxvsig"]
+    ref = O.compute_derivatives(prm, h, "f32")["maxvsig"]
+    assert np.array_equal(got == 0, ref == 0)
+    # 2 c and a wij of rounding
+    assert np.allclose(got, ref, rtol=1e-6, atol=0)
