@@ -458,7 +458,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
                      (c.sweep_symmetric == 1 ||
                       (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity)));
     const OwnPlan plan = own_plan(c, n, c.sweep_slices, kOwnSlicesMax);
-    const bool masses = sweep_grav && (sym || n >= kMassCheckMin);  // the equal-mass check
+    const bool masses = sweep_grav && n >= (sym ? kMassCheckMinSym : kMassCheckMin);  // the equal-mass check
     if (need_list) {
         grow_list_capacity(c, n, s);
         if ((r = ensure_nbr(c, n)) || (r = ensure_list_watch(c, s))) return r;

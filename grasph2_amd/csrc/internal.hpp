@@ -642,6 +642,11 @@ OwnPlan own_plan(const Ctx& c, int64_t n, int slices, int max_planes);
 // it Plummer 1000 14.2 -> 10 us per step, 9500 42.4 -> 38, allocation-free SPH
 // at 20000 240 -> 236; at 24000 271 -> 274)
 constexpr int64_t kMassCheckMin = 24576;
+// and from which the symmetric sweep looks at all masses first (below, the far
+// field's wavefronts look at their own, far_work, and the in-group gravity
+// takes them as they come: Plummer 16384 66.6 -> 61.5 us per step, 50021
+// 434 -> 423)
+constexpr int64_t kMassCheckMinSym = 65536;
 
 // arrays each pass needs, by configuration; 0 or a GRASPH_E_INVALID code
 int check_derivative_arrays(Ctx& c, const grasph_particles* p, uint32_t f, int which);

@@ -65,7 +65,7 @@ __device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, con
         near_part[2 * (size_t)t] = make_float4(x.s, y.s, z.s, 0.0f);
         near_part[2 * (size_t)t + 1] = make_float4(x.c, y.c, z.c, 0.0f);
     };
-    if (um[0] != 0.0f)
+    if (um && um[0] != 0.0f)
         own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
     else
         own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
@@ -226,8 +226,8 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
 // slots of row g, a chunk of 16 at a time; each chunk's partner side (summed
 // over the whole group: one wavefront owns it) goes straight to row g's
 // partials of its group (element 3 (bpart_group_base(J) - boff) on holds
-// group J's; boff: the groups before the column batch; UM: times the common
-// mass m).  The store has no condition: partners of the last chunk past n
+// group J's; boff: the groups before the column batch).  UM: the row's slots
+// have mass mo and the partners mass mp, which the sums take as a factor.  The store has no condition: partners of the last chunk past n
 // (their group's partials are allocated whole) get values nobody reads, and
 // a store behind a branch makes the compiler spill the chunk's registers.
 // The own side is folded every `fold` partners and at the end, so a slot
@@ -242,11 +242,12 @@ static int far_fold(int64_t n) { return n >= kFarFoldMin ? kFarFoldLarge : kFarF
 template <bool UM, bool SOFT>
 __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const int n, const int64_t g, const int b0,
                                           const int b1, const int fold, FarOwn& o, float* __restrict__ bpart,
-                                          const int64_t boff, const float H2, const float m, const int lane)
+                                          const int64_t boff, const float H2, const float mo, const float mp,
+                                          const int lane)
 {
     const int end = min(b1, n);
     if (b0 >= end) {  // a share of the last group past n: zeros in its fragment
-        far_fold_own<UM>(o, m, lane);
+        far_fold_own<UM>(o, mp, lane);
         return;
     }
     float* bp = nullptr;  // row g's partials of the chunk's first partner, for this lane
@@ -259,12 +260,12 @@ __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const i
         const float4 B = load_partner_row<UM>(xs, b + kRow, n, lane);  // unused after the last
         if (b + kRow > end) A = bound_partner_row(A, b, n, lane);
         const float v = far_chunk_rot<UM, SOFT>(A, o, H2);
-        *bp = UM ? v * m : v;
+        *bp = UM ? v * mo : v;
         bp += 3 * kRow;
         A = B;
         terms += kRow;
         if (terms == fold || b + kRow >= end) {
-            far_fold_own<UM>(o, m, lane);
+            far_fold_own<UM>(o, mp, lane);
             terms = 0;
         }
     }
@@ -277,11 +278,16 @@ __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const i
 // own-side sums of row g go to fragment g + k (plain: every fragment is
 // flushed once).  The whole far field keeps a kernel of its own (far_kernel),
 // so the row arithmetic of the batches does not change its code.
-template <bool UM, bool SOFT, bool COL>
+// umass null: each run finds out for itself whether its own slots have one
+// mass and its partners one (one more read of their masses, the first ones
+// with the row's slots; a kernel that looks at all particles first costs 5 us,
+// 8% of a Plummer step at 16384).
+template <bool SOFT, bool COL>
 __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const int n, const int64_t nsb, const int c0,
                                          const int c1, const int64_t U, const int W, const int Q, const int fold,
                                          float4* __restrict__ apart, const bool plain, const int k, const bool merge,
-                                         float* __restrict__ bpart, const float H2, const float m, float* lsum)
+                                         float* __restrict__ bpart, const float H2,
+                                         const float* __restrict__ umass, float* lsum)
 {
     if (k >= W) return;
     const int lane = threadIdx.x & 63, len = kSB / Q;
@@ -296,24 +302,34 @@ __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const in
         const int64_t row = COL ? col_row_units(g, c0, c1, Q) : row_units(g, nsb, Q);
         const int64_t cnt = min(row - s, u1 - u);
         const int first = kSB * (int)(COL ? col_first_group(g, c0) : g + 1) + len * (int)s;
+        const int end = first + len * (int)cnt;
+        float mo, mp = 0.0f, mj = 0.0f;
+        if (!umass) {
+            mp = xs[min(first, n - 1)].w;
+            mj = xs[min(first + lane, min(end, n) - 1)].w;
+        }
         far_load_row(xs, n, g, lane, lsum, apart + (size_t)kFragElems * (g + k), plain, o);
-        far_range<UM, SOFT>(xs, n, g, first, first + len * (int)cnt, fold, o, bpart, boff, H2, m, lane);
+        bool one_mass;
+        if (umass) {
+            one_mass = umass[0] != 0.0f;
+            mo = mp = umass[1];
+        } else {
+            mo = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(o.m[0])));
+            int differ = __float_as_int(mj) ^ __float_as_int(mp);
+#pragma unroll
+            for (int q = 0; q < kNI; ++q) differ |= __float_as_int(o.m[q]) ^ __float_as_int(mo);
+#pragma unroll 4
+            for (int j = first + 64 + lane; j < min(end, n); j += 64)
+                differ |= __float_as_int(xs[j].w) ^ __float_as_int(mp);
+            one_mass = !__any(differ != 0);
+        }
+        if (one_mass)
+            far_range<true, SOFT>(xs, n, g, first, end, fold, o, bpart, boff, H2, mo, mp, lane);
+        else
+            far_range<false, SOFT>(xs, n, g, first, end, fold, o, bpart, boff, H2, 1.0f, 1.0f, lane);
         if (!merge) far_flush_own(o, lane);
         u += cnt;
     }
-}
-
-template <bool SOFT, bool COL>
-__device__ __forceinline__ void far_dispatch(const float4* __restrict__ xs, const int n, const int64_t nsb,
-                                             const int c0, const int c1, const int64_t U, const int W, const int Q,
-                                             const int fold, float4* __restrict__ apart, const int plain,
-                                             const int k, const bool merge, float* __restrict__ bpart,
-                                             const float H2, const float* __restrict__ umass, float* lsum)
-{
-    if (umass[0] != 0.0f)
-        far_work<true, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, k, merge, bpart, H2, umass[1], lsum);
-    else
-        far_work<false, SOFT, COL>(xs, n, nsb, c0, c1, U, W, Q, fold, apart, plain, k, merge, bpart, H2, 1.0f, lsum);
 }
 
 // Wavefronts share a workgroup so that, when their ranges lie in one row (all
@@ -333,8 +349,8 @@ __global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __
     const int k0 = kFarMerge * (int)blockIdx.x;
     const int64_t g = plain ? far_merged_row(k0, U, W, nsb, Q) : -1;
     const bool merge = g >= 0;  // the same for the whole workgroup
-    far_dispatch<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, k0 + wave, merge, bpart, H2, umass,
-                              lsum[wave]);
+    far_work<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, k0 + wave, merge, bpart, H2, umass,
+                          lsum[wave]);
     if (!merge) return;
     __syncthreads();
     float4* const fr = apart + (size_t)kFragElems * (g + k0);
@@ -361,7 +377,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
                                                                    const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
-    far_dispatch<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
+    far_work<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
 }
 
 // Per slot, in a fixed order: the in-group sums, the far own-side fragments
@@ -590,7 +606,7 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
 {
     FarOwn o;
     far_load_row(xk, n, R.g, lane, lsum, frag, plain, o);
-    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kFarFoldLarge, o, bk, 0, H2, m, lane);
+    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kFarFoldLarge, o, bk, 0, H2, m, m, lane);
     far_flush_own(o, lane);
 }
 

@@ -57,3 +57,34 @@ def test_far_shares(n):
     mx, norm = vec_errors(out[0], out[1])
     # both sides within the bound above of the exact sums
     assert mx < 2e-5 and norm < 1e-6, (mx, norm)
+
+
+# Below 65536 particles every run of partners decides for itself whether its
+# row's slots have one mass and its partners one: two masses (most runs have
+# one on each side, some another on each), one particle that differs, all.
+@pytest.mark.parametrize("masses", ["two", "one differs", "none equal"])
+@pytest.mark.parametrize("soft", [True, False])
+def test_far_runs_of_one_mass(masses, soft):
+    n = 5000
+    print("far masses %s soft=%s" % (masses, soft), flush=True)
+    h, prm = ics.plummer(n, seed=7)
+    m = h["posm"][:, 3]
+    if masses == "two":
+        m[n // 3:] *= np.float32(1.7)
+    elif masses == "one differs":
+        m[n - 40] *= np.float32(3.0)
+    else:
+        m *= np.random.default_rng(7).uniform(0.5, 2.0, size=n).astype(np.float32)
+    if not soft:
+        prm.H = 0.0
+    ctx = g.Context(0)
+    ctx.set_option("sweep_symmetric", 1)
+    d = g.DeviceParticles.from_host(h)
+    ctx.compute_derivatives(d, prm)
+    g.hip.synchronize()
+    got = d.download(["acc"])["acc"]
+    d.free()
+    ctx.close()
+    mx, norm = vec_errors(got, O.compute_derivatives(prm, h, "f64")["acc"])
+    # as above; without softening the closest pairs' FP32 separations carry up to 2^-24 |x| / r each
+    assert (mx < 1e-5 and norm < 1e-6) if soft else (mx < 1e-3 and norm < 1e-4), (mx, norm)
