@@ -301,13 +301,12 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
     return L;
 }
 
-// The symmetric sweep's default thresholds (option sweep_symmetric = 2),
-// measured step times, symmetric against one-sided: with neighbour lists
-// (default solids / collision) 106 / 119 against 105 / 113 us at 12500
-// particles, 112 / 124 against 115 / 127 at 14000; gravity alone (Plummer) 69
-// against 66 at 14000, 77 against 76 at 15500, 82 against 94 at 16500.
-constexpr int64_t kSymAutoMinLists = 13312;
-constexpr int64_t kSymAutoMinGravity = 15360;
+// The symmetric sweep's default threshold (option sweep_symmetric = 2),
+// measured step times, symmetric against one-sided: gravity alone (Plummer) 41
+// against 38 us at 9500 particles, 42 against 47 at 11000; with neighbour lists
+// (default solids / collision) 88 / 96 against 89 / 94 at 9500, 89 / 94 against
+// 90 / 99 at 11000.
+constexpr int64_t kSymAutoMin = 10752;
 
 int sym_wgs(const Ctx& c) { return c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(c.cus); }
 
@@ -346,8 +345,10 @@ int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t 
     S.finish = L.finish;
     S.add_acc = add_acc;
     // wavefronts per 64 slots (Plummer steps at 16384: 81.3 us with 4, 77.3
-    // with 8, 77.8 with 16; at 50021: 437 with 1, 416 with 4, 418 with 8)
-    S.near_waves = c.sym_near_shares > 0 ? near_waves_of(c.sym_near_shares) : L.n < 32768 ? 8 : 4;
+    // with 8, 77.8 with 16; at 50021: 437 with 1, 416 with 4, 418 with 8); with
+    // 8 the combine is in the same launch (50021: 379.3 -> 377.8, from 65536
+    // on the same as 4 and two launches)
+    S.near_waves = c.sym_near_shares > 0 ? near_waves_of(c.sym_near_shares) : L.n < 65536 ? 8 : 4;
     S.acc = L.acc;
     S.vel = L.vel;
     S.xvel = L.xvel;
@@ -363,6 +364,12 @@ int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t 
     if (sym_has_far(S)) {
         ProfScope ps(&c, s, KC_FAR);
         if ((e = launch_sym_far(S, P, s)) != hipSuccess) return hip_fail(c, e, "far-field launch");
+    }
+    if (sym_fused(S)) {
+        ProfScope ps(&c, s, KC_SWEEP);
+        if ((e = launch_sym_near_combine(S, P, s)) != hipSuccess)
+            return hip_fail(c, e, "in-group gravity and combine launch");
+        return 0;
     }
     {
         ProfScope ps(&c, s, KC_SWEEP);
@@ -456,7 +463,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     const bool sweep_grav = accel_pass && grav;
     const bool sym = sweep_grav &&
                      (c.sweep_symmetric == 1 ||
-                      (c.sweep_symmetric == 2 && n >= (need_list ? kSymAutoMinLists : kSymAutoMinGravity)));
+                      (c.sweep_symmetric == 2 && n >= kSymAutoMin));
     const OwnPlan plan = own_plan(c, n, c.sweep_slices, kOwnSlicesMax);
     const bool masses = sweep_grav && n >= (sym ? kMassCheckMinSym : kMassCheckMin);  // the equal-mass check
     if (need_list) {

@@ -224,6 +224,8 @@ struct SymLaunch {
 // field, then the combine
 hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_t s);
 hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s);
+bool sym_fused(const SymLaunch& L);
+hipError_t launch_sym_near_combine(const SymLaunch& L, const DevParams& P, hipStream_t s);
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s);
 bool sym_has_far(const SymLaunch& L);
 

@@ -127,7 +127,8 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     // between its slots, and if a part still is, boxes are tested against the
     // slots one by one.  (With the wide box one such wavefront tested every
     // particle: N = 200003, 1736 us instead of 207; with all of them slot by
-    // slot those wavefronts were the last by far: liquid of 8192 TBD us.)
+    // slot those wavefronts were the last by far: liquid of 8192, 20.8 us
+    // instead of 14.9.)
     const auto wide = [&](const float4 l, const float4 h) {
         const float w = fmaxf(h.x - l.x, fmaxf(h.y - l.y, h.z - l.z));
         return (bool)__builtin_amdgcn_readfirstlane(w * w > 4.0f * H2);

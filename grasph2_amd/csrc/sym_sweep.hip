@@ -53,22 +53,25 @@ __device__ __forceinline__ float swap16_sum(float p, float q)
 
 // In-group gravity: a workgroup takes 64 NI slots of a group, its wavefronts
 // an equal share of the group's slots as partners each (whole shares of
-// kGroup / waves, whatever the group holds).  Writes the slot's compensated
-// sums (slot-indexed, two float4).
-template <int NI, bool SOFT>
+// kGroup / waves, whatever the group holds).  store(t, x, y, z) gets every
+// slot's compensated sums.
+template <int NI, bool SOFT, typename F>
 __device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, const int o0, const int g0, const int g1,
-                                              float4* __restrict__ near_part, const float h2,
-                                              const float* __restrict__ um, float* lds)
+                                              const float h2, const float* __restrict__ um, float* lds, F&& store)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
-    auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
-        near_part[2 * (size_t)t] = make_float4(x.s, y.s, z.s, 0.0f);
-        near_part[2 * (size_t)t + 1] = make_float4(x.c, y.c, z.c, 0.0f);
-    };
     if (um && um[0] != 0.0f)
         own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
     else
         own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
+}
+
+// a slot's compensated sums as two float4
+__device__ __forceinline__ void store_near(float4* __restrict__ near_part, const int t, const CSum& x, const CSum& y,
+                                           const CSum& z)
+{
+    near_part[2 * (size_t)t] = make_float4(x.s, y.s, z.s, 0.0f);
+    near_part[2 * (size_t)t + 1] = make_float4(x.c, y.c, z.c, 0.0f);
 }
 
 template <bool SOFT>
@@ -78,7 +81,8 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void ingroup_kernel(const float4
 {
     extern __shared__ float lds[];
     const int o0 = 64 * blockIdx.x, g0 = o0 / kGroup * kGroup;
-    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), near_part, h2, umass, lds);
+    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), h2, umass, lds,
+                           [&](int t, const CSum& x, const CSum& y, const CSum& z) { store_near(near_part, t, x, y, z); });
 }
 
 // One chunk of 16 partners (pj: row lane l holds partner l) against the
@@ -380,6 +384,110 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
     far_work<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
 }
 
+// The far field's part p of PARTS of slot t's sums: the own-side fragments of
+// its row, then the partner-side partials, every PARTS-th from the p-th on.
+template <int PARTS, bool PLAIN>
+__device__ __forceinline__ void far_sums(const float4* __restrict__ apart, const float* __restrict__ bpart,
+                                         const int t, const int p, const int64_t nsb, const int64_t U, const int W,
+                                         const int Q, CSum& x, CSum& y, CSum& z)
+{
+            const int64_t g = t / kGroup, local = t - g * kGroup;
+            if (U > 0 && g < rows_with_units(nsb)) {
+                // one fragment per wavefront that touched the row (every wavefront
+                // has a share: W <= U), or per workgroup of them; eight fragments'
+                // loads in flight before their ordered adds
+                const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
+                const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
+                const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
+                int64_t k = p;
+                for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
+                    float4 f[8], fc[8];
+    #pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const float4* fr = fragment(k + u * PARTS);
+                        f[u] = fr[0];
+                        if (!PLAIN) fc[u] = fr[64];
+                    }
+    #pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
+                        if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
+                    }
+                }
+                for (; k < R.count; k += PARTS) {
+                    const float4* fr = fragment(k);
+                    const float4 f = fr[0];
+                    x.add(f.x); y.add(f.y); z.add(f.z);
+                    if (!PLAIN) {
+                        const float4 fc = fr[64];
+                        x.c += fc.x; y.c += fc.y; z.c += fc.z;
+                    }
+                }
+            }
+            const int64_t base = bpart_group_base(g) + local;
+            const int ng = (int)g;
+            // eight groups' loads in flight before their (ordered) adds
+            int gp = p;
+            for (; gp + 7 * PARTS < ng; gp += 8 * PARTS) {
+                float v[8][3];
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const size_t e = 3 * (size_t)(base + (int64_t)(gp + u * PARTS) * kGroup);
+                    v[u][0] = bpart[e]; v[u][1] = bpart[e + 1]; v[u][2] = bpart[e + 2];
+                }
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
+                }
+            }
+            for (; gp < ng; gp += PARTS) {
+                const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
+                x.add(-bpart[e]); y.add(-bpart[e + 1]); z.add(-bpart[e + 2]);
+            }
+}
+
+// The parts' sums added in part order, in part 0's threads (thread q kSlots +
+// l holds part q of the workgroup's l-th slot).
+template <int PARTS, int SLOTS>
+__device__ __forceinline__ void add_parts(const int p, CSum& x, CSum& y, CSum& z)
+{
+    __shared__ float red[6][PARTS * SLOTS];  // every thread reaches the barrier
+    if (p > 0) {
+        red[0][threadIdx.x] = x.s; red[1][threadIdx.x] = x.c;
+        red[2][threadIdx.x] = y.s; red[3][threadIdx.x] = y.c;
+        red[4][threadIdx.x] = z.s; red[5][threadIdx.x] = z.c;
+    }
+    __syncthreads();
+    if (p > 0) return;
+#pragma unroll
+    for (int q = 1; q < PARTS; ++q) {
+        const int o = (int)threadIdx.x + q * SLOTS;
+        x.add(red[0][o]); x.c += red[1][o];
+        y.add(red[2][o]); y.c += red[3][o];
+        z.add(red[4][o]); z.c += red[5][o];
+    }
+}
+
+// slot t's gravity into the acceleration of its particle
+__device__ __forceinline__ void finish_slot(const int t, CSum x, CSum y, CSum z, const int* __restrict__ perm,
+                                            float4* __restrict__ acc, const int finish, const int add_acc,
+                                            float4* __restrict__ xvel, float* __restrict__ maxvsig,
+                                            const DevParams& P)
+{
+    const int i = perm ? perm[t] : t;
+    if (add_acc) {  // the SPH terms (and environment), summed before the far field was done
+        const float4 a = acc[i];
+        x.add(a.x); y.add(a.y); z.add(a.z);
+    }
+    float ax = x.value(), ay = y.value(), az = z.value();
+    if (finish) {
+        environment_acceleration(P, ax, ay, az);
+        if (xvel) xvel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (maxvsig) maxvsig[i] = 0.0f;
+    }
+    acc[i] = make_float4(ax, ay, az, 0.0f);
+}
+
 // Per slot, in a fixed order: the in-group sums, the far own-side fragments
 // (workgroup order), the far partner-side partials (group order, negated:
 // they were summed as seen from the other side), compensated; then the
@@ -393,9 +501,8 @@ template <int PARTS, bool PLAIN>
 __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
     const int n, const int64_t nsb, const int64_t U, const int W, const int Q, const int grav,
-    const int* __restrict__ perm,
-    const float4* __restrict__ xs, float4* __restrict__ acc, const int finish, const int add_acc,
-    const float4* __restrict__ vel, float4* __restrict__ xvel, float* __restrict__ maxvsig, const DevParams P)
+    const int* __restrict__ perm, float4* __restrict__ acc, const int finish, const int add_acc,
+    float4* __restrict__ xvel, float* __restrict__ maxvsig, const DevParams P)
 {
     constexpr int kSlots = kBlock / PARTS;  // slots per block
     const int p = (int)threadIdx.x / kSlots;
@@ -406,90 +513,36 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
             const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
             x = CSum{a.x, c.x}; y = CSum{a.y, c.y}; z = CSum{a.z, c.z};
         }
-        const int64_t g = t / kGroup, local = t - g * kGroup;
-        if (U > 0 && g < rows_with_units(nsb)) {
-            // one fragment per wavefront that touched the row (every wavefront
-            // has a share: W <= U), or per workgroup of them; eight fragments'
-            // loads in flight before their ordered adds
-            const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
-            const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
-            const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
-            int64_t k = p;
-            for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
-                float4 f[8], fc[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const float4* fr = fragment(k + u * PARTS);
-                    f[u] = fr[0];
-                    if (!PLAIN) fc[u] = fr[64];
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
-                    if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
-                }
-            }
-            for (; k < R.count; k += PARTS) {
-                const float4* fr = fragment(k);
-                const float4 f = fr[0];
-                x.add(f.x); y.add(f.y); z.add(f.z);
-                if (!PLAIN) {
-                    const float4 fc = fr[64];
-                    x.c += fc.x; y.c += fc.y; z.c += fc.z;
-                }
-            }
-        }
-        const int64_t base = bpart_group_base(g) + local;
-        const int ng = (int)g;
-        // eight groups' loads in flight before their (ordered) adds
-        int gp = p;
-        for (; gp + 7 * PARTS < ng; gp += 8 * PARTS) {
-            float v[8][3];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const size_t e = 3 * (size_t)(base + (int64_t)(gp + u * PARTS) * kGroup);
-                v[u][0] = bpart[e]; v[u][1] = bpart[e + 1]; v[u][2] = bpart[e + 2];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
-            }
-        }
-        for (; gp < ng; gp += PARTS) {
-            const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
-            x.add(-bpart[e]); y.add(-bpart[e + 1]); z.add(-bpart[e + 2]);
-        }
+        far_sums<PARTS, PLAIN>(apart, bpart, t, p, nsb, U, W, Q, x, y, z);
     }
-    if constexpr (PARTS > 1) {
-        __shared__ float red[6][kBlock];  // every thread reaches the barrier
-        if (p > 0) {
-            red[0][threadIdx.x] = x.s; red[1][threadIdx.x] = x.c;
-            red[2][threadIdx.x] = y.s; red[3][threadIdx.x] = y.c;
-            red[4][threadIdx.x] = z.s; red[5][threadIdx.x] = z.c;
-        }
-        __syncthreads();
-        if (p > 0) return;
-#pragma unroll
-        for (int q = 1; q < PARTS; ++q) {
-            const int o = (int)threadIdx.x + q * kSlots;
-            x.add(red[0][o]); x.c += red[1][o];
-            y.add(red[2][o]); y.c += red[3][o];
-            z.add(red[4][o]); z.c += red[5][o];
-        }
-    }
-    if (t >= n) return;
-    const int i = perm ? perm[t] : t;
-    if (add_acc) {  // the SPH terms (and environment), summed before the far field was done
-        const float4 a = acc[i];
-        x.add(a.x); y.add(a.y); z.add(a.z);
-    }
-    float ax = x.value(), ay = y.value(), az = z.value();
-    if (finish) {
-        environment_acceleration(P, ax, ay, az);
-        if (xvel) xvel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (maxvsig) maxvsig[i] = 0.0f;
-    }
-    acc[i] = make_float4(ax, ay, az, 0.0f);
+    if constexpr (PARTS > 1) add_parts<PARTS, kSlots>(p, x, y, z);
+    if (p == 0 && t < n) finish_slot(t, x, y, z, perm, acc, finish, add_acc, xvel, maxvsig, P);
+}
+
+// In-group gravity and combine in one launch, for counts at which either
+// takes as long as its launch: a workgroup of kNearFused wavefronts makes 64
+// slots' in-group sums as ingroup_kernel does, then wavefront p is their part
+// p of the combine.  The sums are the two kernels' bit for bit.  Plummer N =
+// 16384: 61.5 -> 59.4 us per step.
+constexpr int kNearFused = 8;
+template <bool SOFT>
+__global__ __launch_bounds__(64 * kNearFused) void near_combine_kernel(
+    const float4* __restrict__ xs, const float4* __restrict__ apart, const float* __restrict__ bpart, const int n,
+    const int64_t nsb, const int64_t U, const int W, const int Q, const float* __restrict__ umass,
+    const int* __restrict__ perm, float4* __restrict__ acc, const int finish, const int add_acc,
+    float4* __restrict__ xvel, float* __restrict__ maxvsig, const DevParams P)
+{
+    __shared__ float lds[own_lds_floats(1, kNearFused)];
+    const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int o0 = 64 * blockIdx.x, g0 = o0 / kGroup * kGroup, t = o0 + lane;
+    CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
+    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), P.H2, umass, lds,
+                           [&](int, const CSum& a, const CSum& b, const CSum& c) {  // wavefront 0's lanes
+                               x = a; y = b; z = c;
+                           });
+    if (t < n) far_sums<kNearFused, true>(apart, bpart, t, p, nsb, U, W, Q, x, y, z);
+    add_parts<kNearFused, 64>(p, x, y, z);
+    if (p == 0 && t < n) finish_slot(t, x, y, z, perm, acc, finish, add_acc, xvel, maxvsig, P);
 }
 
 // After column batch [c0, c1) of the far field (column-batched far field,
@@ -593,8 +646,8 @@ __global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4*
     const int4 bl = blk[xcd_block((int)blockIdx.x, (int)gridDim.x)];  // XCD-contiguous (xcd_block)
     const SymInst S = sinst[bl.x];
     const int g0 = S.off + (bl.y - S.off) / kGroup * kGroup;
-    ingroup_block<4, SOFT>(xs, bl.y, g0, min(S.off + S.n, g0 + kGroup), near_part, insts[bl.x].H2, umass + 2 * bl.x,
-                           lds);
+    ingroup_block<4, SOFT>(xs, bl.y, g0, min(S.off + S.n, g0 + kGroup), insts[bl.x].H2, umass + 2 * bl.x, lds,
+                           [&](int t, const CSum& x, const CSum& y, const CSum& z) { store_near(near_part, t, x, y, z); });
 }
 
 // one piece of a far row of an instance of the batch: group R.g against
@@ -818,6 +871,25 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
     return hipGetLastError();
 }
 
+// both of the next two in one launch, where that is the faster way
+bool sym_fused(const SymLaunch& L)
+{
+    if (L.n <= 0 || !L.grav || L.near_waves != kNearFused) return false;
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
+    return G.ncols == 1 && G.plain;
+}
+hipError_t launch_sym_near_combine(const SymLaunch& L, const DevParams& P, hipStream_t s)
+{
+    const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
+#define GRASPH_FUSED(SOFT)                                                                                            \
+    hipLaunchKernelGGL(near_combine_kernel<SOFT>, dim3((L.n + 63) / 64), dim3(64 * kNearFused), 0, s, L.xs, L.apart, \
+                       L.bpart, L.n, G.nsb, G.units, L.wgs, G.split, L.umass, L.perm, L.acc, L.finish ? 1 : 0,       \
+                       L.add_acc ? 1 : 0, L.xvel, L.maxvsig, P)
+    if (P.H2 > 0.0f) GRASPH_FUSED(true); else GRASPH_FUSED(false);
+#undef GRASPH_FUSED
+    return hipGetLastError();
+}
+
 // combine (after both fields): the acceleration
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
@@ -835,7 +907,7 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
 #define GRASPH_COMBINE(PARTS, PLAIN)                                                                                  \
     hipLaunchKernelGGL((sym_combine_kernel<PARTS, PLAIN>), dim3((L.n + kBlock / PARTS - 1) / (kBlock / PARTS)),        \
                        dim3(kBlock), 0, s, L.near_part, L.apart, L.bpart, L.n, G.nsb, G.units, L.wgs,       \
-                       G.split, L.grav ? 1 : 0, L.perm, L.xs, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0, L.vel,       \
+                       G.split, L.grav ? 1 : 0, L.perm, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0,        \
                        L.xvel, L.maxvsig, P)
     if (G.plain) {
         switch (parts) {

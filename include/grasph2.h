@@ -169,7 +169,7 @@ int grasph_destroy(grasph_ctx* ctx);
  * shape), "sweep_symmetric" (single
  * instance: 1 = gravity between groups of 1024 particles evaluated once per
  * pair for both sides, 0 = the one-sided sweep, 2 = the symmetric sweep from
- * 15360 particles on, 13312 with neighbour lists, the default; results agree to FP32 rounding, the
+ * 10752 particles on, the default; results agree to FP32 rounding, the
  * neighbour lists are identical), "sym_workgroups" (workgroups of the
  * symmetric sweep's far-field kernel, single instances and batches, 0 = two
  * wavefronts per SIMD), "sym_partial_bytes" (single instance: device memory
