@@ -45,11 +45,12 @@ namespace grasph {
 namespace {
 
 constexpr int kBlock = 256, kWaves = kBlock / 64;
-// steps in flight of each pass's walk (for_each_neighbour's D): what hides
-// their latency is wavefronts, and a deeper ring costs them registers
-// (density 48 -> 38 us, strain 101 -> 74, acceleration 101 -> 89 at 200003
-// particles, half of it from dropping 4, 2 and 2 steps to these)
-constexpr int kDeepDensity = 2, kDeepStrain = 1, kDeepAccel = 1;
+// steps in flight of each pass's walk (for_each_neighbour's D; strain: with 4
+// lanes, with 16 one): what hides their latency is wavefronts, and a deeper
+// ring costs them registers.  All three passes at 200003 particles: 238 us
+// with 4, 2 and 2 steps and the terms added in the order of all neighbours
+// (48, 101, 89), now 32, 70 and 90.
+constexpr int kDeepDensity = 2, kDeepStrain = 2, kDeepAccel = 1;
 
 // lambdas are inlined by force: called from the list walk and the overflow
 // scan, they would otherwise stay calls and pass the records through scratch
@@ -90,14 +91,14 @@ struct Lists {
 
 // LPP lanes share a particle (4 or 16): lane l of a wavefront serves
 // particle l / LPP of the wavefront's 64 / LPP, and in step e of the walk
-// neighbour e LPP + l % LPP of its list.  The terms are then added in the
-// list's order whatever LPP is (OrderedSums), so the sums do not depend on
-// it: a batch's equal the single instance's bit for bit, and a list's those
-// of its overflow scan.  Against one lane per particle: 4 to 16 times the
-// wavefronts for small counts (8192 particles: density, strain and
-// acceleration 76 -> 27 us), lists of 16 or 4 particles instead of 64 to wait
-// for, and neighbouring lanes read neighbouring records (512 instances:
-// 4.7 -> 3.9 ms).
+// neighbour e LPP + l % LPP of its list.  A particle has four sums of each
+// quantity, of the neighbours k with k mod 4 = 0, 1, 2, 3 in the list's order,
+// added at the end (ClassSums), whatever LPP is: a batch's results equal the
+// single instance's bit for bit, and a list's those of its overflow scan.
+// Against one lane per particle: 4 to 16 times the wavefronts for small counts
+// (8192 particles: density, strain and acceleration 76 -> 26 us), lists of 16
+// or 4 particles instead of 64 to wait for, and neighbouring lanes read
+// neighbouring records (512 instances: 4.7 -> 3.7 ms).
 template <int LPP>
 __device__ __forceinline__ int pass_slot(const SlotMap& m)
 {
@@ -116,57 +117,119 @@ __device__ __forceinline__ void wave_lds_order()
 __device__ __forceinline__ void acc_add(CSum& a, float v) { a.add(v); }
 __device__ __forceinline__ void acc_add(float& a, float v) { a += v; }
 __device__ __forceinline__ void acc_add(double& a, double v) { a += v; }
-__device__ __forceinline__ float acc_value(const CSum& a) { return a.value(); }
-__device__ __forceinline__ float acc_value(float a) { return a; }
-__device__ __forceinline__ double acc_value(double a) { return a; }
 
-// NC running sums of a particle (A: the accumulator of terms of type T), the
-// terms added in the order of the neighbours: the lanes of a particle write
-// their terms to LDS (kRow apart, so the components' rows start in different
-// banks) and lane s adds all LPP terms of the components s, s + LPP, ....
+// adds a class's sum to another's: nothing when it is zero, so that an
+// infinite gravity without neighbours stays one
+__device__ __forceinline__ void acc_merge(CSum& a, const float s, const float c)
+{
+    if (s != 0.0f) a.add(s);
+    a.c += c;
+}
+
+// NC sums of a particle (A: the accumulator of terms of type T) by classes of
+// neighbours.  With 4 lanes each lane is a class and keeps its own sums (with
+// the terms exchanged through LDS and added by all neighbours' order, the
+// exchange took density and strain at 200003 particles 38 and 74 us, now 32
+// and 70).  With
+// 16 the four lanes of a class write their terms to LDS, side by side, a row
+// per quantity (kRow apart, so the rows start in different banks), and lane
+// 4 q + r adds those of class r of the quantities q, q + 4, ....
 template <int LPP, int NC, typename T, typename A>
-struct OrderedSums {
-    static constexpr int K = (NC + LPP - 1) / LPP;
+struct ClassSums {
+    static constexpr int K = LPP == 4 ? NC : (NC + 3) / 4;
     static constexpr int kRow = 64 + 16 / (int)sizeof(T);
-    static constexpr int kLds = NC * kRow;  // elements of T per wavefront
+    static constexpr int kLds = LPP == 4 ? 4 : NC * kRow;  // elements of T per wavefront
     A a[K];
 
-    // the component of accumulator k (lanes without one repeat the last)
-    __device__ __forceinline__ static int comp(int sub, int k) { return min(sub + k * LPP, NC - 1); }
+    // the quantity of accumulator k in lane sub (lanes without one repeat the last)
+    __device__ __forceinline__ static int quantity(int sub, int k)
+    {
+        return LPP == 4 ? k : min(sub / 4 + 4 * k, NC - 1);
+    }
+    // what the sum of quantity c starts from
+    __device__ __forceinline__ void init(const int c, const T v, const int lane)
+    {
+        const int sub = lane % LPP;
+        if (LPP == 4 ? sub == 0 : sub == 4 * (c % 4)) a[LPP == 4 ? c : c / 4] = start(v);
+    }
     // the step's terms (this lane's in v) of the group's first `rem` lanes
     __device__ __forceinline__ void add(const T (&v)[NC], const int rem, T* lds, const int lane)
     {
         const int sub = lane % LPP;
+        if constexpr (LPP == 4) {
+            if (sub < rem) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) lds[c * kRow + lane] = v[c];
-        wave_lds_order();
-        T w[K][LPP];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const T* row = (const T*)__builtin_assume_aligned(lds + comp(sub, k) * kRow + (lane - sub), 16);
-#pragma unroll
-            for (int u = 0; u < LPP; ++u) w[k][u] = row[u];
-        }
-        wave_lds_order();
-#pragma unroll
-        for (int u = 0; u < LPP; ++u)
-            if (u < rem) {
-#pragma unroll
-                for (int k = 0; k < K; ++k) acc_add(a[k], w[k][u]);
+                for (int c = 0; c < NC; ++c) acc_add(a[c], v[c]);
             }
+        } else {
+            T* const group = lds + (lane - sub);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) group[c * kRow + 4 * (sub % 4) + sub / 4] = v[c];
+            wave_lds_order();
+            T w[K][4];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const T* row = (const T*)__builtin_assume_aligned(group + quantity(sub, k) * kRow + 4 * (sub % 4), 16);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[k][u] = row[u];
+            }
+            wave_lds_order();
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (sub % 4 + 4 * u < rem) {
+#pragma unroll
+                    for (int k = 0; k < K; ++k) acc_add(a[k], w[k][u]);
+                }
+        }
     }
-    // one neighbour's terms, the same in every lane of the group
-    __device__ __forceinline__ void add_one(const T (&v)[NC], T* lds, const int lane)
+    // the terms of neighbour `at`, the same in every lane of the group
+    __device__ __forceinline__ void add_one(const T (&v)[NC], const int at, T* lds, const int lane)
     {
+        const int sub = lane % LPP;
+        if constexpr (LPP == 4) {
+            if (sub == at % 4) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) lds[c * kRow + lane] = v[c];
+                for (int c = 0; c < NC; ++c) acc_add(a[c], v[c]);
+            }
+        } else {
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc_add(a[k], lds[comp(lane % LPP, k) * kRow + lane]);
+            for (int c = 0; c < NC; ++c) lds[c * kRow + lane] = v[c];
+            if (sub % 4 == at % 4) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) acc_add(a[k], lds[quantity(sub, k) * kRow + lane]);
+            }
+        }
     }
     // sum c, in every lane of the group (all lanes of the wavefront take part)
     __device__ __forceinline__ T value(const int c, const int lane) const
     {
-        return __shfl(acc_value(a[c / LPP]), lane - lane % LPP + c % LPP, 64);
+        const A& m = a[LPP == 4 ? c : c / 4];
+        const int first = lane - lane % LPP + (LPP == 4 ? 0 : 4 * (c % 4));  // its class 0
+        return total(m, first);
+    }
+
+  private:
+    __device__ __forceinline__ static CSum start_of(float v, CSum*) { return CSum{v, 0.0f}; }
+    __device__ __forceinline__ static T start_of(T v, T*) { return v; }
+    __device__ __forceinline__ static A start(T v) { return start_of(v, (A*)nullptr); }
+    __device__ __forceinline__ static float total(const CSum& m, const int first)
+    {
+        float s[4], e[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = __shfl(m.s, first + r, 64);
+            e[r] = __shfl(m.c, first + r, 64);
+        }
+        CSum x{s[0], e[0]}, y{s[2], e[2]};
+        acc_merge(x, s[1], e[1]);
+        acc_merge(y, s[3], e[3]);
+        acc_merge(x, y.s, y.c);
+        return x.value();
+    }
+    __device__ __forceinline__ static T total(const T& m, const int first)
+    {
+        return (__shfl(m, first, 64) + __shfl(m, first + 1, 64)) +
+               (__shfl(m, first + 2, 64) + __shfl(m, first + 3, 64));
     }
 };
 
@@ -179,7 +242,8 @@ typedef float vec4 __attribute__((ext_vector_type(4)));
 // partners, same order).
 // step(q, rem): q holds the first PIECES float4 of the neighbour's record (of
 // STRIDE float4 at src); lane sub has one if sub < rem (the others repeat the
-// last).  one(q): a neighbour found by the scan, the same for the whole group.
+// last).  one(q, at): neighbour `at` found by the scan, the same for the whole
+// group.
 //
 // The walk is software-pipelined D deep: while step e is computed, the
 // records of steps e + 1 .. e + D and the indices up to e + 2 D are in
@@ -229,6 +293,7 @@ __device__ __forceinline__ void for_each_neighbour(const vec4* __restrict__ src,
     }
     if (act && cnt > kmax) {
         const float4* const coarse = Ls.coarse + 2 * (size_t)m.coarse0;
+        int at = 0;
         for (int first = 0; first < m.n; first += kBoxCoarse) {
             // a box farther than H holds none of the partners (lists.hip)
             const float4 lo = coarse[2 * (first / kBoxCoarse)], hi = coarse[2 * (first / kBoxCoarse) + 1];
@@ -245,7 +310,7 @@ __device__ __forceinline__ void for_each_neighbour(const vec4* __restrict__ src,
                     vec4 q[PIECES];
 #pragma unroll
                     for (int p = 0; p < PIECES; ++p) q[p] = src[STRIDE * (size_t)j + p];
-                    one(q);
+                    one(q, at++);
                 };
                 // the group's lanes test LPP slots at once
                 unsigned b = (unsigned)(__ballot(is) >> (lane - sub)) & ((1u << LPP) - 1u);
@@ -270,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void density_kernel(const float4* __restric
                                                          float* __restrict__ density, const BlockTables T,
                                                          const DevParams P0)
 {
-    using Rho = OrderedSums<LPP, 1, float, CSum>;
+    using Rho = ClassSums<LPP, 1, float, CSum>;
     __shared__ __attribute__((aligned(16))) float terms[kWaves][Rho::kLds];
     const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
@@ -290,10 +355,10 @@ __global__ __launch_bounds__(kBlock) void density_kernel(const float4* __restric
             term(q, v);
             rho.add(v, rem, lt, lane);
         },
-        [&](const vec4 (&q)[1]) GRASPH_INLINE {
+        [&](const vec4 (&q)[1], int at) GRASPH_INLINE {
             float v[1];
             term(q, v);
-            rho.add_one(v, lt, lane);
+            rho.add_one(v, at, lt, lane);
         });
     float r = rho.value(0, lane);
     if (!act || lane % LPP != 0) return;
@@ -319,7 +384,7 @@ __global__ __launch_bounds__(kBlock) void strain_kernel(
     constexpr int kRot = SOLIDS ? 9 : BALS ? 3 : 0;
     constexpr int NC = kRot + (!SOLIDS && (BALS || INTD) ? 1 : 0);
     constexpr int kTerms = NC > 0 ? NC : 1;
-    using Rates = OrderedSums<LPP, kTerms, double, double>;
+    using Rates = ClassSums<LPP, kTerms, double, double>;
     __shared__ __attribute__((aligned(16))) double terms[kWaves][Rates::kLds];
     const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
@@ -359,17 +424,17 @@ __global__ __launch_bounds__(kBlock) void strain_kernel(
         }
         if constexpr (NC == 0) v[0] = 0.0;
     };
-    for_each_neighbour<kDeepStrain, LPP, 2, 4>(
+    for_each_neighbour<LPP == 4 ? kDeepStrain : 1, LPP, 2, 4>(
         (const vec4*)rec, xs, Ls, t, act, kmax, pi, m, P.H2,
         [&](const vec4 (&q)[2], int rem) GRASPH_INLINE {
             double v[kTerms];
             term(q, v);
             R.add(v, rem, lt, lane);
         },
-        [&](const vec4 (&q)[2]) GRASPH_INLINE {
+        [&](const vec4 (&q)[2], int at) GRASPH_INLINE {
             double v[kTerms];
             term(q, v);
-            R.add_one(v, lt, lane);
+            R.add_one(v, at, lt, lane);
         });
     double exx = 0, eyy = 0, ezz = 0, exy = 0, exz = 0, eyz = 0;  // strain rate (symmetric)
     double rxy = 0, rxz = 0, ryz = 0;                              // rotation rate (antisymmetric)
@@ -464,8 +529,8 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
     const int kmax, float4* __restrict__ acc, float4* __restrict__ xvel, float* __restrict__ maxvsig,
     const int acc_has_gravity, const BlockTables T, const DevParams P0)
 {
-    using Acc = OrderedSums<LPP, 3, float, CSum>;
-    using Xv = OrderedSums<LPP, 3, float, float>;
+    using Acc = ClassSums<LPP, 3, float, CSum>;
+    using Xv = ClassSums<LPP, 3, float, float>;
     __shared__ __attribute__((aligned(16))) float terms[kWaves][(XSPH ? 2 : 1) * Acc::kLds];
     const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63, sub = lane % LPP;
@@ -486,7 +551,9 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
     Xv X{};
     if (acc_has_gravity) {
         const float4 g = acc[i];
-        A.a[0].s = sub == 0 ? g.x : sub == 1 ? g.y : g.z;
+        A.init(0, g.x, lane);
+        A.init(1, g.y, lane);
+        A.init(2, g.z, lane);
     }
     float mv = 0.0f;
 
@@ -554,11 +621,11 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
             A.add(f, rem, lt, lane);
             if constexpr (XSPH) X.add(x, rem, lt + Acc::kLds, lane);
         },
-        [&](const vec4 (&q)[4]) GRASPH_INLINE {
+        [&](const vec4 (&q)[4], int at) GRASPH_INLINE {
             float f[3], x[3];
             term(q, f, x, true);
-            A.add_one(f, lt, lane);
-            if constexpr (XSPH) X.add_one(x, lt + Acc::kLds, lane);
+            A.add_one(f, at, lt, lane);
+            if constexpr (XSPH) X.add_one(x, at, lt + Acc::kLds, lane);
         });
     float fx = A.value(0, lane), fy = A.value(1, lane), fz = A.value(2, lane);
     float xvx = 0.0f, xvy = 0.0f, xvz = 0.0f;
