@@ -52,42 +52,54 @@ ProfScope::~ProfScope()
 // four slots 8: what a compute unit runs at once; or half as many) and
 // `planes` workgroups to cover them, whose sums a second kernel adds.  Half
 // workgroups come in odd numbers only, so the shares alone tell the shape.
-// Both forms keep the same pace, so the one that takes fewer rounds of
-// workgroups over the compute units, times (a share's partners + a
-// wavefront's start), and the second kernel least, is taken (Plummer steps with one / four slots: 6144
-// particles 20.4 / 24.2 us, 9500 37.8 / 38.0, 11000 52.7 / 46.6; allocation-
-// free SPH at 40000 597 / 839; 1000 particles with one workgroup's shares 11.0,
-// with two 12.6, 1500 13.7 and 12.5).
-constexpr int64_t kOwnStart = 32, kOwnShare = 32;  // a start's cost and the least share, in partners
+// Or, with one plane, kOwnSplit lanes to a slot and a share to each.  All
+// forms keep the same pace, so the one that takes fewest rounds of workgroups
+// over the compute units, times (a share's partners + a wavefront's start),
+// the second kernel and the lanes' sums least, is taken (Plummer steps with one / four slots:
+// 6144 particles 20.4 / 24.2 us, 9500 37.8 / 38.0, 11000 52.7 / 46.6;
+// allocation-free SPH at 40000 597 / 839; 1500 particles with one plane 13.7,
+// with two 12.5, with four lanes a slot 9.6).
+constexpr int64_t kOwnStart = 32, kOwnShare = 16;  // a start's cost and the least share, in partners
 constexpr int kOwnSlicesMax = 64;
 
-static int64_t own_shape(const Ctx& c, int64_t n, int slices, int ni, OwnPlan& p)
+static int64_t own_shape(const Ctx& c, int64_t n, int slices, int ni, int split, OwnPlan& p)
 {
     const int full = ni == 4 ? 8 : 16, half = full / 2;  // LDS: the wavefronts' sums in 64 KiB
+    const int shares = slices / split;                   // of the wavefronts
     p.ni = ni;
-    p.waves = slices > half && slices % full && slices % half == 0 ? half : std::min(slices, full);
-    p.planes = (slices + p.waves - 1) / p.waves;
+    p.split = split;
+    p.waves = shares > half && shares % full && shares % half == 0 ? half : std::min(shares, full);
+    p.planes = (shares + p.waves - 1) / p.waves;
     p.len = (int)(((n + p.slices() - 1) / p.slices() + 7) / 8 * 8);
-    const int64_t groups = (n + 64 * ni - 1) / (64 * ni) * p.planes, room = (int64_t)c.cus * (full / p.waves);
+    const int64_t slots = 64 / split * ni, groups = (n + slots - 1) / slots * p.planes;
+    const int64_t room = (int64_t)c.cus * (full / p.waves);
     return (ni == 4 ? 2 : 1) * ((groups + room - 1) / room) * (p.len + kOwnStart) +
-           (p.planes > 1 ? 36 + 4 * p.planes : 0);
+           (p.planes > 1 ? 36 + 4 * p.planes : 0) + (split > 1 ? 8 : 0);
 }
 
-// slices 0: the number of shares (of 32 partners or more) that costs least.
-// As many as give 8 (16) wavefronts per compute unit, whatever that leaves
-// of a last round, took 28.8 us at 5500 particles (now 20.3), 76.6 at 11000.
+// slices 0: the number of shares (of kOwnShare partners or more) that costs
+// least.  As many as give 8 (16) wavefronts per compute unit, whatever that
+// leaves of a last round, took 28.8 us at 5500 particles (now 20.3), 76.6 at
+// 11000.
 OwnPlan own_plan(const Ctx& c, int64_t n, int slices, int max_planes)
 {
-    const auto shape = [&](int s, OwnPlan& p) {
-        if (c.sweep_ni == 2) return own_shape(c, n, s, 2, p);
-        OwnPlan one;
-        const int64_t cost = own_shape(c, n, s, 4, p), cost1 = own_shape(c, n, s, 1, one);
-        if (cost1 < cost) p = one;
-        return std::min(cost, cost1);
+    const auto shape = [&](int s, OwnPlan& best) {
+        if (c.sweep_ni == 2) return own_shape(c, n, s, 2, 1, best);
+        int64_t least = own_shape(c, n, s, 4, 1, best);
+        const auto consider = [&](int split) {
+            OwnPlan p;
+            const int64_t cost = own_shape(c, n, s, 1, split, p);
+            if (cost >= least) return;
+            least = cost;
+            best = p;
+        };
+        consider(1);
+        if (s % kOwnSplit == 0) consider(kOwnSplit);  // 64 shares at most: one plane
+        return least;
     };
     OwnPlan best, p;
-    if (slices > 0 || n < 16 * kOwnShare) {
-        shape(slices > 0 ? slices : (int)std::max<int64_t>(1, n / kOwnShare), best);
+    if (slices > 0 || n < 8 * kOwnShare) {
+        shape(slices > 0 ? slices : (int)std::max<int64_t>(1, n / (2 * kOwnShare)), best);
         return best;
     }
     int64_t least = shape(4, best);
@@ -528,6 +540,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     L.waves = plan.waves;
     L.planes = plan.planes;
     L.slice_len = plan.len;
+    L.split = plan.split;
     L.part = c.part;
     if (masses) {
         // equal masses let the sweep factor the mass out of the gravity sum
@@ -667,7 +680,7 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
         carve_derivative_arrays(sh, m, n, lists, grav, plan.planes);
         need = m.used;
         if (need <= (size_t)GRASPH_NOALLOC_SCRATCH_BYTES || plan.planes == 1) break;
-        plan = c.sweep_slices > 0 ? own_plan(sh, n, plan.waves * (plan.planes - 1), kOwnSlicesMax)
+        plan = c.sweep_slices > 0 ? own_plan(sh, n, plan.slices() / plan.planes * (plan.planes - 1), kOwnSlicesMax)
                                   : own_plan(sh, n, 0, plan.planes - 1);
     }
     if (need > (size_t)GRASPH_NOALLOC_SCRATCH_BYTES)

@@ -170,8 +170,9 @@ struct SweepLaunch {
     float* maxvsig;
     // one-sided gravity: ni particles per lane (1, 2 or 4); `waves` wavefronts
     // of a workgroup and `planes` workgroups share their particles' partners,
-    // slice_len (a multiple of 8) each
-    int ni, waves, planes, slice_len;
+    // slice_len (a multiple of 8) each; split: lanes per particle (1, or with
+    // ni 1 and one plane kOwnSplit, which take a share each)
+    int ni, waves, planes, slice_len, split;
     float4* part;       // [planes][n][2] partial sums when planes > 1
     const float* umass; // {uniform, mass} from launch_mass_check, or null
 };
@@ -632,9 +633,10 @@ inline int check_particles(Ctx& c, const grasph_particles* p)
 // How the one-sided gravity sweep of n particles is cut: `slices` (0:
 // chosen from the count) shares of the partners, as many wavefronts of a
 // workgroup as take them, the rest in planes.
+constexpr int kOwnSplit = 4;
 struct OwnPlan {
-    int ni, waves, planes, len;
-    int slices() const { return waves * planes; }
+    int ni, waves, planes, len, split;
+    int slices() const { return waves * planes * split; }
 };
 // slices: the option sweep_slices, 0 for the automatic choice (of at most
 // max_planes planes)

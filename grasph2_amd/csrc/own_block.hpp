@@ -222,5 +222,75 @@ __device__ __forceinline__ void own_block(const float4* __restrict__ xs, const i
     }
 }
 
+// own_block for few particles: 64 / SPLIT slots, each in SPLIT lanes of a
+// wavefront, the q-th of which takes the share wave SPLIT + q of len partners.  With one slot per lane 1000 particles
+// were 16 workgroups of 16 wavefronts, 64 partners long each; four lanes a
+// slot make that 63 workgroups and 16 partners (Plummer step 11.0 -> 9.6 us,
+// of 4096, in one plane instead of four, 13.7 -> 11.2).
+// Every wavefront of the workgroup calls it; lds as for own_block<1>.
+template <int SPLIT, bool UM, bool SOFT, typename F>
+__device__ __forceinline__ void own_split_block(const float4* __restrict__ xs, const int o0, const int n,
+                                                const int len, const float h2, const float m, const int wave,
+                                                const int waves, float* lds, F&& store)
+{
+    constexpr int kSlots = 64 / SPLIT;  // of the workgroup, and partners of a share in a tile
+    const int lane = threadIdx.x & 63, slot = lane % kSlots, q = lane / kSlots;
+    float4* const tile = reinterpret_cast<float4*>(lds) + 64 * wave;
+    const int j0 = (wave * SPLIT + q) * len, j1 = min(n, j0 + len);
+    auto partner = [&](const int j) {  // past the end: far away and massless
+        float4 v = xs[min(j0 + j + slot, n - 1)];
+        if (j0 + j + slot >= j1) v = make_float4(3.0e18f, 3.0e18f, 3.0e18f, 0.0f);
+        return v;
+    };
+    float4 next = partner(0);
+    OwnAcc<1> a;
+    const float4 own = xs[min(o0 + slot, n - 1)];
+    a.x[0] = own.x; a.y[0] = own.y; a.z[0] = own.z;
+    a.ax[0] = a.ay[0] = a.az[0] = 0.0f;
+    CSum s[3] = {CSum{0.0f, 0.0f}, CSum{0.0f, 0.0f}, CSum{0.0f, 0.0f}};
+    for (int j = 0; j < len; j += kSlots) {
+        tile[lane] = next;
+        __builtin_amdgcn_wave_barrier();
+        next = partner(j + kSlots);
+#pragma unroll
+        for (int g = 0; g < kSlots; g += kOwnPairs) {
+            float4 p[kOwnPairs];
+#pragma unroll
+            for (int r = 0; r < kOwnPairs; ++r) p[r] = tile[lane - slot + g + r];
+            own_pairs<1, UM, SOFT>(p, a, h2);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if ((j + kSlots) % kFold == 0 || j + kSlots >= len) {
+            s[0].add(UM ? a.ax[0] * m : a.ax[0]);
+            s[1].add(UM ? a.ay[0] * m : a.ay[0]);
+            s[2].add(UM ? a.az[0] * m : a.az[0]);
+            a.ax[0] = a.ay[0] = a.az[0] = 0.0f;
+        }
+    }
+    float* const red = lds + 256 * waves;  // [wave][6][64]
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        red[(wave * 6 + c) * 64 + lane] = s[c].s;
+        red[(wave * 6 + 3 + c) * 64 + lane] = s[c].c;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    for (int w = 1; w < waves; ++w)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            s[c].add(red[(w * 6 + c) * 64 + lane]);
+            s[c].c += red[(w * 6 + 3 + c) * 64 + lane];
+        }
+#pragma unroll
+    for (int o = kSlots; o < 64; o <<= 1)  // lanes q = 0: (0 + 1) + (2 + 3)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float v = __shfl_xor(s[c].s, o, 64), e = __shfl_xor(s[c].c, o, 64);
+            s[c].add(v);
+            s[c].c += e;
+        }
+    if (q == 0 && o0 + slot < n) store(o0 + slot, s[0], s[1], s[2]);
+}
+
 }  // namespace
 }  // namespace grasph

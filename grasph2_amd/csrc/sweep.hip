@@ -32,7 +32,8 @@ constexpr int kMassBlocks = 256;  // blocks of the single-instance mass check (f
 // Workgroup (own block blockIdx.x, plane blockIdx.y): its wavefronts' shares
 // of slice_len partners start at plane * waves * slice_len.  One plane: the
 // accelerations; several: the plane's partial sums (2 float4 per particle).
-template <int NI, bool SOFT>
+// SPLIT > 1 (one plane): SPLIT lanes per slot (own_split_block).
+template <int NI, bool SOFT, int SPLIT>
 __global__ __launch_bounds__(64 * kOwnMaxWaves) void own_kernel(const float4* __restrict__ xs,
                                                                 const int* __restrict__ perm, const int n,
                                                                 float4* __restrict__ acc, const int finish,
@@ -43,7 +44,7 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void own_kernel(const float4* __
 {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
-    const int o0 = 64 * NI * blockIdx.x, j0 = (int)blockIdx.y * waves * slice_len;
+    const int o0 = 64 / SPLIT * NI * blockIdx.x, j0 = (int)blockIdx.y * waves * slice_len;
     float4* const pp = part ? part + 2 * (size_t)blockIdx.y * n : nullptr;
     auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
         const int i = perm ? perm[t] : t;
@@ -60,6 +61,13 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void own_kernel(const float4* __
         }
         acc[i] = make_float4(ax, ay, az, 0.0f);
     };
+    if constexpr (SPLIT > 1) {  // one plane
+        if (umass && umass[0] != 0.0f)
+            own_split_block<SPLIT, true, SOFT>(xs, o0, n, slice_len, P.H2, umass[1], wave, waves, lds, store);
+        else
+            own_split_block<SPLIT, false, SOFT>(xs, o0, n, slice_len, P.H2, 1.0f, wave, waves, lds, store);
+        return;
+    } else
     if (umass && umass[0] != 0.0f)  // {uniform, mass} of the particles
         own_block<NI, true, SOFT>(xs, o0, n, j0, n, slice_len, P.H2, umass[1], wave, waves, lds, store);
     else
@@ -288,12 +296,13 @@ __global__ void reset_queue_kernel(int* __restrict__ queue, const int n)
     if (i < n) queue[i] = 0;
 }
 
-template <int NI, bool SOFT>
+template <int NI, bool SOFT, int SPLIT = 1>
 hipError_t launch_own(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 {
-    const dim3 grid((unsigned)((L.n + 64 * NI - 1) / (64 * NI)), (unsigned)L.planes);
-    hipLaunchKernelGGL((own_kernel<NI, SOFT>), grid, dim3(64 * L.waves), sizeof(float) * own_lds_floats(NI, L.waves),
-                       s, L.xs ? L.xs : L.posm, L.perm, L.n, L.acc, L.finish ? 1 : 0, L.xvel, L.maxvsig, P,
+    constexpr int kSlots = 64 / SPLIT * NI;  // of a workgroup
+    const dim3 grid((unsigned)((L.n + kSlots - 1) / kSlots), (unsigned)L.planes);
+    const int lds = own_lds_floats(NI, SPLIT > 1 ? std::max(L.waves, 2) : L.waves);
+    hipLaunchKernelGGL((own_kernel<NI, SOFT, SPLIT>), grid, dim3(64 * L.waves), sizeof(float) * lds, s, L.xs ? L.xs : L.posm, L.perm, L.n, L.acc, L.finish ? 1 : 0, L.xvel, L.maxvsig, P,
                        L.slice_len, L.planes > 1 ? L.part : nullptr, L.umass);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || L.planes == 1) return e;
@@ -336,6 +345,8 @@ hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s)
     }
     if (L.waves < 1 || L.waves > kOwnMaxWaves || L.planes < 1 || L.slice_len < 8 || L.slice_len % 8)
         return hipErrorInvalidValue;
+    if (L.split != 1 && (L.split != kOwnSplit || L.ni != 1 || L.planes != 1)) return hipErrorInvalidValue;
+    if (L.split != 1) return soft ? launch_own<1, true, kOwnSplit>(L, P, s) : launch_own<1, false, kOwnSplit>(L, P, s);
     switch (L.ni) {
         case 1: return soft ? launch_own<1, true>(L, P, s) : launch_own<1, false>(L, P, s);
         case 2: return soft ? launch_own<2, true>(L, P, s) : launch_own<2, false>(L, P, s);

@@ -13,7 +13,7 @@ from tests._util import vec_errors
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 31, 511, 512, 1025, 1537, 5500, 9473, 11000, 14337])
+@pytest.mark.parametrize("n", [1, 31, 127, 128, 511, 512, 1025, 1537, 4096, 4097, 5500, 9473, 11000, 14337])
 def test_automatic_shares(n):
     print("one-sided shares n=%d" % n, flush=True)
     h, prm = ics.plummer(n, seed=n)
