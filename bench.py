@@ -11,20 +11,17 @@ FP64 position drift).  Prints one JSON line.
 value = pair interactions per second = N (N - 1) / (seconds per step): every
 step evaluates softened gravity on all ordered pairs i != j.  The timed
 pass launches the steps one by one, or, for gravity alone (whose step holds
-no Morton re-sort), replays them from a HIP graph of config.graph_steps
+no re-sort of the slots), replays them from a HIP graph of config.graph_steps
 steps captured on a stream of its own (the same kernels and arguments).
 roofline: the dominant kernel, FP32 vector ALU bound, at 20 algorithmic
 FLOPs per ordered gravity pair (FMA = 2, rsqrt = 1), divided by its mean
 duration from HIP events recorded around every launch on the stream it
 runs on, over a second pass of as many steps (the timed pass records no
-events: they lengthen a step by ~2%).  From 16384 particles (the symmetric
-sweep)
-that kernel is the far field (far_kernel): the ordered pairs of particles in
+events: they lengthen a step by ~2%).  From 10752 particles (the symmetric
+sweep) that kernel is the far field (far_kernel): the ordered pairs of particles in
 different groups of 1024 slots, N (N - 1) minus the in-group pairs, 99% of
-the pairs at N = 131072; the near field, the list merge and the SPH
-passes run beside it on a second stream.  Below, it
-is the one-sided sweep over all N (N - 1) pairs (its neighbour search rides
-on the same r^2 and adds no counted FLOPs).
+the pairs at N = 131072; every kernel of a step runs in order on one stream.
+Below, it is the one-sided sweep over all N (N - 1) pairs.
 cpu_baseline: the CPU oracle in FP32 (the same op structure as the
 reference's host path) on a bounded sample of target particles i against
 all j, all three passes; one OpenMP thread per CPU of the process's
@@ -45,9 +42,9 @@ PEAK_HBM_GBPS = 8000.0     # MI355X HBM3E (AMD published)
 # The library's default for the single-instance sweep (option "sweep_symmetric" = 2, include/grasph2.h):
 # from this many particles on, gravity between groups of 1024 is evaluated once per pair for both sides.
 # The roofline stays algorithmic either way: 20 FLOP per ordered pair.
-SYM_AUTO_MIN_LISTS = 16384    # with neighbour lists (SPH on)
-SYM_AUTO_MIN_GRAVITY = 16384  # gravity alone
-SYM_GROUP = 1024  # slots per group of the symmetric sweep; pairs inside a group are the near field's
+SYM_AUTO_MIN_LISTS = 10752    # with neighbour lists (SPH on)
+SYM_AUTO_MIN_GRAVITY = 10752  # gravity alone
+SYM_GROUP = 1024  # slots per group of the symmetric sweep; pairs inside a group are one-sided
 FLOP_GRAVITY_PAIR = 20
 # Per neighbour pair, the FLOPs of the passes' formulas (FMA 2; add, sub, mul 1; sqrt, rsqrt, div 1;
 # compensation 0), data-dependent branches at their typical share: W's inner branch (q < 1/2, 1/8 of
@@ -74,7 +71,7 @@ def parse():
     ap.add_argument("--n", type=int, default=0, help="override the particle count")
     ap.add_argument("--graph", type=int, default=-1, metavar="G",
                     help="steps per captured HIP graph in the timed pass (0: plain launches); default 10 for "
-                         "gravity alone, whose step holds no Morton re-sort, else 0 (the re-sort every "
+                         "gravity alone, whose step holds no re-sort, else 0 (the re-sort every "
                          "reorder_interval steps stays out of graphs)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="target CPU time of the baseline sample")
@@ -229,7 +226,7 @@ def main():
     value = pairs / (ms_step * 1e-3)
 
     sym = kt["far"][1] > 0  # the symmetric sweep ran (its far field was timed)
-    # all kernels of the all-pairs sweep, summed per evaluation (with the symmetric sweep, intervals that overlap)
+    # all kernels of the all-pairs sweep, summed per evaluation (with the symmetric sweep: far field, in-group gravity, combine)
     sweep_ms = (kt["sweep"][0] + kt["far"][0]) / args.steps
     sweep_flops = FLOP_GRAVITY_PAIR * pairs
     if sym:

@@ -2,7 +2,7 @@
 //
 // A batch packs many instances back to back (see grasph_batch in
 // grasph2.h).  Per step:
-//   order   per-instance Morton order (eager, every reorder_interval steps)
+//   order   per-instance Hilbert order (eager, every reorder_interval steps)
 //   lists   the neighbour lists of every instance (lists.hip)
 //   sweep   gravity: the symmetric sweep (sym_sweep.hip), or one persistent
 //           launch whose wavefronts pull (instance, tile) items from an atomic
@@ -50,7 +50,7 @@ struct BatchState {
     int* d_queue = nullptr;
     float* d_ts = nullptr;  // variable step: {current dt, next dt} per instance, zero when the tables are built
     float* d_um = nullptr;  // {uniform, mass} per instance, written before each gravity sweep
-    // slot-ordered positions for the sweep (SPH with a Morton order)
+    // slot-ordered positions for the sweep (SPH with a slot order)
     float4* d_xs = nullptr;
     // symmetric sweep (option batch_symmetric): tables and work arrays
     SymInst* d_sinst = nullptr;
@@ -64,7 +64,7 @@ struct BatchState {
     float4* d_sapart = nullptr;
     float* d_sbpart = nullptr;
 
-    // Morton order
+    // Hilbert order
     float* d_bbox = nullptr;
     uint64_t* d_keys = nullptr;
     uint64_t* d_keys_alt = nullptr;
@@ -324,7 +324,7 @@ int ensure_order(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
         O.key_bits = b.key_bits;
         ProfScope ps(&c, s, KC_REORDER);
         hipError_t e = launch_batch_order(O, s);
-        if (e != hipSuccess) return hip_fail(c, e, "batch Morton order");
+        if (e != hipSuccess) return hip_fail(c, e, "batch slot order");
         b.order_valid = true;
         b.order_src = p->posm;
         b.evals_since_order = 0;
@@ -355,7 +355,7 @@ int device_cus(Ctx& c)
     return cus;
 }
 
-// The slot order of the sweep and the passes: the Morton order for SPH (the
+// The slot order of the sweep and the passes: the Hilbert order for SPH (the
 // neighbour work wants it), none for gravity alone.
 const int* slot_order(const Ctx& c, const BatchState& b)
 {
@@ -692,8 +692,8 @@ int time_sweep(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, 
 }
 
 // time one whole derivative evaluation of the batch (eager, min of reps
-// after a warm-up), milliseconds: the sweeps, the neighbour passes beside
-// the far field and the combine, as a step runs them
+// after a warm-up), milliseconds: the sweeps, the neighbour passes
+// and the combine, as a step runs them
 int time_derivs(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, int reps, double* ms)
 {
     hipEvent_t e0, e1;

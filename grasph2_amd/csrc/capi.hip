@@ -150,7 +150,7 @@ int ensure_order(Ctx& c, const grasph_particles* p, hipStream_t s, bool count_ev
     const int64_t n = p->n;
     if (c.reorder_interval <= 0) return 0;
     if (c.reorder_cap < n || !c.perm) {
-        if (c.no_alloc) return fail(c, GRASPH_E_NOMEM, "the Morton order would need a device allocation");
+        if (c.no_alloc) return fail(c, GRASPH_E_NOMEM, "the slot order would need a device allocation");
         void* bufs[] = {c.perm, c.keys, c.keys_alt, c.vals};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
@@ -162,7 +162,7 @@ int ensure_order(Ctx& c, const grasph_particles* p, hipStream_t s, bool count_ev
             hipMalloc((void**)&c.keys_alt, n * sizeof(uint32_t)) != hipSuccess ||
             hipMalloc((void**)&c.vals, n * sizeof(int)) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(c, GRASPH_E_NOMEM, "device allocation of the Morton order failed");
+            return fail(c, GRASPH_E_NOMEM, "device allocation of the slot order failed");
         }
         c.reorder_cap = n;
     }
@@ -188,7 +188,7 @@ int ensure_order(Ctx& c, const grasph_particles* p, hipStream_t s, bool count_ev
         }
         ProfScope ps(&c, s, KC_REORDER);
         hipError_t e = launch_reorder((const float4*)p->posm, (int)n, c, s);
-        if (e != hipSuccess) return hip_fail(c, e, "Morton reorder");
+        if (e != hipSuccess) return hip_fail(c, e, "slot order");
         c.perm_n = n;
         c.perm_src = p->posm;
         c.evals_since_reorder = 0;
@@ -658,7 +658,7 @@ int derivatives_noalloc(Ctx& c, const grasph_particles* p, const grasph_params* 
 
     // a stand-in context: this context's options and state ({current, next}
     // dt, the mass record), the one-sided sweep on one stream, a fresh
-    // Morton order, buffers from the scratch array, no allocation allowed
+    // slot order, buffers from the scratch array, no allocation allowed
     Ctx sh;
     sh.device = c.device;
     sh.cus = c.cus;

@@ -32,7 +32,7 @@ enum KernelClass {
     KC_INTEGRATE = 4,
     KC_REORDER = 5,
     KC_OTHER = 6,
-    KC_FAR = 7  // far field of the symmetric sweep (the rest of the evaluation runs beside it)
+    KC_FAR = 7  // far field of the symmetric sweep
 };
 
 // Per-device library state.  Scratch grows on demand and is reused.
@@ -52,12 +52,12 @@ struct Ctx {
     int reorder_interval = 8;  // particles move little in 8 steps: the order only affects speed
     int sweep_ni = 1;  // i particles per lane in the single-instance sweep
     int sweep_slices = 0;  // j-split of the single-instance sweep (0: chosen from the occupancy)
-    int sweep_symmetric = 2;  // single instance, far pairs once for both sides (sym_sweep.hip): 0 off, 1 on, 2 from 16384 particles
+    int sweep_symmetric = 2;  // single instance, far pairs once for both sides (sym_sweep.hip): 0 off, 1 on, 2 from kSymAutoMin particles
     int sym_workgroups = 0;   // workgroups of its far kernel (0: 2 wavefronts per SIMD)
-    int sym_near_shares = 0;  // wavefronts per block of its near field (0: chosen from the occupancy)
+    int sym_near_shares = 0;  // wavefronts per 64 slots of its in-group gravity (0: chosen from the count)
     // bytes of partner-side partials one column batch of its far field may take (6 n^2 / 1024 in all)
     int64_t sym_partial_bytes = int64_t(12) << 30;
-    int sym_list_priority = 2;  // its near-field lists ahead of the far field: 0 no, 1 yes, 2 below 49152 particles or past 512 list entries
+    int sym_list_priority = 2;  // kept for callers that set it; without effect
     int batch_symmetric = 1;  // batches: the symmetric sweep for instances of batch_symmetric_min particles or more
     int batch_symmetric_min = 0;
     int cus = 256;         // compute units of the device
@@ -75,7 +75,7 @@ struct Ctx {
     int* mass_flags = nullptr;  // per-256-slot flags of the check when the gather makes them
     int64_t mass_flags_cap = 0;
 
-    // Morton order of the i side (slot t -> particle perm[t])
+    // Hilbert order of the i side (slot t -> particle perm[t])
     int* perm = nullptr;
     int64_t perm_n = 0;
     const void* perm_src = nullptr;  // posm pointer the order was computed for
@@ -440,8 +440,8 @@ hipError_t launch_mass_check(const float4* posm, const BatchInst* insts, int n_i
                              hipStream_t s);
 hipError_t launch_reset_queue(int* queue, int n, hipStream_t s);
 
-// Batched Morton order: per-instance bounding boxes, keys (instance, Z-order
-// cell), one radix sort; perm maps each instance's slots into its own range.
+// Batched Hilbert order: per-instance bounding boxes, keys (instance, cell
+// along the curve), one radix sort; perm maps each instance's slots into its own range.
 struct BatchOrder {
     const float4* posm;
     const int* inst_of;      // instance of every particle
@@ -540,8 +540,8 @@ struct InvLaunch {
 int inv_blocks(int n);
 hipError_t launch_invariants(const InvLaunch& L, const grasph_params& prm, hipStream_t s);
 
-// Morton reorder: perm[t] = particle index of the t-th particle along a
-// Z-order curve over the bounding box of posm.
+// Slot order: perm[t] = particle index of the t-th particle along a
+// Hilbert curve over the bounding box of posm.
 size_t reorder_tmp_bytes(int n);
 hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s);
 // Slot-ordered copies for the sweep and the list passes (perm null: the

@@ -2,7 +2,7 @@
 // :72,122,238) that the passes of nbr_passes.hip walk (gfx950).
 //
 // Boxes: every 8 consecutive slots of an instance have a bounding box, and
-// every 512 slots one.  In slot (Morton) order these are small, and a box
+// every 512 slots one.  In slot (Hilbert) order these are small, and a box
 // farther than H from a particle holds none of its neighbours: the box gaps
 // and their squared sum round like the exact pair distance (rounding is
 // monotonic), so they never exceed it.

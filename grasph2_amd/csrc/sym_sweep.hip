@@ -231,9 +231,10 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
 // over the whole group: one wavefront owns it) goes straight to row g's
 // partials of its group (element 3 (bpart_group_base(J) - boff) on holds
 // group J's; boff: the groups before the column batch).  UM: the row's slots
-// have mass mo and the partners mass mp, which the sums take as a factor.  The store has no condition: partners of the last chunk past n
-// (their group's partials are allocated whole) get values nobody reads, and
-// a store behind a branch makes the compiler spill the chunk's registers.
+// have mass mo and the partners mass mp, which the sums take as a factor.  The
+// store has no condition: partners of the last chunk past n (their group's
+// partials are allocated whole) get values nobody reads, and a store behind a
+// branch makes the compiler spill the chunk's registers.
 // The own side is folded every `fold` partners and at the end, so a slot
 // adds at most that many terms in plain FP32 before they join its LDS sum
 // (and at most kFoldsPerFlush such sums before they join the compensated
@@ -391,59 +392,59 @@ __device__ __forceinline__ void far_sums(const float4* __restrict__ apart, const
                                          const int t, const int p, const int64_t nsb, const int64_t U, const int W,
                                          const int Q, CSum& x, CSum& y, CSum& z)
 {
-            const int64_t g = t / kGroup, local = t - g * kGroup;
-            if (U > 0 && g < rows_with_units(nsb)) {
-                // one fragment per wavefront that touched the row (every wavefront
-                // has a share: W <= U), or per workgroup of them; eight fragments'
-                // loads in flight before their ordered adds
-                const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
-                const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
-                const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
-                int64_t k = p;
-                for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
-                    float4 f[8], fc[8];
-    #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const float4* fr = fragment(k + u * PARTS);
-                        f[u] = fr[0];
-                        if (!PLAIN) fc[u] = fr[64];
-                    }
-    #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
-                        if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
-                    }
-                }
-                for (; k < R.count; k += PARTS) {
-                    const float4* fr = fragment(k);
-                    const float4 f = fr[0];
-                    x.add(f.x); y.add(f.y); z.add(f.z);
-                    if (!PLAIN) {
-                        const float4 fc = fr[64];
-                        x.c += fc.x; y.c += fc.y; z.c += fc.z;
-                    }
-                }
+    const int64_t g = t / kGroup, local = t - g * kGroup;
+    if (U > 0 && g < rows_with_units(nsb)) {
+        // one fragment per wavefront that touched the row (every wavefront
+        // has a share: W <= U), or per workgroup of them; eight fragments'
+        // loads in flight before their ordered adds
+        const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
+        const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
+        const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
+        int64_t k = p;
+        for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
+            float4 f[8], fc[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float4* fr = fragment(k + u * PARTS);
+                f[u] = fr[0];
+                if (!PLAIN) fc[u] = fr[64];
             }
-            const int64_t base = bpart_group_base(g) + local;
-            const int ng = (int)g;
-            // eight groups' loads in flight before their (ordered) adds
-            int gp = p;
-            for (; gp + 7 * PARTS < ng; gp += 8 * PARTS) {
-                float v[8][3];
-    #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const size_t e = 3 * (size_t)(base + (int64_t)(gp + u * PARTS) * kGroup);
-                    v[u][0] = bpart[e]; v[u][1] = bpart[e + 1]; v[u][2] = bpart[e + 2];
-                }
-    #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
-                }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
+                if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
             }
-            for (; gp < ng; gp += PARTS) {
-                const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
-                x.add(-bpart[e]); y.add(-bpart[e + 1]); z.add(-bpart[e + 2]);
+        }
+        for (; k < R.count; k += PARTS) {
+            const float4* fr = fragment(k);
+            const float4 f = fr[0];
+            x.add(f.x); y.add(f.y); z.add(f.z);
+            if (!PLAIN) {
+                const float4 fc = fr[64];
+                x.c += fc.x; y.c += fc.y; z.c += fc.z;
             }
+        }
+    }
+    const int64_t base = bpart_group_base(g) + local;
+    const int ng = (int)g;
+    // eight groups' loads in flight before their (ordered) adds
+    int gp = p;
+    for (; gp + 7 * PARTS < ng; gp += 8 * PARTS) {
+        float v[8][3];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const size_t e = 3 * (size_t)(base + (int64_t)(gp + u * PARTS) * kGroup);
+            v[u][0] = bpart[e]; v[u][1] = bpart[e + 1]; v[u][2] = bpart[e + 2];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
+        }
+    }
+    for (; gp < ng; gp += PARTS) {
+        const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
+        x.add(-bpart[e]); y.add(-bpart[e + 1]); z.add(-bpart[e + 2]);
+    }
 }
 
 // The parts' sums added in part order, in part 0's threads (thread q kSlots +

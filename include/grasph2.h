@@ -139,23 +139,21 @@ int grasph_version(void);
  * when ctx is NULL).  Never NULL. */
 const char* grasph_last_error(const grasph_ctx* ctx);
 
-/* Per-device context: owns scratch (neighbour lists, Morton order, partial
+/* Per-device context: owns scratch (neighbour lists, slot order, partial
  * sums, timing events).  Not thread-safe; use one context per host thread. */
 int grasph_create(int device, grasph_ctx** out);
 int grasph_destroy(grasph_ctx* ctx);
 
 /* Tuning knobs.  Keys: "max_neighbours" (list capacity per particle,
  * default 160; a particle with more neighbours takes an exact scan of all
- * partners, with the same results; above 512, four lanes share each
- * particle's neighbours in the single-instance passes, which splits their
- * sums four ways: equal to FP32 rounding), "max_neighbours_grow" (1 = after an
+ * partners, with the same results bit for bit), "max_neighbours_grow" (1 = after a
  * single-instance evaluation whose lists overflowed, a later one raises
  * max_neighbours to 1.25 times the largest count seen, in steps of 32, up
  * to 4096 and 16 GiB of lists; the count is stored in host memory by the
  * list kernel and read without waiting, and not during graph capture; the
  * default; 0 = fixed; batches keep the capacity last set),
  * "reorder_interval"
- * (Morton re-sort every k derivative evaluations, default 8; 0 = never;
+ * (slots re-sorted along a Hilbert curve every k derivative evaluations, default 8; 0 = never;
  * the order changes only the order of compensated sums, not which pairs
  * are found; a new particle count or position array re-sorts at once,
  * and an array allocated at a freed one's address counts as the same
@@ -200,8 +198,8 @@ int grasph_get_option(const grasph_ctx* ctx, const char* key, int64_t* value);
 /* computeDerivatives(pb)                       src/computeDerivatives.h:315-328
  * Runs the passes the flags select, in the reference's order:
  * density summation (:320), strain rate / Balsara / density rate (:323),
- * acceleration (:327).  Fused here into one all-pairs sweep (gravity,
- * density, neighbour list) plus two neighbour-list passes.
+ * acceleration (:327).  Here an all-pairs gravity sweep, the neighbour
+ * lists, and one pass over the lists for each.
  * With GRASPH_VARIABLE_TIMESTEP the acceleration pass (here and in
  * grasph_calc_acceleration) sets the context's next dt to max_timestep, as
  * calcAcceleration::do_after sets nextTS (:305-308). */
@@ -213,12 +211,12 @@ int grasph_compute_derivatives(grasph_ctx* ctx, const grasph_particles* p,
  * forbid hipMalloc).  The same passes and results as
  * grasph_compute_derivatives with options sweep_symmetric = 0 and
  * reorder_interval = 1 (and sweep_slices as chosen below), computed
- * without any device allocation: every work array (Morton order and sort
+ * without any device allocation: every work array (slot order and sort
  * storage, slot-ordered positions and records, neighbour lists, the
  * j-split's partial sums) is cut from one static device array of
  * GRASPH_NOALLOC_SCRATCH_BYTES per GPU, held from library load until the
  * process ends.  Runs on `stream` alone (no second stream), re-sorts the
- * Morton order on every call and records no timing events.  The j-split
+ * slot order on every call and records no timing events.  The j-split
  * ("sweep_slices", automatic when 0) is reduced until the arrays fit; when
  * even one slice does not fit, returns GRASPH_E_INVALID and says how many
  * bytes the call needs.  With SPH and the default 160 neighbours per list a
