@@ -77,9 +77,9 @@ struct BatchState {
     const void* order_src = nullptr;
     int64_t evals_since_order = 0;
 
-    // neighbour lists (and their boxes: fine ones, then coarse ones) and pass records
+    // neighbour lists (and their boxes: fine, then coarse, then mid ones) and pass records
     float4* d_box = nullptr;
-    int64_t n_fine = 0;
+    int64_t n_fine = 0, n_coarse = 0;
     int* d_nbr = nullptr;
     int* d_cnt = nullptr;
     int64_t nbr_cap = 0;  // slots * kmax allocated
@@ -254,11 +254,12 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
             hipMalloc((void**)&b.d_vals, nt * sizeof(int)) != hipSuccess ||
             hipMalloc((void**)&b.d_perm, nt * sizeof(int)) != hipSuccess ||
             hipMalloc((void**)&b.d_xs, nt * sizeof(float4)) != hipSuccess ||
-            hipMalloc((void**)&b.d_box, 2 * (size_t)std::max(1, fine0 + coarse0) * sizeof(float4)) != hipSuccess) {
+            hipMalloc((void**)&b.d_box, 2 * (size_t)std::max(1, fine0 + (1 + kBoxCoarse / kBoxMid) * coarse0) * sizeof(float4)) != hipSuccess) {
             (void)hipGetLastError();
             return fail(c, GRASPH_E_NOMEM, "device allocation of the batch order failed");
         }
         b.n_fine = fine0;
+        b.n_coarse = coarse0;
         b.sort_bytes = batch_order_tmp_bytes((int)p->n, b.key_bits);
         if (hipMalloc(&b.d_sort_tmp, std::max<size_t>(b.sort_bytes, 1)) != hipSuccess) {
             (void)hipGetLastError();
@@ -392,6 +393,7 @@ int batch_lists(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s)
     L.n = (int)b.ntotal;
     L.fine = b.d_box;
     L.coarse = b.d_box + 2 * b.n_fine;
+    L.mid = b.d_box + 2 * (b.n_fine + b.n_coarse);
     L.nbr = b.d_nbr;
     L.nbr_cnt = b.d_cnt;
     L.kmax = b.kmax;

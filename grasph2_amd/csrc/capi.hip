@@ -499,13 +499,14 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         mass_flags = masses;
         if ((perm && (r = grow(c, c.xs, c.xs_cap, n, "slot-ordered positions"))) ||
             (r = grow(c, c.rec, c.rec_cap, n, "slot records")) ||
-            (r = grow(c, c.box, c.box_cap, 2 * (fine_boxes(n) + coarse_boxes(n)), "neighbour-search boxes")) ||
+            (r = grow(c, c.box, c.box_cap, 2 * all_boxes(n), "neighbour-search boxes")) ||
             (mass_flags && (r = grow(c, c.mass_flags, c.mass_flags_cap, gather_blocks, "mass-check flags"))))
             return r;
         ProfScope ps(&c, s, KC_REORDER);
         hipError_t e = launch_gather(perm, (int)n, (const float4*)p->posm, reads_vel ? (const float4*)p->vel : nullptr,
                                      gdens ? p->density : nullptr, perm ? c.xs : nullptr, c.rec, s,
-                                     mass_flags ? c.mass_flags : nullptr, c.box, c.box + 2 * fine_boxes(n),
+                                     mass_flags ? c.mass_flags : nullptr, c.box, c.box + 2 * (fine_boxes(n) + coarse_boxes(n)),
+                                     c.box + 2 * fine_boxes(n),
                                      c.list_max_dev);
         if (e != hipSuccess) return hip_fail(c, e, "slot-order gather launch");
         if (perm) xs = c.xs;
@@ -519,6 +520,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         N.H2 = P.H2;
         N.fine = c.box;
         N.coarse = c.box + 2 * fine_boxes(n);
+        N.mid = c.box + 2 * (fine_boxes(n) + coarse_boxes(n));
         N.nbr = c.nbr;
         N.nbr_cnt = c.nbr_cnt;
         N.kmax = c.max_neighbours;
@@ -619,9 +621,9 @@ void carve_derivative_arrays(Ctx& sh, Carve& k, int64_t n, bool lists, bool grav
         sh.sort_tmp_bytes = reorder_tmp_bytes((int)n);
         sh.sort_tmp = k.take<unsigned char>((int64_t)std::max<size_t>(sh.sort_tmp_bytes, 1));
         sh.bbox = k.take<float>(257 * 6);
-        // the boxes go where the sort's keys were: 32 B per 8 and per 512 slots
+        // the boxes go where the sort's keys were: 32 B per 8, 64 and 512 slots
         // in 8 B per slot (below 64 slots: in room of their own)
-        sh.box_cap = 2 * (fine_boxes(n) + coarse_boxes(n));
+        sh.box_cap = 2 * all_boxes(n);
         sh.box = n < 64 ? k.take<float4>(sh.box_cap) : reinterpret_cast<float4*>(sh.keys);
         sh.xs = k.take<float4>(n);
         sh.xs_cap = n;

@@ -93,7 +93,7 @@ struct Ctx {
     int* nbr_cnt = nullptr;
     int64_t nbr_cap_n = 0;
     int nbr_cap_k = 0;
-    float4* box = nullptr;  // the lists' boxes: fine, then coarse
+    float4* box = nullptr;  // the lists' boxes: fine, then coarse, then mid
     int64_t box_cap = 0;
     int64_t last_list_n = 0;  // particles of the last neighbour list built
     float4* part = nullptr;   // partial sums of a j-split sweep
@@ -281,12 +281,15 @@ hipError_t launch_sym_batch_far(const SymBatchLaunch& L, hipStream_t s);
 hipError_t launch_sym_batch_combine(const SymBatchLaunch& L, hipStream_t s);
 inline bool sym_batch_has_far(const SymBatchLaunch& L) { return L.ntotal > 0 && L.n_blk > 0 && L.grav && L.nrows > 0; }
 
-// Neighbour lists (lists.hip): bounding boxes of every kBoxFine and every
+// Neighbour lists (lists.hip): bounding boxes of every kBoxFine, kBoxMid and
 // kBoxCoarse consecutive slots of an instance, two float4 (lo, hi) each, then
-// one list per slot.
-constexpr int kBoxFine = 8, kBoxCoarse = 512;
+// one list per slot.  A box array holds all fine ones, all coarse ones, then
+// the mid ones (a batch's: kBoxCoarse / kBoxMid per coarse box).
+constexpr int kBoxFine = 8, kBoxMid = 64, kBoxCoarse = 512;
 inline int64_t fine_boxes(int64_t n) { return (n + kBoxFine - 1) / kBoxFine; }
+inline int64_t mid_boxes(int64_t n) { return (n + kBoxMid - 1) / kBoxMid; }
 inline int64_t coarse_boxes(int64_t n) { return (n + kBoxCoarse - 1) / kBoxCoarse; }
+inline int64_t all_boxes(int64_t n) { return fine_boxes(n) + coarse_boxes(n) + mid_boxes(n); }
 struct BatchInst;
 struct ListLaunch {
     const float4* xs;  // slot-ordered positions
@@ -294,6 +297,7 @@ struct ListLaunch {
     float H2;          // one instance
     float4* fine;      // boxes: one instance's come from the gather, a batch's are made here
     float4* coarse;
+    float4* mid;
     int* nbr;
     int* nbr_cnt;
     int kmax;
@@ -381,9 +385,9 @@ __device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_bl
 
 // The boxes of the kBoxCoarse slots first + threadIdx.x of an instance of n
 // (a workgroup of as many threads; p: this thread's slot, act: below n) into
-// the instance's fine and coarse arrays.
+// the instance's fine, mid and coarse arrays.
 __device__ inline void block_boxes(const float4 p, const bool act, const int first, const int n,
-                                   float4* __restrict__ fine, float4* __restrict__ coarse)
+                                   float4* __restrict__ fine, float4* __restrict__ mid, float4* __restrict__ coarse)
 {
     constexpr int kWaves = kBoxCoarse / 64;
     __shared__ float red[6][kWaves];
@@ -403,9 +407,15 @@ __device__ inline void block_boxes(const float4 p, const bool act, const int fir
             fine[2 * f + 1] = make_float4(v[3], v[4], v[5], 0.0f);
         }
     }
-    if (lane == 0)
+    if (lane == 0) {
+        if (act) {
+            const int f = (first + (int)threadIdx.x) / kBoxMid;
+            mid[2 * f] = make_float4(v[0], v[1], v[2], 0.0f);
+            mid[2 * f + 1] = make_float4(v[3], v[4], v[5], 0.0f);
+        }
 #pragma unroll
         for (int c = 0; c < 6; ++c) red[c][wave] = v[c];
+    }
     __syncthreads();  // every thread of the workgroup gets here
     if (threadIdx.x == 0 && first < n) {
 #pragma unroll
@@ -548,12 +558,13 @@ hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s);
 // identity): xs[t] = posm[perm[t]] when xs is given, and the slot records'
 // position/mass and velocity/density (vel or density null: zeros there).
 // With mass_flags (one int per kGatherBlock slots) also the per-block half of
-// the equal-mass check, which launch_mass_final completes; with fine and
+// the equal-mass check, which launch_mass_final completes; with fine, mid and
 // coarse the lists' boxes (one instance), and list_max cleared.
 constexpr int kGatherBlock = kBoxCoarse;
 hipError_t launch_gather(const int* perm, int n, const float4* posm, const float4* vel, const float* density,
                          float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags = nullptr,
-                         float4* fine = nullptr, float4* coarse = nullptr, int* list_max = nullptr);
+                         float4* fine = nullptr, float4* mid = nullptr, float4* coarse = nullptr,
+                         int* list_max = nullptr);
 hipError_t launch_mass_final(const float4* posm, const int* mass_flags, int nflags, float* umass, hipStream_t s);
 
 // environmentAcceleration and the zero XVEL / MAXVSIG stores of

@@ -1,28 +1,35 @@
 // lists.hip -- the neighbour lists (0 < r^2 <= H^2, src/computeDerivatives.h
 // :72,122,238) that the passes of nbr_passes.hip walk (gfx950).
 //
-// Boxes: every 8 consecutive slots of an instance have a bounding box, and
-// every 512 slots one.  In slot (Hilbert) order these are small, and a box
+// Boxes: every 8, every 64 and every 512 consecutive slots of an instance have
+// a bounding box.  In slot (Hilbert) order these are small, and a box
 // farther than H from a particle holds none of its neighbours: the box gaps
 // and their squared sum round like the exact pair distance (rounding is
 // monotonic), so they never exceed it.
 //
 // One wavefront makes the lists of 8 slots.  Lane l tests box l of 64 boxes
-// of 512 against the 8 slots' own box, then lane l box l of the 64 boxes of 8
-// in each that is near, then the particles of the near ones, 64 at a time:
-// those within H of the own box are collected in LDS, in slot order.  Lane
+// of 512 against the 8 slots' own box; the 64 lanes then test the boxes of 64
+// in 8 near ones at a time (instances of up to 8192 particles begin here),
+// then the boxes of 8 in 8 near ones of these, then the particles of the near
+// ones, 64 at a time: those within H of the own box are collected in LDS, in slot order.  Lane
 // l = 8 i + j takes slot i against every eighth of them from the j-th on; the
 // 64 lanes' hits in one ballot give slot i its partners as a byte in slot
 // order, so a partner's place in the list is the count so far plus the bits
 // below it: the lists come out in increasing slot order, complete and one to a
 // slot, whatever the launch shape.
 //
-// What bounds it: instructions, 1150 vector ones per wavefront, and the
-// stores (each 4 bytes of a line of its own).  8 slots meet ~70 boxes within
+// What bounds it: instructions, about 1000 vector ones per wavefront, and the
+// chain of dependent loads from level to level.  8 slots meet ~70 boxes within
 // H = 2.5 spacings, 560 particles, for ~65 neighbours each, of which ~250 come
 // within H of their box: testing the slots against those instead of all 560
 // took N = 200003 from 126 to 92 us, 65536 squeezed ones (430 partners each)
-// from 190 to 137, 512 instances from 1.63 to 1.15 ms.
+// from 190 to 137, 512 instances from 1.63 to 1.15 ms.  The boxes of 64 save
+// most of the tests of boxes of 8 (12 to 16 boxes of 512 are near, with 64 of
+// 8 each), and with lists short enough for 8 wavefronts per SIMD took SPH
+// steps without gravity at 200003 particles from 283 to 275 us, default solids
+// at 16384 from 103 to 99, three single passes at 20011 from 221 to 212.  The
+// stores (4 bytes, each to a line of its own) do not bound it: collected in
+// LDS and written side by side, the same steps took 277 to 286, 103 and 226.
 #include "internal.hpp"
 
 namespace grasph {
@@ -31,9 +38,13 @@ namespace {
 constexpr int kBoxThreads = kBoxCoarse;  // slots of a coarse box: one workgroup
 constexpr int kTile = 32;                // slots per workgroup of the list kernel
 constexpr int kListThreads = 8 * kTile;
-constexpr int kBoxList = 384;            // near fine boxes a wavefront collects before it tests them
+constexpr int kBoxList = 256;            // near fine boxes a wavefront collects before it tests them
+constexpr int kMidList = 128;            // near mid boxes it collects before it tests their fine ones
+// instances of so many mid boxes test them without the coarse ones (allocation-free steps of 8192 particles 81.4 us
+// with the coarse ones, 81.1 without; a two-round test costs what the coarse round and its chain do)
+constexpr int kMidDirect = 128;
 constexpr int kAhead = 2;                // loads of 8 boxes' partners in flight
-constexpr int kPartners = 256;           // close partners a wavefront collects before it tests them
+constexpr int kPartners = 192;           // close partners a wavefront collects before it tests them
 
 #define GRASPH_INLINE __attribute__((always_inline))
 typedef float vec4 __attribute__((ext_vector_type(4)));
@@ -67,7 +78,8 @@ __device__ __forceinline__ float lane_value(const float v, const int lane)
 __global__ __launch_bounds__(kBoxThreads) void batch_box_kernel(const float4* __restrict__ xs,
                                                                 const int4* __restrict__ blk,
                                                                 const BatchInst* __restrict__ insts,
-                                                                float4* __restrict__ fine, float4* __restrict__ coarse)
+                                                                float4* __restrict__ fine, float4* __restrict__ mid,
+                                                                float4* __restrict__ coarse)
 {
     const int4 bl = blk[blockIdx.x];
     const BatchInst I = insts[bl.x];
@@ -76,13 +88,15 @@ __global__ __launch_bounds__(kBoxThreads) void batch_box_kernel(const float4* __
     const int t = first + (int)threadIdx.x;
     const bool act = t < I.n;
     const float4 p = act ? xs[I.off + t] : make_float4(0.f, 0.f, 0.f, 0.f);
-    block_boxes(p, act, first, I.n, fine + 2 * (size_t)I.fine0, coarse + 2 * (size_t)I.coarse0);
+    block_boxes(p, act, first, I.n, fine + 2 * (size_t)I.fine0, mid + 2 * (size_t)(kBoxCoarse / kBoxMid) * I.coarse0,
+                coarse + 2 * (size_t)I.coarse0);
 }
 
 template <bool BATCH>
 __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __restrict__ xs, const int n0,
                                                             const float4* __restrict__ fine0,
                                                             const float4* __restrict__ coarse0,
+                                                            const float4* __restrict__ mid0,
                                                             int* __restrict__ nbr, int* __restrict__ nbr_cnt,
                                                             const int kmax, const float h2,
                                                             const int4* __restrict__ blk,
@@ -91,13 +105,15 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
 {
     // one wavefront's rows are its own: no barrier
     __shared__ int boxes[kTile / kBoxFine][kBoxList];
+    __shared__ int mids[kTile / kBoxFine][kMidList];
+    __shared__ int coarses[kTile / kBoxFine][64];
     __shared__ vec4 partners[kTile / kBoxFine][kPartners];
     // XCD-contiguous (xcd_block): neighbouring tiles read the same partners
     const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     int off = 0, n = n0, first;  // the instance's slots [off, off + n); this wavefront's 8, instance-relative
     float H2 = h2;
-    const float4 *fine = fine0, *coarse = coarse0;
+    const float4 *fine = fine0, *coarse = coarse0, *mid = mid0;
     if (BATCH) {
         const int4 bl = blk[tile / (256 / kTile)];  // of 256 slots
         const BatchInst I = insts[bl.x];
@@ -106,6 +122,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         H2 = I.H2;
         fine += 2 * (size_t)I.fine0;
         coarse += 2 * (size_t)I.coarse0;
+        mid += 2 * (size_t)(kBoxCoarse / kBoxMid) * I.coarse0;
         first = bl.y - off + kTile * (tile % (256 / kTile)) + kBoxFine * wave;
     } else {
         first = kTile * tile + kBoxFine * wave;
@@ -119,7 +136,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         const float4 p = xs[off + t];
         xi = p.x; yi = p.y; zi = p.z;
     }
-    const int nf = (n + kBoxFine - 1) / kBoxFine, nc = (n + kBoxCoarse - 1) / kBoxCoarse;
+    const int nf = (n + kBoxFine - 1) / kBoxFine, nm = (n + kBoxMid - 1) / kBoxMid, nc = (n + kBoxCoarse - 1) / kBoxCoarse;
     float4 lo = fine[2 * (first / kBoxFine)], hi = fine[2 * (first / kBoxFine) + 1];
     // Eight slots that span a jump of the slot order (where the curve leaves
     // the particles and comes back) have a box that says little.  Where it is
@@ -232,31 +249,59 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
             }
         }
     };
-    int m = 0;  // boxes collected
-    for (int c0 = 0; c0 < nc; c0 += 64) {
-        const int c = min(c0 + lane, nc - 1);
-        uint64_t mc = __builtin_amdgcn_ballot_w64(c0 + lane < nc && near(coarse[2 * c], coarse[2 * c + 1]));
-        while (mc) {
-            // two coarse boxes at a time, their fine boxes' loads in flight together
-            const int f0 = (c0 + __builtin_ctzll(mc)) * (kBoxCoarse / kBoxFine);
-            mc &= mc - 1;
-            const int f1 = mc ? (c0 + __builtin_ctzll(mc)) * (kBoxCoarse / kBoxFine) : nf;  // nf: none
-            mc &= mc - 1;
-            const int fa = min(f0 + lane, nf - 1), fb = min(f1 + lane, nf - 1);
-            const float4 la = fine[2 * fa], ha = fine[2 * fa + 1], lb = fine[2 * fb], hb = fine[2 * fb + 1];
-            const uint64_t ma = __builtin_amdgcn_ballot_w64(f0 + lane < nf && near(la, ha));
-            const uint64_t mb = __builtin_amdgcn_ballot_w64(f1 + lane < nf && near(lb, hb));
-            const uint64_t lower = (1ull << lane) - 1ull;
-            if ((ma >> lane) & 1) box[m + __builtin_popcountll(ma & lower)] = f0 + lane;
+    int* const mbox = mids[wave];
+    int* const cbox = coarses[wave];
+    const uint64_t lower = (1ull << lane) - 1ull;
+    int m = 0, mm = 0;  // fine boxes, mid boxes collected
+    // The fine boxes of the mid boxes collected, 16 mid boxes at a time, their
+    // loads in flight together.
+    auto test_mids = [&]() {
+        wave_lds_order();
+        for (int b = 0; b < mm; b += 16) {
+            const int ua = b + i, ub = ua + 8;
+            const int fa = kBoxMid / kBoxFine * mbox[min(ua, mm - 1)] + j, fb = kBoxMid / kBoxFine * mbox[min(ub, mm - 1)] + j;
+            const int ca = min(fa, nf - 1), cb = min(fb, nf - 1);
+            const float4 la = fine[2 * ca], ha = fine[2 * ca + 1], lb = fine[2 * cb], hb = fine[2 * cb + 1];
+            const uint64_t ma = __builtin_amdgcn_ballot_w64(ua < mm && fa < nf && near(la, ha));
+            const uint64_t mb = __builtin_amdgcn_ballot_w64(ub < mm && fb < nf && near(lb, hb));
+            if ((ma >> lane) & 1) box[m + __builtin_popcountll(ma & lower)] = fa;
             m += __builtin_popcountll(ma);
-            if ((mb >> lane) & 1) box[m + __builtin_popcountll(mb & lower)] = f1 + lane;
+            if ((mb >> lane) & 1) box[m + __builtin_popcountll(mb & lower)] = fb;
             m += __builtin_popcountll(mb);
             if (m > kBoxList - 128) {
                 test_boxes(m);
                 m = 0;
             }
         }
+        wave_lds_order();
+        mm = 0;
+    };
+    if (nm <= kMidDirect) {
+        for (int b = 0; b < nm; b += 64) {
+            const int q = b + lane, cq = min(q, nm - 1);
+            const uint64_t ms = __builtin_amdgcn_ballot_w64(q < nm && near(mid[2 * cq], mid[2 * cq + 1]));
+            if ((ms >> lane) & 1) mbox[mm + __builtin_popcountll(ms & lower)] = q;
+            mm += __builtin_popcountll(ms);
+            if (mm > kMidList - 64) test_mids();
+        }
     }
+    for (int c0 = nm <= kMidDirect ? nc : 0; c0 < nc; c0 += 64) {
+        const int c = min(c0 + lane, nc - 1);
+        const uint64_t mc = __builtin_amdgcn_ballot_w64(c0 + lane < nc && near(coarse[2 * c], coarse[2 * c + 1]));
+        const int cc = __builtin_popcountll(mc);  // near coarse boxes: their mid boxes, 8 coarse ones at a time
+        if ((mc >> lane) & 1) cbox[__builtin_popcountll(mc & lower)] = c;
+        wave_lds_order();
+        for (int b = 0; b < cc; b += 8) {
+            const int u = b + i, q = kBoxCoarse / kBoxMid * cbox[min(u, cc - 1)] + j, cq = min(q, nm - 1);
+            const float4 l2 = mid[2 * cq], h2 = mid[2 * cq + 1];
+            const uint64_t ms = __builtin_amdgcn_ballot_w64(u < cc && q < nm && near(l2, h2));
+            if ((ms >> lane) & 1) mbox[mm + __builtin_popcountll(ms & lower)] = q;
+            mm += __builtin_popcountll(ms);
+            if (mm > kMidList - 64) test_mids();
+        }
+        wave_lds_order();
+    }
+    test_mids();
     test_boxes(m);
     test_partners();
     if (j == 0 && t < n) nbr_cnt[off + t] = cnt;
@@ -278,7 +323,7 @@ hipError_t launch_lists(const ListLaunch& L, hipStream_t s)
 {
     if (L.n <= 0) return hipSuccess;
     hipLaunchKernelGGL(list_kernel<false>, dim3((L.n + kTile - 1) / kTile), dim3(kListThreads), 0, s, L.xs, L.n,
-                       L.fine, L.coarse, L.nbr, L.nbr_cnt, L.kmax, L.H2, nullptr, nullptr, L.max_dev, L.max_host);
+                       L.fine, L.coarse, L.mid, L.nbr, L.nbr_cnt, L.kmax, L.H2, nullptr, nullptr, L.max_dev, L.max_host);
     return hipGetLastError();
 }
 
@@ -286,9 +331,9 @@ hipError_t launch_batch_lists(const ListLaunch& L, hipStream_t s)
 {
     if (L.n <= 0 || L.n_blk <= 0) return hipSuccess;
     hipLaunchKernelGGL(batch_box_kernel, dim3(L.n_blk), dim3(kBoxThreads), 0, s, L.xs, L.blk, L.insts, L.fine,
-                       L.coarse);
+                       L.mid, L.coarse);
     hipLaunchKernelGGL(list_kernel<true>, dim3(256 / kTile * L.n_blk), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
-                       L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk, L.insts, nullptr, nullptr);
+                       L.mid, L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk, L.insts, nullptr, nullptr);
     return hipGetLastError();
 }
 

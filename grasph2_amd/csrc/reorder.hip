@@ -276,7 +276,8 @@ __global__ __launch_bounds__(kBlock) void batch_keys(const float4* __restrict__ 
 __global__ __launch_bounds__(kGatherBlock) void gather_kernel(
     const int* __restrict__ perm, const int n, const float4* __restrict__ posm, const float4* __restrict__ vel,
     const float* __restrict__ density, float4* __restrict__ xs, SlotRec* __restrict__ rec,
-    int* __restrict__ mass_flags, float4* __restrict__ fine, float4* __restrict__ coarse, int* __restrict__ list_max)
+    int* __restrict__ mass_flags, float4* __restrict__ fine, float4* __restrict__ mid,
+    float4* __restrict__ coarse, int* __restrict__ list_max)
 {
     const int t = blockIdx.x * kGatherBlock + threadIdx.x;
     int bad = 0;
@@ -297,20 +298,20 @@ __global__ __launch_bounds__(kGatherBlock) void gather_kernel(
         bad = __syncthreads_or(bad);
         if (threadIdx.x == 0) mass_flags[blockIdx.x] = bad;
     }
-    if (fine) block_boxes(p, t < n, blockIdx.x * kGatherBlock, n, fine, coarse);
+    if (fine) block_boxes(p, t < n, blockIdx.x * kGatherBlock, n, fine, mid, coarse);
 }
 
 }  // namespace
 
 hipError_t launch_gather(const int* perm, int n, const float4* posm, const float4* vel, const float* density,
-                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags, float4* fine, float4* coarse,
+                         float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags, float4* fine, float4* mid, float4* coarse,
                          int* list_max)
 {
     if (n <= 0) return hipSuccess;
-    if (!posm || (xs && !perm) || (fine && !coarse)) return hipErrorInvalidValue;
+    if (!posm || (xs && !perm) || (fine && !(mid && coarse))) return hipErrorInvalidValue;
     static_assert(kGatherBlock == kBoxCoarse, "a workgroup of the gather makes one coarse box");
     hipLaunchKernelGGL(gather_kernel, dim3((n + kGatherBlock - 1) / kGatherBlock), dim3(kGatherBlock), 0, s, perm, n,
-                       posm, vel, density, xs, rec, mass_flags, fine, coarse, list_max);
+                       posm, vel, density, xs, rec, mass_flags, fine, mid, coarse, list_max);
     return hipGetLastError();
 }
 

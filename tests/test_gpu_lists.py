@@ -106,3 +106,21 @@ def test_order_by_rank_and_by_sort(kind, n):
     ctx.close()
     want = brute_counts(h["posm"][:, :3], prm.H)
     assert (pairs, mx) == (int(want.sum()), int(want.max()))
+
+
+# boxes of 64 tested directly up to 8192 particles, from there through the boxes of 512 (64 of them a round: two
+# rounds from 32769); with H of 12 spacings every box is near and the collected ones are worked off in between
+@pytest.mark.parametrize("n,spacings", [(4097, 12.0), (8192, 2.5), (8193, 2.5), (8193, 12.0), (33000, 2.5)])
+def test_counts_at_edges_of_the_box_search(n, spacings):
+    print("box search n=%d spacings=%g" % (n, spacings), flush=True)
+    h, prm = particles("ball", n, np.random.default_rng(n))
+    prm.H = spacings * (4.2 / n) ** (1.0 / 3.0)
+    ctx = g.Context(0)
+    d = g.DeviceParticles.from_host(h)
+    ctx.calc_density(d, prm)
+    pairs, mx, over = ctx.neighbour_stats()
+    d.free()
+    ctx.close()
+    want = brute_counts(h["posm"][:, :3], prm.H)
+    assert (pairs, mx) == (int(want.sum()), int(want.max()))
+    assert over == int(np.count_nonzero(want > 160))
