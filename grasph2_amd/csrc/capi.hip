@@ -492,6 +492,11 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
     const int* perm = need_list ? order_of(c) : nullptr;
     const float4* xs = (const float4*)p->posm;
     const int gather_blocks = (int)((n + kGatherBlock - 1) / kGatherBlock);
+    // calcAcceleration::do_after sets nextTS = max_timestep
+    // (computeDerivatives.h:305-308): the next integrate(pb, true) takes
+    // min(max_timestep, this step's criteria), so dt can grow again.  No pass
+    // reads it, so with lists the gather does it.
+    const bool reset_dt = accel_pass && (f & GRASPH_VARIABLE_TIMESTEP);
     bool mass_flags = false;  // the gather makes the equal-mass check's per-block flags
     if (need_list) {
         const bool reads_vel = strain_pass || (accel_pass && sph);
@@ -505,9 +510,9 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         ProfScope ps(&c, s, KC_REORDER);
         hipError_t e = launch_gather(perm, (int)n, (const float4*)p->posm, reads_vel ? (const float4*)p->vel : nullptr,
                                      gdens ? p->density : nullptr, perm ? c.xs : nullptr, c.rec, s,
-                                     mass_flags ? c.mass_flags : nullptr, c.box, c.box + 2 * (fine_boxes(n) + coarse_boxes(n)),
-                                     c.box + 2 * fine_boxes(n),
-                                     c.list_max_dev);
+                                     mass_flags ? c.mass_flags : nullptr, c.box,
+                                     c.box + 2 * (fine_boxes(n) + coarse_boxes(n)), c.box + 2 * fine_boxes(n),
+                                     c.list_max_dev, reset_dt ? c.ts + 1 : nullptr, P.ts_max);
         if (e != hipSuccess) return hip_fail(c, e, "slot-order gather launch");
         if (perm) xs = c.xs;
     }
@@ -581,10 +586,7 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         hipError_t e = launch_accel(N, P, s);
         if (e != hipSuccess) return hip_fail(c, e, "acceleration pass launch");
     }
-    if (accel_pass && (f & GRASPH_VARIABLE_TIMESTEP)) {
-        // calcAcceleration::do_after sets nextTS = max_timestep
-        // (computeDerivatives.h:305-308): the next integrate(pb, true) takes
-        // min(max_timestep, this step's criteria), so dt can grow again.
+    if (reset_dt && !need_list) {
         hipError_t e = launch_vts_set_next(c.ts, 1, nullptr, P, 1, s);
         if (e != hipSuccess) return hip_fail(c, e, "time-step reset launch");
     }

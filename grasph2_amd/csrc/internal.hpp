@@ -559,12 +559,13 @@ hipError_t launch_reorder(const float4* posm, int n, Ctx& c, hipStream_t s);
 // position/mass and velocity/density (vel or density null: zeros there).
 // With mass_flags (one int per kGatherBlock slots) also the per-block half of
 // the equal-mass check, which launch_mass_final completes; with fine, mid and
-// coarse the lists' boxes (one instance), and list_max cleared.
+// coarse the lists' boxes (one instance), and list_max cleared;
+// with ts_next that set to ts_max.
 constexpr int kGatherBlock = kBoxCoarse;
 hipError_t launch_gather(const int* perm, int n, const float4* posm, const float4* vel, const float* density,
                          float4* xs, SlotRec* rec, hipStream_t s, int* mass_flags = nullptr,
                          float4* fine = nullptr, float4* mid = nullptr, float4* coarse = nullptr,
-                         int* list_max = nullptr);
+                         int* list_max = nullptr, float* ts_next = nullptr, float ts_max = 0.0f);
 hipError_t launch_mass_final(const float4* posm, const int* mass_flags, int nflags, float* umass, hipStream_t s);
 
 // environmentAcceleration and the zero XVEL / MAXVSIG stores of
