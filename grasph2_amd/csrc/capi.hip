@@ -284,9 +284,10 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
 // empty steps).  Passes called one by one / SPH without gravity, 16 against 4
 // lanes: 4096 particles 119 against 139 us / 47 against 57, 8192 144 against
 // 159 / 54 against 59, 11000 198 against 209 / 63 against 59, 16384 213
-// against 222 / 64 against 60.
+// against 222 / 64 against 60.  And 16 where the lists have grown long
+// (kLongLists): 65536 squeezed particles 1151 against 1181 us.
 constexpr int64_t kPassLanes16Max = 10240;
-int pass_lanes(int64_t n) { return n <= kPassLanes16Max ? 16 : 4; }
+int pass_lanes(int64_t n, int kmax) { return n <= kPassLanes16Max || kmax > kLongLists ? 16 : 4; }
 
 NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
 {
@@ -302,8 +303,8 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
     L.nbr_cnt = c.nbr_cnt;
     L.coarse = c.box + 2 * fine_boxes(p->n);
     L.n = (int)p->n;
-    L.lanes = pass_lanes(L.n);
     L.kmax = c.max_neighbours;
+    L.lanes = pass_lanes(L.n, L.kmax);
     L.balsara = p->balsara;
     L.density_dt = p->density_dt;
     L.dstress_dt = p->dstress_dt;

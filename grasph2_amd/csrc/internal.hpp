@@ -349,7 +349,34 @@ __device__ inline int xcd_block(int b, int nb)
     return x * q + min(x, r) + i;
 }
 
-// What one block of a per-particle pass works on.
+// The same in runs of c blocks: 8 c blocks after another are dealt to the XCDs
+// c to each, what is left at the end as xcd_block deals it.
+__device__ inline int xcd_runs(int b, int nb, int c)
+{
+    constexpr int kXcds = 8;
+    const int run = kXcds * c, full = nb / run * run;
+    if (b >= full) return full + xcd_block(b - full, nb - full);
+    const int r = b % run;
+    return b - r + r % kXcds * c + r / kXcds;
+}
+
+// A single instance's lists have grown long (capacity past this, bodies crushed
+// together): dense parts, contiguous in slot order, hold most neighbours.
+// Whole eighths then leave most of the work to an XCD or two, and 4 lanes per
+// particle wait for the longest list of 16: the passes take runs of kXcdRun
+// slots and 16 lanes.  131072 particles after impact (1e8 neighbours, up to
+// 3021 each), density, strain and acceleration: 0.55 + 0.95 + 1.09 ms before,
+// 0.45 + 0.67 + 0.79 with runs of 2048, 0.42 + 0.65 + 0.76 with 4096, 0.47 +
+// 0.70 + 0.83 with 8192 (5.77 ms a step before, 5.0 with 4096, 5.13 with 8192).
+// Runs read more halo than eighths: evenly squeezed spheres, whose eighths hold
+// the same work, lose by them (131072 particles 3423 against 3524 us, 90000
+// 1738 against 1789, 65536 1160 against 1229: an eighth there is 8192 slots and
+// stays), and with short lists 200003 particles 274 against 278.
+constexpr int kLongLists = 512, kXcdRun = 4096, kXcdRunMin = 65536;
+__device__ inline int xcd_run(int n, int kmax) { return kmax > kLongLists && n > kXcdRunMin ? kXcdRun : 0; }
+
+// What one block of a per-particle pass works on (run: slots per XCD in turn, 0
+// for whole eighths).
 struct SlotMap {
     int slot0, slot_end, off, n, inst, coarse0;
     // element c of particle i in an array of 6 (resp. 3) planes per instance
@@ -358,10 +385,11 @@ struct SlotMap {
 };
 
 template <bool BATCH>
-__device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_block = 256)
+__device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_block = 256, int run = 0)
 {
     SlotMap m;
-    const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
+    const int blk = BATCH || run == 0 ? xcd_block((int)blockIdx.x, (int)gridDim.x)
+                                      : xcd_runs((int)blockIdx.x, (int)gridDim.x, run / slots_per_block);
     if (BATCH) {
         const int parts = 256 / slots_per_block;  // blocks per entry of the table
         const int4 b = T.blk[blk / parts];

@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void density_kernel(const float4* __restric
 {
     using Rho = ClassSums<LPP, 1, float, CSum>;
     __shared__ __attribute__((aligned(16))) float terms[kWaves][Rho::kLds];
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP, xcd_run((int)nstride, kmax));
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
     const bool act = t0 < m.slot_end;
     const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kBlock) void strain_kernel(
     constexpr int kTerms = NC > 0 ? NC : 1;
     using Rates = ClassSums<LPP, kTerms, double, double>;
     __shared__ __attribute__((aligned(16))) double terms[kWaves][Rates::kLds];
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP, xcd_run((int)nstride, kmax));
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63;
     const bool act = t0 < m.slot_end;
     const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges
@@ -532,7 +532,7 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
     using Acc = ClassSums<LPP, 3, float, CSum>;
     using Xv = ClassSums<LPP, 3, float, float>;
     __shared__ __attribute__((aligned(16))) float terms[kWaves][(XSPH ? 2 : 1) * Acc::kLds];
-    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP);
+    const SlotMap m = slot_map<BATCH>(T, (int)nstride, kBlock / LPP, xcd_run((int)nstride, kmax));
     const int t0 = pass_slot<LPP>(m), lane = threadIdx.x & 63, sub = lane % LPP;
     const bool act = t0 < m.slot_end;
     const int t = act ? t0 : m.slot_end - 1;  // lanes past the end only take part in the wavefront's exchanges

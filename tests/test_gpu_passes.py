@@ -103,3 +103,15 @@ def test_rigid_rotation_counts_the_same_pairs():
     assert np.array_equal(got == 0, ref == 0)
     # 2 c and a wij of rounding
     assert np.allclose(got, ref, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("kind,n", [("solid", 65536), ("solid", 65537), ("xsph", 65599), ("solid", 98500)])
+def test_long_list_capacity_changes_nothing(kind, n):
+    """A capacity past 512 takes 16 lanes a particle and, from 65537 particles on, blocks dealt to the XCDs in runs
+    (whole runs up to 65536 and 98304 slots' worth of them, and what is left at the end)."""
+    print("long lists kind=%s n=%d" % (kind, n), flush=True)
+    h, prm = workload(kind, n)
+    a = run(h, prm, 0)
+    b = run(h, prm, 544)
+    for f in a:
+        assert np.array_equal(a[f], b[f]), f
