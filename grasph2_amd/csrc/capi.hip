@@ -199,8 +199,7 @@ int ensure_order(Ctx& c, const grasph_particles* p, hipStream_t s, bool count_ev
 
 const int* order_of(Ctx& c) { return c.reorder_interval > 0 ? c.perm : nullptr; }
 
-// whether work enqueued on s is being captured into a graph (then the
-// event query and the copy would break the capture)
+// whether work enqueued on s is being captured into a graph
 bool stream_capturing(hipStream_t s)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -531,7 +530,9 @@ int derivatives(Ctx& c, const grasph_particles* p, const grasph_params* prm, voi
         N.nbr_cnt = c.nbr_cnt;
         N.kmax = c.max_neighbours;
         N.max_dev = c.list_max_dev;
-        N.max_host = c.max_neighbours_grow ? c.list_max_host : nullptr;
+        // not under capture: replays would report counts whose growth frees
+        // the lists that the graph points to
+        N.max_host = c.max_neighbours_grow && c.list_max_host && !stream_capturing(s) ? c.list_max_host : nullptr;
         ProfScope ps(&c, s, KC_SWEEP);
         hipError_t e = launch_lists(N, s);
         if (e != hipSuccess) return hip_fail(c, e, "neighbour list launch");

@@ -150,7 +150,9 @@ int grasph_destroy(grasph_ctx* ctx);
  * single-instance evaluation whose lists overflowed, a later one raises
  * max_neighbours to 1.25 times the largest count seen, in steps of 32, up
  * to 4096 and 16 GiB of lists; the count is stored in host memory by the
- * list kernel and read without waiting, and not during graph capture; the
+ * list kernel and read without waiting; work captured into a graph reports
+ * nothing, but its lists go when a later eager evaluation of this context
+ * raises the capacity: capture again then, or keep it fixed; the
  * default; 0 = fixed; batches keep the capacity last set),
  * "reorder_interval"
  * (slots re-sorted along a Hilbert curve every k derivative evaluations, default 8; 0 = never;
