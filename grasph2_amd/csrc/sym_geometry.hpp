@@ -117,14 +117,14 @@ __device__ __host__ inline int64_t row_of_unit(int64_t u, int64_t nsb, int Q = 1
 // (N = 50021: 8 pieces leave the fullest of 2048 shares 9% above the mean,
 // 64 pieces 0.7%; Plummer step 419 -> 391 us, N = 17000 111 -> 83).
 constexpr int kMinSplit = 2, kMaxSplit = 64;
-__device__ __host__ inline int far_split(int64_t n, int64_t wanted)
+__device__ __host__ inline int far_split(int64_t n, int64_t wanted, int most = kMaxSplit)
 {
     const int64_t nsb = (n + kSB - 1) / kSB;
     const int64_t u1 = row_prefix(rows_with_units(nsb), nsb, 1);
     if (u1 <= 0 || wanted <= 0) return kMinSplit;
     int best = kMinSplit;
     int64_t best_num = 0, best_den = 1;  // makespan as the fraction num / den super-blocks
-    for (int Q = kMinSplit; Q <= kMaxSplit; Q *= 2) {
+    for (int Q = kMinSplit; Q <= most; Q *= 2) {
         const int64_t U = u1 * Q, W = wanted < U ? wanted : U;
         const int64_t num = (U + W - 1) / W;
         if (Q == kMinSplit || num * best_den < best_num * Q) {
@@ -135,13 +135,31 @@ __device__ __host__ inline int far_split(int64_t n, int64_t wanted)
     }
     return best;
 }
+// The most partners whose terms a slot adds in plain FP32 before they join its
+// LDS sum: a piece of a partner group by the rule above with 16 pieces at most
+// (512 down to 64 by the count: 131072 particles 512, 165000 128, 262144 64),
+// and 128 below 131072.  Of the plain sums only this one grows with the count,
+// and it shows: with a fixed 512 from 131072 on the error against FP64 (equal /
+// unequal masses) is 4.13e-8 / 5.32e-8 of the norm at 165000 and 3.88e-8 /
+// 4.68e-8 at 262144, with the rule 3.64e-8 / 4.15e-8 and 3.53e-8 / 3.78e-8, for
+// 2.8% and 3.9% of the step.  At 65536 128 instead of the piece's 512 gives
+// 3.86e-8 / 5.48e-8 instead of 4.67e-8 / 6.96e-8 for 1.6%; at 131072 it would
+// cost 2.2%.
+constexpr int kMaxFoldSplit = 16, kShortFold = 128;
+constexpr int64_t kShortFoldBelow = 131072;
+__device__ __host__ inline int far_fold(int64_t n, int64_t wanted)
+{
+    const int piece = kSB / far_split(n, wanted, kMaxFoldSplit);
+    return n < kShortFoldBelow && piece > kShortFold ? kShortFold : piece;
+}
 // the workgroup whose share [k U / W, (k + 1) U / W) holds unit u
 __device__ __host__ inline int64_t wg_of_unit(int64_t u, int64_t U, int64_t W) { return ((u + 1) * W - 1) / U; }
 // Wavefronts of the whole far field's workgroups: workgroup K's are k =
 // kFarMerge K and the next.  Where all of them are there and work on one row,
 // their own-side sums leave as one fragment, wavefront kFarMerge K's
-// (far_merged_row: that row, else -1).  Only plain fragments are merged.
-constexpr int kFarMerge = 4;
+// (far_merged_row: that row, else -1).  Only plain fragments are merged; a
+// merged one has corrections.
+constexpr int kFarMerge = 8;
 __device__ __host__ inline int64_t far_merged_row(int64_t k0, int64_t U, int64_t W, int64_t nsb, int Q)
 {
     if (k0 + kFarMerge > W) return -1;
@@ -204,7 +222,8 @@ __device__ __host__ inline int64_t bpart_group_base(int64_t h) { return (int64_t
 // kFoldsPerFlush folds and at the end of its stay on the row.  The first flush
 // writes the sums (their corrections are exactly zero).  When no stay has more
 // than kFoldsPerFlush folds, every fragment is flushed once: it is
-// plain, and neither the far field nor the combine touch its corrections;
+// plain, and neither the far field nor the combine touch its corrections
+// (except a merged one's, which its wavefronts' sums leave);
 // otherwise the first flush writes zero corrections too.
 constexpr int kFoldsPerFlush = 16;
 constexpr int kFragElems = 2 * kGroup;

@@ -23,6 +23,7 @@
 // one-sided sweep.
 // Every sum is in a fixed order, so results do not vary from run to run.
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -238,12 +239,8 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
 // The own side is folded every `fold` partners and at the end, so a slot
 // adds at most that many terms in plain FP32 before they join its LDS sum
 // (and at most kFoldsPerFlush such sums before they join the compensated
-// fragment): 512 from 131072 particles on, where a fold every 128 costs 1.3%
-// of the step and the sums of many workgroups average their rounding; 128
-// below (N = 50021: error against FP64 5.3e-8 of the norm, 6.8e-8 with 512,
-// for 1.4% of the step) and 512 in batches.
-constexpr int kFarFoldLarge = 512, kFarFoldSmall = 128, kFarFoldMin = 131072;
-static int far_fold(int64_t n) { return n >= kFarFoldMin ? kFarFoldLarge : kFarFoldSmall; }
+// fragment): far_fold's number, in batches half a group.
+constexpr int kBatchFold = 512;
 template <bool UM, bool SOFT>
 __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const int n, const int64_t g, const int b0,
                                           const int b1, const int fold, FarOwn& o, float* __restrict__ bpart,
@@ -368,7 +365,8 @@ __global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __
 #pragma unroll
             for (int w = 1; w < kFarMerge; ++w) v[c].add(lsum[w][kGroup * c + slot]);
         }
-        fr[128 * q + lane] = make_float4(v[0].value(), v[1].value(), v[2].value(), 0.0f);  // frag_elem(slot)
+        fr[128 * q + lane] = make_float4(v[0].s, v[1].s, v[2].s, 0.0f);  // frag_elem(slot)
+        fr[128 * q + lane + 64] = make_float4(v[0].c, v[1].c, v[2].c, 0.0f);
     }
 }
 
@@ -399,30 +397,39 @@ __device__ __forceinline__ void far_sums(const float4* __restrict__ apart, const
         // loads in flight before their ordered adds
         const RowFragments R = row_fragments(row_prefix(g, nsb, Q), row_prefix(g + 1, nsb, Q), U, W, PLAIN);
         const float4* const row = apart + (size_t)kFragElems * g + frag_elem((int)local);
-        const auto fragment = [&](const int64_t e) { return row + (size_t)kFragElems * R.wavefront(e); };
-        int64_t k = p;
-        for (; k + 7 * PARTS < R.count; k += 8 * PARTS) {
-            float4 f[8], fc[8];
+        // fragments [e0, e1), with their corrections
+        const auto add = [&](const int64_t e0, const int64_t e1, auto corrections) {
+            int64_t k = e0 + p;
+            for (; k + 7 * PARTS < e1; k += 8 * PARTS) {
+                float4 f[8], fc[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const float4* fr = fragment(k + u * PARTS);
-                f[u] = fr[0];
-                if (!PLAIN) fc[u] = fr[64];
-            }
+                for (int u = 0; u < 8; ++u) {
+                    const float4* fr = row + (size_t)kFragElems * R.wavefront(k + u * PARTS);
+                    f[u] = fr[0];
+                    if constexpr (corrections) fc[u] = fr[64];
+                }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
-                if (!PLAIN) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
+                for (int u = 0; u < 8; ++u) {
+                    x.add(f[u].x); y.add(f[u].y); z.add(f[u].z);
+                    if constexpr (corrections) { x.c += fc[u].x; y.c += fc[u].y; z.c += fc[u].z; }
+                }
             }
-        }
-        for (; k < R.count; k += PARTS) {
-            const float4* fr = fragment(k);
-            const float4 f = fr[0];
-            x.add(f.x); y.add(f.y); z.add(f.z);
-            if (!PLAIN) {
-                const float4 fc = fr[64];
-                x.c += fc.x; y.c += fc.y; z.c += fc.z;
+            for (; k < e1; k += PARTS) {
+                const float4* fr = row + (size_t)kFragElems * R.wavefront(k);
+                const float4 f = fr[0];
+                x.add(f.x); y.add(f.y); z.add(f.z);
+                if constexpr (corrections) {
+                    const float4 fc = fr[64];
+                    x.c += fc.x; y.c += fc.y; z.c += fc.z;
+                }
             }
+        };
+        if constexpr (PLAIN) {
+            add(0, R.lead, std::false_type());
+            add(R.lead, R.lead + R.merged, std::true_type());
+            add(R.lead + R.merged, R.count, std::false_type());
+        } else {
+            add(0, R.count, std::true_type());
         }
     }
     const int64_t base = bpart_group_base(g) + local;
@@ -660,7 +667,7 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
 {
     FarOwn o;
     far_load_row(xk, n, R.g, lane, lsum, frag, plain, o);
-    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kFarFoldLarge, o, bk, 0, H2, m, m, lane);
+    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kBatchFold, o, bk, 0, H2, m, m, lane);
     far_flush_own(o, lane);
 }
 
@@ -801,7 +808,7 @@ SymGeom sym_geometry(int64_t n, int wgs, int64_t col_elems)
     G.wgs = far_workgroups(wgs, G.units);
     G.near_elems = 2 * n;
     G.apart_elems = (int64_t)kFragElems * (G.groups + wgs);
-    G.plain = fragments_plain(far_folds(G.units, G.wgs, G.split, far_fold(n)));
+    G.plain = fragments_plain(far_folds(G.units, G.wgs, G.split, far_fold(n, wgs)));
     G.bpart_elems = 3 * bpart_group_base(G.groups);
     G.ncols = 1;
     if (G.bpart_elems > col_elems) {
@@ -834,7 +841,7 @@ template <bool SOFT>
 void launch_far_column(const SymLaunch& L, const SymCol& C, const int split, const DevParams& P, hipStream_t s)
 {
     hipLaunchKernelGGL((far_column_kernel<SOFT>), dim3(C.wgs), dim3(kFarThreads), 0, s, L.xs, L.n, C.c0, C.c1,
-                       C.units, C.wgs, split, far_fold(L.n), L.apart, C.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                       C.units, C.wgs, split, far_fold(L.n, L.wgs), L.apart, C.plain ? 1 : 0, L.bpart, P.H2, L.umass);
 }
 
 void launch_column_combine(const SymLaunch& L, const SymCol& C, const int split, const bool first, const bool last,
@@ -857,15 +864,15 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
         const int far_groups = (L.wgs + kFarMerge - 1) / kFarMerge;
         if (P.H2 > 0.0f)
             hipLaunchKernelGGL((far_kernel<true>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                               L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         else
             hipLaunchKernelGGL((far_kernel<false>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, far_fold(L.n), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+                               L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
         return hipGetLastError();
     }
     const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
     for (int b = 0; b < G.ncols; ++b) {
-        const SymCol C = sym_column(G.split, far_fold(L.n), L.wgs, c[b], c[b + 1]);
+        const SymCol C = sym_column(G.split, far_fold(L.n, L.wgs), L.wgs, c[b], c[b + 1]);
         if (P.H2 > 0.0f) launch_far_column<true>(L, C, G.split, P, s); else launch_far_column<false>(L, C, G.split, P, s);
         if (b + 1 < G.ncols) launch_column_combine(L, C, G.split, b == 0, false, P, s);
     }
@@ -899,7 +906,7 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
     if (G.ncols > 1 && sym_has_far(L)) {
         // the last column batch's combine, which finishes
         const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
-        const SymCol C = sym_column(G.split, far_fold(L.n), L.wgs, c[G.ncols - 1], c[G.ncols]);
+        const SymCol C = sym_column(G.split, far_fold(L.n, L.wgs), L.wgs, c[G.ncols - 1], c[G.ncols]);
         launch_column_combine(L, C, G.split, false, true, P, s);
         return hipGetLastError();
     }
@@ -948,7 +955,7 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
             for (int h = 0; h < batch_row_pieces(u); ++h) {
                 const int units = (int)(batch_piece_begin(u, h + 1) - batch_piece_begin(u, h));
                 T.rows.push_back(SymRow{k, g, h, units});
-                T.plain = T.plain && fragments_plain((int64_t)units * kGroup / kFarFoldLarge);
+                T.plain = T.plain && fragments_plain((int64_t)units * kGroup / kBatchFold);
             }
         }
         row0 += S.nrows;
