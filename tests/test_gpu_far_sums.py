@@ -62,3 +62,29 @@ def test_own_chains(groups):
     total = m.astype(np.float64).sum()
     rms = np.sqrt(np.mean((got / total - 1.0) ** 2))
     assert rms < 1.15e-7, rms
+
+
+@pytest.mark.parametrize("waves", [0, 4])
+def test_in_group_chains(waves):
+    """Inside a group, 64 slots in one point and the 960 others, masses in
+    [1, 2), in the other.  As above with 64 a chain, 15 of them: 1.15e-7 /
+    sqrt(960 / 64), and the result's own 1.7e-8: 3.4e-8, times 1.4 for the sample."""
+    print("in-group chains waves=%d" % waves, flush=True)
+    ctx = g.Context(0)
+    ctx.set_option("sweep_symmetric", 1)
+    ctx.set_option("sym_near_shares", waves)
+    prm = ics.plummer_params(2.0)
+    off = []
+    for seed in range(64):
+        h = g.host_particles(1024, ("posm", "vel", "acc"))
+        h["posm"][:, 3] = np.random.default_rng(seed).uniform(1.0, 2.0, size=1024).astype(np.float32)
+        h["posm"][:960, :3] = 2.0
+        d = g.DeviceParticles.from_host(h)
+        ctx.compute_derivatives(d, prm)
+        g.hip.synchronize()
+        got = 32.0 * d.download(["acc"])["acc"][960:, 0].astype(np.float64)
+        d.free()
+        off.append(got / h["posm"][:960, 3].astype(np.float64).sum() - 1.0)
+    ctx.close()
+    rms = np.sqrt(np.mean(np.square(off)))
+    assert rms < 4.8e-8, rms
