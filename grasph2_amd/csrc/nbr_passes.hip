@@ -564,7 +564,7 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
         const PairSep sep = pair_sep(rx, ry, rz, P);
         const double s = dw_over_r_f64(sep, P);
         const float gx = (float)(s * (double)rx), gy = (float)(s * (double)ry), gz = (float)(s * (double)rz);
-        const float rho2 = rhoi + qb.w, irho2 = AV || XSPH ? rcp_f32(rho2) : 0.0f;  // twice the mean density
+        const float rho2 = rhoi + qb.w;  // twice the mean density
         const float mj = pj.w;
         const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
         float II = 0.0f;
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
             const float wij = (rx * vx + ry * vy + rz * vz) * (float)sep.ir;
             const float vsig = __builtin_fmaf(-3.0f, wij, P.c + P.c);
             const float b = BALS ? bi + qb.z : 2.0f;
-            const float II0 = div_f32(-0.5f * P.alpha * b * wij * vsig, rho2, irho2);
+            const float II0 = -0.25f * b * P.alpha * wij * vsig / (0.5f * rho2);
             II = wij < 0.0f ? II0 : 0.0f;
             if (BALS && counts && wij < 0.0f) mv = fmaxf(mv, vsig);
         }
@@ -607,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
         if (XSPH) {  // :291-294
             const float qf = (float)sep.q, om = 1.0f - qf;
             const float w = P.Wpref * (qf < 0.5f ? __builtin_fmaf(-6.0f * qf * qf, om, 1.0f) : 2.0f * om * om * om);
-            const float fx = div_f32(2.0f * mj, rho2, irho2) * w;
+            const float fx = 2.0f * mj / rho2 * w;
             x[0] = -fx * vx;
             x[1] = -fx * vy;
             x[2] = -fx * vz;

@@ -86,20 +86,6 @@ __device__ inline double div_f64(double a, double b)
     const double e = __builtin_fma(-b, y, 1.0);
     return __builtin_amdgcn_div_fixup(a * __builtin_fma(y, __builtin_fma(e, e, e), y), b, a);
 }
-// 1 / b for div_f32 below (b's exponent well inside FP32's range)
-__device__ inline float rcp_f32(float b)
-{
-    const float y = __builtin_amdgcn_rcpf(b);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-// a / b, y = rcp_f32(b): rounded once (an error of at most half an ulp and
-// 2^-20 of one), zeros, infinities and NaN as in IEEE division
-__device__ inline float div_f32(float a, float b, float y)
-{
-    const float q = a * y;
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
-}
-
 // A pair's separation in FP64 from the FP32 coordinate differences: 1 / r and
 // q = r / H.
 struct PairSep {
