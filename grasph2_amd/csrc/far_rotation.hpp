@@ -71,8 +71,8 @@ __device__ __forceinline__ float ror(float v)
 }
 
 // One rotation in plain code (no softening: coincident particles exert
-// nothing, computeDerivatives.h:226).
-template <bool UM>
+// nothing, computeDerivatives.h:226).  WIDE: far_rotation_soft's.
+template <bool UM, bool WIDE>
 __device__ __forceinline__ void far_rotation_hard(FarPartner& p, FarOwn& o)
 {
     float px = 0.0f, py = 0.0f, pz = 0.0f;
@@ -83,7 +83,11 @@ __device__ __forceinline__ void far_rotation_hard(FarPartner& p, FarOwn& o)
         const float inv = __builtin_amdgcn_rsqf(d2);
         float s = inv * inv;
         s = (d2 > 0.0f) ? s * inv : 0.0f;
-        const float sa = UM ? s : p.m * s, sb = UM ? s : s * o.m[q];
+        float sa = UM ? s : p.m * s, sb = UM ? s : s * o.m[q];
+        if (!UM && WIDE) {
+            sa = d2 > 0.0f ? (p.m * inv) * (inv * inv) : 0.0f;
+            sb = d2 > 0.0f ? (o.m[q] * inv) * (inv * inv) : 0.0f;
+        }
         o.ax[q] = fmaf(dx, sa, o.ax[q]); o.ay[q] = fmaf(dy, sa, o.ay[q]); o.az[q] = fmaf(dz, sa, o.az[q]);
         px = fmaf(dx, sb, px); py = fmaf(dy, sb, py); pz = fmaf(dz, sb, pz);
     }
@@ -127,6 +131,10 @@ __device__ __forceinline__ void far_rotation_hard(FarPartner& p, FarOwn& o)
 // unequal masses: the slot's mass for the partner side, the partner's for the slot's
 #define GRASPH_FAR_MASS(q, d, x, y, z, t)                                                                          \
     "v_mul_f32 v" #t ", v" #d ", %[m" #q "]\n v_mul_f32 v" #d ", %[jm], v" #d "\n"
+// the same from 1/r and 1/r^2, each mass joining 1/r first; v130 in passing
+#define GRASPH_FAR_WIDE(q, d, x, y, z, t)                                                                          \
+    "v_mul_f32 v130, v" #d ", %[m" #q "]\n v_mul_f32 v" #d ", %[jm], v" #d "\n"                                   \
+    "v_mul_f32 v" #d ", v" #t ", v" #d "\n v_mul_f32 v" #t ", v130, v" #t "\n"
 // slot q's sums and its partner side with the factor in register f; op starts (v_mul) or continues (v_fmac) P
 #define GRASPH_FAR_SUMS(q, d, x, y, z, f, op)                                                                      \
     "v_fmac_f32 %[ax" #q "], v" #x ", v" #d "\n" op " %[px], v" #x ", v" #f "\n"                                    \
@@ -152,11 +160,14 @@ __device__ __forceinline__ void far_rotation_hard(FarPartner& p, FarOwn& o)
     GRASPH_FAR_ROR("v_add_f32_dpp", "tx", ", %[px]") GRASPH_FAR_ROR("v_add_f32_dpp", "ty", ", %[py]")              \
     GRASPH_FAR_ROR("v_add_f32_dpp", "tz", ", %[pz]") GRASPH_FAR_ROR("v_mov_b32_dpp", "jx", "")                     \
     GRASPH_FAR_ROR("v_mov_b32_dpp", "jy", "") GRASPH_FAR_ROR("v_mov_b32_dpp", "jz", "")
-#define GRASPH_FAR_CUBE "s_setprio 0\n" GRASPH_FAR_SLOTS(GRASPH_FAR_INV2) GRASPH_FAR_SLOTS(GRASPH_FAR_INV3)
+#define GRASPH_FAR_SQUARE "s_setprio 0\n" GRASPH_FAR_SLOTS(GRASPH_FAR_INV2)
+#define GRASPH_FAR_CUBE GRASPH_FAR_SQUARE GRASPH_FAR_SLOTS(GRASPH_FAR_INV3)
 
 // One rotation with softening; the partner's mass rotates for the next one.
 // (Early-clobber outputs: the block writes them before its last input is read.)
-template <bool UM>
+// WIDE, unequal masses: the masses join 1/r, not 1/r^3, as in own_block.hpp, one
+// multiply per pair more.
+template <bool UM, bool WIDE>
 __device__ __forceinline__ void far_rotation_soft(FarPartner& p, FarOwn& o, const float h2)
 {
     if constexpr (UM) {
@@ -167,12 +178,17 @@ __device__ __forceinline__ void far_rotation_soft(FarPartner& p, FarOwn& o, cons
                      : GRASPH_FAR_CLOBBERS);
     } else {
         const float jm = p.m;
-        asm volatile(GRASPH_FAR_HEAD GRASPH_FAR_ROR("v_mov_b32_dpp", "nm", "") GRASPH_FAR_CUBE
-                         GRASPH_FAR_SLOTS(GRASPH_FAR_MASS) GRASPH_FAR_SLOT0(GRASPH_FAR_START_M)
-                             GRASPH_FAR_SLOTS1(GRASPH_FAR_SUMS_M)
-                     : GRASPH_FAR_PARTNER, [nm] "+&v"(p.m) GRASPH_FAR_SLOTS(GRASPH_FAR_OUT)
-                     : [h2] "v"(h2), [jm] "v"(jm) GRASPH_FAR_SLOTS(GRASPH_FAR_IN) GRASPH_FAR_SLOTS(GRASPH_FAR_MASS_IN)
-                     : GRASPH_FAR_CLOBBERS);
+#define GRASPH_FAR_UNEQUAL(FACTORS, ...)                                                                           \
+    asm volatile(GRASPH_FAR_HEAD GRASPH_FAR_ROR("v_mov_b32_dpp", "nm", "") FACTORS                                 \
+                     GRASPH_FAR_SLOT0(GRASPH_FAR_START_M) GRASPH_FAR_SLOTS1(GRASPH_FAR_SUMS_M)                     \
+                 : GRASPH_FAR_PARTNER, [nm] "+&v"(p.m) GRASPH_FAR_SLOTS(GRASPH_FAR_OUT)                            \
+                 : [h2] "v"(h2), [jm] "v"(jm) GRASPH_FAR_SLOTS(GRASPH_FAR_IN) GRASPH_FAR_SLOTS(GRASPH_FAR_MASS_IN) \
+                 : GRASPH_FAR_CLOBBERS, ##__VA_ARGS__)
+        if constexpr (WIDE)
+            GRASPH_FAR_UNEQUAL(GRASPH_FAR_SQUARE GRASPH_FAR_SLOTS(GRASPH_FAR_WIDE), "v130");
+        else
+            GRASPH_FAR_UNEQUAL(GRASPH_FAR_CUBE GRASPH_FAR_SLOTS(GRASPH_FAR_MASS));
+#undef GRASPH_FAR_UNEQUAL
     }
 }
 

@@ -60,6 +60,8 @@ struct OwnAcc {
 #define GRASPH_OWN_RSQ(q, r, d, x, y, z, t) GRASPH_FAR_RSQ(q, d, x, y, z, t)
 #define GRASPH_OWN_INV2(q, r, d, x, y, z, t) GRASPH_FAR_INV2(q, d, x, y, z, t)
 #define GRASPH_OWN_INV3(q, r, d, x, y, z, t) GRASPH_FAR_INV3(q, d, x, y, z, t)
+// the mass joins 1/r: m / r is in range where 1 / r^3 alone is not (r past 10^13 or
+// below 10^-13, with masses to match)
 #define GRASPH_OWN_MASS(q, r, d, x, y, z, t) "v_mul_f32 v" #d ", %[jm" #r "], v" #d "\n"
 #define GRASPH_OWN_SUMS(q, r, d, x, y, z, t)                                                                       \
     "v_fmac_f32 %[ax" #q "], v" #x ", v" #d "\n v_fmac_f32 %[ay" #q "], v" #y ", v" #d "\n"                         \
@@ -71,7 +73,7 @@ struct OwnAcc {
 #define GRASPH_OWN_BODY(PAIRS, MASS)                                                                               \
     "v_mov_b32 v96, %[h2]\n" PAIRS(GRASPH_OWN_SUB) PAIRS(GRASPH_OWN_R2X) PAIRS(GRASPH_OWN_R2Y)                      \
     PAIRS(GRASPH_OWN_R2Z) "s_setprio 1\n" PAIRS(GRASPH_OWN_RSQ) "s_setprio 0\n s_nop 0\n"                          \
-    PAIRS(GRASPH_OWN_INV2) PAIRS(GRASPH_OWN_INV3) MASS PAIRS(GRASPH_OWN_SUMS)
+    PAIRS(GRASPH_OWN_INV2) MASS PAIRS(GRASPH_OWN_INV3) PAIRS(GRASPH_OWN_SUMS)
 #define GRASPH_OWN_ASM(PAIRS, SUMS, SLOTS, PARTNERS, MASSES)                                                       \
     if constexpr (UM)                                                                                              \
         asm volatile(GRASPH_OWN_BODY(PAIRS, "") : SUMS : [h2] "v"(h2), SLOTS, PARTNERS : GRASPH_OWN_CLOBBERS);     \
@@ -96,9 +98,7 @@ __device__ __forceinline__ void own_pairs(const float4 (&p)[kOwnPairs / NI], Own
                 const float dx = p[r].x - a.x[q], dy = p[r].y - a.y[q], dz = p[r].z - a.z[q];
                 const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
                 const float inv = __builtin_amdgcn_rsqf(d2);
-                float s = inv * inv;
-                s = (d2 > 0.0f) ? s * inv : 0.0f;
-                if (!UM) s = p[r].w * s;
+                const float s = (d2 > 0.0f) ? (UM ? inv : p[r].w * inv) * (inv * inv) : 0.0f;
                 a.ax[q] = fmaf(dx, s, a.ax[q]); a.ay[q] = fmaf(dy, s, a.ay[q]); a.az[q] = fmaf(dz, s, a.az[q]);
             }
     } else if constexpr (NI == 1) {

@@ -90,16 +90,16 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void ingroup_kernel(const float4
 // lane's kNI slots.  Own side into o.a*; returns the partner side: lanes
 // 0-15 hold partner l's x, lanes 16-31 partner l - 16's z, lanes 32-47
 // partner l - 32's y (UM: without the common mass; else with the slots' masses).
-template <bool UM, bool SOFT>
+template <bool UM, bool SOFT, bool WIDE>
 __device__ __forceinline__ float far_chunk_rot(const float4 pj, FarOwn& o, const float H2)
 {
     FarPartner p{pj.x, pj.y, pj.z, pj.w, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
     for (int k = 0; k < kRow; ++k) {
         if constexpr (SOFT)
-            far_rotation_soft<UM>(p, o, H2);
+            far_rotation_soft<UM, WIDE>(p, o, H2);
         else
-            far_rotation_hard<UM>(p, o);
+            far_rotation_hard<UM, WIDE>(p, o);
     }
     // the last rotation's contribution, then home
     const float tx = ror<1>(ror<1>(p.tx) + p.px), ty = ror<1>(ror<1>(p.ty) + p.py), tz = ror<1>(ror<1>(p.tz) + p.pz);
@@ -241,7 +241,7 @@ __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int
 // (and at most kFoldsPerFlush such sums before they join the compensated
 // fragment): far_fold's number, in batches half a group.
 constexpr int kBatchFold = 512;
-template <bool UM, bool SOFT>
+template <bool UM, bool SOFT, bool WIDE>
 __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const int n, const int64_t g, const int b0,
                                           const int b1, const int fold, FarOwn& o, float* __restrict__ bpart,
                                           const int64_t boff, const float H2, const float mo, const float mp,
@@ -261,7 +261,7 @@ __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const i
                  3 * (lane & (kRow - 1)) + partner_comp_rot(lane);
         const float4 B = load_partner_row<UM>(xs, b + kRow, n, lane);  // unused after the last
         if (b + kRow > end) A = bound_partner_row(A, b, n, lane);
-        const float v = far_chunk_rot<UM, SOFT>(A, o, H2);
+        const float v = far_chunk_rot<UM, SOFT, WIDE>(A, o, H2);
         *bp = UM ? v * mo : v;
         bp += 3 * kRow;
         A = B;
@@ -284,7 +284,7 @@ __device__ __forceinline__ void far_range(const float4* __restrict__ xs, const i
 // mass and its partners one (one more read of their masses, the first ones
 // with the row's slots; a kernel that looks at all particles first costs 5 us,
 // 8% of a Plummer step at 16384).
-template <bool SOFT, bool COL>
+template <bool SOFT, bool COL, bool WIDE>
 __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const int n, const int64_t nsb, const int c0,
                                          const int c1, const int64_t U, const int W, const int Q, const int fold,
                                          float4* __restrict__ apart, const bool plain, const int k, const bool merge,
@@ -326,9 +326,9 @@ __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const in
             one_mass = !__any(differ != 0);
         }
         if (one_mass)
-            far_range<true, SOFT>(xs, n, g, first, end, fold, o, bpart, boff, H2, mo, mp, lane);
+            far_range<true, SOFT, false>(xs, n, g, first, end, fold, o, bpart, boff, H2, mo, mp, lane);
         else
-            far_range<false, SOFT>(xs, n, g, first, end, fold, o, bpart, boff, H2, 1.0f, 1.0f, lane);
+            far_range<false, SOFT, WIDE>(xs, n, g, first, end, fold, o, bpart, boff, H2, 1.0f, 1.0f, lane);
         if (!merge) far_flush_own(o, lane);
         u += cnt;
     }
@@ -338,7 +338,11 @@ __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const in
 // but two a row), their own-side sums leave as one fragment: a fragment per
 // wavefront was 34 MB written and read again, whatever the count (Plummer
 // N = 16384: 69.6 -> 66.6 us per step, 50021: 441 -> 434).
-template <bool SOFT>
+// WIDE (below kWideBelow particles, down to where the one-sided sweep takes over):
+// unequal masses in any units, as there (unequal masses, N = 13000: 51.6 -> 53.6 us
+// a step; from 16384 on 1 / r^3 has to be in range by itself).
+constexpr int kWideBelow = 16384;
+template <bool SOFT, bool WIDE>
 __global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __restrict__ xs, const int n,
                                                                const int64_t nsb, const int64_t U, const int W,
                                                                const int Q, const int fold,
@@ -351,7 +355,7 @@ __global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __
     const int k0 = kFarMerge * (int)blockIdx.x;
     const int64_t g = plain ? far_merged_row(k0, U, W, nsb, Q) : -1;
     const bool merge = g >= 0;  // the same for the whole workgroup
-    far_work<SOFT, false>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, k0 + wave, merge, bpart, H2, umass,
+    far_work<SOFT, false, WIDE>(xs, n, nsb, 1, (int)nsb, U, W, Q, fold, apart, plain, k0 + wave, merge, bpart, H2, umass,
                           lsum[wave]);
     if (!merge) return;
     __syncthreads();
@@ -380,7 +384,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void far_column_kernel(const float4
                                                                    const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
-    far_work<SOFT, true>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
+    far_work<SOFT, true, false>(xs, n, 0, c0, c1, U, W, Q, fold, apart, plain, blockIdx.x, false, bpart, H2, umass, lsum);
 }
 
 // The far field's part p of PARTS of slot t's sums: the own-side fragments of
@@ -667,7 +671,7 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
 {
     FarOwn o;
     far_load_row(xk, n, R.g, lane, lsum, frag, plain, o);
-    far_range<UM, SOFT>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kBatchFold, o, bk, 0, H2, m, m, lane);
+    far_range<UM, SOFT, false>(xk, n, R.g, kGroup * j0, kGroup * (j0 + R.units), kBatchFold, o, bk, 0, H2, m, m, lane);
     far_flush_own(o, lane);
 }
 
@@ -862,12 +866,15 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
     const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     if (G.ncols == 1) {
         const int far_groups = (L.wgs + kFarMerge - 1) / kFarMerge;
-        if (P.H2 > 0.0f)
-            hipLaunchKernelGGL((far_kernel<true>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
-        else
-            hipLaunchKernelGGL((far_kernel<false>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb, G.units,
-                               L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass);
+#define GRASPH_FAR(SOFT, WIDE)                                                                                       \
+    hipLaunchKernelGGL((far_kernel<SOFT, WIDE>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb,     \
+                       G.units, L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass)
+        const bool soft = P.H2 > 0.0f, wide = L.n < kWideBelow;
+        if (soft && wide) GRASPH_FAR(true, true);
+        else if (soft) GRASPH_FAR(true, false);
+        else if (wide) GRASPH_FAR(false, true);
+        else GRASPH_FAR(false, false);
+#undef GRASPH_FAR
         return hipGetLastError();
     }
     const std::vector<int> c = sym_columns(G.nsb, L.col_elems);
