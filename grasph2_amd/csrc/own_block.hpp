@@ -22,11 +22,10 @@
 namespace grasph {
 namespace {
 
-constexpr int kFold = 128;        // partners per plain partial sum before the compensated add
-// the same for the pairs inside a group of the symmetric sweep, a larger part of
-// all (error against FP64 of the norm with 128: 4.44e-8 at 16384 particles, with
-// 64 4.37e-8; at 5000 with unequal masses 8.59e-8, 7.65e-8)
-constexpr int kGroupFold = 64;
+// partners per plain partial sum before the compensated add (error against FP64
+// of the norm with 128 and 64, unequal masses: 8000 particles 1.13e-7, 8.64e-8; pairs
+// inside a group at 16384 4.44e-8, 4.37e-8 of all; for 0.5% of the step)
+constexpr int kFold = 64;
 constexpr int kOwnPairs = 8;      // pairs per asm block
 constexpr int kOwnMaxWaves = 16;  // wavefronts sharing their own slots
 
@@ -115,9 +114,8 @@ __device__ __forceinline__ void own_pairs(const float4 (&p)[kOwnPairs / NI], Own
 }
 
 // Compensated gravity of the lane's slots from the partners [j0, j1), in
-// order, FOLD (64 or 128) at a time in plain FP32; tile: 64 float4 of this
-// wavefront's; m the common mass when UM.
-template <int NI, bool UM, bool SOFT, int FOLD>
+// order; tile: 64 float4 of this wavefront's; m the common mass when UM.
+template <int NI, bool UM, bool SOFT>
 __device__ __forceinline__ void own_sweep(const float4* __restrict__ xs, const int j0, const int j1, OwnAcc<NI>& a,
                                           CSum (&s)[NI][3], const float h2, const float m, float4* tile,
                                           const int lane)
@@ -154,15 +152,13 @@ __device__ __forceinline__ void own_sweep(const float4* __restrict__ xs, const i
             }
         }
         __builtin_amdgcn_wave_barrier();
-        static_assert(FOLD == 64 || FOLD == 128);
-        if (FOLD == 64 || ((j - j0) & 64) || j + 64 >= j1) {  // FOLD partners, or the end
+        static_assert(kFold == 64);  // a tile
 #pragma unroll
-            for (int q = 0; q < NI; ++q) {
-                s[q][0].add(UM ? a.ax[q] * m : a.ax[q]);
-                s[q][1].add(UM ? a.ay[q] * m : a.ay[q]);
-                s[q][2].add(UM ? a.az[q] * m : a.az[q]);
-                a.ax[q] = a.ay[q] = a.az[q] = 0.0f;
-            }
+        for (int q = 0; q < NI; ++q) {
+            s[q][0].add(UM ? a.ax[q] * m : a.ax[q]);
+            s[q][1].add(UM ? a.ay[q] * m : a.ay[q]);
+            s[q][2].add(UM ? a.az[q] * m : a.az[q]);
+            a.ax[q] = a.ay[q] = a.az[q] = 0.0f;
         }
     }
 }
@@ -179,7 +175,7 @@ __host__ __device__ constexpr int own_lds_floats(int ni, int waves)
 // [j0 + wave len, j0 + (wave + 1) len).  store(t, x, y, z) gets every slot's
 // sums, the shares' added in share order.  With several wavefronts they are
 // the whole workgroup, and every thread calls it.
-template <int NI, bool UM, bool SOFT, int FOLD = kFold, typename F>
+template <int NI, bool UM, bool SOFT, typename F>
 __device__ __forceinline__ void own_block(const float4* __restrict__ xs, const int o0, const int o1, const int j0,
                                           const int j1, const int len, const float h2, const float m,
                                           const int wave, const int waves, float* lds, F&& store)
@@ -195,7 +191,7 @@ __device__ __forceinline__ void own_block(const float4* __restrict__ xs, const i
         s[q][0] = s[q][1] = s[q][2] = CSum{0.0f, 0.0f};
     }
     const int b = j0 + wave * len, e = min(j1, b + len);
-    own_sweep<NI, UM, SOFT, FOLD>(xs, b, e, a, s, h2, m, reinterpret_cast<float4*>(lds) + 64 * wave, lane);
+    own_sweep<NI, UM, SOFT>(xs, b, e, a, s, h2, m, reinterpret_cast<float4*>(lds) + 64 * wave, lane);
     if (waves == 1) {
 #pragma unroll
         for (int q = 0; q < NI; ++q)

@@ -13,7 +13,7 @@
 // particle perm[t].  The pair loop is own_block.hpp's: up to 16 wavefronts of
 // a workgroup share 64 or 256 own slots and add their sums in LDS; with more
 // shares than that, planes of workgroups write partial sums that a second
-// kernel adds.  Sums are plain FP32 over blocks of 128 partners, then
+// kernel adds.  Sums are plain FP32 over blocks of 64 partners, then
 // compensated (TwoSum).
 //
 // The batched kernel runs the same code persistently over a queue of work
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kBlock) void no_gravity_kernel(const int n, float4*
 // in ping-pong.  Softened, the self pair is in the sum and is taken back
 // where r^2, as the oracle rounds it, is 0 (cand: softened squared distance
 // that every such pair stays below).
-constexpr int kChunk = 8;
+constexpr int kChunk = 8, kPotFold = 128;  // partners per plain partial sum
 template <bool SOFT>
 __device__ __forceinline__ void pot_chunk(const float4 (&pj)[kChunk], const float xi, const float yi, const float zi,
                                           float& phi, const float H2, const float cand)
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kBlock) void pot_kernel(const float4* __restrict__ 
 #pragma unroll
         for (int c = 0; c < kChunk; ++c) A[c] = posm[ja + c];
         pot_chunk<SOFT>(B, p.x, p.y, p.z, phi, H2, cand);
-        if (((k + 1) % (kFold / kChunk)) == kFold / kChunk - 1) fold();
+        if (((k + 1) % (kPotFold / kChunk)) == kPotFold / kChunk - 1) fold();
     }
     if (k < nchunks) pot_chunk<SOFT>(A, p.x, p.y, p.z, phi, H2, cand);
     if (nfull < n) {  // the last partial chunk, padded with far-away massless partners

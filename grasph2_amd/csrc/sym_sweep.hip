@@ -62,9 +62,9 @@ __device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, con
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
     if (um && um[0] != 0.0f)
-        own_block<NI, true, SOFT, kGroupFold>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
+        own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
     else
-        own_block<NI, false, SOFT, kGroupFold>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
+        own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
 }
 
 // a slot's compensated sums as two float4

@@ -1,4 +1,5 @@
-"""The far field's own-side sums (csrc/sym_sweep.hip), alone: every group but
+"""Plain FP32 chains of the gravity sums, alone.  The far field's own side
+(csrc/sym_sweep.hip): every group but
 the last in one point, the last group's particles in another, so that each far
 pair's factor is a power of two (r^2 + H^2 = 16, dx = 2: m_j / 32 exactly) or
 nothing.  What a slot of the first groups is off by is the rounding of its sum
@@ -64,15 +65,16 @@ def test_own_chains(groups):
     assert rms < 1.15e-7, rms
 
 
-@pytest.mark.parametrize("waves", [0, 4])
-def test_in_group_chains(waves):
-    """Inside a group, 64 slots in one point and the 960 others, masses in
+@pytest.mark.parametrize("symmetric,waves,slices", [(1, 0, 0), (1, 4, 0), (0, 0, 1), (0, 0, 3)])
+def test_in_group_and_one_sided_chains(symmetric, waves, slices):
+    """Inside a group, or one-sided, 64 slots in one point and the 960 others, masses in
     [1, 2), in the other.  As above with 64 a chain, 15 of them: 1.15e-7 /
     sqrt(960 / 64), and the result's own 1.7e-8: 3.4e-8, times 1.4 for the sample."""
-    print("in-group chains waves=%d" % waves, flush=True)
+    print("in-group chains sym=%d waves=%d slices=%d" % (symmetric, waves, slices), flush=True)
     ctx = g.Context(0)
-    ctx.set_option("sweep_symmetric", 1)
+    ctx.set_option("sweep_symmetric", symmetric)
     ctx.set_option("sym_near_shares", waves)
+    ctx.set_option("sweep_slices", slices)
     prm = ics.plummer_params(2.0)
     off = []
     for seed in range(64):
