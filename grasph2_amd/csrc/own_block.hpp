@@ -224,15 +224,16 @@ __device__ __forceinline__ void own_block(const float4* __restrict__ xs, const i
 }
 
 // own_block for few particles: 64 / SPLIT slots, each in SPLIT lanes of a
-// wavefront, the q-th of which takes the share wave SPLIT + q of len partners.  With one slot per lane 1000 particles
-// were 16 workgroups of 16 wavefronts, 64 partners long each; four lanes a
-// slot make that 63 workgroups and 16 partners (Plummer step 11.0 -> 9.6 us,
-// of 4096, in one plane instead of four, 13.7 -> 11.2).
+// wavefront, the q-th of which takes the share wave SPLIT + q of len partners,
+// whose masses are taken as they come.  With one slot per lane 1000 particles
+// were 16 workgroups of 16 wavefronts, 64 partners long each; four lanes a slot
+// make that 63 workgroups of 11 wavefronts and 24 partners (Plummer step 11.0 ->
+// 9.6 us, of 4096, in one plane instead of four, 13.7 -> 11.2).
 // Every wavefront of the workgroup calls it; lds as for own_block<1>.
-template <int SPLIT, bool UM, bool SOFT, typename F>
+template <int SPLIT, bool SOFT, typename F>
 __device__ __forceinline__ void own_split_block(const float4* __restrict__ xs, const int o0, const int n,
-                                                const int len, const float h2, const float m, const int wave,
-                                                const int waves, float* lds, F&& store)
+                                                const int len, const float h2, const int wave, const int waves,
+                                                float* lds, F&& store)
 {
     constexpr int kSlots = 64 / SPLIT;  // of the workgroup, and partners of a share in a tile
     const int lane = threadIdx.x & 63, slot = lane % kSlots, q = lane / kSlots;
@@ -258,13 +259,13 @@ __device__ __forceinline__ void own_split_block(const float4* __restrict__ xs, c
             float4 p[kOwnPairs];
 #pragma unroll
             for (int r = 0; r < kOwnPairs; ++r) p[r] = tile[lane - slot + g + r];
-            own_pairs<1, UM, SOFT>(p, a, h2);
+            own_pairs<1, false, SOFT>(p, a, h2);
         }
         __builtin_amdgcn_wave_barrier();
         if ((j + kSlots) % kFold == 0 || j + kSlots >= len) {
-            s[0].add(UM ? a.ax[0] * m : a.ax[0]);
-            s[1].add(UM ? a.ay[0] * m : a.ay[0]);
-            s[2].add(UM ? a.az[0] * m : a.az[0]);
+            s[0].add(a.ax[0]);
+            s[1].add(a.ay[0]);
+            s[2].add(a.az[0]);
             a.ax[0] = a.ay[0] = a.az[0] = 0.0f;
         }
     }

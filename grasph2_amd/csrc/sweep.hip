@@ -61,14 +61,9 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void own_kernel(const float4* __
         }
         acc[i] = make_float4(ax, ay, az, 0.0f);
     };
-    if constexpr (SPLIT > 1) {  // one plane
-        if (umass && umass[0] != 0.0f)
-            own_split_block<SPLIT, true, SOFT>(xs, o0, n, slice_len, P.H2, umass[1], wave, waves, lds, store);
-        else
-            own_split_block<SPLIT, false, SOFT>(xs, o0, n, slice_len, P.H2, 1.0f, wave, waves, lds, store);
-        return;
-    } else
-    if (umass && umass[0] != 0.0f)  // {uniform, mass} of the particles
+    if constexpr (SPLIT > 1)  // one plane, no mass check
+        own_split_block<SPLIT, SOFT>(xs, o0, n, slice_len, P.H2, wave, waves, lds, store);
+    else if (umass && umass[0] != 0.0f)  // {uniform, mass} of the particles
         own_block<NI, true, SOFT>(xs, o0, n, j0, n, slice_len, P.H2, umass[1], wave, waves, lds, store);
     else
         own_block<NI, false, SOFT>(xs, o0, n, j0, n, slice_len, P.H2, 1.0f, wave, waves, lds, store);
@@ -345,7 +340,7 @@ hipError_t launch_sweep(const SweepLaunch& L, const DevParams& P, hipStream_t s)
     }
     if (L.waves < 1 || L.waves > kOwnMaxWaves || L.planes < 1 || L.slice_len < 8 || L.slice_len % 8)
         return hipErrorInvalidValue;
-    if (L.split != 1 && (L.split != kOwnSplit || L.ni != 1 || L.planes != 1)) return hipErrorInvalidValue;
+    if (L.split != 1 && (L.split != kOwnSplit || L.ni != 1 || L.planes != 1 || L.umass)) return hipErrorInvalidValue;
     if (L.split != 1) return soft ? launch_own<1, true, kOwnSplit>(L, P, s) : launch_own<1, false, kOwnSplit>(L, P, s);
     switch (L.ni) {
         case 1: return soft ? launch_own<1, true>(L, P, s) : launch_own<1, false>(L, P, s);
