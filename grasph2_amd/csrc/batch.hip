@@ -563,6 +563,7 @@ int batch_passes(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s
     N.nbr = b.d_nbr;
     N.nbr_cnt = b.d_cnt;
     N.coarse = b.d_box + 2 * b.n_fine;
+    N.mid = b.d_box + 2 * (b.n_fine + b.n_coarse);
     N.n = (int)b.ntotal;
     N.lanes = 4;
     N.kmax = b.kmax;

@@ -303,6 +303,7 @@ NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
     L.nbr = c.nbr;
     L.nbr_cnt = c.nbr_cnt;
     L.coarse = c.box + 2 * fine_boxes(p->n);
+    L.mid = c.box + 2 * (fine_boxes(p->n) + coarse_boxes(p->n));
     L.n = (int)p->n;
     L.kmax = c.max_neighbours;
     L.lanes = pass_lanes(L.n, L.kmax);

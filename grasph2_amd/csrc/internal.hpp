@@ -514,6 +514,7 @@ struct NbrLaunch {
     const int* nbr;
     const int* nbr_cnt;
     const float4* coarse;  // the lists' boxes of 512 slots
+    const float4* mid;     // and of 64
     int n;
     int kmax;
     float* balsara;
