@@ -220,6 +220,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     // The partners in the m boxes of box[] within H of this wavefront's own
     // box, collected: 8 boxes at a time, kAhead times as many on their way.
     auto test_boxes = [&](const int m) {
+        if (m == 0) return;  // box[m - 1] is read
         wave_lds_order();
         int at[kAhead];
         vec4 q[kAhead];
