@@ -217,6 +217,15 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         wave_lds_order();
         np = 0;
     };
+    // The particles collected: the `close` lanes' of p, slots a of the instance.
+    const auto collect = [&](vec4 p, const int a, const bool close) GRASPH_INLINE {
+        const uint64_t all = __builtin_amdgcn_ballot_w64(close);
+        p.w = __int_as_float(off + a);
+        if (close)
+            part[np + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0))] = p;
+        np += __builtin_popcountll(all);
+        if (np > kPartners - 72) test_partners();
+    };
     // The partners in the m boxes of box[] within H of this wavefront's own
     // box, collected: 8 boxes at a time, kAhead times as many on their way.
     auto test_boxes = [&](const int m) {
@@ -235,18 +244,13 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
                 const int a = at[u];
-                vec4 p = q[u];
+                const vec4 p = q[u];
                 fetch(b0 + 8 * (u + kAhead), at[u], q[u]);
                 const float4 at4 = make_float4(p.x, p.y, p.z, 0.0f);
                 bool close = boxes_near(lo, hi, at4, at4, H2);
                 if (jump) close = close || boxes_near(lo2, hi2, at4, at4, H2);
                 close = close && a < n;
-                const uint64_t all = __builtin_amdgcn_ballot_w64(close);
-                p.w = __int_as_float(off + a);
-                if (close)
-                    part[np + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0))] = p;
-                np += __builtin_popcountll(all);
-                if (np > kPartners - 72) test_partners();
+                collect(p, a, close);
             }
         }
     };
@@ -258,6 +262,53 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     // loads in flight together.
     auto test_mids = [&]() {
         wave_lds_order();
+        // The wavefront's slots lie apart and most boxes in a row are near: the
+        // slot order keeps nothing together here (option reorder_interval 0, or
+        // bodies small beside the distance of a stray particle, on which the
+        // curve's cells depend).  Every particle of the boxes is then tested
+        // against the 8 slots, 64 particles a load.  60000 particles in random
+        // order 2244 -> 1280 us a derivative call, one of them 3000 radii away
+        // 1912 -> 1230 (all-pairs lists beside the gravity took 1458 and 1508).
+        if (each && mm > kMidList / 4 && mbox[mm - 1] - mbox[0] < 2 * mm) {
+            test_boxes(m);
+            m = 0;
+            // the slots as registers of the loop (the compiler read their lanes anew for
+            // every 64 particles: list kernel 1237 us, 673 now), a third of them vector
+            // ones: all would leave 6 wavefronts a SIMD instead of 8
+            float sx[kBoxFine], sy[kBoxFine], sz[kBoxFine];
+#pragma unroll
+            for (int q = 0; q < kBoxFine; ++q) {
+                const float4 o = slot(q);  // NaN past the end: nothing is close
+                sx[q] = o.x; sy[q] = o.y; sz[q] = o.z;
+                __asm__ volatile("" : "+v"(sx[q]), "+s"(sy[q]), "+s"(sz[q]));
+            }
+            const float limit = fmaf(H2, 1.0f + 1.0f / (1 << 20), 1e-37f);  // within H, as the pairs round it
+            const auto first_of = [&](const int b) GRASPH_INLINE {
+                return kBoxMid * __builtin_amdgcn_readfirstlane(mbox[min(b, mm - 1)]);
+            };
+            const auto load = [&](const int a) GRASPH_INLINE {
+                return *reinterpret_cast<const vec4*>(xj + a + (uint32_t)min(lane, n - 1 - a));
+            };
+            int ahead = first_of(0);
+            vec4 next = load(ahead);
+            for (int b = 0; b < mm; ++b) {
+                const int a = ahead;
+                const vec4 p = next;
+                ahead = first_of(b + 1);
+                next = load(ahead);
+                float d = INFINITY;
+#pragma unroll
+                for (int q = 0; q < kBoxFine; ++q) {
+                    const float dx = p.x - sx[q], dy = p.y - sy[q], dz = p.z - sz[q];
+                    d = fminf(d, fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
+                }
+                const bool close = d <= limit && lane < n - a;
+                if (__builtin_amdgcn_ballot_w64(close)) collect(p, a + lane, close);
+            }
+            wave_lds_order();
+            mm = 0;
+            return;
+        }
         for (int b = 0; b < mm; b += 16) {
             const int ua = b + i, ub = ua + 8;
             const int fa = kBoxMid / kBoxFine * mbox[min(ua, mm - 1)] + j, fb = kBoxMid / kBoxFine * mbox[min(ub, mm - 1)] + j;
