@@ -45,8 +45,8 @@ struct BatchState {
     int* d_inst_of = nullptr;
     int4* d_items = nullptr;
     int n_items = 0;
-    int4* d_blk = nullptr;
-    int n_blk = 0;
+    int4* d_blk = nullptr;    // (instance, first, end) of every 256 slots, then of every 64 and of every 32
+    int n_blk = 0, n_blk64 = 0, n_blk32 = 0;
     int* d_queue = nullptr;
     float* d_ts = nullptr;  // variable step: {current dt, next dt} per instance, zero when the tables are built
     float* d_um = nullptr;  // {uniform, mass} per instance, written before each gravity sweep
@@ -56,8 +56,8 @@ struct BatchState {
     SymInst* d_sinst = nullptr;
     SymRow* d_srows = nullptr;
     int n_srows = 0;
-    int4* d_sblk = nullptr;  // 256-slot blocks of the instances in the symmetric sweep
-    int n_sblk = 0;
+    int4* d_sblk = nullptr;  // 256-slot, then 64-slot blocks of the instances in the symmetric sweep
+    int n_sblk = 0, n_sblk64 = 0;
     int64_t sym_min = -1;    // the size threshold the tables were built with (-1: none)
     bool sym_plain = true;  // SymBatchTables::plain
     float4* d_snear = nullptr;
@@ -125,7 +125,7 @@ void free_tables(BatchState& b)
     b.d_sinst = nullptr; b.d_srows = nullptr; b.d_box = nullptr; b.d_snear = nullptr;
     b.d_sapart = nullptr; b.d_sbpart = nullptr; b.d_sblk = nullptr;
     b.n_srows = 0;
-    b.n_sblk = 0;
+    b.n_sblk = b.n_sblk64 = 0;
     b.sym_min = -1;
     b.sym_plain = true;
     b.d_insts = nullptr; b.d_prm = nullptr; b.d_inst_of = nullptr; b.d_items = nullptr; b.d_blk = nullptr;
@@ -135,7 +135,7 @@ void free_tables(BatchState& b)
     b.sort_bytes = 0;
     b.order_valid = false;
     b.n_items = 0;
-    b.n_blk = 0;
+    b.n_blk = b.n_blk64 = b.n_blk32 = 0;
 }
 
 template <typename T>
@@ -223,7 +223,7 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
         std::vector<BatchInst> insts(n_inst);
         std::vector<DevParams> prm(n_inst);
         std::vector<int> inst_of((size_t)p->n);
-        std::vector<int4> blk;
+        std::vector<int4> blk, blk64, blk32;
         int fine0 = 0, coarse0 = 0;
         for (int k = 0; k < n_inst; ++k) {
             prm[k] = make_dev_params(&bt->params[k]);
@@ -232,10 +232,15 @@ int prepare(Ctx& c, const grasph_particles* p, const grasph_batch* bt)
             fine0 += (int)fine_boxes(n);
             coarse0 += (int)coarse_boxes(n);
             for (int64_t i = off; i < off + n; ++i) inst_of[(size_t)i] = k;
-            for (int64_t s = off; s < off + n; s += 256)
-                blk.push_back(make_int4(k, (int)s, (int)std::min<int64_t>(s + 256, off + n), 0));
+            append_blocks(blk, k, off, off + n, 256);
+            append_blocks(blk64, k, off, off + n, 64);
+            append_blocks(blk32, k, off, off + n, 32);
         }
         b.n_blk = (int)blk.size();
+        b.n_blk64 = (int)blk64.size();
+        b.n_blk32 = (int)blk32.size();
+        blk.insert(blk.end(), blk64.begin(), blk64.end());
+        blk.insert(blk.end(), blk32.begin(), blk32.end());
         if ((r = upload(c, b.d_insts, insts, "batch instance table")) || (r = upload(c, b.d_prm, prm, "batch params")) ||
             (r = upload(c, b.d_inst_of, inst_of, "batch instance map")) || (r = upload(c, b.d_blk, blk, "batch blocks")))
             return r;
@@ -343,6 +348,8 @@ BlockTables tables(const BatchState& b)
     T.insts = b.d_insts;
     T.prm = b.d_prm;
     T.nblocks = b.n_blk;
+    T.blk64 = b.d_blk + b.n_blk;
+    T.nblocks64 = b.n_blk64;
     return T;
 }
 
@@ -399,6 +406,8 @@ int batch_lists(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s)
     L.kmax = b.kmax;
     L.blk = b.d_blk;
     L.n_blk = b.n_blk;
+    L.blk32 = b.d_blk + b.n_blk + b.n_blk64;
+    L.n_blk32 = b.n_blk32;
     L.insts = b.d_insts;
     ProfScope ps(&c, s, KC_SWEEP);
     hipError_t e = launch_batch_lists(L, s);
@@ -439,8 +448,11 @@ int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStrea
 int ensure_sym(Ctx& c, BatchState& b)
 {
     if (b.d_sinst && b.sym_min == c.batch_symmetric_min) return 0;
-    const SymBatchTables T = sym_batch_tables(b.offsets, c.batch_symmetric_min);
+    SymBatchTables T = sym_batch_tables(b.offsets, c.batch_symmetric_min);
     int r;
+    b.n_sblk = (int)T.blk.size();
+    b.n_sblk64 = (int)T.blk64.size();
+    T.blk.insert(T.blk.end(), T.blk64.begin(), T.blk64.end());
     free_ptr(b.d_sinst); free_ptr(b.d_srows); free_ptr(b.d_sblk);
     b.d_sinst = nullptr; b.d_srows = nullptr; b.d_sblk = nullptr;
     if ((r = upload(c, b.d_sinst, T.insts, "batch symmetric-sweep instances")) ||
@@ -448,7 +460,6 @@ int ensure_sym(Ctx& c, BatchState& b)
         (r = upload(c, b.d_sblk, T.blk, "batch symmetric-sweep blocks")))
         return r;
     b.n_srows = (int)T.rows.size();
-    b.n_sblk = (int)T.blk.size();
     b.sym_min = c.batch_symmetric_min;
     b.sym_plain = T.plain;
     // fresh arrays for the new tables (upload()-style: free, then allocate)
@@ -488,6 +499,8 @@ int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStr
     L.prm = b.d_prm;
     L.blk = b.d_sblk;
     L.n_blk = b.n_sblk;
+    L.blk64 = b.d_sblk + b.n_sblk;
+    L.n_blk64 = b.n_sblk64;
     L.rows = b.d_srows;
     L.nrows = b.n_srows;
     L.plain = b.sym_plain;

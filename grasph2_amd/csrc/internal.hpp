@@ -241,10 +241,15 @@ struct SymInst {
 struct SymRow {
     int inst, g, piece, units;  // piece `piece` of far row g of instance inst: units partner groups
 };
+// [begin, end) of instance k in blocks of `slots`
+inline void append_blocks(std::vector<int4>& blk, int k, int64_t begin, int64_t end, int slots)
+{
+    for (int64_t s = begin; s < end; s += slots) blk.push_back(make_int4(k, (int)s, (int)std::min(s + slots, end), 0));
+}
 struct SymBatchTables {
     std::vector<SymInst> insts;  // every instance; those below min_n have n = 0
     std::vector<SymRow> rows;    // longest first
-    std::vector<int4> blk;       // 256-slot blocks (instance, first, end) of the instances in the sweep
+    std::vector<int4> blk, blk64;  // 256-slot and 64-slot blocks (instance, first, end) of the instances in the sweep
     int64_t apart_elems = 0, bpart_elems = 0;
     bool plain = true;  // no row piece flushes its fragment twice
 };
@@ -259,8 +264,10 @@ struct SymBatchLaunch {
     const SymInst* sinst;
     const BatchInst* insts;
     const DevParams* prm;
-    const int4* blk;      // 256-slot blocks of the instances in the sweep
+    const int4* blk;      // 256-slot and 64-slot blocks of the instances in the sweep
     int n_blk;
+    const int4* blk64;
+    int n_blk64;
     const SymRow* rows;
     int nrows;
     int* queue;           // one work counter
@@ -303,8 +310,10 @@ struct ListLaunch {
     int kmax;
     int* max_dev;      // largest count of an overflowed list: of this evaluation (0 before it), and
     int* max_host;     // the host's copy; null: not reported
-    const int4* blk;   // batch: 256-slot blocks of all instances
+    const int4* blk;   // batch: 256-slot and 32-slot blocks of all instances
     int n_blk;
+    const int4* blk32;
+    int n_blk32;
     const BatchInst* insts;
 };
 hipError_t launch_lists(const ListLaunch& L, hipStream_t s);
@@ -332,6 +341,11 @@ struct BlockTables {
     const BatchInst* insts;
     const DevParams* prm;  // per-instance parameters
     int nblocks;           // 0: one instance, the grid covers all slots
+    // the same cut into blocks of 64 slots, one list pass workgroup each (with four
+    // to a block of 256, most of them empty, 2000 instances of 50 took 55 us in the
+    // strain and the acceleration pass, now 19)
+    const int4* blk64;
+    int nblocks64;
 };
 
 // Workgroups are dealt to the GPU's 8 XCDs in turn (workgroup b to XCD
@@ -391,11 +405,10 @@ __device__ inline SlotMap slot_map(const BlockTables& T, int n, int slots_per_bl
     const int blk = BATCH || run == 0 ? xcd_block((int)blockIdx.x, (int)gridDim.x)
                                       : xcd_runs((int)blockIdx.x, (int)gridDim.x, run / slots_per_block);
     if (BATCH) {
-        const int parts = 256 / slots_per_block;  // blocks per entry of the table
-        const int4 b = T.blk[blk / parts];
+        const int4 b = slots_per_block == 64 ? T.blk64[blk] : T.blk[blk];  // 64 or 256
         const BatchInst I = T.insts[b.x];
         m.inst = b.x;
-        m.slot0 = b.y + blk % parts * slots_per_block;
+        m.slot0 = b.y;
         m.slot_end = b.z;
         m.off = I.off;
         m.n = I.n;
@@ -422,17 +435,19 @@ __device__ inline void block_boxes(const float4 p, const bool act, const int fir
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float v[6] = {act ? p.x : INFINITY,  act ? p.y : INFINITY,  act ? p.z : INFINITY,
                   act ? p.x : -INFINITY, act ? p.y : -INFINITY, act ? p.z : -INFINITY};
+    if (__any(act)) {  // else the wavefront's slots are past the end
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+        for (int o = 1; o < 64; o <<= 1) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v[c] = fminf(v[c], __shfl_xor(v[c], o, 64));
-            v[c + 3] = fmaxf(v[c + 3], __shfl_xor(v[c + 3], o, 64));
-        }
-        if (o == kBoxFine / 2 && (lane & (kBoxFine - 1)) == 0 && act) {
-            const int f = (first + (int)threadIdx.x) / kBoxFine;
-            fine[2 * f] = make_float4(v[0], v[1], v[2], 0.0f);
-            fine[2 * f + 1] = make_float4(v[3], v[4], v[5], 0.0f);
+            for (int c = 0; c < 3; ++c) {
+                v[c] = fminf(v[c], __shfl_xor(v[c], o, 64));
+                v[c + 3] = fmaxf(v[c + 3], __shfl_xor(v[c + 3], o, 64));
+            }
+            if (o == kBoxFine / 2 && (lane & (kBoxFine - 1)) == 0 && act) {
+                const int f = (first + (int)threadIdx.x) / kBoxFine;
+                fine[2 * f] = make_float4(v[0], v[1], v[2], 0.0f);
+                fine[2 * f + 1] = make_float4(v[3], v[4], v[5], 0.0f);
+            }
         }
     }
     if (lane == 0) {

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     float H2 = h2;
     const float4 *fine = fine0, *coarse = coarse0, *mid = mid0;
     if (BATCH) {
-        const int4 bl = blk[tile / (256 / kTile)];  // of 256 slots
+        const int4 bl = blk[tile];
         const BatchInst I = insts[bl.x];
         off = I.off;
         n = I.n;
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
         fine += 2 * (size_t)I.fine0;
         coarse += 2 * (size_t)I.coarse0;
         mid += 2 * (size_t)(kBoxCoarse / kBoxMid) * I.coarse0;
-        first = bl.y - off + kTile * (tile % (256 / kTile)) + kBoxFine * wave;
+        first = bl.y - off + kBoxFine * wave;
     } else {
         first = kTile * tile + kBoxFine * wave;
     }
@@ -381,11 +381,12 @@ hipError_t launch_lists(const ListLaunch& L, hipStream_t s)
 
 hipError_t launch_batch_lists(const ListLaunch& L, hipStream_t s)
 {
-    if (L.n <= 0 || L.n_blk <= 0) return hipSuccess;
+    if (L.n <= 0 || L.n_blk <= 0 || L.n_blk32 <= 0) return hipSuccess;
+    static_assert(kTile == 32, "the batch's blocks of the list kernel");
     hipLaunchKernelGGL(batch_box_kernel, dim3(L.n_blk), dim3(kBoxThreads), 0, s, L.xs, L.blk, L.insts, L.fine,
                        L.mid, L.coarse);
-    hipLaunchKernelGGL(list_kernel<true>, dim3(256 / kTile * L.n_blk), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
-                       L.mid, L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk, L.insts, nullptr, nullptr);
+    hipLaunchKernelGGL(list_kernel<true>, dim3(L.n_blk32), dim3(kListThreads), 0, s, L.xs, 0, L.fine, L.coarse,
+                       L.mid, L.nbr, L.nbr_cnt, L.kmax, 0.0f, L.blk32, L.insts, nullptr, nullptr);
     return hipGetLastError();
 }
 

@@ -677,7 +677,7 @@ inline dim3 grid_plain(const NbrLaunch& L)  // per-particle kernels without a li
 inline dim3 grid_of(const NbrLaunch& L)
 {
     const int per = kBlock / L.lanes;  // particles per block
-    return dim3(L.T.nblocks > 0 ? L.T.nblocks * L.lanes : (L.n + per - 1) / per);
+    return dim3(L.T.nblocks > 0 ? L.T.nblocks64 : (L.n + per - 1) / per);
 }
 
 template <bool BATCH, int LPP>

@@ -53,18 +53,19 @@ __device__ __forceinline__ float swap16_sum(float p, float q)
 // ------------------------------------------------------------------ kernels
 
 // In-group gravity: a workgroup takes 64 NI slots of a group, its wavefronts
-// an equal share of the group's slots as partners each (whole shares of
-// kGroup / waves, whatever the group holds).  store(t, x, y, z) gets every
-// slot's compensated sums.
+// a share of len (times their number at least the group's slots) of the
+// group's slots as partners each.  store(t, x, y, z) gets every slot's
+// compensated sums.
 template <int NI, bool SOFT, typename F>
 __device__ __forceinline__ void ingroup_block(const float4* __restrict__ xs, const int o0, const int g0, const int g1,
-                                              const float h2, const float* __restrict__ um, float* lds, F&& store)
+                                              const int len, const float h2, const float* __restrict__ um, float* lds,
+                                              F&& store)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
     if (um && um[0] != 0.0f)
-        own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, um[1], wave, waves, lds, store);
+        own_block<NI, true, SOFT>(xs, o0, g1, g0, g1, len, h2, um[1], wave, waves, lds, store);
     else
-        own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, kGroup / waves, h2, 1.0f, wave, waves, lds, store);
+        own_block<NI, false, SOFT>(xs, o0, g1, g0, g1, len, h2, 1.0f, wave, waves, lds, store);
 }
 
 // a slot's compensated sums as two float4
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(64 * kOwnMaxWaves) void ingroup_kernel(const float4
 {
     extern __shared__ float lds[];
     const int o0 = 64 * blockIdx.x, g0 = o0 / kGroup * kGroup;
-    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), h2, umass, lds,
+    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), kGroup / (int)(blockDim.x >> 6), h2, umass, lds,
                            [&](int t, const CSum& x, const CSum& y, const CSum& z) { store_near(near_part, t, x, y, z); });
 }
 
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(64 * kNearFused) void near_combine_kernel(
     const int p = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int o0 = 64 * blockIdx.x, g0 = o0 / kGroup * kGroup, t = o0 + lane;
     CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
-    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), P.H2, umass, lds,
+    ingroup_block<1, SOFT>(xs, o0, g0, min(n, g0 + kGroup), kGroup / kNearFused, P.H2, umass, lds,
                            [&](int, const CSum& a, const CSum& b, const CSum& c) {  // wavefront 0's lanes
                                x = a; y = b; z = c;
                            });
@@ -646,7 +647,8 @@ __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
 // (instance, group) from a counter, longest first, so each row's own-side
 // sums leave as one fragment, numbered by the instance's first row + g.
 
-template <bool SOFT>
+// NI 4: blk has blocks of 256 slots, NI 1: of 64.
+template <int NI, bool SOFT>
 __global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4* __restrict__ xs,
                                                                    const int4* __restrict__ blk,
                                                                    const SymInst* __restrict__ sinst,
@@ -654,12 +656,15 @@ __global__ __launch_bounds__(kBlock) void sym_batch_ingroup_kernel(const float4*
                                                                    float4* __restrict__ near_part,
                                                                    const float* __restrict__ umass)
 {
-    __shared__ float lds[own_lds_floats(4, kBlock / 64)];
+    constexpr int kWaves = kBlock / 64;
+    __shared__ float lds[own_lds_floats(NI, kWaves)];
     const int4 bl = blk[xcd_block((int)blockIdx.x, (int)gridDim.x)];  // XCD-contiguous (xcd_block)
     const SymInst S = sinst[bl.x];
     const int g0 = S.off + (bl.y - S.off) / kGroup * kGroup;
-    ingroup_block<4, SOFT>(xs, bl.y, g0, min(S.off + S.n, g0 + kGroup), insts[bl.x].H2, umass + 2 * bl.x, lds,
-                           [&](int t, const CSum& x, const CSum& y, const CSum& z) { store_near(near_part, t, x, y, z); });
+    const int g1 = min(S.off + S.n, g0 + kGroup);
+    const int len = ((g1 - g0 + kWaves - 1) / kWaves + 7) / 8 * 8;  // even shares: small groups keep all wavefronts busy
+    ingroup_block<NI, SOFT>(xs, bl.y, g0, g1, len, insts[bl.x].H2, umass + 2 * bl.x, lds,
+                            [&](int t, const CSum& x, const CSum& y, const CSum& z) { store_near(near_part, t, x, y, z); });
 }
 
 // one piece of a far row of an instance of the batch: group R.g against
@@ -950,9 +955,10 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
         SymInst S;
         S.off = (int)offsets[k];
         S.n = sym ? (int)n : 0;  // instances left to the one-sided sweep: nothing here
-        if (sym)
-            for (int64_t s = offsets[k]; s < offsets[k + 1]; s += 256)
-                T.blk.push_back(make_int4(k, (int)s, (int)std::min<int64_t>(s + 256, offsets[k + 1]), 0));
+        if (sym) {
+            append_blocks(T.blk, k, offsets[k], offsets[k + 1], 256);
+            append_blocks(T.blk64, k, offsets[k], offsets[k + 1], 64);
+        }
         S.nsb = (int)((S.n + kSB - 1) / kSB);
         S.nrows = (int)rows_with_units(S.nsb);
         S.row0 = row0;
@@ -975,15 +981,23 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
     return T;
 }
 
+// Blocks of 64 slots, one a lane, where those of 256 leave the GPU idle (so many
+// workgroups fill it once: 16 x 4096 particles 48 against 34 us, 32 x
+// 4096 56 either way, 512 x 1000 165 against 172) or leave an eighth of the lanes
+// without a slot (2000 x 50: 20 us with 256, 8 with 64).
+constexpr int kNearBlocksMin = 512;
 hipError_t launch_sym_batch_ingroup(const SymBatchLaunch& L, hipStream_t s)
 {
     if (L.ntotal <= 0 || L.n_blk <= 0 || !L.grav) return hipSuccess;
-    if (L.soft)
-        hipLaunchKernelGGL(sym_batch_ingroup_kernel<true>, dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk, L.sinst,
-                           L.insts, L.near_part, L.umass);
-    else
-        hipLaunchKernelGGL(sym_batch_ingroup_kernel<false>, dim3(L.n_blk), dim3(kBlock), 0, s, L.xs, L.blk, L.sinst,
-                           L.insts, L.near_part, L.umass);
+    const bool small = L.n_blk < kNearBlocksMin || 9 * (int64_t)L.n_blk64 < 32 * (int64_t)L.n_blk;
+#define GRASPH_NEAR(NI, SOFT, N, BLK)                                                                                \
+    hipLaunchKernelGGL((sym_batch_ingroup_kernel<NI, SOFT>), dim3(N), dim3(kBlock), 0, s, L.xs, BLK, L.sinst, L.insts, \
+                       L.near_part, L.umass)
+    if (small && L.soft) GRASPH_NEAR(1, true, L.n_blk64, L.blk64);
+    else if (small) GRASPH_NEAR(1, false, L.n_blk64, L.blk64);
+    else if (L.soft) GRASPH_NEAR(4, true, L.n_blk, L.blk);
+    else GRASPH_NEAR(4, false, L.n_blk, L.blk);
+#undef GRASPH_NEAR
     return hipGetLastError();
 }
 
