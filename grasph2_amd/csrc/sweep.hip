@@ -245,7 +245,9 @@ __global__ __launch_bounds__(64) void combine_kernel(const float4* __restrict__ 
 // (inst, slot0, ni) covers slots [slot0, slot0 + 64 ni) of instance inst
 // with ni particles per lane (chosen per size bucket) against all of the
 // instance's particles [off, off + n); its slots are the same range of perm.
-// Every wavefront leaves the loop once the counter passes n_items.  NIMAX
+// A wavefront's first item is its own number, the next come from the counter
+// (2000 instances of 50: 134 us a derivative call with the first from there
+// too); it leaves the loop past n_items.  NIMAX
 // is the largest ni of the items.
 template <int NIMAX, bool SOFT>
 __global__ __launch_bounds__(kBlock) void batch_sweep_kernel(const float4* __restrict__ xs,
@@ -260,11 +262,9 @@ __global__ __launch_bounds__(kBlock) void batch_sweep_kernel(const float4* __res
     auto store = [&](const int t, const CSum& x, const CSum& y, const CSum& z) {
         acc[perm ? perm[t] : t] = make_float4(x.value(), y.value(), z.value(), 0.0f);
     };
-    for (;;) {
-        int w = 0;
-        if ((threadIdx.x & 63) == 0) w = atomicAdd(queue, 1);
-        w = __builtin_amdgcn_readfirstlane(w);
-        if (w >= n_items) break;
+    const int waves = (int)(gridDim.x * blockDim.x) >> 6;
+    int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    while (w < n_items) {
         const int4 it = items[w];
         const BatchInst I = insts[it.x];
         const int e = I.off + I.n;
@@ -280,6 +280,10 @@ __global__ __launch_bounds__(kBlock) void batch_sweep_kernel(const float4* __res
         } else {
             own_block<1, false, SOFT>(xs, it.y, e, I.off, e, I.n, I.H2, 1.0f, 0, 1, tile, store);
         }
+        if (waves >= n_items) break;
+        w = 0;
+        if ((threadIdx.x & 63) == 0) w = atomicAdd(queue, 1);
+        w = __builtin_amdgcn_readfirstlane(w) + waves;
     }
 }
 
@@ -309,11 +313,12 @@ hipError_t launch_own(const SweepLaunch& L, const DevParams& P, hipStream_t s)
 template <bool SOFT>
 hipError_t launch_b(const BatchSweepLaunch& L, hipStream_t s)
 {
+    const int blocks = std::min(L.blocks, (L.n_items + L.waves_per_block - 1) / L.waves_per_block);
     if (L.ni_max == 2)
-        hipLaunchKernelGGL((batch_sweep_kernel<2, SOFT>), dim3(L.blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
+        hipLaunchKernelGGL((batch_sweep_kernel<2, SOFT>), dim3(blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
                            L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, L.umass);
     else
-        hipLaunchKernelGGL((batch_sweep_kernel<1, SOFT>), dim3(L.blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
+        hipLaunchKernelGGL((batch_sweep_kernel<1, SOFT>), dim3(blocks), dim3(64 * L.waves_per_block), 0, s, L.xs,
                            L.perm, L.items, L.n_items, L.insts, L.queue, L.acc, L.umass);
     return hipGetLastError();
 }

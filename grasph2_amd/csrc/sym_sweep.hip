@@ -680,9 +680,10 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
     far_flush_own(o, lane);
 }
 
-// Persistent far field over the batch's rows; every wavefront leaves once
-// the counter passes nrows.  plain: no piece has more than kFoldsPerFlush
-// units.
+// Persistent far field over the batch's rows: a wavefront's first is its own
+// number, the next come from the counter; it leaves past nrows.  (With the
+// first from the counter too, where few rows end up was a race: 384 of them
+// 545 or 580 us.)  plain: no piece has more than kFoldsPerFlush units.
 template <bool SOFT>
 __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
     const float4* __restrict__ xs, const SymInst* __restrict__ sinst, const BatchInst* __restrict__ insts,
@@ -691,11 +692,9 @@ __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
 {
     __shared__ float lsum[3 * kGroup];
     const int lane = threadIdx.x;
-    for (;;) {
-        int r = 0;
-        if (lane == 0) r = atomicAdd(queue, 1);
-        r = __builtin_amdgcn_readfirstlane(__shfl(r, 0, 64));
-        if (r >= nrows) break;
+    const int waves = gridDim.x;
+    int r = blockIdx.x;
+    while (r < nrows) {
         const SymRow R = rows[r];
         const SymInst S = sinst[R.inst];
         const float H2 = insts[R.inst].H2;
@@ -709,6 +708,10 @@ __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
             batch_far_row<true, SOFT>(xk, S.n, R, j0, lsum, frag, plain, bk, H2, m, lane);
         else
             batch_far_row<false, SOFT>(xk, S.n, R, j0, lsum, frag, plain, bk, H2, 1.0f, lane);
+        if (waves >= nrows) break;
+        r = 0;
+        if (lane == 0) r = atomicAdd(queue, 1);
+        r = __builtin_amdgcn_readfirstlane(r) + waves;
     }
 }
 
