@@ -608,14 +608,15 @@ __global__ __launch_bounds__(kBlock) void accel_kernel(
             f[1] = st * gy;
             f[2] = st * gz;
         }
-        if (AV) {
-            f[0] = __builtin_fmaf(-II, gx, f[0]);
-            f[1] = __builtin_fmaf(-II, gy, f[1]);
-            f[2] = __builtin_fmaf(-II, gz, f[2]);
-        }
         f[0] *= mj;
         f[1] *= mj;
         f[2] *= mj;
+        if (AV) {  // the mass joins II first: II times the gradient can be below FP32's range where m II is not
+            const float mII = mj * II;
+            f[0] = __builtin_fmaf(-mII, gx, f[0]);
+            f[1] = __builtin_fmaf(-mII, gy, f[1]);
+            f[2] = __builtin_fmaf(-mII, gz, f[2]);
+        }
         if (XSPH) {  // :291-294
             const float qf = (float)sep.q, om = 1.0f - qf;
             const float w = P.Wpref * (qf < 0.5f ? __builtin_fmaf(-6.0f * qf * qf, om, 1.0f) : 2.0f * om * om * om);
