@@ -707,6 +707,9 @@ constexpr int64_t kMassCheckMin = 24576;
 // takes them as they come: Plummer 16384 66.6 -> 61.5 us per step, 50021
 // 434 -> 423)
 constexpr int64_t kMassCheckMinSym = 65536;
+// below so many particles the symmetric sweep keeps what the one-sided sweep gives:
+// unequal masses in any units, and gravity that the SPH terms join, not the reverse
+constexpr int64_t kSymOneSided = 16384;
 
 // arrays each pass needs, by configuration; 0 or a GRASPH_E_INVALID code
 int check_derivative_arrays(Ctx& c, const grasph_particles* p, uint32_t f, int which);

@@ -339,10 +339,9 @@ __device__ __forceinline__ void far_work(const float4* __restrict__ xs, const in
 // but two a row), their own-side sums leave as one fragment: a fragment per
 // wavefront was 34 MB written and read again, whatever the count (Plummer
 // N = 16384: 69.6 -> 66.6 us per step, 50021: 441 -> 434).
-// WIDE (below kWideBelow particles, down to where the one-sided sweep takes over):
+// WIDE (below kSymOneSided particles, down to where the one-sided sweep takes over):
 // unequal masses in any units, as there (unequal masses, N = 13000: 51.6 -> 53.6 us
 // a step; from 16384 on 1 / r^3 has to be in range by itself).
-constexpr int kWideBelow = 16384;
 template <bool SOFT, bool WIDE>
 __global__ __launch_bounds__(64 * kFarMerge, 2) void far_kernel(const float4* __restrict__ xs, const int n,
                                                                const int64_t nsb, const int64_t U, const int W,
@@ -877,7 +876,7 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 #define GRASPH_FAR(SOFT, WIDE)                                                                                       \
     hipLaunchKernelGGL((far_kernel<SOFT, WIDE>), dim3(far_groups), dim3(64 * kFarMerge), 0, s, L.xs, L.n, G.nsb,     \
                        G.units, L.wgs, G.split, far_fold(L.n, L.wgs), L.apart, G.plain ? 1 : 0, L.bpart, P.H2, L.umass)
-        const bool soft = P.H2 > 0.0f, wide = L.n < kWideBelow;
+        const bool soft = P.H2 > 0.0f, wide = L.n < kSymOneSided;
         if (soft && wide) GRASPH_FAR(true, true);
         else if (soft) GRASPH_FAR(true, false);
         else if (wide) GRASPH_FAR(false, true);
