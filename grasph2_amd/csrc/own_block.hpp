@@ -10,7 +10,8 @@
 // the v_rsq_f32 have to come in runs.  A wavefront copies 64 partners at a
 // time into LDS and reads them back one by one, the same for every lane; 8
 // pairs at a time go through one asm block.  Every slot meets the partners in
-// their order whatever NI is, so NI does not change a bit of the result.
+// their order whatever NI is, so with the same shares NI does not change a bit of
+// the result (own_plan chooses other shares for another NI, though).
 // Measured: Plummer steps of 1000 particles 59 -> 11 us (28 with one share
 // per slot block, 14 with the equal-mass check), of 8192 ~100 -> 31; pairs
 // inside the groups of the 512-instance ensemble 1.34 -> 1.10 ms.

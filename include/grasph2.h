@@ -162,9 +162,10 @@ int grasph_destroy(grasph_ctx* ctx);
  * particles until the next re-sort: slower, never wrong),
  * "profile" (1 = record HIP events around each kernel), "sweep_i_per_lane"
  * (particles per lane of the one-sided sweep: 2, or 1 = chosen from the
- * count, the default; the results are the same bit for bit), "sweep_slices"
- * (j-split of the sweep, 0 = automatic; past a workgroup's 8 or 16 wavefronts
- * rounded up to whole workgroups),
+ * count, the default; the j-split depends on it, so results agree to FP32
+ * rounding),
+ * "sweep_slices" (j-split of the sweep, 0 = automatic; past a workgroup's 8 or
+ * 16 wavefronts rounded up to whole workgroups),
  * "batch_waves_per_block", "batch_blocks_per_cu" (batched sweep launch
  * shape), "sweep_symmetric" (single
  * instance: 1 = gravity between groups of 1024 particles evaluated once per
