@@ -479,7 +479,8 @@ int ensure_sym(Ctx& c, BatchState& b)
 
 // The symmetric gravity sweep over the batch's larger instances, in order on
 // s (mass_done: launch_sweep_only has run the mass check).  add_acc: acc
-// holds the SPH terms, the gravity joins them.
+// holds the SPH terms, the gravity joins them; else the finishing launch or the
+// acceleration pass follows.
 int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStream_t s, bool mass_done, bool add_acc)
 {
     int r;
@@ -490,13 +491,10 @@ int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStr
     L.xs = L.perm ? b.d_xs : (const float4*)p->posm;
     L.ntotal = (int)b.ntotal;
     L.n_inst = b.n_inst;
-    L.grav = true;
-    L.finish = false;  // the finishing launch of the batch follows
     L.add_acc = add_acc;
     L.soft = all_soft(b);
     L.sinst = b.d_sinst;
     L.insts = b.d_insts;
-    L.prm = b.d_prm;
     L.blk = b.d_sblk;
     L.n_blk = b.n_sblk;
     L.blk64 = b.d_sblk + b.n_sblk;
@@ -507,9 +505,6 @@ int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStr
     L.queue = b.d_queue + 1;
     L.wgs = c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(device_cus(c));
     L.acc = (float4*)p->acc;
-    L.vel = (const float4*)p->vel;
-    L.xvel = (float4*)p->xvel;
-    L.maxvsig = p->maxvsig;
     L.near_part = b.d_snear;
     L.apart = b.d_sapart;
     L.bpart = b.d_sbpart;

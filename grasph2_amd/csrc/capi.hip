@@ -274,7 +274,6 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
     L.n = (int)p->n;
     L.acc = (float4*)p->acc;
     L.pot = c.pot;
-    L.vel = (const float4*)p->vel;
     L.xvel = (float4*)p->xvel;
     L.maxvsig = p->maxvsig;
     return L;
@@ -356,7 +355,6 @@ int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t 
     S.xs = L.xs ? L.xs : L.posm;
     S.perm = L.perm;
     S.n = L.n;
-    S.grav = L.grav;
     S.finish = L.finish;
     S.add_acc = add_acc;
     // wavefronts per 64 slots (Plummer steps at 16384: 81.3 us with 4, 77.3
@@ -365,7 +363,6 @@ int run_sym_sweep(Ctx& c, const SweepLaunch& L, const DevParams& P, hipStream_t 
     // on the same as 4 and two launches)
     S.near_waves = c.sym_near_shares > 0 ? near_waves_of(c.sym_near_shares) : L.n < 65536 ? 8 : 4;
     S.acc = L.acc;
-    S.vel = L.vel;
     S.xvel = L.xvel;
     S.maxvsig = L.maxvsig;
     S.umass = L.umass;

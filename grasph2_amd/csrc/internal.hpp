@@ -165,7 +165,6 @@ struct SweepLaunch {
     float* pot;         // written when want_pot
     bool grav, want_pot;
     bool finish;        // apply environmentAcceleration, zero xvel / maxvsig (SPH off)
-    const float4* vel;
     float4* xvel;
     float* maxvsig;
     // one-sided gravity: ni particles per lane (1, 2 or 4); `waves` wavefronts
@@ -205,15 +204,13 @@ struct SymLaunch {
     const float4* xs;   // slot-ordered positions + masses
     const int* perm;    // slot -> particle, or null
     int n;
-    bool grav;
     bool finish;        // as SweepLaunch::finish
     bool add_acc;       // acc already holds the SPH terms: the combine adds the gravity to them
     int near_waves;     // in-group gravity: wavefronts sharing 64 slots
     float4* acc;
-    const float4* vel;
     float4* xvel;
     float* maxvsig;
-    const float* umass; // {uniform, mass} (grav)
+    const float* umass; // {uniform, mass}, or null
     int wgs;            // workgroups of the far kernel
     float4* near_part;
     float4* apart;        // own-side fragments (kFragElems each)
@@ -259,11 +256,10 @@ struct SymBatchLaunch {
     const float4* xs;     // slot-ordered positions + masses of the batch
     const int* perm;      // slot -> particle, or null
     int ntotal, n_inst;
-    bool grav, finish, soft;
+    bool soft;
     bool add_acc;         // acc already holds the SPH terms: the combine adds the gravity to them
     const SymInst* sinst;
     const BatchInst* insts;
-    const DevParams* prm;
     const int4* blk;      // 256-slot and 64-slot blocks of the instances in the sweep
     int n_blk;
     const int4* blk64;
@@ -275,9 +271,6 @@ struct SymBatchLaunch {
     bool plain;           // SymBatchTables::plain
     const float* umass;   // {uniform, mass} per instance
     float4* acc;
-    const float4* vel;
-    float4* xvel;
-    float* maxvsig;
     float4* near_part;
     float4* apart;        // own-side fragments (kFragElems each)
     float* bpart;
@@ -286,7 +279,7 @@ struct SymBatchLaunch {
 hipError_t launch_sym_batch_ingroup(const SymBatchLaunch& L, hipStream_t s);
 hipError_t launch_sym_batch_far(const SymBatchLaunch& L, hipStream_t s);
 hipError_t launch_sym_batch_combine(const SymBatchLaunch& L, hipStream_t s);
-inline bool sym_batch_has_far(const SymBatchLaunch& L) { return L.ntotal > 0 && L.n_blk > 0 && L.grav && L.nrows > 0; }
+inline bool sym_batch_has_far(const SymBatchLaunch& L) { return L.ntotal > 0 && L.n_blk > 0 && L.nrows > 0; }
 
 // Neighbour lists (lists.hip): bounding boxes of every kBoxFine, kBoxMid and
 // kBoxCoarse consecutive slots of an instance, two float4 (lo, hi) each, then

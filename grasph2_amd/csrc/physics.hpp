@@ -17,7 +17,7 @@ namespace grasph {
 struct DevParams {
     uint32_t flags;
     int32_t dim;
-    float H, H2, Wpref, dWpref;
+    float H, H2, Wpref;
     float rho0, BULK, dBULKdP, c, c2, shear, Y, tanfr, cohesion, alpha;
     float mateps, matexp, normalsep, Wnorm, xsph, dt;
     float cax, cay, caz;
@@ -46,13 +46,6 @@ __host__ __device__ inline float spline_prefactor(int dim, float h)
     if (dim == 2) return 40.0f / (7.0f * float(M_PI) * h * h);
     return 8.0f / (float(M_PI) * h * h * h);
 }
-// src/sph/kernel.h:68-87
-__host__ __device__ inline float dspline_prefactor(int dim, float h)
-{
-    if (dim == 1) return 24.0f / (3.0f * h * h);
-    if (dim == 2) return 240.0f / (7.0f * float(M_PI) * h * h * h);
-    return 48.0f / (float(M_PI) * h * h * h * h);
-}
 
 // src/sph/kernel.h:130-136 (cubic B-spline, support radius h)
 __host__ __device__ inline float w_spline(float r, float h, float factor)
@@ -60,13 +53,6 @@ __host__ __device__ inline float w_spline(float r, float h, float factor)
     const float q = r / h;
     return factor * ((q <= 1.0f) ? ((q < 0.5f) ? (6.0f * q * q * q - 6.0f * q * q + 1.0f)
                                                : 2.0f * (1.0f - q) * (1.0f - q) * (1.0f - q))
-                                 : 0.0f);
-}
-// src/sph/kernel.h:169-175
-__host__ __device__ inline float dw_spline(float r, float h, float factor)
-{
-    const float q = r / h;
-    return factor * ((q <= 1.0f) ? ((q < 0.5f) ? (3.0f * q * q - 2.0f * q) : -1.0f * (1.0f - q) * (1.0f - q))
                                  : 0.0f);
 }
 
@@ -170,15 +156,7 @@ struct CSum {
     __device__ inline float value() const { return s + c; }
 };
 
-// src/sph/models.h:187-192
-__device__ inline float balsara_switch(float divv, float cx, float cy, float cz, float c, float h)
-{
-    const float absdiv = fabsf(divv);
-    const float abscurl = sqrtf(cx * cx + cy * cy + cz * cz);
-    return absdiv / (absdiv + abscurl + 0.0001f * c / h);
-}
-
-// the same from FP64 sums, rounded once
+// src/sph/models.h:187-192 from FP64 sums, rounded once
 __device__ inline float balsara_switch_f64(double divv, double cx, double cy, double cz, float c, float h)
 {
     const double absdiv = fabs(divv);
@@ -214,7 +192,6 @@ __host__ inline DevParams make_dev_params(const grasph_params* p)
     d.H = p->H;
     d.H2 = p->H * p->H;
     d.Wpref = spline_prefactor(d.dim, d.H);
-    d.dWpref = dspline_prefactor(d.dim, d.H);
     d.rho0 = p->rho0; d.BULK = p->BULK; d.dBULKdP = p->dBULKdP;
     d.c = p->SOUNDSPEED; d.c2 = p->SOUNDSPEED * p->SOUNDSPEED;
     d.shear = p->shear; d.Y = p->Y; d.tanfr = p->tanfr; d.cohesion = p->cohesion; d.alpha = p->alpha;
@@ -233,6 +210,7 @@ __host__ inline DevParams make_dev_params(const grasph_params* p)
     const double h = p->H;
     d.invH64 = h > 0.0 ? 1.0 / h : 0.0;
     d.Wpref64 = d.dim == 1 ? 4.0 / (3.0 * h) : d.dim == 2 ? 40.0 / (7.0 * M_PI * h * h) : 8.0 / (M_PI * h * h * h);
+    // src/sph/kernel.h:68-87
     const double dW = d.dim == 1 ? 24.0 / (3.0 * h * h) : d.dim == 2 ? 240.0 / (7.0 * M_PI * h * h * h)
                                                                      : 48.0 / (M_PI * h * h * h * h);
     d.Wi64 = -6.0 * d.Wpref64;

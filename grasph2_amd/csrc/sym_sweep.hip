@@ -512,7 +512,7 @@ __device__ __forceinline__ void finish_slot(const int t, CSum x, CSum y, CSum z,
 template <int PARTS, bool PLAIN>
 __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
-    const int n, const int64_t nsb, const int64_t U, const int W, const int Q, const int grav,
+    const int n, const int64_t nsb, const int64_t U, const int W, const int Q,
     const int* __restrict__ perm, float4* __restrict__ acc, const int finish, const int add_acc,
     float4* __restrict__ xvel, float* __restrict__ maxvsig, const DevParams P)
 {
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
     const int p = (int)threadIdx.x / kSlots;
     const int t = blockIdx.x * kSlots + ((int)threadIdx.x - p * kSlots);
     CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
-    if (grav && t < n) {
+    if (t < n) {
         if (p == 0) {
             const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
             x = CSum{a.x, c.x}; y = CSum{a.y, c.y}; z = CSum{a.z, c.z};
@@ -534,7 +534,8 @@ __global__ __launch_bounds__(kBlock) void sym_combine_kernel(
 // In-group gravity and combine in one launch, for counts at which either
 // takes as long as its launch: a workgroup of kNearFused wavefronts makes 64
 // slots' in-group sums as ingroup_kernel does, then wavefront p is their part
-// p of the combine.  The sums are the two kernels' bit for bit.  Plummer N =
+// p of the combine.  The in-group sums are the two kernels'
+// bit for bit; the combine has 8 parts whatever the count.  Plummer N =
 // 16384: 61.5 -> 59.4 us per step.
 constexpr int kNearFused = 8;
 template <bool SOFT>
@@ -641,10 +642,10 @@ __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
 // ------------------------------------------------------------------ batches
 // The same sweep over the larger instances of a batch (slot indices are
 // the batch's; the smaller instances stay with the one-sided persistent
-// sweep).  Differences: no shares in the near field (the batch has
-// wavefronts to spare); the far kernel is persistent and takes whole rows
-// (instance, group) from a counter, longest first, so each row's own-side
-// sums leave as one fragment, numbered by the instance's first row + g.
+// sweep).  Differences: four wavefronts share the in-group gravity of a block
+// of slots; the far kernel is persistent and takes rows (instance, group), cut
+// into kBatchPieces pieces at most, longest first; each piece's own-side sums
+// leave as a fragment, numbered by the instance's first row + g and the piece.
 
 // NI 4: blk has blocks of 256 slots, NI 1: of 64.
 template <int NI, bool SOFT>
@@ -715,15 +716,13 @@ __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
 }
 
 // Per slot of the instances in the sweep (256-slot block table), as
-// sym_combine_kernel: near partial, the row's one own-side fragment, the
+// sym_combine_kernel: near partial, the row's pieces' own-side fragments, the
 // partner-side partials (group order, negated).
 template <bool PLAIN>
 __global__ __launch_bounds__(kBlock) void sym_batch_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
-    const SymInst* __restrict__ sinst, const int4* __restrict__ blk, const int grav, const int* __restrict__ perm,
-    const float4* __restrict__ xs, float4* __restrict__ acc, const int finish, const int add_acc,
-    const float4* __restrict__ vel, float4* __restrict__ xvel, float* __restrict__ maxvsig,
-    const DevParams* __restrict__ prm)
+    const SymInst* __restrict__ sinst, const int4* __restrict__ blk, const int* __restrict__ perm,
+    float4* __restrict__ acc, const int add_acc)
 {
     const int4 bl = blk[blockIdx.x];
     const int t = bl.y + threadIdx.x;
@@ -731,56 +730,48 @@ __global__ __launch_bounds__(kBlock) void sym_batch_combine_kernel(
     const int k = bl.x;
     const SymInst S = sinst[k];
     CSum x{0.0f, 0.0f}, y{0.0f, 0.0f}, z{0.0f, 0.0f};
-    if (grav) {
-        const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
-        x.add(a.x); y.add(a.y); z.add(a.z);
-        x.c += c.x; y.c += c.y; z.c += c.z;
-        const int local = t - S.off;
-        const int g = local / kGroup, lg = local - g * kGroup;
-        if (g < S.nrows) {
-            const int pieces = batch_row_pieces(row_units(g, S.nsb));
-            for (int h = 0; h < pieces; ++h) {
-                const float4* fr = apart + (size_t)kFragElems * ((size_t)kBatchPieces * (S.row0 + g) + h) + frag_elem(lg);
-                const float4 f = fr[0];
-                x.add(f.x); y.add(f.y); z.add(f.z);
-                if (!PLAIN) {
-                    const float4 fc = fr[64];
-                    x.c += fc.x; y.c += fc.y; z.c += fc.z;
-                }
+    const float4 a = near_part[2 * (size_t)t], c = near_part[2 * (size_t)t + 1];
+    x.add(a.x); y.add(a.y); z.add(a.z);
+    x.c += c.x; y.c += c.y; z.c += c.z;
+    const int local = t - S.off;
+    const int g = local / kGroup, lg = local - g * kGroup;
+    if (g < S.nrows) {
+        const int pieces = batch_row_pieces(row_units(g, S.nsb));
+        for (int h = 0; h < pieces; ++h) {
+            const float4* fr = apart + (size_t)kFragElems * ((size_t)kBatchPieces * (S.row0 + g) + h) + frag_elem(lg);
+            const float4 f = fr[0];
+            x.add(f.x); y.add(f.y); z.add(f.z);
+            if (!PLAIN) {
+                const float4 fc = fr[64];
+                x.c += fc.x; y.c += fc.y; z.c += fc.z;
             }
         }
-        const float* bk = bpart + S.bpart0;
-        const int64_t base = bpart_group_base(g) + lg;
-        int gp = 0;  // eight groups' loads in flight before their (ordered) adds
-        for (; gp + 8 <= g; gp += 8) {
-            float v[8][3];
+    }
+    const float* bk = bpart + S.bpart0;
+    const int64_t base = bpart_group_base(g) + lg;
+    int gp = 0;  // eight groups' loads in flight before their (ordered) adds
+    for (; gp + 8 <= g; gp += 8) {
+        float v[8][3];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const size_t e = 3 * (size_t)(base + (int64_t)(gp + u) * kGroup);
-                v[u][0] = bk[e]; v[u][1] = bk[e + 1]; v[u][2] = bk[e + 2];
-            }
+        for (int u = 0; u < 8; ++u) {
+            const size_t e = 3 * (size_t)(base + (int64_t)(gp + u) * kGroup);
+            v[u][0] = bk[e]; v[u][1] = bk[e + 1]; v[u][2] = bk[e + 2];
+        }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
-            }
+        for (int u = 0; u < 8; ++u) {
+            x.add(-v[u][0]); y.add(-v[u][1]); z.add(-v[u][2]);
         }
-        for (; gp < g; ++gp) {
-            const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
-            x.add(-bk[e]); y.add(-bk[e + 1]); z.add(-bk[e + 2]);
-        }
+    }
+    for (; gp < g; ++gp) {
+        const size_t e = 3 * (size_t)(base + (int64_t)gp * kGroup);
+        x.add(-bk[e]); y.add(-bk[e + 1]); z.add(-bk[e + 2]);
     }
     const int i = perm ? perm[t] : t;
     if (add_acc) {  // the SPH terms (and environment), summed before the far field was done
         const float4 a = acc[i];
         x.add(a.x); y.add(a.y); z.add(a.z);
     }
-    float ax = x.value(), ay = y.value(), az = z.value();
-    if (finish) {
-        environment_acceleration(prm[k], ax, ay, az);
-        if (xvel) xvel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (maxvsig) maxvsig[i] = 0.0f;
-    }
-    acc[i] = make_float4(ax, ay, az, 0.0f);
+    acc[i] = make_float4(x.value(), y.value(), z.value(), 0.0f);
 }
 
 }  // namespace
@@ -834,7 +825,7 @@ SymGeom sym_geometry(int64_t n, int wgs, int64_t col_elems)
 // gravity inside the groups
 hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
-    if (L.n <= 0 || !L.grav) return hipSuccess;
+    if (L.n <= 0) return hipSuccess;
     const int w = L.near_waves;  // a power of two: the shares cover the group exactly
     if (w < 1 || w > kOwnMaxWaves || (w & (w - 1))) return hipErrorInvalidValue;
     const dim3 grid((L.n + 63) / 64), block(64 * w);
@@ -846,7 +837,7 @@ hipError_t launch_sym_ingroup(const SymLaunch& L, const DevParams& P, hipStream_
     return hipGetLastError();
 }
 
-bool sym_has_far(const SymLaunch& L) { return L.n > 0 && L.grav && sym_geometry(L.n, L.wgs).units > 0; }
+bool sym_has_far(const SymLaunch& L) { return L.n > 0 && sym_geometry(L.n, L.wgs).units > 0; }
 
 template <bool SOFT>
 void launch_far_column(const SymLaunch& L, const SymCol& C, const int split, const DevParams& P, hipStream_t s)
@@ -896,7 +887,7 @@ hipError_t launch_sym_far(const SymLaunch& L, const DevParams& P, hipStream_t s)
 // both of the next two in one launch, where that is the faster way
 bool sym_fused(const SymLaunch& L)
 {
-    if (L.n <= 0 || !L.grav || L.near_waves != kNearFused) return false;
+    if (L.n <= 0 || L.near_waves != kNearFused) return false;
     const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     return G.ncols == 1 && G.plain;
 }
@@ -915,7 +906,7 @@ hipError_t launch_sym_near_combine(const SymLaunch& L, const DevParams& P, hipSt
 // combine (after both fields): the acceleration
 hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_t s)
 {
-    if (L.n <= 0 || !(L.grav || L.finish)) return hipSuccess;
+    if (L.n <= 0) return hipSuccess;
     const SymGeom G = sym_geometry(L.n, L.wgs, L.col_elems);
     if (G.ncols > 1 && sym_has_far(L)) {
         // the last column batch's combine, which finishes
@@ -924,12 +915,13 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
         launch_column_combine(L, C, G.split, false, true, P, s);
         return hipGetLastError();
     }
-    // threads per slot: about 2^17 threads or more in all
+    // threads per slot: about 2^17 threads or more in all (below 65536 particles the fused launch takes the
+    // combine, unless option sym_near_shares asks for another in-group shape)
     const int parts = L.n >= 98304 ? 1 : L.n >= 49152 ? 2 : L.n >= 24576 ? 4 : 8;
 #define GRASPH_COMBINE(PARTS, PLAIN)                                                                                  \
     hipLaunchKernelGGL((sym_combine_kernel<PARTS, PLAIN>), dim3((L.n + kBlock / PARTS - 1) / (kBlock / PARTS)),        \
                        dim3(kBlock), 0, s, L.near_part, L.apart, L.bpart, L.n, G.nsb, G.units, L.wgs,       \
-                       G.split, L.grav ? 1 : 0, L.perm, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0,        \
+                       G.split, L.perm, L.acc, L.finish ? 1 : 0, L.add_acc ? 1 : 0,        \
                        L.xvel, L.maxvsig, P)
     if (G.plain) {
         switch (parts) {
@@ -990,7 +982,7 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
 constexpr int kNearBlocksMin = 512;
 hipError_t launch_sym_batch_ingroup(const SymBatchLaunch& L, hipStream_t s)
 {
-    if (L.ntotal <= 0 || L.n_blk <= 0 || !L.grav) return hipSuccess;
+    if (L.ntotal <= 0 || L.n_blk <= 0) return hipSuccess;
     const bool small = L.n_blk < kNearBlocksMin || 9 * (int64_t)L.n_blk64 < 32 * (int64_t)L.n_blk;
 #define GRASPH_NEAR(NI, SOFT, N, BLK)                                                                                \
     hipLaunchKernelGGL((sym_batch_ingroup_kernel<NI, SOFT>), dim3(N), dim3(kBlock), 0, s, L.xs, BLK, L.sinst, L.insts, \
@@ -1019,15 +1011,13 @@ hipError_t launch_sym_batch_far(const SymBatchLaunch& L, hipStream_t s)
 
 hipError_t launch_sym_batch_combine(const SymBatchLaunch& L, hipStream_t s)
 {
-    if (L.ntotal <= 0 || L.n_blk <= 0 || !(L.grav || L.finish)) return hipSuccess;
+    if (L.ntotal <= 0 || L.n_blk <= 0) return hipSuccess;
     if (L.plain)
         hipLaunchKernelGGL(sym_batch_combine_kernel<true>, dim3(L.n_blk), dim3(kBlock), 0, s, L.near_part, L.apart,
-                           L.bpart, L.sinst, L.blk, L.grav ? 1 : 0, L.perm, L.xs, L.acc, L.finish ? 1 : 0,
-                           L.add_acc ? 1 : 0, L.vel, L.xvel, L.maxvsig, L.prm);
+                           L.bpart, L.sinst, L.blk, L.perm, L.acc, L.add_acc ? 1 : 0);
     else
         hipLaunchKernelGGL(sym_batch_combine_kernel<false>, dim3(L.n_blk), dim3(kBlock), 0, s, L.near_part, L.apart,
-                           L.bpart, L.sinst, L.blk, L.grav ? 1 : 0, L.perm, L.xs, L.acc, L.finish ? 1 : 0,
-                           L.add_acc ? 1 : 0, L.vel, L.xvel, L.maxvsig, L.prm);
+                           L.bpart, L.sinst, L.blk, L.perm, L.acc, L.add_acc ? 1 : 0);
     return hipGetLastError();
 }
 
