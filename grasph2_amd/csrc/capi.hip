@@ -281,12 +281,13 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
 
 // Lanes per particle of the passes: 16 while the particles' 4 would leave the
 // GPU's SIMDs idle, 4 from there (16 lanes walk short lists in few, partly
-// empty steps).  Passes called one by one / SPH without gravity, 16 against 4
-// lanes: 4096 particles 119 against 139 us / 47 against 57, 8192 144 against
-// 159 / 54 against 59, 11000 198 against 209 / 63 against 59, 16384 213
-// against 222 / 64 against 60.  And 16 where the lists have grown long
-// (kLongLists): 65536 squeezed particles 1151 against 1181 us.
-constexpr int64_t kPassLanes16Max = 10240;
+// empty steps).  Passes called one by one on bodies in contact / a liquid without
+// gravity, 16 against 4 lanes: 4096 particles 79 against 99 us / 27 against 36,
+// 8192 81 against 97 / 33 against 40, 16384 107 against 120 / 39 against 42, 24000
+// 123 against 127 / 46 against 48, 30000 126 against 125 / 56 against 53.  And 16
+// where the lists have grown long (kLongLists): 65537 squeezed particles 1115
+// against 1211 us.
+constexpr int64_t kPassLanes16Max = 24576;
 int pass_lanes(int64_t n, int kmax) { return n <= kPassLanes16Max || kmax > kLongLists ? 16 : 4; }
 
 NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)

@@ -11,16 +11,25 @@
 
 namespace grasph {
 
-// Neighbour lists come in tiles of 64 slots: entry k of slot t lies at
-// list_entry(t, k, kmax) of its plane, so a wavefront's k-th entries are one
-// 256-byte line and a wavefront's whole list is contiguous (a plane laid out
-// as [k][slot] puts each entry of a long list in another part of a
-// gigabyte-sized array, and the page-table walks made merging and walking
-// long lists several times slower).  A plane holds list_plane(n, kmax)
-// entries.
+// Neighbour lists come in tiles of 64 slots, contiguous (as planes [k][slot]
+// each entry of a long list lay in another part of a gigabyte-sized array, and
+// the page-table walks made walking them several times slower); in a tile four
+// entries of a slot side by side, then the next slot's four, then all slots'
+// next four (single entries if kmax is no multiple of 4): entry k of slot t lies
+// at list_entry(t, k, kmax).  So a 128-byte line holds four entries of 8 slots, which
+// is what one wavefront of the list kernel fills within a few steps, and 4 lanes
+// of a pass read a slot's next four together.  With a row of 64 slots per entry
+// the lines left the L2 half written: collision after impact (1e8 neighbours,
+// 131072 particles) lists 0.85 ms, now 0.36, passes 0.42 + 0.65 + 0.75, now 0.30 +
+// 0.54 + 0.61; 65537 squeezed particles 1229 -> 1115 us, SPH without gravity at
+// 100000 149 -> 142.  A plane holds list_plane(n, kmax) entries.
+__host__ __device__ inline int list_chunk(int kmax) { return kmax % 4 ? 1 : 4; }
+__host__ __device__ inline uint32_t list_mask(int kmax) { return ~(uint32_t)(list_chunk(kmax) - 1); }
+// of entry k from the list's entry 0; increases with k
+__host__ __device__ inline uint32_t list_offset(uint32_t k, uint32_t mask) { return k + 63u * (k & mask); }
 __host__ __device__ inline size_t list_entry(int t, int k, int kmax)
 {
-    return ((size_t)(t >> 6) * (size_t)kmax + (size_t)k) * 64 + (size_t)(t & 63);
+    return (size_t)(t >> 6) * (size_t)kmax * 64 + (size_t)(t & 63) * (size_t)list_chunk(kmax) + list_offset(k, list_mask(kmax));
 }
 __host__ __device__ inline size_t list_plane(int64_t n, int kmax) { return (size_t)((n + 63) / 64) * 64 * (size_t)kmax; }
 
@@ -372,13 +381,13 @@ __device__ inline int xcd_runs(int b, int nb, int c)
 // Whole eighths then leave most of the work to an XCD or two, and 4 lanes per
 // particle wait for the longest list of 16: the passes take runs of kXcdRun
 // slots and 16 lanes.  131072 particles after impact (1e8 neighbours, up to
-// 3021 each), density, strain and acceleration: 0.55 + 0.95 + 1.09 ms before,
-// 0.45 + 0.67 + 0.79 with runs of 2048, 0.42 + 0.65 + 0.76 with 4096, 0.47 +
-// 0.70 + 0.83 with 8192 (5.77 ms a step before, 5.0 with 4096, 5.13 with 8192).
-// Runs read more halo than eighths: evenly squeezed spheres, whose eighths hold
-// the same work, lose by them (131072 particles 3423 against 3524 us, 90000
-// 1738 against 1789, 65536 1160 against 1229: an eighth there is 8192 slots and
-// stays), and with short lists 200003 particles 274 against 278.
+// 3021 each), density, strain and acceleration: 0.40 + 0.79 + 0.92 ms with 4 lanes and
+// runs, 0.37 + 0.67 + 0.78 with 16 and whole eighths, 0.30 + 0.54 + 0.61 with both (a
+// step 4.90, 4.48 and 4.13 ms).  Runs read more halo than eighths: evenly squeezed
+// spheres, whose eighths hold the same work, lose by them (131072 particles 3094
+// against 3193 us, 90000 1678 against 1754, 65537 1058 against 1115; to 65536 an
+// eighth is 8192 slots at most and stays), and with short lists 200003 particles
+// 274 against 278.
 constexpr int kLongLists = 512, kXcdRun = 4096, kXcdRunMin = 65536;
 __device__ inline int xcd_run(int n, int kmax) { return kmax > kLongLists && n > kXcdRunMin ? kXcdRun : 0; }
 

@@ -27,9 +27,9 @@
 // most of the tests of boxes of 8 (12 to 16 boxes of 512 are near, with 64 of
 // 8 each), and with lists short enough for 8 wavefronts per SIMD took SPH
 // steps without gravity at 200003 particles from 283 to 275 us, default solids
-// at 16384 from 103 to 99, three single passes at 20011 from 221 to 212.  The
-// stores (4 bytes, each to a line of its own) do not bound it: collected in
-// LDS and written side by side, the same steps took 277 to 286, 103 and 226.
+// at 16384 from 103 to 99, three single passes at 20011 from 221 to 212.  A
+// wavefront's stores fill lines of its own (list_entry): where lists are long they
+// decide (internal.hpp).
 #include "internal.hpp"
 
 namespace grasph {
@@ -193,8 +193,9 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
     };
     // entry k of this lane's slot, in bytes from the wavefront's first tile of
     // the lists (which its 8 slots may leave, in a batch)
-    char* const lists = reinterpret_cast<char*>(nbr + list_entry(off + first, 0, kmax) - ((off + first) & 63));
-    const uint32_t column = 4u * (uint32_t)(((off + t) >> 6 != (off + first) >> 6 ? kmax * 64 : 0) + ((off + t) & 63));
+    char* const lists = reinterpret_cast<char*>(nbr + list_entry((off + first) & ~63, 0, kmax));
+    const uint32_t column = 4u * (uint32_t)(((off + t) >> 6 != (off + first) >> 6 ? kmax * 64 : 0) + ((off + t) & 63) * list_chunk(kmax));
+    const uint32_t mask = list_mask(kmax);
     const uint32_t bit = 1u << j, below = bit - 1u;
     const int shift = 8 * (i & 3);
     const float4* const xj = xs + off;
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const float4* __rest
             const uint32_t half = lane < 32 ? (uint32_t)hits : (uint32_t)(hits >> 32);
             const uint32_t mine = (half >> shift) & 0xffu;
             const int k = cnt + __builtin_popcount(mine & below);
-            if (hit && k < kmax) *reinterpret_cast<int*>(lists + (column + 256u * (uint32_t)k)) = __float_as_int(q.w);
+            if (hit && k < kmax) *reinterpret_cast<int*>(lists + (column + 4u * list_offset((uint32_t)k, mask))) = __float_as_int(q.w);
             cnt += __builtin_popcount(mine);
         }
         wave_lds_order();

@@ -256,8 +256,10 @@ __device__ __forceinline__ void for_each_neighbour(const vec4* __restrict__ src,
     // list's last entry (a lane without a list walks entry 0 of slot t's
     // overflowed one, or reads slot 0 from a count of 0)
     const int* list = cnt > 0 ? Ls.nbr + list_entry(t, 0, kmax) : Ls.cnt + t;
-    const int last = max(c - 1, 0);
-    const auto index = [&](int e) GRASPH_INLINE { return list[64 * (uint64_t)(uint32_t)min(e * LPP + sub, last)]; };
+    const uint32_t mask = list_mask(kmax), lane0 = list_offset((uint32_t)sub, mask);
+    const uint32_t last = list_offset((uint32_t)max(c - 1, 0), mask);
+    static_assert(LPP % 4 == 0);  // a step's entries begin a chunk
+    const auto index = [&](int e) GRASPH_INLINE { return list[min((uint32_t)(64 * LPP * e) + lane0, last)]; };
     const auto fetch = [&](int j, vec4 (&r)[PIECES]) GRASPH_INLINE {
 #pragma unroll
         for (int q = 0; q < PIECES; ++q) r[q] = src[STRIDE * (uint64_t)(uint32_t)j + q];

@@ -13,7 +13,7 @@ from tests._util import vec_errors
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [300, 11000])  # 16 and 4 lanes per particle
+@pytest.mark.parametrize("n", [300, 25000])  # 16 and 4 lanes per particle
 @pytest.mark.parametrize("rho,mass,speed", [(1.5e38, 1e20, 1e9), (1.0, 1e-3, 1.0), (2.0e-39, 1e-38, 1.0)])
 def test_mean_density(n, rho, mass, speed):
     print("density range n=%d rho=%g" % (n, rho), flush=True)

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kind", ["solid", "xsph"])
 @pytest.mark.parametrize("n,reach", [(3, 4.0), (6, 4.0), (18, 4.0), (40, 1.0), (65, 0.6), (65, 4.0), (513, 0.5), (577, 1.0),
-                                     (1100, 1.3), (10300, 0.7)])
+                                     (1100, 1.3), (25000, 0.8)])
 def test_scan_equals_list(kind, n, reach):
     print("scan kind=%s n=%d reach=%g" % (kind, n, reach), flush=True)
     h, prm = workload(kind, n)

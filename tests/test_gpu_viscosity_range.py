@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("solid", [False, True])
-@pytest.mark.parametrize("n", [300, 11000])  # 16 and 4 lanes per particle
+@pytest.mark.parametrize("n", [300, 25000])  # 16 and 4 lanes per particle
 def test_slow_flow_of_large_bodies(n, solid):
     print("viscosity range n=%d solid=%s" % (n, solid), flush=True)
     rng = np.random.default_rng(n)
