@@ -281,13 +281,14 @@ SweepLaunch sweep_base(Ctx& c, const grasph_particles* p)
 
 // Lanes per particle of the passes: 16 while the particles' 4 would leave the
 // GPU's SIMDs idle, 4 from there (16 lanes walk short lists in few, partly
-// empty steps).  Passes called one by one on bodies in contact / a liquid without
-// gravity, 16 against 4 lanes: 4096 particles 79 against 99 us / 27 against 36,
-// 8192 81 against 97 / 33 against 40, 16384 107 against 120 / 39 against 42, 24000
-// 123 against 127 / 46 against 48, 30000 126 against 125 / 56 against 53.  And 16
-// where the lists have grown long (kLongLists): 65537 squeezed particles 1115
-// against 1211 us.
-constexpr int64_t kPassLanes16Max = 24576;
+// empty steps).  Passes called one by one on bodies in contact / these without
+// gravity / a step of default solids (16 neighbours each), 16 against 4 lanes: 4096
+// particles 86 against 107 us / 43 against 64 / 45 against 45, 10000 132 against 148
+// / 54 against 69 / 81 against 78, 16384 164 against 178 / 60 against 72 / 103
+// against 98, 24000 229 against 235 / 70 against 75 / 167 against 159: from the line
+// on what short lists lose weighs as much as what longer ones gain.  And 16 where
+// the lists have grown long (kLongLists): 65537 squeezed particles 1115 against 1211 us.
+constexpr int64_t kPassLanes16Max = 10240;
 int pass_lanes(int64_t n, int kmax) { return n <= kPassLanes16Max || kmax > kLongLists ? 16 : 4; }
 
 NbrLaunch nbr_base(Ctx& c, const grasph_particles* p)
