@@ -49,7 +49,7 @@ constexpr int kBlock = 256, kWaves = kBlock / 64;
 // lanes, with 16 one): what hides their latency is wavefronts, and a deeper
 // ring costs them registers.  All three passes at 200003 particles: 238 us
 // with 4, 2 and 2 steps and the terms added in the order of all neighbours
-// (48, 101, 89), now 32, 70 and 90.
+// (48, 101, 89), now 29, 65 and 83.
 constexpr int kDeepDensity = 2, kDeepStrain = 2, kDeepAccel = 1;
 
 // lambdas are inlined by force: called from the list walk and the overflow
@@ -130,8 +130,8 @@ __device__ __forceinline__ void acc_merge(CSum& a, const float s, const float c)
 // NC sums of a particle (A: the accumulator of terms of type T) by classes of
 // neighbours.  With 4 lanes each lane is a class and keeps its own sums (with
 // the terms exchanged through LDS and added by all neighbours' order, the
-// exchange took density and strain at 200003 particles 38 and 74 us, now 32
-// and 70).  With
+// exchange took density and strain at 200003 particles 38 and 74 us, without
+// it 32 and 70).  With
 // 16 the four lanes of a class write their terms to LDS, side by side, a row
 // per quantity (kRow apart, so the rows start in different banks), and lane
 // 4 q + r adds those of class r of the quantities q, q + 4, ....

@@ -36,7 +36,7 @@ def own_sums(n, masses):
 @pytest.mark.parametrize("n", [5 * 1024, 11 * 1024, 16 * 1024])  # a wavefront has 16, 32 and 64 partners
 def test_merged_wavefronts_lose_nothing(n):
     """Integer masses of 18 bits: a wavefront's sum (at most 64 of them) is
-    exact, four wavefronts' need up to 26 bits, and the whole one, an odd
+    exact, eight wavefronts' need up to 27 bits, and the whole one, an odd
     number just below the middle between two floats, has to round down."""
     print("far merge n=%d" % n, flush=True)
     m = np.random.default_rng(n).integers(1 << 17, 1 << 18, size=1024)
