@@ -60,6 +60,7 @@ struct BatchState {
     int n_sblk = 0, n_sblk64 = 0;
     int64_t sym_min = -1;    // the size threshold the tables were built with (-1: none)
     bool sym_plain = true;  // SymBatchTables::plain
+    int sym_most = 0;       // SymBatchTables::most
     float4* d_snear = nullptr;
     float4* d_sapart = nullptr;
     float* d_sbpart = nullptr;
@@ -448,7 +449,7 @@ int launch_sweep_only(Ctx& c, BatchState& b, const grasph_particles* p, hipStrea
 int ensure_sym(Ctx& c, BatchState& b)
 {
     if (b.d_sinst && b.sym_min == c.batch_symmetric_min) return 0;
-    SymBatchTables T = sym_batch_tables(b.offsets, c.batch_symmetric_min);
+    SymBatchTables T = sym_batch_tables(b.offsets, c.batch_symmetric_min, sym_default_workgroups(device_cus(c)));
     int r;
     b.n_sblk = (int)T.blk.size();
     b.n_sblk64 = (int)T.blk64.size();
@@ -462,6 +463,7 @@ int ensure_sym(Ctx& c, BatchState& b)
     b.n_srows = (int)T.rows.size();
     b.sym_min = c.batch_symmetric_min;
     b.sym_plain = T.plain;
+    b.sym_most = T.most;
     // fresh arrays for the new tables (upload()-style: free, then allocate)
     void* old[] = {b.d_snear, b.d_sapart, b.d_sbpart};
     for (void* q : old) free_ptr(q);
@@ -502,6 +504,7 @@ int run_sym_sweep_batch(Ctx& c, BatchState& b, const grasph_particles* p, hipStr
     L.rows = b.d_srows;
     L.nrows = b.n_srows;
     L.plain = b.sym_plain;
+    L.most = b.sym_most;
     L.queue = b.d_queue + 1;
     L.wgs = c.sym_workgroups > 0 ? c.sym_workgroups : sym_default_workgroups(device_cus(c));
     L.acc = (float4*)p->acc;

@@ -257,10 +257,11 @@ struct SymBatchTables {
     std::vector<SymRow> rows;    // longest first
     std::vector<int4> blk, blk64;  // 256-slot and 64-slot blocks (instance, first, end) of the instances in the sweep
     int64_t apart_elems = 0, bpart_elems = 0;
+    int most = 4;       // pieces of a row at most (kBatchPieces to kBatchPiecesMost)
     bool plain = true;  // no row piece flushes its fragment twice
 };
-// instances of at least min_n particles take the symmetric sweep
-SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n);
+// instances of at least min_n particles take the symmetric sweep; wgs: wavefronts of the far field that run at once
+SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n, int64_t wgs);
 struct SymBatchLaunch {
     const float4* xs;     // slot-ordered positions + masses of the batch
     const int* perm;      // slot -> particle, or null
@@ -275,6 +276,7 @@ struct SymBatchLaunch {
     int n_blk64;
     const SymRow* rows;
     int nrows;
+    int most;             // SymBatchTables::most
     int* queue;           // one work counter
     int wgs;
     bool plain;           // SymBatchTables::plain

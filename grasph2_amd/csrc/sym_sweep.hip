@@ -644,7 +644,7 @@ __global__ __launch_bounds__(kBlock) void sym_column_combine_kernel(
 // the batch's; the smaller instances stay with the one-sided persistent
 // sweep).  Differences: four wavefronts share the in-group gravity of a block
 // of slots; the far kernel is persistent and takes rows (instance, group), cut
-// into kBatchPieces pieces at most, longest first; each piece's own-side sums
+// into kBatchPieces or a few more pieces, longest first; each piece's own-side sums
 // leave as a fragment, numbered by the instance's first row + g and the piece.
 
 // NI 4: blk has blocks of 256 slots, NI 1: of 64.
@@ -687,8 +687,8 @@ __device__ __forceinline__ void batch_far_row(const float4* __restrict__ xk, con
 template <bool SOFT>
 __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
     const float4* __restrict__ xs, const SymInst* __restrict__ sinst, const BatchInst* __restrict__ insts,
-    const SymRow* __restrict__ rows, const int nrows, int* __restrict__ queue, float4* __restrict__ apart,
-    const int plain, float* __restrict__ bpart, const float* __restrict__ umass)
+    const SymRow* __restrict__ rows, const int nrows, const int most, int* __restrict__ queue,
+    float4* __restrict__ apart, const int plain, float* __restrict__ bpart, const float* __restrict__ umass)
 {
     __shared__ float lsum[3 * kGroup];
     const int lane = threadIdx.x;
@@ -702,8 +702,8 @@ __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
         float* const bk = bpart + S.bpart0;
         const bool um = umass[2 * R.inst] != 0.0f;
         const float m = umass[2 * R.inst + 1];
-        const int j0 = R.g + 1 + (int)batch_piece_begin(row_units(R.g, S.nsb), R.piece);
-        float4* const frag = apart + (size_t)kFragElems * ((size_t)kBatchPieces * (S.row0 + R.g) + R.piece);
+        const int j0 = R.g + 1 + (int)batch_piece_begin(row_units(R.g, S.nsb), R.piece, most);
+        float4* const frag = apart + (size_t)kFragElems * ((size_t)most * (S.row0 + R.g) + R.piece);
         if (um)
             batch_far_row<true, SOFT>(xk, S.n, R, j0, lsum, frag, plain, bk, H2, m, lane);
         else
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(kFarThreads, 2) void sym_batch_far_kernel(
 template <bool PLAIN>
 __global__ __launch_bounds__(kBlock) void sym_batch_combine_kernel(
     const float4* __restrict__ near_part, const float4* __restrict__ apart, const float* __restrict__ bpart,
-    const SymInst* __restrict__ sinst, const int4* __restrict__ blk, const int* __restrict__ perm,
+    const SymInst* __restrict__ sinst, const int4* __restrict__ blk, const int most, const int* __restrict__ perm,
     float4* __restrict__ acc, const int add_acc)
 {
     const int4 bl = blk[blockIdx.x];
@@ -736,9 +736,9 @@ __global__ __launch_bounds__(kBlock) void sym_batch_combine_kernel(
     const int local = t - S.off;
     const int g = local / kGroup, lg = local - g * kGroup;
     if (g < S.nrows) {
-        const int pieces = batch_row_pieces(row_units(g, S.nsb));
+        const int pieces = batch_row_pieces(row_units(g, S.nsb), most);
         for (int h = 0; h < pieces; ++h) {
-            const float4* fr = apart + (size_t)kFragElems * ((size_t)kBatchPieces * (S.row0 + g) + h) + frag_elem(lg);
+            const float4* fr = apart + (size_t)kFragElems * ((size_t)most * (S.row0 + g) + h) + frag_elem(lg);
             const float4 f = fr[0];
             x.add(f.x); y.add(f.y); z.add(f.z);
             if (!PLAIN) {
@@ -937,10 +937,19 @@ hipError_t launch_sym_combine(const SymLaunch& L, const DevParams& P, hipStream_
     return hipGetLastError();
 }
 
-SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n)
+SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min_n, int64_t wgs)
 {
     SymBatchTables T;
     const int n_inst = (int)offsets.size() - 1;
+    const auto pieces = [&](int most) {
+        int64_t count = 0;
+        for (int k = 0; k < n_inst; ++k) {
+            const int64_t n = offsets[k + 1] - offsets[k], nsb = n >= min_n ? (n + kSB - 1) / kSB : 0;
+            for (int64_t g = 0; g < rows_with_units(nsb); ++g) count += batch_row_pieces(row_units(g, nsb), most);
+        }
+        return count;
+    };
+    while (T.most < kBatchPiecesMost && pieces(T.most) < wgs) T.most *= 2;
     int row0 = 0;
     int64_t bpart0 = 0;
     for (int k = 0; k < n_inst; ++k) {
@@ -959,8 +968,8 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
         S.bpart0 = bpart0;
         for (int g = 0; g < S.nrows; ++g) {
             const int64_t u = row_units(g, S.nsb);
-            for (int h = 0; h < batch_row_pieces(u); ++h) {
-                const int units = (int)(batch_piece_begin(u, h + 1) - batch_piece_begin(u, h));
+            for (int h = 0; h < batch_row_pieces(u, T.most); ++h) {
+                const int units = (int)(batch_piece_begin(u, h + 1, T.most) - batch_piece_begin(u, h, T.most));
                 T.rows.push_back(SymRow{k, g, h, units});
                 T.plain = T.plain && fragments_plain((int64_t)units * kGroup / kBatchFold);
             }
@@ -970,7 +979,7 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
         T.insts.push_back(S);
     }
     std::stable_sort(T.rows.begin(), T.rows.end(), [](const SymRow& a, const SymRow& b) { return a.units > b.units; });
-    T.apart_elems = (int64_t)kFragElems * kBatchPieces * row0;
+    T.apart_elems = (int64_t)kFragElems * T.most * row0;
     T.bpart_elems = bpart0;
     return T;
 }
@@ -1002,10 +1011,10 @@ hipError_t launch_sym_batch_far(const SymBatchLaunch& L, hipStream_t s)
     if ((e = launch_reset_queue(L.queue, 1, s)) != hipSuccess) return e;
     if (L.soft)
         hipLaunchKernelGGL((sym_batch_far_kernel<true>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.sinst, L.insts,
-                           L.rows, L.nrows, L.queue, L.apart, L.plain ? 1 : 0, L.bpart, L.umass);
+                           L.rows, L.nrows, L.most, L.queue, L.apart, L.plain ? 1 : 0, L.bpart, L.umass);
     else
         hipLaunchKernelGGL((sym_batch_far_kernel<false>), dim3(L.wgs), dim3(kFarThreads), 0, s, L.xs, L.sinst, L.insts,
-                           L.rows, L.nrows, L.queue, L.apart, L.plain ? 1 : 0, L.bpart, L.umass);
+                           L.rows, L.nrows, L.most, L.queue, L.apart, L.plain ? 1 : 0, L.bpart, L.umass);
     return hipGetLastError();
 }
 
@@ -1014,10 +1023,10 @@ hipError_t launch_sym_batch_combine(const SymBatchLaunch& L, hipStream_t s)
     if (L.ntotal <= 0 || L.n_blk <= 0) return hipSuccess;
     if (L.plain)
         hipLaunchKernelGGL(sym_batch_combine_kernel<true>, dim3(L.n_blk), dim3(kBlock), 0, s, L.near_part, L.apart,
-                           L.bpart, L.sinst, L.blk, L.perm, L.acc, L.add_acc ? 1 : 0);
+                           L.bpart, L.sinst, L.blk, L.most, L.perm, L.acc, L.add_acc ? 1 : 0);
     else
         hipLaunchKernelGGL(sym_batch_combine_kernel<false>, dim3(L.n_blk), dim3(kBlock), 0, s, L.near_part, L.apart,
-                           L.bpart, L.sinst, L.blk, L.perm, L.acc, L.add_acc ? 1 : 0);
+                           L.bpart, L.sinst, L.blk, L.most, L.perm, L.acc, L.add_acc ? 1 : 0);
     return hipGetLastError();
 }
 
