@@ -949,7 +949,7 @@ SymBatchTables sym_batch_tables(const std::vector<int64_t>& offsets, int64_t min
         }
         return count;
     };
-    while (T.most < kBatchPiecesMost && pieces(T.most) < wgs) T.most *= 2;
+    while (T.most < kBatchPiecesMost && pieces(T.most) < std::min(wgs, pieces(2 * T.most))) T.most *= 2;
     int row0 = 0;
     int64_t bpart0 = 0;
     for (int k = 0; k < n_inst; ++k) {
