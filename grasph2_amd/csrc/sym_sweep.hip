@@ -212,17 +212,26 @@ template <bool UM>
 __device__ __forceinline__ void far_fold_own(FarOwn& o, const float m, const int lane)
 {
     if (o.folds == kFoldsPerFlush) far_flush_own(o, lane);
-    const int l = own_lane(lane);
-    const bool first = o.folds == 0;
+    float* const sum = o.lsum + own_lane(lane);
+    float old[3][kNI];  // all read before the first is used: one by one they waited 32 times a fold
+    if (o.folds > 0) {
+#pragma unroll
+        for (int q = 0; q < kNI; ++q)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) old[c][q] = sum[kGroup * c + 64 * q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < kNI; ++q) old[0][q] = old[1][q] = old[2][q] = 0.0f;
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < kNI; ++q) {
-        const int slot = 64 * q + l;
         const float ax = UM ? o.ax[q] * m : o.ax[q];
         const float ay = UM ? o.ay[q] * m : o.ay[q];
         const float az = UM ? o.az[q] * m : o.az[q];
-        o.lsum[slot] = first ? ax : o.lsum[slot] + ax;
-        o.lsum[kGroup + slot] = first ? ay : o.lsum[kGroup + slot] + ay;
-        o.lsum[2 * kGroup + slot] = first ? az : o.lsum[2 * kGroup + slot] + az;
+        sum[64 * q] = old[0][q] + ax;
+        sum[kGroup + 64 * q] = old[1][q] + ay;
+        sum[2 * kGroup + 64 * q] = old[2][q] + az;
         o.ax[q] = o.ay[q] = o.az[q] = 0.0f;
     }
     ++o.folds;
