@@ -25,8 +25,8 @@
 // rotation is one asm block: for all 16 slots the differences (odd
 // registers) and r^2 + H^2 (even registers), then the 16 v_rsq_f32 and the 6
 // DPP instructions in one run at priority 1, then the rest.  With it
-// far_kernel alone on the GPU takes 2.31 ms for the 8.52e9 unordered pairs of
-// N = 131072 (3.20 before, 148 TFLOP/s at 20 per ordered pair now), and
+// far_kernel alone on the GPU takes 2.28 ms for the 8.52e9 unordered pairs of
+// N = 131072 (3.20 before, 150 TFLOP/s at 20 per ordered pair now), and
 // 165 ms for N = 1048576 with unequal masses (231 before).
 #pragma once
 

@@ -142,9 +142,9 @@ __device__ __host__ inline int far_split(int64_t n, int64_t wanted, int most = k
 // and it shows: with a fixed 512 from 131072 on the error against FP64 (equal /
 // unequal masses) is 4.13e-8 / 5.32e-8 of the norm at 165000 and 3.88e-8 /
 // 4.68e-8 at 262144, with the rule 3.64e-8 / 4.15e-8 and 3.53e-8 / 3.78e-8, for
-// 2.8% and 3.9% of the step.  At 65536 128 instead of the piece's 512 gives
-// 3.86e-8 / 5.48e-8 instead of 4.67e-8 / 6.96e-8 for 1.6%; at 131072 it would
-// cost 2.2%.
+// 2.2% and 3.3% of the step.  At 65536 128 instead of the piece's 512 gives
+// 3.86e-8 / 5.48e-8 instead of 4.67e-8 / 6.96e-8 for 1.8%; at 131072 it would
+// cost 1.6%.
 constexpr int kMaxFoldSplit = 16, kShortFold = 128;
 constexpr int64_t kShortFoldBelow = 131072;
 __device__ __host__ inline int far_fold(int64_t n, int64_t wanted)
